@@ -74,8 +74,12 @@ template <class Chain> constexpr bool is_gather_chain() {
 template <class WP, class Plane> __device__ __forceinline__ u32 masked_row_offset(int y, const Plane& plane) {
     if constexpr (requires { WP::kLaneMasked; }) return WP::row_offset(y, plane); else return 0u;
 }
-template <class WP, class Plane, class V> __device__ __forceinline__ void masked_put(const Plane& plane, u32 row_off, u32 lane_off, const V& v) {
-    if constexpr (requires { WP::kLaneMasked; }) WP::put_masked(plane, row_off, lane_off, v);
+template <class WP, bool STREAM, class Plane, class V> __device__ __forceinline__ void masked_put(const Plane& plane, u32 row_off, u32 lane_off, const V& v) {
+    if constexpr (requires { WP::kLaneMasked; }) WP::template put_masked<STREAM>(plane, row_off, lane_off, v);
+}
+// Whether the chain's writer has a streaming form (see kStreamOutputBytes) for the bilinear kernel to choose.
+template <class Chain> constexpr bool writer_streams() {
+    if constexpr (requires { Chain::Write::Plane::kLaneMasked; }) return Chain::Write::Plane::kLaneMasked; else return false;
 }
 
 // (The geometry a launcher hands to kernels that renumber their workgroups -- TileGeom, division_magic, the limits that
@@ -256,7 +260,7 @@ constexpr int kGatherBY = FKD_GATHER_BY;
 // source); only stores are predicated.
 // The tile's work once the plane's parameters are in registers: q (the plane's read), ops, wpar (the plane's write), the
 // output extent aw x ah, the plane z, the tile's first column tx0 and its row of tiles.
-template <class Chain, int XI, int YI, class Q, class OPS, class WPAR>
+template <class Chain, int XI, int YI, bool STREAM, class Q, class OPS, class WPAR>
 __device__ __forceinline__ void gather_tile(const typename Chain::Params& p, const Q& q, const OPS& ops, const WPAR& wpar,
                                             int aw, int ah, int z, int tx0, u32 tile_row) {
     using Root = ResizeRoot<typename Chain::Read>;
@@ -457,7 +461,7 @@ __device__ __forceinline__ void gather_tile(const typename Chain::Params& p, con
             if constexpr (MASKED) {
                 const u32 row_off = masked_row_offset<WP>(y, oplane);
 #pragma unroll
-                for (int i = 0; i < XI; ++i) masked_put<WP>(oplane, row_off, lane_off[i], res[i].v);
+                for (int i = 0; i < XI; ++i) masked_put<WP, STREAM>(oplane, row_off, lane_off[i], res[i].v);
             } else if constexpr (FKD_GATHER_ADJ && XI > 1) {
                 if (xof(XI - 1) < aw) {
                     WP::template put_run<XI>(orow, xof(0), res);
@@ -539,7 +543,7 @@ __device__ __forceinline__ void gather_tile(const typename Chain::Params& p, con
     }
 }
 
-template <class Chain, int XI, int YI>
+template <class Chain, int XI, int YI, bool STREAM>
 __device__ __forceinline__ void gather_body(const typename Chain::Params& p, const TileGeom& g) {
     using Root = ResizeRoot<typename Chain::Read>;
     using RZ = typename Root::Resize;
@@ -574,7 +578,7 @@ __device__ __forceinline__ void gather_body(const typename Chain::Params& p, con
     if (tin >= per_plane) return;
     const u32 tile_row = gg.tiles_x_magic ? u32(((unsigned long long)tin * gg.tiles_x_magic) >> 32) : tin / gg.tiles_x;
     const int tx0 = int(tin - tile_row * gg.tiles_x) * TW;
-    gather_tile<Chain, XI, YI>(p, q, ops, wpar, aw, ah, z, tx0, tile_row);
+    gather_tile<Chain, XI, YI, STREAM>(p, q, ops, wpar, aw, ah, z, tx0, tile_row);
 }
 
 // ---- strip form of the bilinear kernel: narrow outputs (batches of small planes) -------------------------------------
@@ -624,7 +628,7 @@ template <class Chain> constexpr bool strip_capable() {
     }
 }
 
-template <class Chain>
+template <class Chain, bool STREAM>
 __device__ __forceinline__ void strip_body(const typename Chain::Params& p, const u32 first_late_workgroup) {
     using Root = ResizeRoot<typename Chain::Read>;
     using RZ = typename Root::Resize;
@@ -782,7 +786,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
                 asm volatile("" : "+v"(off));
                 if (g + kStripStep * k >= aw) off = WP::kMaskedOut;
             }
-            WP::put_masked(oplane, 0u, off, res);
+            WP::template put_masked<STREAM>(oplane, 0u, off, res);
         };
         // One step of taps is in flight behind the step being blended.  The steps are written out (a plane has at most
         // kStripMaxSteps of them) and the only branches leave the kernel: every step issues the same accesses in the same
@@ -811,14 +815,14 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     run_static(IntTag<0>{});
 }
 
-template <class Chain>
+template <class Chain, bool STREAM>
 __global__ __launch_bounds__(kStripThreads) void k_strip(const typename Chain::Params p, const u32 first_late_workgroup) {
-    if constexpr (strip_capable<Chain>()) strip_body<Chain>(p, first_late_workgroup);
+    if constexpr (strip_capable<Chain>()) strip_body<Chain, STREAM>(p, first_late_workgroup);
 }
 
-template <class Chain, int XI, int YI>
+template <class Chain, int XI, int YI, bool STREAM>
 __global__ __launch_bounds__(kGatherBX * kGatherBY) void k_gather(const typename Chain::Params p, const TileGeom g) {
-    gather_body<Chain, XI, YI>(p, g);
+    gather_body<Chain, XI, YI, STREAM>(p, g);
 }
 
 // ---- per-chain constants shared by the ahead-of-time and the run-time launchers ---------------------------
@@ -891,20 +895,28 @@ template <class D> __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_diverg
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
-                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u};
+                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u,
+                       is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) DivergentBody<Chain>::run(p);
     else if constexpr (is_gather_chain<Chain>()) {
         if constexpr (strip_capable<Chain>()) {
-            if (g.tiles_x == 0u) { strip_body<Chain>(p, g.n_tiles); return; }      // wave uniform: the launcher chose the strip form
+            if (g.tiles_x == 0u) {                       // wave uniform: the launcher chose the strip form
+                if (g.stream != 0u) strip_body<Chain, true>(p, g.n_tiles);
+                else strip_body<Chain, false>(p, g.n_tiles);
+                return;
+            }
         }
-        gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI>(p, g);
+        if constexpr (writer_streams<Chain>()) {
+            if (g.stream != 0u) { gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, true>(p, g); return; }
+        }
+        gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, false>(p, g);
     }
     else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>()>(p, 0u, &g);
 }

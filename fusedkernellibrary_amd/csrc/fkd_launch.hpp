@@ -31,13 +31,13 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     const unsigned gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);
     dim3 grid(gx, gy, p.active_z);
     const dim3 block(kRowsBX, kRowsBY, 1);
-    TileGeom g{0u, 0u, 0u, 0u};
+    TileGeom g{};
     if constexpr (rows_in_bands<Chain>()) {
         // gathering reads, larger launches: a one-dimensional grid whose workgroups the kernel renumbers into one band per XCD
         if ((unsigned long long)gx * gy > 0x7fffff00ull) return hipErrorInvalidConfiguration;
         if (gx * gy >= kRowsBandBlocks) {
             grid = dim3(rows_band_chunk(gx * gy) * 8u, 1, p.active_z);
-            g = TileGeom{gx, gy, gx * gy * p.active_z, division_magic(gx, gx * gy)};
+            g = TileGeom{gx, gy, gx * gy * p.active_z, division_magic(gx, gx * gy), 0u};
         }
     }
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
@@ -64,6 +64,8 @@ template <class Chain>
 hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int XI = FKD_GATHER_XI, YI = FKD_GATHER_YI;
     constexpr int TW = kGatherBX * XI, TH = kGatherBY * YI;
+    constexpr bool kStreams = writer_streams<Chain>();
+    const bool streamed = kStreams && (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(typename Chain::Value) > kStreamOutputBytes;
     if constexpr (strip_capable<Chain>()) {
         // Narrow outputs (batches of small planes): the strip form, whose workgroups own 8 whole rows of a plane.
         // (an output without columns has no workgroup in the tile form's grid: it falls through and launches nothing)
@@ -72,7 +74,9 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
             if (info) *info = LaunchInfo{"strip", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned(kStripMaxWidth * 16 + (kStripThreads / 64) * 4)};
             if (grid.x == 0 || grid.z == 0) return hipSuccess;
             if (grid.z > 65535u) return hipErrorInvalidConfiguration;
-            return launch_by_pointer(&k_strip<Chain>, grid, block, stream, p, strip_first_late_workgroup((unsigned long long)grid.x * grid.z));
+            const unsigned first_late = strip_first_late_workgroup((unsigned long long)grid.x * grid.z);
+            if (streamed) return launch_by_pointer(&k_strip<Chain, kStreams>, grid, block, stream, p, first_late);
+            return launch_by_pointer(&k_strip<Chain, false>, grid, block, stream, p, first_late);
         }
     }
     TileGeom g;
@@ -85,7 +89,9 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
     if (info) *info = LaunchInfo{"gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
     if (g.n_tiles == 0) return hipSuccess;
     if (grid.z > 65535u) return hipErrorInvalidConfiguration;
-    return launch_by_pointer(&k_gather<Chain, XI, YI>, grid, block, stream, p, g);
+    g.stream = streamed ? 1u : 0u;
+    if (streamed) return launch_by_pointer(&k_gather<Chain, XI, YI, kStreams>, grid, block, stream, p, g);
+    return launch_by_pointer(&k_gather<Chain, XI, YI, false>, grid, block, stream, p, g);
 }
 
 // Several chains in one launch: the grid of the rows kernel over the largest extent, alignment decided per plane on

@@ -40,6 +40,7 @@ using fkd::JitMeta;
 using fkd::TileGeom;
 using fkd::division_magic;
 using fkd::kRowsBandBlocks;
+using fkd::kStreamOutputBytes;
 using fkd::strip_first_late_workgroup;
 
 struct JitKernel {
@@ -203,7 +204,8 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     unsigned active[4];
     memcpy(active, blob, sizeof(active));   // Chain::Params starts with active_w, active_h, active_z, reserved (bit 0: strip form allowed)
     const JitMeta& m = k->meta;
-    TileGeom g{0, 0, 0, 0};
+    TileGeom g{0, 0, 0, 0, 0};
+    g.stream = (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes ? 1u : 0u;
     unsigned grid[3], block[3] = {64, 4, 1};
     const char* kind = m.gather ? "gather_jit" : "rows_jit";
     if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {

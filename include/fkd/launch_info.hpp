@@ -20,7 +20,17 @@ struct TileGeom {
     // floor(2^32 / tiles_x) + 1 when (t * magic) >> 32 == t / tiles_x for every tile number t of a plane, else 0: the
     // division then costs two scalar multiplications instead of a float reciprocal on the vector unit.
     unsigned tiles_x_magic;
+    // bilinear kernel with a planar writer: 1 when the launch's output is streamed past the last-level cache
+    unsigned stream;
 };
+// Planar outputs of the bilinear kernel above this many bytes are stored with the non-temporal hint.  Written through the
+// L2 they are kept by the 256 MB last-level cache, which pushes the source images out of it; every tap line then comes from
+// HBM between the writes, one isolated read at a time, and each costs the channel a turn from writing to reading and back.
+// 64 crops of a 3840x2160 image to 640x640 (314 MB out, 25 MB of source): 77 us written through, 60 us non-temporal, although
+// the stores alone take 55 us either way.  The line lies where the two cross (64 crops of a 1920x1080 image; written through /
+// non-temporal): 224x224, 38 MB 9.8 / 10.2 us; 288x288, 64 MB 14.4 / 14.6; 320x320, 79 MB 17.2 / 16.4; 384x384, 113 MB 26.9 /
+// 21.6; 512x512, 201 MB 48.8 / 35.1.
+constexpr unsigned long long kStreamOutputBytes = 64ull << 20;
 // The magic for dividing numbers below `limit` by d, or 0 when there is none.
 inline unsigned division_magic(unsigned d, unsigned limit) {
     if (d == 0) return 0;
@@ -50,6 +60,7 @@ struct JitMeta {
     unsigned max_planes;      // most planes (grid z) a launch may have, 0: no limit of the kernel's own
     unsigned strip_width;     // gather kernel: outputs up to this width are launched in strip form (TileGeom::tiles_x == 0), 0: never
     unsigned bands;           // rows kernel: 1 when launches of kRowsBandBlocks blocks per plane or more take the bands form of grid
+    unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
 };
 
 } // namespace fkd

@@ -2877,15 +2877,15 @@ template <class T, bool TRANSPOSED = false> struct TensorSplit {
     }
     FKD_DEV static u32 lane_offset(int x, bool valid) { return valid ? u32(x) * u32(sizeof(B)) : kMaskedOut; }
     FKD_DEV static u32 row_offset(int y, const PlaneRef& r) { return u32(y) * r.pitch; }
-    FKD_DEV static void put_masked(const PlaneRef& r, u32 row_off, u32 lane_off, const T& v) {
-#ifndef FKD_STORE_AUX
-#define FKD_STORE_AUX (1 | 16)
-#endif
-        constexpr int kThrough = FKD_STORE_AUX;     // sc0 sc1: written through the L2, as gstore_through
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<0>(v)), r.rsrc, lane_off, row_off, kThrough);
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<1>(v)), r.rsrc, lane_off, row_off + r.chan_bytes, kThrough);
-        if constexpr (cn_v<T> > 2) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<2>(v)), r.rsrc, lane_off, row_off + 2u * r.chan_bytes, kThrough);
-        if constexpr (cn_v<T> > 3) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<3>(v)), r.rsrc, lane_off, row_off + 3u * r.chan_bytes, kThrough);
+    // STREAM: the launch writes more than the last-level cache should give up for it (kStreamOutputBytes).  The stores then
+    // carry the non-temporal hint, which keeps the output out of that cache; otherwise they are written through the L2
+    // (sc0 sc1, as gstore_through), which is faster while output and source fit the cache together.
+    template <bool STREAM> FKD_DEV static void put_masked(const PlaneRef& r, u32 row_off, u32 lane_off, const T& v) {
+        constexpr int kPolicy = STREAM ? 2 : (1 | 16);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<0>(v)), r.rsrc, lane_off, row_off, kPolicy);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<1>(v)), r.rsrc, lane_off, row_off + r.chan_bytes, kPolicy);
+        if constexpr (cn_v<T> > 2) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<2>(v)), r.rsrc, lane_off, row_off + 2u * r.chan_bytes, kPolicy);
+        if constexpr (cn_v<T> > 3) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(u32, chan<3>(v)), r.rsrc, lane_off, row_off + 3u * r.chan_bytes, kPolicy);
     }
     struct RowRef { B* p; size_t px; };
     FKD_DEV static RowRef row(int y, int z, const Params& p) { return RowRef{at(p, 0, y, z), G::channel_elements(p)}; }

@@ -1,0 +1,43 @@
+"""Planar outputs of the bilinear kernel on both sides of the size from which they are stored past the last-level cache
+(64 MiB): the two kinds of store leave the same bytes, the oracle's, in both forms of the kernel and in a chain compiled on
+first use."""
+import numpy as np
+import pytest
+
+import fkl_cases as cases
+import oracle_lib as ol
+import workloads as wl
+from fusedkernellibrary_amd import last_launch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dst,kernel", [((293, 298), None), ((293, 299), None),      # 67 057 152 and 67 282 176 bytes: ragged rows
+                                        ((251, 348), "strip"), ((251, 349), "strip")])
+def test_batches_around_the_limit(dst, kernel):
+    import torch
+    c = wl.config3(width=640 if kernel else 641, height=359, min_side=2, span=340)      # rows that share their alignment, or not
+    src = torch.from_numpy(c["src"]).cuda()
+    out = torch.full((64, 3, dst[1], dst[0]), -7.0, dtype=torch.float32, device="cuda")
+    cases.crop_resize_norm_split(src, c["rects"], dst, c["sub"], c["div"], out)
+    torch.cuda.synchronize()
+    if kernel:
+        assert last_launch()["kernel"] == kernel
+    want = ol.oracle_crop_resize_norm_split(c["src"], c["rects"], dst, c["sub"], c["div"])
+    assert out.cpu().numpy().tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("dst", [(1365, 1365), (1366, 1366), (201, 9275)])           # 67 076 100, 67 174 416 and 67 113 900 bytes
+def test_a_chain_compiled_on_first_use(dst):
+    import torch
+    rng = np.random.RandomState(11)
+    img = rng.randint(0, 256, (200, 320, 3)).astype(np.uint8)
+    rects = np.array([[10, 20, 300, 60], [40, 0, 50, 200], [100, 50, 120, 120]], np.int32)
+    bg, mul = np.array([0.25, 128.5, 255.0], np.float32), np.array([0.5, 2.0, 1.0 / 255.0], np.float32)
+    out = torch.full((3, 3, dst[1], dst[0]), -7.0, dtype=torch.float32, device="cuda")
+    cases.uncompiled_letterbox_split_b3(torch.from_numpy(img).cuda(), rects, dst, bg, mul, out)
+    torch.cuda.synchronize()
+    want = np.zeros((3, 3, dst[1], dst[0]), np.float32)
+    reads = [ol.read_2d(img, 3, crop=rects[i], resize=dst, ar=ol.PRESERVE_AR, bg=tuple(bg) + (0.0,)) for i in range(3)]
+    ol.execute(reads, [ol.op(ol.MUL, tuple(mul) + (0.0,))], [ol.write(ol.TENSOR_SPLIT, want, 3, dst[0], dst[1], 3, 3)])
+    assert out.cpu().numpy().tobytes() == want.tobytes()
