@@ -4,7 +4,8 @@
 //
 //  rows kernel    one thread produces V = 4 horizontally adjacent outputs of one row of plane z.  Reads and
 //                 writes of 4 elements move as dwordx3 / dwordx4 accesses (12 bytes for uchar3, 16 for float,
-//                 48 for float3) that consecutive lanes make contiguous, so a wave64 touches whole cache lines.
+//                 48 for float3) that consecutive lanes make contiguous, so a wave64 touches whole cache lines;
+//                 rows may start at any byte and have any width.
 //                 Each thread handles ROWS rows so several independent loads are in flight per lane.
 //                 Plane z = workgroup index in z: horizontal (batch) fusion, per-plane parameters are wave
 //                 uniform and come out of the kernel-argument segment through scalar loads.
@@ -101,11 +102,14 @@ constexpr unsigned long long kStreamElements = 1ull << 26;   // launches over mo
 #endif
 
 // The full-width part of the rows kernel: every lane has V elements in each of its ROWS rows.  MODE as in
-// detail::load_run.
-template <class Chain, int V, int ROWS, int MODE>
-__device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 kernarg_offset, int x0, int ybase, int z, int ah) {
+// detail::load_run.  TAIL: rows that are not a multiple of V wide; the lane at a row's end, which has fewer than V elements
+// left, works on the row's last V elements and stores only those from x0 on (the others are its neighbour's; what it read
+// there is not used, so a chain that works in place is none the wiser).
+template <class Chain, int V, int ROWS, int MODE, bool TAIL = false>
+__device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 kernarg_offset, int first, int ybase, int z, int aw, int ah) {
     using R = typename Chain::Read;
     using W = typename Chain::Write;
+    const int x0 = TAIL && first + V > aw ? aw - V : first;
 
     // All loads first, unconditionally (rows past the end re-read the last row, which is in bounds), so every
     // lane has ROWS independent wide loads in flight before the first use; only the stores are predicated.
@@ -128,7 +132,15 @@ __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 k
         Slot<typename Chain::Value> row[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) row[i].v = out[r * V + i + FKD_TEST_INDEX_OFFSET].v;
-        if (y < ah) W::template exec_row<V, MODE>(x0, y, z, row, p.write);
+        if (y >= ah) continue;
+        if constexpr (TAIL) {
+            if (x0 != first) {
+#pragma unroll
+                for (int i = 1; i < V; ++i) if (x0 + i >= first) W::exec(x0 + i, y, z, row[i].v, p.write);
+                continue;
+            }
+        }
+        W::template exec_row<V, MODE>(x0, y, z, row, p.write);
     }
 }
 
@@ -171,25 +183,36 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     const int ybase = (block_y * kRowsBY + threadIdx.y) * ROWS;
     if (x0 >= aw || ybase >= ah) return;
     // Wave-cooperative accesses (mode 2 of load_run / store_run) need every lane of the wave on a full run.
-    constexpr bool kExchange = ALIGNED && (detail::wave_exchange_ok<typename R::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
+    constexpr bool kExchange = (detail::wave_exchange_ok<typename R::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
     if constexpr (kExchange) {
         if (int(block_x * kRowsBX + kRowsBX) * V <= aw) {
-            rows_full<Chain, V, ROWS, 2>(p, kernarg_offset, x0, ybase, z, ah);
+            rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign>(p, kernarg_offset, x0, ybase, z, aw, ah);
             return;
         }
     }
     // A launch over more elements than the last-level cache could hold between two launches reads them with the
     // non-temporal hint (100 images of 1920x1080 uchar3: 225 -> 209 us); smaller inputs are left to the caches, where a
     // pipeline's previous stage may have put them (the hint costs 15 % on a 33 MB image that is still cached).
-    constexpr bool kMayStream = ALIGNED && !Chain::kLongChain && !kExchange;
-    if constexpr (kMayStream) {
-        if (x0 + V <= aw && (unsigned long long)(u32(aw)) * u32(ah) * gridDim.z > kStreamElements) {
-            rows_full<Chain, V, ROWS, 1 | 4>(p, kernarg_offset, x0, ybase, z, ah);
+    constexpr bool kMayStream = !Chain::kLongChain && !kExchange;
+    const bool stream = kMayStream && (unsigned long long)(u32(aw)) * u32(ah) * gridDim.z > kStreamElements;
+    // The wave at the end of rows whose width is no multiple of V (wave uniform).  Its lanes make the accesses of the other
+    // waves, at whatever alignment the row's last V elements have; element by element, each behind the one before, the
+    // last lane's three elements took longer than the rest of the launch (100 operations on 511x512 floats, four launches:
+    // 43.0 -> 22.9 us; a 1919x1079 warp 11.1 -> 8.7 us).
+    if constexpr (V > 1 && any_x<R>()) {
+        if (aw % V != 0 && aw >= V && int(block_x * kRowsBX + kRowsBX) * V > aw) {
+            if constexpr (kMayStream) {
+                if (stream) { rows_full<Chain, V, ROWS, 0 | 4, true>(p, kernarg_offset, x0, ybase, z, aw, ah); return; }
+            }
+            rows_full<Chain, V, ROWS, 0, true>(p, kernarg_offset, x0, ybase, z, aw, ah);
             return;
         }
     }
     if (x0 + V <= aw) {
-        rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0>(p, kernarg_offset, x0, ybase, z, ah);
+        if constexpr (kMayStream) {
+            if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4>(p, kernarg_offset, x0, ybase, z, aw, ah); return; }
+        }
+        rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0>(p, kernarg_offset, x0, ybase, z, aw, ah);
     } else {
         for (int r = 0; r < ROWS; ++r) {
             const int y = ybase + r;

@@ -50,7 +50,8 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
 template <class Chain>
 hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int V = RowsConfig<Chain>::V, ROWS = RowsConfig<Chain>::ROWS;
-    // Wide (dwordx3/x4) accesses need every row start dword aligned; checked here, once per launch, on the host.
+    // Runs move as wide accesses at any alignment; that every row start is dword aligned (checked here, once per launch, on
+    // the host) tells readers of grouped samples that a run starts on a group.
     const bool aligned = Chain::Read::rows_aligned(p.read, 0) && Chain::Write::rows_aligned(p.write);
     if constexpr (ROWS > 1) {
         const unsigned long long gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);

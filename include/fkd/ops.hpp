@@ -30,6 +30,15 @@ inline std::string istr(long long v) { return std::to_string(v); }
 // vectors that the backend can only legalise through scratch or LDS.
 template <class T> struct alignas(sizeof(T) % 4 != 0 ? 4 : alignof(T)) Slot { T v; };
 
+namespace detail {
+// How a run of elements is accessed (the mode of exec_row, load_run and store_run; p is the run's address).  Low two bits: 0:
+// nothing is known about p.  1: p is dword aligned.  2: all 64 lanes of the wave are in this
+// call with consecutive runs (lane i at p0 + i * V elements), and p is dword aligned unless kAnyAlign is set.  Bit 2 (value
+// 4): the launch reads more than the caches hold, loads carry the non-temporal hint.
+constexpr int kAnyAlign = 16;
+constexpr bool aligned_mode(int mode) { return (mode & 3) != 0 && (mode & kAnyAlign) == 0; }
+} // namespace detail
+
 // Facts about values that only types can vouch for, used where an operation may be shortened if its input is tame.
 // finite_taps<B>: the taps of read B, after everything fused into it, are finite numbers whatever the image holds
 // (integer pixels through operations without run-time parameters); a tap with weight zero then contributes a zero and can
@@ -43,6 +52,10 @@ template <class Op> constexpr bool finite_map() {
 }
 template <class R> constexpr bool bounded_out() {
     if constexpr (requires { R::kBoundedOut; }) return R::kBoundedOut; else return false;
+}
+// any_x<R>: read R's exec_row may start at any element of the row, not only at a multiple of the run's length.
+template <class R> constexpr bool any_x() {
+    if constexpr (requires { R::kAnyX; }) return R::kAnyX; else return false;
 }
 template <class T> constexpr bool small_integer_base() {
     return !(__is_same(base_t<T>, f32) || __is_same(base_t<T>, f64)) && sizeof(base_t<T>) <= 2;
@@ -102,6 +115,22 @@ typedef u32 u32x4_t __attribute__((ext_vector_type(4)));
 typedef u32x2_t u32x2_a4 __attribute__((aligned(4)));
 typedef u32x3_t u32x3_a4 __attribute__((aligned(4)));
 typedef u32x4_t u32x4_a4 __attribute__((aligned(4)));
+// The same at any byte address: the hardware takes global accesses of any width at any byte alignment.
+typedef u16 u16_a1 __attribute__((aligned(1)));
+typedef u32 u32_a1 __attribute__((aligned(1)));
+typedef u32x2_t u32x2_a1 __attribute__((aligned(1)));
+typedef u32x3_t u32x3_a1 __attribute__((aligned(1)));
+typedef u32x4_t u32x4_a1 __attribute__((aligned(1)));
+template <int N, bool ALIGNED> struct DwordsAt;      // N dwords at a dword boundary (ALIGNED) or at any byte
+template <> struct DwordsAt<1, true> { using type = u32; };
+template <> struct DwordsAt<2, true> { using type = u32x2_a4; };
+template <> struct DwordsAt<3, true> { using type = u32x3_a4; };
+template <> struct DwordsAt<4, true> { using type = u32x4_a4; };
+template <> struct DwordsAt<1, false> { using type = u32_a1; };
+template <> struct DwordsAt<2, false> { using type = u32x2_a1; };
+template <> struct DwordsAt<3, false> { using type = u32x3_a1; };
+template <> struct DwordsAt<4, false> { using type = u32x4_a1; };
+template <int N, bool ALIGNED> using dwords_at = typename DwordsAt<N, ALIGNED>::type;
 
 // One whole-dword store (1-4 dwords).  Output is written once and not read again by the kernel, so the stores carry
 // the non-temporal hint: the L2s then hand the lines on early instead of keeping them dirty until the kernel ends,
@@ -145,39 +174,39 @@ template <class T> FKD_DEV void store_elem(T* p, const T& v) {
     }
 }
 
-template <int W, bool STREAM = false> FKD_DEV void load_words(const void* p, u32 (&w)[W]) {
+template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_words(const void* p, u32 (&w)[W]) {
     static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
-        w[0] = gload_run<STREAM>(gconst<u32>(p));
+        w[0] = gload_run<STREAM>(gconst<dwords_at<1, ALIGNED>>(p));
     } else if constexpr (W == 2) {
-        const u32x2_t v = gload_run<STREAM>(gconst<u32x2_a4>(p));
+        const u32x2_t v = gload_run<STREAM>(gconst<dwords_at<2, ALIGNED>>(p));
         w[0] = v.x; w[1] = v.y;
     } else if constexpr (W == 3) {
-        const u32x3_t v = gload_run<STREAM>(gconst<u32x3_a4>(p));
+        const u32x3_t v = gload_run<STREAM>(gconst<dwords_at<3, ALIGNED>>(p));
         w[0] = v.x; w[1] = v.y; w[2] = v.z;
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
-            const u32x4_t v = gload_run<STREAM>(gconst<u32x4_a4>(p) + i);
+            const u32x4_t v = gload_run<STREAM>(gconst<dwords_at<4, ALIGNED>>(p) + i);
             w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
         }
     }
 }
-template <int W> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
+template <int W, bool ALIGNED = true> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
     static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
-        gstore(gmut<u32>(p), w[0]);
+        gstore<dwords_at<1, ALIGNED>>(gmut<dwords_at<1, ALIGNED>>(p), w[0]);
     } else if constexpr (W == 2) {
-        u32x2_t v; v.x = w[0]; v.y = w[1];
-        gstore(gmut<u32x2_a4>(p), v);
+        dwords_at<2, ALIGNED> v; v.x = w[0]; v.y = w[1];
+        gstore(gmut<dwords_at<2, ALIGNED>>(p), v);
     } else if constexpr (W == 3) {
-        u32x3_t v; v.x = w[0]; v.y = w[1]; v.z = w[2];
-        gstore(gmut<u32x3_a4>(p), v);
+        dwords_at<3, ALIGNED> v; v.x = w[0]; v.y = w[1]; v.z = w[2];
+        gstore(gmut<dwords_at<3, ALIGNED>>(p), v);
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
-            u32x4_t v; v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
-            gstore(gmut<u32x4_a4>(p) + i, v);
+            dwords_at<4, ALIGNED> v; v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
+            gstore(gmut<dwords_at<4, ALIGNED>>(p) + i, v);
         }
     }
 }
@@ -244,11 +273,10 @@ template <class T, int V, int W> FKD_DEV void unpack_words(const u32 (&w)[W], Sl
     unpack_words_impl<T, V, W>(w, out, MakeSeq<V>{});
 }
 
-// V consecutive elements starting at p.  ALIGNED promises that p is dword aligned (the launcher checks every
-// row start of every plane on the host before it picks the kernel variant): the run then moves as one wide
-// access per <= 16 bytes (global_load_dwordx3 for four uchar3, dwordx4 for four floats), which consecutive
-// lanes make contiguous.  Without the promise, or when the run is not a whole number of dwords, elements move
-// one by one.
+// V consecutive elements starting at p move as one wide access per <= 16 bytes (global_load_dwordx3 for four uchar3, dwordx4
+// for four floats), which consecutive lanes make contiguous, at any byte alignment of p: rows of 1279 uchar3 start at every
+// one, and moved byte by byte they were bound by the number of accesses (100 images of 510x333: 40 us byte by byte, 20 us so;
+// 4 of 1279x719: 37.2 and 25.2 us per 4 launches).  Runs that are not a whole number of dwords move element by element.
 template <class T> constexpr bool wide_ok(int v) {
     const int bytes = int(sizeof(T)) * v;
     return v > 1 && bytes % 4 == 0 && (bytes <= 16 || bytes % 16 == 0) && sizeof(T) == sizeof(base_t<T>) * cn_v<T>;
@@ -277,14 +305,14 @@ FKD_DEV void wave_exchange_fence() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
-template <int W, bool STREAM> FKD_DEV void load_words_wave(const void* p, u32 (&w)[W]) {
+template <int W, bool STREAM, bool ALIGNED> FKD_DEV void load_words_wave(const void* p, u32 (&w)[W]) {
     const u32 lane = threadIdx.x;
     u32* stage = wave_stage();
     // p is this lane's run; the segment starts W dwords per lane earlier
     const char* seg = reinterpret_cast<const char*>(p) - size_t(lane) * (W * 4);
     u32x4_t q[W / 4];
 #pragma unroll
-    for (int k = 0; k < W / 4; ++k) q[k] = gload_run<STREAM>(gconst<u32x4_a4>(seg + k * 1024 + lane * 16));
+    for (int k = 0; k < W / 4; ++k) q[k] = gload_run<STREAM>(gconst<dwords_at<4, ALIGNED>>(seg + k * 1024 + lane * 16));
     wave_exchange_fence();   // the previous exchange's reads come first
 #pragma unroll
     for (int k = 0; k < W / 4; ++k) *reinterpret_cast<u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)) = q[k];
@@ -295,7 +323,7 @@ template <int W, bool STREAM> FKD_DEV void load_words_wave(const void* p, u32 (&
         w[4 * j] = v.x; w[4 * j + 1] = v.y; w[4 * j + 2] = v.z; w[4 * j + 3] = v.w;
     }
 }
-template <int W> FKD_DEV void store_words_wave(void* p, const u32 (&w)[W]) {
+template <int W, bool ALIGNED> FKD_DEV void store_words_wave(void* p, const u32 (&w)[W]) {
     const u32 lane = threadIdx.x;
     u32* stage = wave_stage();
     char* seg = reinterpret_cast<char*>(p) - size_t(lane) * (W * 4);
@@ -308,25 +336,22 @@ template <int W> FKD_DEV void store_words_wave(void* p, const u32 (&w)[W]) {
     wave_exchange_fence();
 #pragma unroll
     for (int k = 0; k < W / 4; ++k)
-        gstore(gmut<u32x4_a4>(seg + k * 1024 + lane * 16), *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
+        gstore<dwords_at<4, ALIGNED>>(gmut<dwords_at<4, ALIGNED>>(seg + k * 1024 + lane * 16), *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
 }
 
-// Low two bits of the mode: 0: nothing is known about p.  1: p is dword aligned.  2: as 1, and all 64 lanes of the
-// wave are in this call with consecutive runs (lane i at p0 + i * V elements).  Bit 2 (value 4): the launch reads more
-// than the caches hold, loads carry the non-temporal hint.
 template <class T, int V, int MODE_BITS> FKD_DEV void load_run(const T* p, Slot<T> (&out)[V]) {
     constexpr int MODE = MODE_BITS & 3;
     constexpr bool STREAM = (MODE_BITS & 4) != 0;
-    constexpr bool ALIGNED = MODE != 0;
+    constexpr bool ALIGNED = aligned_mode(MODE_BITS);
     if constexpr (MODE == 2 && wave_exchange_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
-        load_words_wave<W, STREAM>(p, w);
+        load_words_wave<W, STREAM, ALIGNED>(p, w);
         unpack_words<T, V, W>(w, out);
-    } else if constexpr (ALIGNED && wide_ok<T>(V)) {
+    } else if constexpr (wide_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
-        load_words<W, STREAM>(p, w);
+        load_words<W, STREAM, ALIGNED>(p, w);
         if constexpr (sizeof(base_t<T>) < 4) {
             // Keep each dword an opaque scalar: otherwise the optimiser rewrites "shift and mask a vector lane"
             // into byte-vector extracts (<12 x i8>), which the backend can only legalise through scratch memory.
@@ -341,13 +366,13 @@ template <class T, int V, int MODE_BITS> FKD_DEV void load_run(const T* p, Slot<
 }
 template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot<T> (&in)[V]) {
     constexpr int MODE = MODE_BITS & 3;
-    constexpr bool ALIGNED = MODE != 0;
+    constexpr bool ALIGNED = aligned_mode(MODE_BITS);
     if constexpr (MODE == 2 && wave_exchange_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
         pack_words<T, V, W>(in, w);
-        store_words_wave<W>(p, w);
-    } else if constexpr (ALIGNED && wide_ok<T>(V)) {
+        store_words_wave<W, ALIGNED>(p, w);
+    } else if constexpr (wide_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
         pack_words<T, V, W>(in, w);
@@ -357,7 +382,7 @@ template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot
 #pragma unroll
             for (int i = 0; i < W; ++i) asm("" : "+v"(w[i]));
         }
-        store_words<W>(p, w);
+        store_words<W, ALIGNED>(p, w);
     } else {
 #pragma unroll
         for (int i = 0; i < V; ++i) store_elem(p + i, in[i].v);
@@ -371,11 +396,6 @@ template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot
 // of 4 bytes (up to 16) moves as one access.  Runs of 3 and 6 bytes (uchar3, a uchar3 pair, ushort3) move as one or
 // two whole dwords when OVERREAD allows touching up to 3 bytes past the run (the caller guarantees those bytes are
 // inside the allocation); otherwise channel by channel.
-typedef u16 u16_a1 __attribute__((aligned(1)));
-typedef u32 u32_a1 __attribute__((aligned(1)));
-typedef u32x2_t u32x2_a1 __attribute__((aligned(1)));
-typedef u32x3_t u32x3_a1 __attribute__((aligned(1)));
-typedef u32x4_t u32x4_a1 __attribute__((aligned(1)));
 template <class T, int V = 1> constexpr int overread_bytes() {
     constexpr int n = int(sizeof(T)) * V;
     return (n == 1 || n == 2 || n % 4 == 0 || n > 16) ? 0 : (n + 3) / 4 * 4 - n;
@@ -1463,6 +1483,7 @@ template <class T> struct Read2D {
     using Out = T;
     using Params = RawPtr2D<const T>;
     static constexpr bool kTapCursor = true;
+    static constexpr bool kAnyX = true;
     static constexpr bool kFiniteTaps = !(__is_same(base_t<T>, f32) || __is_same(base_t<T>, f64));
     static constexpr bool kBoundedOut = small_integer_base<T>();
     FKD_NAME("Read2D<" + type_name<T>() + ">")
@@ -1552,6 +1573,7 @@ template <class T> struct Read3D {
     using Out = T;
     using Params = RawPtr3D<const T>;
     static constexpr bool kTapCursor = false;
+    static constexpr bool kAnyX = true;
     static constexpr bool kBoundedOut = small_integer_base<T>();
     FKD_NAME("Read3D<" + type_name<T>() + ">")
 #if defined(FKD_EXEC_CODE)
@@ -1719,6 +1741,7 @@ template <bool VU> struct ReadNV {
     using Out = Vec<u8, 3>;
     using Params = RawNV12;
     static constexpr bool kTapCursor = true;
+    static constexpr bool kAnyX = true;
     static constexpr bool kFiniteTaps = true;
     static constexpr bool kBoundedOut = true;
     FKD_NAME(VU ? "ReadNV21" : "ReadNV12")
@@ -1736,11 +1759,20 @@ template <bool VU> struct ReadNV {
 #endif
 #if defined(FKD_DEVICE_CODE)
     template <int V, int A> FKD_DEV static void exec_row(int x, int y, int z, const Params& p, Slot<Out> (&out)[V]) {
-        if constexpr (V == 4 && (A & 3) != 0) {
-            // four pixels: their luma is one dword, their two chroma pairs another (x is a multiple of four here)
-            const u32 luma = *detail::gconst<u32>(p.data + size_t(y) * p.pitch + x);
-            u32 uv = *detail::gconst<u32>(p.data + size_t(p.pitch) * p.height + size_t(y >> 1) * p.pitch + x);
-            u32 l = luma;
+        if constexpr (V == 4) {
+            // four pixels: their luma is one dword, their two chroma pairs another (x is even here: a multiple of four unless
+            // the run is the last one of a row)
+            constexpr bool ALIGNED = detail::aligned_mode(A);
+            if constexpr (!ALIGNED) {
+                if ((x & 1) != 0) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) out[i].v = exec(x + i, y, z, p);
+                    return;
+                }
+            }
+            using Dword = detail::dwords_at<1, ALIGNED>;
+            u32 l = *detail::gconst<Dword>(p.data + size_t(y) * p.pitch + x);
+            u32 uv = *detail::gconst<Dword>(p.data + size_t(p.pitch) * p.height + size_t(y >> 1) * p.pitch + x);
             asm("" : "+v"(l), "+v"(uv));     // keep the dwords whole: bytes leave through v_cvt_f32_ubyteN / v_bfe
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1833,6 +1865,7 @@ template <int PF> struct ReadYUV {
     using B = typename PixelBase<PF>::type;
     using Out = Vec<B, 3>;
     using Params = RawYUV;
+    static constexpr bool kAnyX = true;
     static constexpr bool kTapCursor = false;
     FKD_NAME("ReadYUV<" + istr(PF) + ">")
 #if defined(FKD_EXEC_CODE)
@@ -1858,9 +1891,17 @@ template <int PF> struct ReadYUV {
 #endif
 #if defined(FKD_DEVICE_CODE)
     template <int V, int A> FKD_DEV static void exec_row(int x, int y, int z, const Params& p, Slot<Out> (&out)[V]) {
-        if constexpr (V == 4 && (A & 3) != 0) {
-            // Four pixels as whole dwords (x is a multiple of four here): packed 4:2:2 holds them in two groups of four
+        if constexpr (V == 4) {
+            // Four pixels as whole dwords (x is even here: a multiple of four unless the run is the last one of a row): packed 4:2:2 holds them in two groups of four
             // samples, semi-planar formats in four luma samples and two chroma pairs.
+            constexpr bool ALIGNED = detail::aligned_mode(A);
+            if constexpr (!ALIGNED) {
+                if ((x & 1) != 0) {
+#pragma unroll
+                    for (int i = 0; i < V; ++i) out[i].v = exec(x + i, y, z, p);
+                    return;
+                }
+            }
             constexpr int S = int(sizeof(B));                 // bytes per sample
             constexpr int kBits = 8 * S;
             constexpr u32 kMask = S == 1 ? 0xffu : 0xffffu;
@@ -1869,11 +1910,8 @@ template <int PF> struct ReadYUV {
                 u32 l[S], c[S];
                 const u8* lp = p.data + size_t(y) * p.pitch + size_t(x) * S;
                 const u8* cp = p.data + size_t(p.pitch) * p.height + size_t(L::k420 ? y >> 1 : y) * p.pitch + size_t(x) * S;
-                if constexpr (S == 1) { l[0] = *detail::gconst<u32>(lp); c[0] = *detail::gconst<u32>(cp); }
-                else {
-                    const detail::u32x2_t a = *detail::gconst<detail::u32x2_a4>(lp), b = *detail::gconst<detail::u32x2_a4>(cp);
-                    l[0] = a.x; l[1] = a.y; c[0] = b.x; c[1] = b.y;
-                }
+                detail::load_words<S, false, ALIGNED>(lp, l);
+                detail::load_words<S, false, ALIGNED>(cp, c);
 #pragma unroll
                 for (int i = 0; i < S; ++i) asm("" : "+v"(l[i]), "+v"(c[i]));
 #pragma unroll
@@ -1885,8 +1923,7 @@ template <int PF> struct ReadYUV {
             } else {
                 u32 g[2 * S];
                 const u8* gp = p.data + size_t(y) * p.pitch + size_t(x) * 2 * S;
-                if constexpr (S == 1) { const detail::u32x2_t a = *detail::gconst<detail::u32x2_a4>(gp); g[0] = a.x; g[1] = a.y; }
-                else { const detail::u32x4_t a = *detail::gconst<detail::u32x4_a4>(gp); g[0] = a.x; g[1] = a.y; g[2] = a.z; g[3] = a.w; }
+                detail::load_words<2 * S, false, ALIGNED>(gp, g);
 #pragma unroll
                 for (int i = 0; i < 2 * S; ++i) asm("" : "+v"(g[i]));
 #pragma unroll
@@ -1937,6 +1974,7 @@ template <class Back> struct Crop {
     using Out = typename Back::Out;
     struct Params { i32 x, y, w, h; typename Back::Params back; };
     static constexpr bool kTapCursor = Back::kTapCursor;
+    static constexpr bool kAnyX = any_x<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>();
     FKD_NAME("Crop<" + Back::name() + ">")
     FKD_HD static bool strip_ok(const Params& p) {
@@ -2066,7 +2104,7 @@ template <int BT, class Back> struct Border {
     // other for their lanes cost a 16-pixel pad of a 2160p image 9.8 instead of 8.8 us); with a constant border it differs
     // from lane to lane.  Either way the wave-cooperative access mode is not handed on.
     template <int V, int A> FKD_DEV static void exec_row(int x, int y, int z, const Params& p, Slot<Out> (&out)[V]) {
-        constexpr int kLaneMode = (A & 3) != 0 ? ((A & 4) | 1) : 0;
+        constexpr int kLaneMode = detail::aligned_mode(A) ? ((A & 4) | 1) : 0;
         const int w = Back::width(p.back), h = Back::height(p.back);
         const bool run_inside = x >= 0 && x + V <= w;
         if constexpr (BT == 0) {
@@ -2121,6 +2159,7 @@ template <class Back, class... Ops> struct FusedRead {
     using Out = typename FoldOut<typename Back::Out, Ops...>::type;
     struct Params { typename Back::Params back; Tup<typename Ops::Params...> ops; };
     static constexpr bool kTapCursor = Back::kTapCursor;
+    static constexpr bool kAnyX = any_x<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>() && (finite_map<Ops>() && ...);
     FKD_NAME("FusedRead<" + Back::name() + OpList<Ops...>::names() + ">")
     FKD_HD static bool strip_ok(const Params& p) {
@@ -2375,6 +2414,7 @@ template <int WT, class Back> struct Warp {
         typename Back::Params back;
     };
     static constexpr bool kTapCursor = false;
+    static constexpr bool kAnyX = true;
     static constexpr bool kGatherRead = true;     // taps are scattered: one element per thread
     static constexpr bool kPairTaps = [] {
         if constexpr (requires { Back::kTapPair; }) return Back::kTapCursor && Back::kTapPair; else return false;
@@ -2563,6 +2603,7 @@ template <int N, class PlaneOp> struct BatchRead {
     static constexpr int kBatch = N;
     struct Params { typename PlaneOp::Params plane[N]; };
     static constexpr bool kTapCursor = false;
+    static constexpr bool kAnyX = any_x<PlaneOp>();
     static constexpr bool kBoundedOut = bounded_out<PlaneOp>();
     FKD_NAME("BatchRead<" + istr(N) + "," + PlaneOp::name() + ">")
     FKD_HD static bool strip_ok(const Params& p, u32 planes) {
@@ -2595,6 +2636,7 @@ template <int N, class PlaneOp> struct BatchReadDefault {
     static constexpr int kBatch = N;
     struct Params { typename PlaneOp::Params plane[N]; i32 used; Out def; };
     static constexpr bool kTapCursor = false;
+    static constexpr bool kAnyX = any_x<PlaneOp>();
     FKD_NAME("BatchReadDefault<" + istr(N) + "," + PlaneOp::name() + ">")
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static Out exec(int x, int y, int z, const Params& p) {
@@ -2682,6 +2724,7 @@ template <class T> struct DualRead2D {
     using Out = Two<T, T>;
     using One = Read2D<T>;
     struct Params { typename One::Params a, b; };
+    static constexpr bool kAnyX = true;
     FKD_NAME("DualRead2D<" + type_name<T>() + ">")
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static Out exec(int x, int y, int z, const Params& p) { return Out{One::exec(x, y, z, p.a), One::exec(x, y, z, p.b)}; }

@@ -1,0 +1,127 @@
+"""Rows of the pointwise chains at every byte alignment and every remainder of their width: images whose first byte, pitch and
+width are anything, where a lane's run is one wide access at any address and the lane at a row's end works on the row's last run.
+Results are the oracle's bit for bit and nothing beside the image is touched."""
+import numpy as np
+import pytest
+
+import fkl_cases as cases
+import oracle_lib as ol
+
+pytestmark = pytest.mark.gpu
+
+FILL = 0xA5
+
+
+class Placed:
+    """A (h, w, c) image in the middle of a device buffer of FILL bytes, `offset` bytes past an aligned address, rows `pitch`
+    bytes apart."""
+    def __init__(self, shape, dtype, offset, pad_bytes, device, data=None):
+        import torch
+        h, row = shape[0], int(np.prod(shape[1:])) * np.dtype(dtype).itemsize
+        self.shape, self.dtype, self.row, self.pitch, self.start = shape, np.dtype(dtype), row, row + pad_bytes, 256 + offset
+        host = np.full(self.start + self.pitch * h + 256, FILL, np.uint8)
+        if data is not None:
+            self._rows(host)[:] = np.ascontiguousarray(data).view(np.uint8).reshape(h, row)
+        self.buf = torch.from_numpy(host).to(device)
+
+    def _rows(self, host):
+        return np.lib.stride_tricks.as_strided(host[self.start:], (self.shape[0], self.row), (self.pitch, 1))
+
+    def view(self):
+        """The image as the case drivers take it: a byte-strided tensor of its first row's address."""
+        import torch
+        size = self.dtype.itemsize
+        kind = {1: torch.uint8, 2: torch.int16, 4: torch.float32}[size]
+        assert self.start % size == 0 and self.pitch % size == 0
+        inner = [int(np.prod(self.shape[i + 1:])) for i in range(1, len(self.shape))]
+        return self.buf[self.start % size:self.buf.numel() // size * size].view(kind).as_strided(self.shape, [self.pitch // size] + inner, self.start // size)
+
+    def read(self):
+        host = self.buf.cpu().numpy()
+        rows = self._rows(host)
+        got = np.array(rows).view(self.dtype).reshape(self.shape)
+        rows[:] = FILL
+        assert (host == FILL).all(), "a byte beside the image was written"
+        return got
+
+
+WIDTHS = (1, 2, 3, 4, 5, 7, 9, 63, 255, 256, 257, 258, 259, 260, 511, 513, 1022, 1023)
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+def test_uchar3_images(device, offset):
+    import torch
+    rng = np.random.RandomState(7 + offset)
+    mul, add = rng.uniform(0.5, 2.0, (4, 3)).astype(np.float32), rng.uniform(-64, 64, (4, 3)).astype(np.float32)
+    for n, w in enumerate(WIDTHS):
+        h, pad = (1, 2, 9)[n % 3], (0, 1, 2, 5)[(n + offset) % 4]
+        imgs = [rng.randint(0, 256, (h, w, 3)).astype(np.uint8) for _ in range(4)]
+        want = ol.oracle_batch_muladd_sat(imgs, mul, add)
+        srcs = [Placed((h, w, 3), np.uint8, offset, pad, device, a) for a in imgs]
+        outs = [Placed((h, w, 3), np.uint8, (offset + 1) % 4, pad, device) for _ in imgs]
+        cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [o.view() for o in outs])
+        cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [s.view() for s in srcs])      # in place
+        torch.cuda.synchronize()
+        for a, b, c in zip(srcs, outs, want):
+            assert np.array_equal(b.read(), c) and np.array_equal(a.read(), c), (w, h, pad, offset)
+
+
+@pytest.mark.parametrize("n_ops", [1, 3, 100])
+def test_float_chains(device, n_ops):
+    import torch
+    rng = np.random.RandomState(n_ops)
+    for n, w in enumerate(WIDTHS):
+        h, pad = (1, 3, 9)[n % 3], 4 * (n % 3)
+        img = rng.uniform(-1, 1, (h, w)).astype(np.float32)
+        src, out = Placed((h, w), np.float32, 4 * (n % 4), pad, device, img), Placed((h, w), np.float32, 4, pad, device)
+        cases.add_mul_chain(src.view(), n_ops, 0.5, 1.0001, out.view())
+        torch.cuda.synchronize()
+        want = ol.oracle_add_mul_chain(img, n_ops, np.float32(0.5), np.float32(1.0001))
+        assert out.read().tobytes() == want.tobytes(), (w, h, pad)
+
+
+def test_streamed_launches(device):
+    """More than 2^26 elements: the loads of every kind of wave carry the non-temporal hint."""
+    import torch
+    rng = np.random.RandomState(5)
+    w, h = 1021, 661                                     # 100 * 1021 * 661 = 67 488 100
+    img = [rng.randint(0, 256, (h, w, 3)).astype(np.uint8) for _ in range(2)]
+    dev = [torch.from_numpy(a).to(device) for a in img]
+    outs = torch.zeros((100, h, w, 3), dtype=torch.uint8, device=device)
+    mul, add = rng.uniform(0.5, 2.0, (100, 3)).astype(np.float32), rng.uniform(-64, 64, (100, 3)).astype(np.float32)
+    cases.batch_muladd_sat([dev[i % 2] for i in range(100)], mul, add, [outs[i] for i in range(100)])
+    torch.cuda.synchronize()
+    for i in (0, 1, 50, 99):
+        want = ol.oracle_batch_muladd_sat([img[i % 2]], mul[i:i + 1], add[i:i + 1])[0]
+        assert np.array_equal(outs[i].cpu().numpy(), want), i
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_NV21, 0, 0), (ol.PF_P010, 0, 2), (ol.PF_P210, 1, 1), (ol.PF_Y210, 0, 1),
+                                      (ol.PF_UYVY, 1, 1)])
+def test_video_frames_to_rgb(device, pf, cr, cp):
+    """Even widths (packed and semi-planar formats have no others), on both sides of a run, a wave and two waves."""
+    import torch
+    dt = np.uint16 if ol.PF_WIDE[pf] else np.uint8
+    rng = np.random.RandomState(70 + pf)
+    for n, w in enumerate((2, 4, 6, 10, 254, 256, 258, 260, 510, 514, 1022)):
+        h, size = (2, 6, 12)[n % 3], np.dtype(dt).itemsize
+        rows, cols = ol.frame_shape(pf, w, h)
+        buf = rng.randint(0, 1024 if ol.PF_WIDE[pf] else 256, (rows, cols)).astype(dt)
+        frame = Placed((rows, cols), dt, size * (n % 4), size * (n % 3), device, buf)
+        out = Placed((h, w, 3), np.float32, 4 * (n % 4), 4 * (n % 2), device)
+        cases.yuv_to_rgb(pf, cr, cp, frame.view(), w, h, out.view())
+        torch.cuda.synchronize()
+        assert out.read().tobytes() == ol.oracle_yuv_to_rgb(pf, cr, cp, buf, w, h).tobytes(), (w, h)
+
+
+@pytest.mark.parametrize("w", [1, 255, 257, 511, 1023])
+def test_warps(device, w):
+    import torch
+    rng = np.random.RandomState(w)
+    img = rng.randint(0, 256, (61, 83, 3)).astype(np.uint8)
+    m = np.array([[0.9, -0.2, 4.5], [0.15, 1.1, -3.25]], np.float32)
+    for h in (1, 7):
+        out = Placed((h, w, 3), np.float32, 4, 4, device)
+        cases.warp(torch.from_numpy(img).to(device), m, False, (w, h), out.view())
+        torch.cuda.synchronize()
+        assert out.read().tobytes() == ol.oracle_warp(img, 3, m, (w, h), False).tobytes(), h
