@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52067000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "e9eddcc335d428f4c532638230867500632c96a9f79d2e6743f7a14b78178f2d"
+TRAFFIC_C3_SOURCES_SHA256 = "527f181da43b06098af2f9141166396799491a63182fb0c4beba6bfb4bdac09d"
 
 
 def device_sources_sha256():

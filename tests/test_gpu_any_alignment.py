@@ -125,3 +125,26 @@ def test_warps(device, w):
         cases.warp(torch.from_numpy(img).to(device), m, False, (w, h), out.view())
         torch.cuda.synchronize()
         assert out.read().tobytes() == ol.oracle_warp(img, 3, m, (w, h), False).tobytes(), h
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_NV21, 1, 0), (ol.PF_P010, 0, 2), (ol.PF_P210, 1, 1), (ol.PF_Y210, 0, 0),
+                                      (ol.PF_UYVY, 1, 2)])
+def test_rgb_to_video_frames(device, pf, cr, cp):
+    """Both parities of both extents: the last chroma block of an odd one belongs to a single column or row.  Launches of
+    2 048 workgroups and more give a thread two rows."""
+    import torch
+    dt = np.uint16 if ol.PF_WIDE[pf] else np.uint8
+    size = np.dtype(dt).itemsize
+    rng = np.random.RandomState(90 + pf)
+    sizes = [(w, (1, 2, 5, 12)[n % 4]) for n, w in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 254, 255, 256, 257, 258, 259, 260, 510, 513))]
+    for n, (w, h) in enumerate(sizes + [(1021, 4100), (1026, 4097)]):
+        rgb = rng.randint(0, 1024 if ol.PF_WIDE[pf] else 256, (h, w, 3)).astype(dt)
+        rows, cols = ol.frame_shape(pf, w + (w & 1), h + (h & 1))
+        if pf in (ol.PF_NV12, ol.PF_NV21, ol.PF_P010, ol.PF_P210):
+            rows = h + (h + 1) // 2 if pf != ol.PF_P210 else 2 * h     # chroma rows start right after `height` luma rows
+        start = np.full((rows, cols), 9, dt)
+        frame = Placed((rows, cols), dt, size * (n % 4), size * (n % 3), device, start)
+        src = Placed((h, w, 3), dt, size * ((n + 1) % 4), size * (n % 2), device, rgb)
+        cases.rgb_to_yuv(pf, cr, cp, src.view(), frame.view())
+        torch.cuda.synchronize()
+        assert np.array_equal(frame.read(), ol.oracle_rgb_to_yuv(pf, cr, cp, rgb, start)), (w, h)
