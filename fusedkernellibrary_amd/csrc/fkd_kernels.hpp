@@ -96,29 +96,36 @@ constexpr unsigned long long kStreamElements = 1ull << 26;   // launches over mo
 // FKD_TEST_UNRESOLVED_INDEX defined, the rows kernel indexes its values with an offset that is zero when the kernel runs
 // but unknown when it is compiled (an index the optimiser cannot resolve keeps the array in memory).  Zero otherwise.
 #ifdef FKD_TEST_UNRESOLVED_INDEX
-#define FKD_TEST_INDEX_OFFSET int(p.active_w >> 31)
+#define FKD_TEST_INDEX_OFFSET int(p.reserved >> 31)
 #else
 #define FKD_TEST_INDEX_OFFSET 0
 #endif
 
-// The full-width part of the rows kernel: every lane has V elements in each of its ROWS rows.  MODE as in
-// detail::load_run.  TAIL: rows that are not a multiple of V wide; the lane at a row's end, which has fewer than V elements
-// left, works on the row's last V elements and stores only those from x0 on (the others are its neighbour's; what it read
-// there is not used, so a chain that works in place is none the wiser).
-template <class Chain, int V, int ROWS, int MODE, bool TAIL = false>
-__device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 kernarg_offset, int first, int ybase, int z, int aw, int ah) {
+// One wave's part of the rows kernel: V elements of each of ROWS rows per lane, row r from element x[r] on.  MODE as in
+// detail::load_run.  EDGE: the wave's segment of 64 * V elements, which begins at seg[r], reaches past the end of the row
+// (kRowEnd: lanes that have no element inside are not here) or past either end (kRowEnds: all lanes of the wave are here).  A
+// lane that has fewer than V of its elements inside, or none, then works on the first or last V elements of the row, and only
+// the elements of the segment are stored; what a lane reads beside its own is not used or its neighbour's in the same wave,
+// so a chain that works in place is none the wiser.
+constexpr int kRowEnd = 1, kRowEnds = 2;
+template <class Chain, int V, int ROWS, int MODE, int EDGE = 0>
+__device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 kernarg_offset, const int (&seg)[ROWS], const int (&x)[ROWS],
+                                          int ybase, int z, int aw, int ah) {
     using R = typename Chain::Read;
     using W = typename Chain::Write;
-    const int x0 = TAIL && first + V > aw ? aw - V : first;
 
     // All loads first, unconditionally (rows past the end re-read the last row, which is in bounds), so every
     // lane has ROWS independent wide loads in flight before the first use; only the stores are predicated.
     Slot<typename R::Out> in[ROWS * V];
+    int x0[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
         const int y = ybase + r < ah ? ybase + r : ah - 1;
+        x0[r] = x[r];
+        if constexpr (EDGE == kRowEnd) x0[r] = x[r] < aw - V ? x[r] : aw - V;
+        if constexpr (EDGE == kRowEnds) x0[r] = x[r] < 0 ? 0 : (x[r] < aw - V ? x[r] : aw - V);
         Slot<typename R::Out> row[V];
-        R::template exec_row<V, MODE>(x0, y, z, p.read, row);
+        R::template exec_row<V, MODE>(x0[r], y, z, p.read, row);
 #pragma unroll
         for (int i = 0; i < V; ++i) in[r * V + i].v = row[i].v;
     }
@@ -133,16 +140,26 @@ __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 k
 #pragma unroll
         for (int i = 0; i < V; ++i) row[i].v = out[r * V + i + FKD_TEST_INDEX_OFFSET].v;
         if (y >= ah) continue;
-        if constexpr (TAIL) {
-            if (x0 != first) {
+        if constexpr (EDGE == kRowEnds && has_edge_store<W, V>()) {
+            W::template exec_edge<V>(seg[r], x0[r], aw, y, z, row, p.write);
+        } else if constexpr (EDGE != 0) {
+            if (x0[r] == x[r]) {
+                W::template exec_row<V, MODE>(x0[r], y, z, row, p.write);
+            } else if (EDGE == kRowEnd || (x[r] > -V && x[r] < aw)) {
 #pragma unroll
-                for (int i = 1; i < V; ++i) if (x0 + i >= first) W::exec(x0 + i, y, z, row[i].v, p.write);
-                continue;
+                for (int i = 0; i < V; ++i) {
+                    if (EDGE == kRowEnd && i == 0) continue;              // (the first of the row's last V is never the lane's)
+                    if (x0[r] + i >= x[r] && (EDGE == kRowEnd || x0[r] + i < x[r] + V)) W::exec(x0[r] + i, y, z, row[i].v, p.write);
+                }
             }
+        } else {
+            W::template exec_row<V, MODE>(x0[r], y, z, row, p.write);
         }
-        W::template exec_row<V, MODE>(x0, y, z, row, p.write);
     }
 }
+
+// Whether waves may take runs that start anywhere in a row.
+template <class Chain> constexpr bool rows_any_x(int v) { return v > 1 && any_x<typename Chain::Read>(); }
 
 // Chains whose read gathers its taps from wherever the coordinates fall (warps, bilinear reads without a tap cursor): their
 // larger launches number the workgroups of a plane so that each XCD works on a contiguous band of the output.
@@ -161,7 +178,8 @@ template <class Chain> constexpr bool rows_in_bands() {
 // `kernarg_offset`: where p sits inside the kernel-argument segment (0 when the chain's parameter block is the
 // kernel's first argument); long chains fetch their operations' parameters from there.  BANDS: the launch has the bands
 // form of grid (see rows_band_chunk).
-template <class Chain, int V, int ROWS, bool ALIGNED, bool BANDS = false>
+// SHIFT: the launch's grid has room for segments that begin left of a row (Chain::row_phase_bound).
+template <class Chain, int V, int ROWS, bool ALIGNED, bool BANDS = false, bool SHIFT = false>
 __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     using R = typename Chain::Read;
     using W = typename Chain::Write;
@@ -179,40 +197,75 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
             block_x = tin - block_y * gx;
         }
     }
-    const int x0 = (block_x * kRowsBX + threadIdx.x) * V;
-    const int ybase = (block_y * kRowsBY + threadIdx.y) * ROWS;
-    if (x0 >= aw || ybase >= ah) return;
     // Wave-cooperative accesses (mode 2 of load_run / store_run) need every lane of the wave on a full run.
     constexpr bool kExchange = (detail::wave_exchange_ok<typename R::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
-    if constexpr (kExchange) {
-        if (int(block_x * kRowsBX + kRowsBX) * V <= aw) {
-            rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign>(p, kernarg_offset, x0, ybase, z, aw, ah);
-            return;
-        }
-    }
     // A launch over more elements than the last-level cache could hold between two launches reads them with the
     // non-temporal hint (100 images of 1920x1080 uchar3: 225 -> 209 us); smaller inputs are left to the caches, where a
     // pipeline's previous stage may have put them (the hint costs 15 % on a 33 MB image that is still cached).
     constexpr bool kMayStream = !Chain::kLongChain && !kExchange;
     const bool stream = kMayStream && (unsigned long long)(u32(aw)) * u32(ah) * gridDim.z > kStreamElements;
-    // The wave at the end of rows whose width is no multiple of V (wave uniform).  Its lanes make the accesses of the other
-    // waves, at whatever alignment the row's last V elements have; element by element, each behind the one before, the
-    // last lane's three elements took longer than the rest of the launch (100 operations on 511x512 floats, four launches:
-    // 43.0 -> 22.9 us; a 1919x1079 warp 11.1 -> 8.7 us).
-    if constexpr (V > 1 && any_x<R>()) {
-        if (aw % V != 0 && aw >= V && int(block_x * kRowsBX + kRowsBX) * V > aw) {
-            if constexpr (kMayStream) {
-                if (stream) { rows_full<Chain, V, ROWS, 0 | 4, true>(p, kernarg_offset, x0, ybase, z, aw, ah); return; }
+    if constexpr (rows_any_x<Chain>(V)) {
+        // A wave owns a segment of 64 * V elements of a row.  Segments are counted from the row's start or, in launches with
+        // room for it (row_phase_bound), from the last line boundary before it, so that every wave but the two at a row's ends
+        // stores whole lines: a line shared by two waves leaves the chip as two partial writes.
+        if (aw >= V) {
+            const int yw = (block_y * kRowsBY + __builtin_amdgcn_readfirstlane(int(threadIdx.y))) * ROWS;
+            if (yw >= ah) return;
+            constexpr int kWhole = kExchange ? 2 | detail::kAnyAlign : 0;
+            int seg[ROWS], x[ROWS];
+            bool whole = true;
+            auto go = [&](auto edge_tag) {
+                constexpr int EDGE = decltype(edge_tag)::value;
+                if constexpr (kMayStream) {
+                    if (stream) { rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | 4, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
+                }
+                rows_full<Chain, V, ROWS, EDGE ? 0 : kWhole, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah);
+            };
+            if constexpr (SHIFT && has_row_phase<W>()) {
+                const u32 bound = Chain::row_phase_bound(p.reserved);
+                if (bound != 0u) {
+                    bool outside = true;
+#pragma unroll
+                    for (int r = 0; r < ROWS; ++r) {
+                        const int phase = W::row_phase(yw + r < ah ? yw + r : ah - 1, z, p.write) & int(bound);
+                        seg[r] = int(block_x) * kRowsBX * V - (phase % x_group<R>() == 0 ? phase : 0);
+                        whole = whole && seg[r] >= 0 && seg[r] + kRowsBX * V <= aw;
+                        outside = outside && seg[r] >= aw;
+                        x[r] = seg[r] + int(threadIdx.x) * V;
+                    }
+                    if (outside) return;                                   // (wave uniform, as `whole`)
+                    if (whole) go(IntTag<0>{}); else go(IntTag<kRowEnds>{});
+                    return;
+                }
             }
-            rows_full<Chain, V, ROWS, 0, true>(p, kernarg_offset, x0, ybase, z, aw, ah);
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) { seg[r] = int(block_x) * kRowsBX * V; x[r] = seg[r] + int(threadIdx.x) * V; }
+            whole = seg[0] + kRowsBX * V <= aw;
+            if (whole) { go(IntTag<0>{}); return; }
+            if (x[0] >= aw) return;
+            go(IntTag<kRowEnd>{});
             return;
         }
     }
-    if (x0 + V <= aw) {
-        if constexpr (kMayStream) {
-            if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4>(p, kernarg_offset, x0, ybase, z, aw, ah); return; }
+    const int x0 = (block_x * kRowsBX + threadIdx.x) * V;
+    const int ybase = (block_y * kRowsBY + threadIdx.y) * ROWS;
+    if (x0 >= aw || ybase >= ah) return;
+    int same[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) same[r] = x0;
+    if (!rows_any_x<Chain>(V) && x0 + V <= aw) {
+        if constexpr (!rows_any_x<Chain>(V)) {
+            if constexpr (kExchange) {
+                if (int(block_x * kRowsBX + kRowsBX) * V <= aw) {
+                    rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign>(p, kernarg_offset, same, same, ybase, z, aw, ah);
+                    return;
+                }
+            }
+            if constexpr (kMayStream) {
+                if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4>(p, kernarg_offset, same, same, ybase, z, aw, ah); return; }
+            }
+            rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0>(p, kernarg_offset, same, same, ybase, z, aw, ah);
         }
-        rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0>(p, kernarg_offset, x0, ybase, z, aw, ah);
     } else {
         for (int r = 0; r < ROWS; ++r) {
             const int y = ybase + r;
@@ -231,7 +284,7 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
 
 template <class Chain, int V, int ROWS, bool ALIGNED>
 __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_rows(const typename Chain::Params p, const TileGeom g) {
-    rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>()>(p, 0u, &g);
+    rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), true>(p, 0u, &g);
 }
 
 // Whether the rows of plane z of the read and of the write all start on dword boundaries, decided on the device
@@ -245,9 +298,10 @@ template <class Op, class P> FKD_DEV bool write_plane_aligned(const P& p, int z)
     if constexpr (requires { Op::plane_rows_aligned(p, z); }) return Op::plane_rows_aligned(p, z);
     else return Op::rows_aligned(p);
 }
-template <class Chain, int V, int ROWS, bool BANDS = false>
+template <class Chain, int V, int ROWS, bool BANDS = false, bool SHIFT = false>
 __device__ __forceinline__ void rows_auto_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     const int z = blockIdx.z;
+    if constexpr (rows_any_x<Chain>(V)) { rows_body<Chain, V, ROWS, false, BANDS, SHIFT>(p, kernarg_offset, bands); return; }
     const bool aligned = read_plane_aligned<typename Chain::Read>(p.read, z) && write_plane_aligned<typename Chain::Write>(p.write, z);
     if (aligned) rows_body<Chain, V, ROWS, true, BANDS>(p, kernarg_offset, bands);
     else rows_body<Chain, V, ROWS, false, BANDS>(p, kernarg_offset, bands);
@@ -941,7 +995,7 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
         }
         gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, false>(p, g);
     }
-    else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>()>(p, 0u, &g);
+    else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), true>(p, 0u, &g);
 }
 
 } // namespace fkd

@@ -27,7 +27,7 @@ constexpr unsigned kRowsSmallGrid = 2048;
 
 template <class Chain, int V, int ROWS>
 hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info, bool aligned) {
-    const unsigned gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);
+    const unsigned gx = (p.active_w + rows_phase_bound(p.reserved) + kRowsBX * V - 1) / (kRowsBX * V);
     const unsigned gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);
     dim3 grid(gx, gy, p.active_z);
     const dim3 block(kRowsBX, kRowsBY, 1);
@@ -43,7 +43,9 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
     if (grid.y > 65535u || grid.z > 65535u) return hipErrorInvalidConfiguration;
-    if (aligned) return launch_by_pointer(&k_rows<Chain, V, ROWS, true>, grid, block, stream, p, g);
+    if constexpr (!rows_any_x<Chain>(V)) {     // (the others take runs at any alignment, one kernel for both)
+        if (aligned) return launch_by_pointer(&k_rows<Chain, V, ROWS, true>, grid, block, stream, p, g);
+    }
     return launch_by_pointer(&k_rows<Chain, V, ROWS, false>, grid, block, stream, p, g);
 }
 

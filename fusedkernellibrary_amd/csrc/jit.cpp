@@ -41,6 +41,7 @@ using fkd::TileGeom;
 using fkd::division_magic;
 using fkd::kRowsBandBlocks;
 using fkd::kStreamOutputBytes;
+using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
 struct JitKernel {
@@ -228,7 +229,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[2] = active[2];
         block[1] = m.by;
     } else {
-        grid[0] = (active[0] + 64 * m.v - 1) / (64 * m.v);
+        grid[0] = (active[0] + (m.max_planes != 0 ? 0u : rows_phase_bound(active[3])) + 64 * m.v - 1) / (64 * m.v);
         grid[1] = (active[1] + 4 * m.rows - 1) / (4 * m.rows);
         grid[2] = active[2];
         if (m.bands && (unsigned long long)grid[0] * grid[1] >= kRowsBandBlocks) {

@@ -43,6 +43,10 @@ inline unsigned division_magic(unsigned d, unsigned limit) {
 inline constexpr unsigned rows_band_chunk(unsigned blocks) { return (blocks + 7u) / 8u; }
 constexpr unsigned kRowsBandBlocks = 4096;
 
+// Bits 8 to 15 of a chain's Params::reserved: by how many elements at most the rows kernel's waves begin left of a row so
+// that they store whole lines (Chain::finalize_write); the grid has to reach that much further.
+inline constexpr unsigned rows_phase_bound(unsigned reserved) { return (reserved >> 8) & 0xffu; }
+
 // Strip form of the bilinear kernel: a launch of at most kStripOneRoundWorkgroups workgroups (eight per compute unit: every
 // workgroup resident from the start) runs with wave priorities; the kernel is told the number of the first workgroup that
 // counts as started late, or 0 for a launch whose waves keep the default priority (see the kernels' header).

@@ -57,6 +57,65 @@ template <class R> constexpr bool bounded_out() {
 template <class R> constexpr bool any_x() {
     if constexpr (requires { R::kAnyX; }) return R::kAnyX; else return false;
 }
+// x_group<R>: ... and is at its best from multiples of this many.
+template <class R> constexpr int x_group() {
+    if constexpr (requires { R::kXGroup; }) return R::kXGroup; else return 1;
+}
+// How far the rows of an image of T are from line boundaries: a row of T at address a starts row_phase(a) elements after the
+// start of an element that lies on one (0 where none does, or where a row starts on a boundary).  The phase s solves
+// s * sizeof(T) = a modulo the line; sizeof(T) is a power of two or three times one, and 3 * 43 = 129.  For half a line it is
+// the same number modulo half the period.
+constexpr u32 kLineBytes = 128;
+template <class T> constexpr u32 row_phase_unit() {      // the power of two in sizeof(T), 0 for sizes that have no phase
+    constexpr u32 n = u32(sizeof(T));
+    constexpr u32 unit = n & (0u - n);
+    return n / unit == 1u || n / unit == 3u ? (unit < kLineBytes ? unit : 0u) : 0u;
+}
+template <class T> FKD_HD int row_phase_of(size_t address) {
+    constexpr u32 unit = row_phase_unit<T>();
+    if constexpr (unit == 0u) {
+        return 0;
+    } else {
+        const u32 a = u32(address) & (kLineBytes - 1u);
+        if (a % unit != 0u) return 0;
+        return int(((a / unit) * (u32(sizeof(T)) == unit ? 1u : 43u)) & (kLineBytes / unit - 1u));
+    }
+}
+// The largest phase of the rows of an image: 0 when all of them start on line boundaries.
+template <class T> FKD_HD u32 row_phase_bound_of(const void* data, size_t pitch, size_t plane_bytes = 0) {
+    constexpr u32 unit = row_phase_unit<T>();
+    if (unit == 0u || ((reinterpret_cast<size_t>(data) | pitch | plane_bytes) % kLineBytes) == 0) return 0u;
+    return kLineBytes / unit - 1u;
+}
+// has_edge_store<W, V>: write W has a form of its own for the waves at a row's ends.
+template <class W, int V> constexpr bool has_edge_store() {
+    if constexpr (requires { W::template kEdgeStore<V>; }) return W::template kEdgeStore<V>; else return false;
+}
+// Which of the bounds `full` (whole lines), half of it (half lines) and 0 (segments counted from the row's start) a launch
+// takes whose rows are `width` elements and whose output is `bytes`.  Whole lines pay where the output is large enough to be
+// bound by the memory and the row is several segments of 256 long.
+// us, counted from the row's start / whole lines / half lines: NV12 to float3 at 3838x2160 27.5 / 20.1 / 20.6, at 1922x1080
+// 6.9 / 6.65 / 6.8, at 642x482 (3.7 MB, 4 launches) 13.8 / 16.6; floats at 3839x2159 12.2 / 11.4 / 11.7, 4 of 1921x1080 19.6 /
+// 17.5 / 17.7.  A segment more per row costs its empty waves: 100 uchar3 images of 644x480 (3 segments, 4 with whole lines)
+// 35.1 / 40.1 / 33.8, of 510x333 (2, 3) 19.6 / 20.4 / 20.2, 4 of 1279x719 (5, 6) 6.0 / 6.3 / 6.3, but 100 of 1023x768 (4, 5;
+// 236 MB) 110 / 91.6 / 92.9.  Elements of no whole dwords are stored byte by byte at a row's ends, so they need more output: 4
+// images of 1400x700 (11.8 MB, 4 launches) 23.6 / 24.9, of 1900x1000 (22.8 MB) 9.8 / 9.25.  Elements of several dwords go
+// through LDS there: NV12 to float3 at 1282x720 (11 MB, 4 launches) 16.9 / 20.4, at 2500x1400 11.2 / 10.4.
+constexpr u32 kPhaseMinWidth = 512;
+constexpr unsigned long long kPhaseAnyBytes = 128ull << 20;
+template <class T> constexpr unsigned long long phase_min_bytes() { return sizeof(T) % 4 != 0 ? 16000000 : sizeof(T) > 4 ? 24000000 : 6000000; }
+inline u32 phase_bound_for(u32 full, u32 width, unsigned long long bytes, unsigned long long min_bytes) {
+    if (full == 0u || width < kPhaseMinWidth || bytes < min_bytes) return 0u;
+    const u32 half = (full & 1u) != 0u ? full >> 1 : (full >> 2) << 1;      // n - 1 or 2 * (n - 1), n a power of two
+    auto segments = [&](u32 bound) { return (width + bound + 255u) / 256u; };
+    const u32 plain = segments(0u);
+    if (segments(full) == plain) return full;
+    if (segments(half) == plain) return half;
+    return bytes >= kPhaseAnyBytes || plain >= 8u ? full : 0u;
+}
+template <class W> constexpr bool has_row_phase() {
+    if constexpr (requires { W::kRowPhase; }) return W::kRowPhase; else return false;
+}
 template <class T> constexpr bool small_integer_base() {
     return !(__is_same(base_t<T>, f32) || __is_same(base_t<T>, f64)) && sizeof(base_t<T>) <= 2;
 }
@@ -386,6 +445,38 @@ template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot
     } else {
 #pragma unroll
         for (int i = 0; i < V; ++i) store_elem(p + i, in[i].v);
+    }
+}
+
+// The counterpart of store_run for the two waves at a row's ends, whose segment of 64 * V elements reaches past an end of the
+// row (`aw` elements long): the segment begins at element seg of the row, the lane holds the V elements from x on (0 <= x <=
+// aw - V), between them the lanes hold all elements of the segment that lie in the row, and those are stored.  Runs of 32, 48
+// or 64 bytes leave as dense instructions here too.
+template <class T, int V> FKD_DEV void store_run_edge(T* row, int seg, int x, int aw, const Slot<T> (&in)[V]) {
+    static_assert(wave_exchange_ok<T>(V) && sizeof(T) % 4 == 0, "whole dwords per element");
+    constexpr int W = int(sizeof(T)) * V / 4, E = int(sizeof(T)) / 4;
+    const int lane = int(threadIdx.x);
+    u32 w[W];
+    pack_words<T, V, W>(in, w);
+    u32* stage = wave_stage();
+    wave_exchange_fence();
+    const int at = (x - seg) * E;
+#pragma unroll
+    for (int j = 0; j < W; ++j) if (u32(at + j) < u32(64 * W)) stage[stage_at<W>(u32(at + j))] = w[j];
+    wave_exchange_fence();
+    const int lo = seg < 0 ? -seg * E : 0, hi = (aw - seg < 64 * V ? aw - seg : 64 * V) * E;      // dwords of the segment that exist
+    char* base = reinterpret_cast<char*>(row) + ptrdiff_t(seg) * ptrdiff_t(sizeof(T));
+#pragma unroll
+    for (int k = 0; k < W / 4; ++k) {
+        const int f = k * 256 + lane * 4;
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(f)));
+        if (f >= lo && f + 4 <= hi) {
+            gstore<dwords_at<4, false>>(gmut<dwords_at<4, false>>(base + f * 4), v);
+        } else {
+            const u32 d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) if (f + i >= lo && f + i < hi) gstore<u32_a1>(gmut<u32_a1>(base + (f + i) * 4), d[i]);
+        }
     }
 }
 
@@ -1741,6 +1832,7 @@ template <bool VU> struct ReadNV {
     using Out = Vec<u8, 3>;
     using Params = RawNV12;
     static constexpr bool kTapCursor = true;
+    static constexpr int kXGroup = 2;
     static constexpr bool kAnyX = true;
     static constexpr bool kFiniteTaps = true;
     static constexpr bool kBoundedOut = true;
@@ -1865,6 +1957,7 @@ template <int PF> struct ReadYUV {
     using B = typename PixelBase<PF>::type;
     using Out = Vec<B, 3>;
     using Params = RawYUV;
+    static constexpr int kXGroup = 2;
     static constexpr bool kAnyX = true;
     static constexpr bool kTapCursor = false;
     FKD_NAME("ReadYUV<" + istr(PF) + ">")
@@ -1975,6 +2068,7 @@ template <class Back> struct Crop {
     struct Params { i32 x, y, w, h; typename Back::Params back; };
     static constexpr bool kTapCursor = Back::kTapCursor;
     static constexpr bool kAnyX = any_x<Back>();
+    static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>();
     FKD_NAME("Crop<" + Back::name() + ">")
     FKD_HD static bool strip_ok(const Params& p) {
@@ -2160,6 +2254,7 @@ template <class Back, class... Ops> struct FusedRead {
     struct Params { typename Back::Params back; Tup<typename Ops::Params...> ops; };
     static constexpr bool kTapCursor = Back::kTapCursor;
     static constexpr bool kAnyX = any_x<Back>();
+    static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>() && (finite_map<Ops>() && ...);
     FKD_NAME("FusedRead<" + Back::name() + OpList<Ops...>::names() + ">")
     FKD_HD static bool strip_ok(const Params& p) {
@@ -2604,6 +2699,7 @@ template <int N, class PlaneOp> struct BatchRead {
     struct Params { typename PlaneOp::Params plane[N]; };
     static constexpr bool kTapCursor = false;
     static constexpr bool kAnyX = any_x<PlaneOp>();
+    static constexpr int kXGroup = x_group<PlaneOp>();
     static constexpr bool kBoundedOut = bounded_out<PlaneOp>();
     FKD_NAME("BatchRead<" + istr(N) + "," + PlaneOp::name() + ">")
     FKD_HD static bool strip_ok(const Params& p, u32 planes) {
@@ -2637,6 +2733,7 @@ template <int N, class PlaneOp> struct BatchReadDefault {
     struct Params { typename PlaneOp::Params plane[N]; i32 used; Out def; };
     static constexpr bool kTapCursor = false;
     static constexpr bool kAnyX = any_x<PlaneOp>();
+    static constexpr int kXGroup = x_group<PlaneOp>();
     FKD_NAME("BatchReadDefault<" + istr(N) + "," + PlaneOp::name() + ">")
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static Out exec(int x, int y, int z, const Params& p) {
@@ -2692,6 +2789,9 @@ template <class T> struct Write2D {
     using In = T;
     using Params = RawPtr2D<T>;
     FKD_NAME("Write2D<" + type_name<T>() + ">")
+    static constexpr bool kRowPhase = true;
+    static constexpr unsigned long long kPhaseMin = phase_min_bytes<T>();
+    FKD_HD static u32 row_phase_bound(const Params& p) { return row_phase_bound_of<T>(p.data, p.pitch); }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static void exec(int x, int y, int, const T& v, const Params& p) {
         detail::store_elem(detail::row_ptr(p.data, p.pitch, x, y), v);
@@ -2702,6 +2802,11 @@ template <class T> struct Write2D {
         detail::store_run<T, V, A>(detail::row_ptr(p.data, p.pitch, x, y), v);
     }
     FKD_HD static bool rows_aligned(const Params& p) { return detail::dword_aligned(p.data) && p.pitch % 4 == 0; }
+    template <int V> static constexpr bool kEdgeStore = detail::wave_exchange_ok<T>(V);
+    template <int V> FKD_DEV static void exec_edge(int seg, int x, int aw, int y, int, const Slot<T> (&v)[V], const Params& p) {
+        detail::store_run_edge<T, V>(detail::row_ptr(p.data, p.pitch, 0, y), seg, x, aw, v);
+    }
+    FKD_DEV static int row_phase(int y, int, const Params& p) { return row_phase_of<T>(reinterpret_cast<size_t>(p.data) + size_t(y) * p.pitch); }
     // Row cursor: one address computation per row, one add per element.
     // The part of the parameters one plane needs (all of them here).
     using Plane = Write2D;
@@ -2815,6 +2920,11 @@ template <class T> struct TensorWrite {
     using In = T;
     using Params = RawPtr3D<T>;
     FKD_NAME("TensorWrite<" + type_name<T>() + ">")
+    static constexpr bool kRowPhase = true;
+    static constexpr unsigned long long kPhaseMin = phase_min_bytes<T>();
+    FKD_HD static u32 row_phase_bound(const Params& p) {
+        return row_phase_bound_of<T>(p.data, p.pitch, p.planes > 1 ? size_t(p.plane_pitch) * p.color_planes : 0);
+    }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static T* plane(const Params& p, int z) {
         return reinterpret_cast<T*>(reinterpret_cast<char*>(p.data) + size_t(p.plane_pitch) * p.color_planes * z);
@@ -2830,6 +2940,11 @@ template <class T> struct TensorWrite {
     FKD_HD static bool rows_aligned(const Params& p) {
         return detail::dword_aligned(p.data) && p.pitch % 4 == 0 && (size_t(p.plane_pitch) * p.color_planes) % 4 == 0;
     }
+    template <int V> static constexpr bool kEdgeStore = detail::wave_exchange_ok<T>(V);
+    template <int V> FKD_DEV static void exec_edge(int seg, int x, int aw, int y, int z, const Slot<T> (&v)[V], const Params& p) {
+        detail::store_run_edge<T, V>(detail::row_ptr(plane(p, z), p.pitch, 0, y), seg, x, aw, v);
+    }
+    FKD_DEV static int row_phase(int y, int z, const Params& p) { return row_phase_of<T>(reinterpret_cast<size_t>(detail::row_ptr(plane(p, z), p.pitch, 0, y))); }
     // The part of the parameters one plane needs (all of them here).
     using Plane = TensorWrite;
     FKD_DEV static const Params& plane_params(const Params& p, int) { return p; }
@@ -2977,6 +3092,14 @@ template <int PF> struct WriteYUV {
     using B = typename PixelBase<PF>::type;
     using In = Vec<B, 3>;
     using Params = RawYUVOut;
+    // (rows of luma samples or of groups of two pixels; runs start at even pixels)
+    using Group = Vec<B, L::kSemiPlanar ? 2 : 4>;
+    static constexpr bool kRowPhase = true;
+    static constexpr unsigned long long kPhaseMin = phase_min_bytes<u32>();
+    FKD_HD static u32 row_phase_bound(const Params& p) {
+        const u32 groups = row_phase_bound_of<Group>(p.data, p.pitch);
+        return groups != 0u ? 2u * groups : 0u;
+    }
     FKD_NAME("WriteYUV<" + istr(PF) + ">")
 #if defined(FKD_EXEC_CODE)
     struct RowRef { char* row; char* crow; bool chroma_row; int last_x; };
@@ -3063,6 +3186,9 @@ template <int PF> struct WriteYUV {
         }
     }
     FKD_HD static bool rows_aligned(const Params&) { return true; }   // any alignment
+    FKD_DEV static int row_phase(int y, int, const Params& p) {
+        return 2 * row_phase_of<Group>(reinterpret_cast<size_t>(p.data) + size_t(y) * p.pitch);
+    }
     using Plane = WriteYUV;
     FKD_DEV static const Params& plane_params(const Params& p, int) { return p; }
 #endif
@@ -3073,6 +3199,14 @@ template <int N, class W> struct BatchWrite {
     using In = typename W::In;
     struct Params { typename W::Params plane[N]; };
     FKD_NAME("BatchWrite<" + istr(N) + "," + W::name() + ">")
+    static constexpr bool kRowPhase = has_row_phase<W>();
+    static constexpr unsigned long long kPhaseMin = [] { if constexpr (has_row_phase<W>()) return W::kPhaseMin; else return 0ull; }();
+    FKD_HD static u32 row_phase_bound(const Params& p) {
+        if constexpr (kRowPhase) {
+            for (int i = 0; i < N; ++i) if (const u32 b = W::row_phase_bound(p.plane[i])) return b;      // one bound per type
+        }
+        return 0u;
+    }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static void exec(int x, int y, int z, const In& v, const Params& p) { W::exec(x, y, z, v, p.plane[z]); }
 #endif
@@ -3085,6 +3219,11 @@ template <int N, class W> struct BatchWrite {
         return true;
     }
     FKD_HD static bool plane_rows_aligned(const Params& p, int z) { return W::rows_aligned(p.plane[z]); }
+    template <int V> static constexpr bool kEdgeStore = has_edge_store<W, V>();
+    template <int V> FKD_DEV static void exec_edge(int seg, int x, int aw, int y, int z, const Slot<In> (&v)[V], const Params& p) {
+        W::template exec_edge<V>(seg, x, aw, y, z, v, p.plane[z]);
+    }
+    FKD_DEV static int row_phase(int y, int z, const Params& p) { return W::row_phase(y, z, p.plane[z]); }
     using Plane = W;
     FKD_DEV static const typename W::Params& plane_params(const Params& p, int z) { return p.plane[z]; }
     using RowRef = typename W::RowRef;
@@ -3220,13 +3359,18 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     // Host, once read AND write are filled in: bit 0 of `reserved` tells the launcher that every active plane meets what
     // the strip form of the bilinear kernel asks of its source and destination (that form has no other way to decline a
     // plane).  A parameter block that never came through here keeps the bit clear and gets the tile form.
+    // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
+    // phase_bound_for).
     static constexpr u32 kStripChecked = 1u;
     static void finalize_write(Params& p) {
+        if constexpr (any_x<R>() && has_row_phase<W>())
+            p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
         if constexpr (requires { R::strip_ok(p.read, p.active_z); W::strip_ok(p.write); }) {
             if (R::strip_ok(p.read, p.active_z) && W::strip_ok(p.write)) p.reserved |= kStripChecked;
         }
     }
 #endif
+    FKD_HD static u32 row_phase_bound(u32 reserved) { return (reserved >> 8) & 0xffu; }
 #if defined(FKD_EXEC_CODE)
     static_assert(__is_same(Value, typename W::In), "the write operation does not take the type the chain produces");
     FKD_DEV static Value compute(const typename R::Out& v, const Params& p) {

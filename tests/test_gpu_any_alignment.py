@@ -148,3 +148,72 @@ def test_rgb_to_video_frames(device, pf, cr, cp):
         cases.rgb_to_yuv(pf, cr, cp, src.view(), frame.view())
         torch.cuda.synchronize()
         assert np.array_equal(frame.read(), ol.oracle_rgb_to_yuv(pf, cr, cp, rgb, start)), (w, h)
+
+
+# Outputs of 6 MB and more (16 MB for uchar3, 24 MB for float3) with rows of 512 elements and more, whose waves' segments begin at line boundaries: whole lines, half
+# lines and rows that all start on a boundary.
+@pytest.mark.parametrize("w,h,pad", [(1921, 700, 1), (2051, 700, 0), (1924, 900, 2), (644, 2100, 2), (1024, 1400, 0)])
+def test_line_aligned_segments_uchar3(device, w, h, pad):
+    import torch
+    rng = np.random.RandomState(w)
+    mul, add = rng.uniform(0.5, 2.0, (4, 3)).astype(np.float32), rng.uniform(-64, 64, (4, 3)).astype(np.float32)
+    imgs = [rng.randint(0, 256, (h, w, 3)).astype(np.uint8) for _ in range(4)]
+    want = ol.oracle_batch_muladd_sat(imgs, mul, add)
+    srcs = [Placed((h, w, 3), np.uint8, 3, pad, device, a) for a in imgs]
+    outs = [Placed((h, w, 3), np.uint8, 0 if w == 1024 else i, 0 if w == 1024 else pad, device) for i in range(4)]
+    cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [o.view() for o in outs])
+    cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [s.view() for s in srcs])      # in place
+    torch.cuda.synchronize()
+    for a, b, c in zip(srcs, outs, want):
+        assert np.array_equal(b.read(), c) and np.array_equal(a.read(), c)
+
+
+@pytest.mark.parametrize("w,h,offset", [(1921, 1080, 4), (2049, 790, 0), (1536, 1000, 12), (1536, 1000, 0)])
+@pytest.mark.parametrize("n_ops", [1, 100])
+def test_line_aligned_segments_floats(device, n_ops, w, h, offset):
+    import torch
+    img = np.random.RandomState(w).uniform(-1, 1, (h, w)).astype(np.float32)
+    src, out = Placed((h, w), np.float32, 0, 0, device, img), Placed((h, w), np.float32, offset, 0, device)
+    cases.add_mul_chain(src.view(), n_ops, 0.5, 1.0001, out.view())
+    torch.cuda.synchronize()
+    assert out.read().tobytes() == ol.oracle_add_mul_chain(img, n_ops, np.float32(0.5), np.float32(1.0001)).tobytes()
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_P010, 0, 2), (ol.PF_UYVY, 1, 1)])
+@pytest.mark.parametrize("w,h,offset", [(966, 2080, 4), (2050, 1000, 8), (770, 2600, 0), (1280, 1600, 0)])
+def test_line_aligned_segments_video_to_rgb(device, pf, cr, cp, w, h, offset):
+    import torch
+    dt = np.uint16 if ol.PF_WIDE[pf] else np.uint8
+    rows, cols = ol.frame_shape(pf, w, h)
+    buf = np.random.RandomState(w).randint(0, 1024 if ol.PF_WIDE[pf] else 256, (rows, cols)).astype(dt)
+    frame, out = Placed((rows, cols), dt, 0, 0, device, buf), Placed((h, w, 3), np.float32, offset, 0, device)
+    cases.yuv_to_rgb(pf, cr, cp, frame.view(), w, h, out.view())
+    torch.cuda.synchronize()
+    assert out.read().tobytes() == ol.oracle_yuv_to_rgb(pf, cr, cp, buf, w, h).tobytes()
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_NV21, 1, 0), (ol.PF_P010, 0, 2), (ol.PF_UYVY, 1, 2)])
+@pytest.mark.parametrize("w,h", [(2050, 1000), (2047, 1001), (1922, 1080)])
+def test_line_aligned_segments_rgb_to_video(device, pf, cr, cp, w, h):
+    import torch
+    dt = np.uint16 if ol.PF_WIDE[pf] else np.uint8
+    rgb = np.random.RandomState(w).randint(0, 1024 if ol.PF_WIDE[pf] else 256, (h, w, 3)).astype(dt)
+    rows, cols = ol.frame_shape(pf, w + (w & 1), h + (h & 1))
+    if pf in (ol.PF_NV12, ol.PF_NV21, ol.PF_P010):
+        rows = h + (h + 1) // 2
+    start = np.full((rows, cols), 9, dt)
+    frame, src = Placed((rows, cols), dt, 0, 0, device, start), Placed((h, w, 3), dt, 0, 0, device, rgb)
+    cases.rgb_to_yuv(pf, cr, cp, src.view(), frame.view())
+    torch.cuda.synchronize()
+    assert np.array_equal(frame.read(), ol.oracle_rgb_to_yuv(pf, cr, cp, rgb, start))
+
+
+@pytest.mark.parametrize("w,h,offset", [(961, 2101, 4), (1025, 2000, 8)])
+def test_line_aligned_segments_warp(device, w, h, offset):
+    import torch
+    img = np.random.RandomState(w).randint(0, 256, (h, w, 3)).astype(np.uint8)
+    m = np.array([[0.99, -0.12, 4.5], [0.12, 0.99, -3.25]], np.float32)
+    out = Placed((h, w, 3), np.float32, offset, 0, device)
+    cases.warp(torch.from_numpy(img).to(device), m, False, (w, h), out.view())
+    torch.cuda.synchronize()
+    assert out.read().tobytes() == ol.oracle_warp(img, 3, m, (w, h), False).tobytes()
