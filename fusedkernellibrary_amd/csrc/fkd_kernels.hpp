@@ -667,8 +667,7 @@ __device__ __forceinline__ void gather_body(const typename Chain::Params& p, con
 // thread, and handed round through 4 KB of LDS; what depends on the row is worked out once per lane and serves all its
 // pixels.  So the fixed work of a wave is spread over seven pixels per lane instead of four, nearly all of it on the
 // vector unit (the scalar unit is shared by the four SIMDs of a compute unit and was as busy as they were).
-// What the form asks of every plane -- source rows that share their alignment (pitch a multiple of 4), source smaller
-// than 2 GB and at least two columns wide, output plane smaller than 2 GB -- is checked on the host when the parameter
+// What the form asks of every plane -- source smaller than 2 GB and at least two columns wide, output plane smaller than 2 GB -- is checked on the host when the parameter
 // block is made (Chain::finalize_write, bit 0 of Params::reserved); launchers take the tile form when the bit is clear.
 // Taps come through a buffer resource whose extent ends with the image, so windows that reach past the last row read
 // zeros in bytes nobody uses and no lane needs a narrower access; the row is part of the lane's offset.
@@ -748,6 +747,10 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     if constexpr (RZ::kAR != IGNORE_AR) { ox = q.x1; oy = q.y1; }
     const int sw = Back::width(q.back), sh = Back::height(q.back);
     const detail::TapImage image = Back::tap_image_bounded(z, q.back);
+    // Rows that do not share their alignment: a column's entry then holds the byte offset of its first tap, and where in its
+    // dword the window begins is only known together with the row (one more instruction per pixel and line).  Otherwise it
+    // holds the offset of the window.  (wave uniform, as the plane)
+    const bool any_pitch = ((Back::tap_row_offset(1, q.back) - Back::tap_row_offset(0, q.back)) & 3u) != 0u;
     const int steps = (aw + kStripStep - 1) / kStripStep;
     if (steps == 0) return;                                             // no columns: nothing to write (the whole workgroup leaves)
 
@@ -765,7 +768,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         u32 flags = pp.shift | (clamped ? kClamped : 0u);
         if constexpr (RZ::kAR != IGNORE_AR) flags |= (x >= q.x1 && x <= q.x2) ? 0u : kOutsideX;
         detail::u32x4_t e;
-        e.x = __builtin_bit_cast(u32, ax); e.y = __builtin_bit_cast(u32, bx); e.z = pp.off; e.w = flags;
+        e.x = __builtin_bit_cast(u32, ax); e.y = __builtin_bit_cast(u32, bx); e.z = pp.off + pp.shift; e.w = flags;
         return e;
     };
 
@@ -785,17 +788,21 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     if constexpr (RZ::kAR != IGNORE_AR) yin = yc >= q.y1 && yc <= q.y2;
 
     struct StepTaps { detail::u32x4_t e; typename Back::PairBits ab, cd; };
-    auto fetch = [&](StepTaps& s) {
+    auto fetch = [&](StepTaps& s, bool any) {
         // (v_alignbyte_b32 takes the bytes to drop from bits 0-1 of its operand, so the flags may ride along)
         detail::PairPrep pa, pb;
         pa.off = s.e.z + row_a; pa.shift = s.e.w;
         pb.off = s.e.z + row_b; pb.shift = s.e.w;
+        if (any) {
+            pa.shift = pa.off; pa.off &= ~3u;
+            pb.shift = pb.off; pb.off &= ~3u;
+        }
         s.ab = Back::pair_load_prepared(image, 0u, pa, q.back);
         s.cd = Back::pair_load_prepared(image, 0u, pb, q.back);
     };
-    auto request = [&](int k, StepTaps& s) {
+    auto request = [&](int k, StepTaps& s, bool any) {
         s.e = column[g + kStripStep * k];
-        fetch(s);
+        fetch(s, any);
         __builtin_amdgcn_sched_barrier(0);      // the next step's taps leave before anything waits for this step's
     };
     // The taps of step 0 are requested before the table exists, from the lane's own working out of its first column:
@@ -804,7 +811,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     {
         bool unused;
         first.e = column_entry(g, unused);
-        fetch(first);
+        fetch(first, true);                         // (the general form serves both)
     }
 
     // ---- the column table: one column per thread (the workgroup has as many threads as the form has columns).  Columns
@@ -815,6 +822,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     {
         bool clamped = false;
         detail::u32x4_t e = column_entry(t, clamped);
+        e.z &= any_pitch ? ~0u : ~3u;
         if (t >= steps * kStripStep) { e.z = kNoWindow; clamped = false; }
         column[t] = e;
         const bool any = __builtin_amdgcn_ballot_w64(clamped) != 0ull;
@@ -831,9 +839,10 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     const u32 out0 = yvalid ? WP::row_offset(y, oplane) + WP::lane_offset(g, true) : WP::kMaskedOut;
     const bool partial = (aw & (kStripStep - 1)) != 0;             // the last step has columns beyond the output
 
-    auto run = [&](auto static_tag, auto clamp_tag) {
+    auto run = [&](auto static_tag, auto clamp_tag, auto pitch_tag) {
         constexpr bool STATIC = decltype(static_tag)::value != 0;
         constexpr bool CLAMP = decltype(clamp_tag)::value != 0;
+        constexpr bool ANY = decltype(pitch_tag)::value != 0;
         auto produce = [&](int k, const StepTaps& s) {
             // (k is known where the steps are written out: one comparison in four of the steps)
             if ((k == 3 || k == 4) && k == falls[0]) __builtin_amdgcn_s_setprio(2);
@@ -871,20 +880,21 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         // in the instruction's immediate offset, and there is no loop bookkeeping.  The request behind the last step meets
         // a column without a window.
         StepTaps sa = first, sb;
-        request(1, sb);
+        request(1, sb, ANY);
 #pragma unroll
         for (int k = 0; k < kStripMaxSteps; k += 2) {
-            if (k > 0) request(k + 1, sb);
+            if (k > 0) request(k + 1, sb, ANY);
             produce(k, sa);
             if (k + 1 >= steps) return;
-            if (k + 2 < kStripMaxSteps) request(k + 2, sa);
+            if (k + 2 < kStripMaxSteps) request(k + 2, sa, ANY);
             produce(k + 1, sb);
             if (k + 2 >= steps) return;
         }
     };
     auto run_static = [&](auto static_tag) {
-        if (some_clamped) run(static_tag, IntTag<1>{});
-        else run(static_tag, IntTag<0>{});
+        if (any_pitch) run(static_tag, IntTag<1>{}, IntTag<1>{});
+        else if (some_clamped) run(static_tag, IntTag<1>{}, IntTag<0>{});
+        else run(static_tag, IntTag<0>{}, IntTag<0>{});
     };
     if constexpr (Chain::kQuick) {
         if (Chain::ops_static(ops)) { run_static(IntTag<1>{}); return; }
@@ -983,15 +993,16 @@ template <class Chain> constexpr JitMeta jit_meta() {
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) DivergentBody<Chain>::run(p);
     else if constexpr (is_gather_chain<Chain>()) {
+        const bool streamed = (g.n_tiles & kStreamFlag) != 0u;
         if constexpr (strip_capable<Chain>()) {
             if (g.tiles_x == 0u) {                       // wave uniform: the launcher chose the strip form
-                if (g.stream != 0u) strip_body<Chain, true>(p, g.n_tiles);
+                if (streamed) strip_body<Chain, true>(p, g.n_tiles & ~kStreamFlag);
                 else strip_body<Chain, false>(p, g.n_tiles);
                 return;
             }
         }
         if constexpr (writer_streams<Chain>()) {
-            if (g.stream != 0u) { gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, true>(p, g); return; }
+            if (streamed) { gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, true>(p, g); return; }
         }
         gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, false>(p, g);
     }

@@ -37,7 +37,7 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
         if ((unsigned long long)gx * gy > 0x7fffff00ull) return hipErrorInvalidConfiguration;
         if (gx * gy >= kRowsBandBlocks) {
             grid = dim3(rows_band_chunk(gx * gy) * 8u, 1, p.active_z);
-            g = TileGeom{gx, gy, gx * gy * p.active_z, division_magic(gx, gx * gy), 0u};
+            g = TileGeom{gx, gy, gx * gy * p.active_z, division_magic(gx, gx * gy)};
         }
     }
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
@@ -92,7 +92,6 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
     if (info) *info = LaunchInfo{"gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
     if (g.n_tiles == 0) return hipSuccess;
     if (grid.z > 65535u) return hipErrorInvalidConfiguration;
-    g.stream = streamed ? 1u : 0u;
     if (streamed) return launch_by_pointer(&k_gather<Chain, XI, YI, kStreams>, grid, block, stream, p, g);
     return launch_by_pointer(&k_gather<Chain, XI, YI, false>, grid, block, stream, p, g);
 }

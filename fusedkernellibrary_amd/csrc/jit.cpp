@@ -40,6 +40,7 @@ using fkd::JitMeta;
 using fkd::TileGeom;
 using fkd::division_magic;
 using fkd::kRowsBandBlocks;
+using fkd::kStreamFlag;
 using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
@@ -205,8 +206,8 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     unsigned active[4];
     memcpy(active, blob, sizeof(active));   // Chain::Params starts with active_w, active_h, active_z, reserved (bit 0: strip form allowed)
     const JitMeta& m = k->meta;
-    TileGeom g{0, 0, 0, 0, 0};
-    g.stream = (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes ? 1u : 0u;
+    TileGeom g{0, 0, 0, 0};
+    const bool streamed = m.gather && (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes;
     unsigned grid[3], block[3] = {64, 4, 1};
     const char* kind = m.gather ? "gather_jit" : "rows_jit";
     if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {
@@ -217,12 +218,12 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[1] = 1;
         grid[2] = active[2];
         block[1] = m.by;
-        g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]);
+        g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]) | (streamed ? kStreamFlag : 0u);
     } else if (m.gather) {
         const unsigned tw = 64 * m.xi, th = m.by * m.yi;
         g.tiles_x = (active[0] + tw - 1) / tw;
         g.tiles_y = (active[1] + th - 1) / th;
-        g.n_tiles = g.tiles_x * g.tiles_y * active[2];
+        g.n_tiles = streamed ? kStreamFlag : 0u;       // (the kernel counts its tiles itself)
         g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
         grid[0] = (g.tiles_x * g.tiles_y + 7u) / 8u * 8u;
         grid[1] = 1;

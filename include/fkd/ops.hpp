@@ -13,6 +13,9 @@
 #pragma once
 
 #include "types.hpp"
+#if !defined(FKD_DEVICE_CODE)
+#include "launch_info.hpp"
+#endif
 
 namespace fkd {
 
@@ -1578,11 +1581,11 @@ template <class T> struct Read2D {
     static constexpr bool kFiniteTaps = !(__is_same(base_t<T>, f32) || __is_same(base_t<T>, f64));
     static constexpr bool kBoundedOut = small_integer_base<T>();
     FKD_NAME("Read2D<" + type_name<T>() + ">")
-    // What the strip form of the bilinear kernel asks of a source image (checked on the host, see Chain::finalize): rows
-    // that share their alignment, byte offsets below 2 GB (the offset 2 GB itself marks a column without a window), two
-    // columns.
-    FKD_HD static bool strip_ok(const Params& p) {
-        return p.pitch % 4 == 0 && size_t(p.pitch) * p.height < 0x7ffffff0ull && p.width >= 2 && p.height >= 1;
+    // What the strip form of the bilinear kernel asks of a source image (checked on the host, see Chain::finalize_write):
+    // byte offsets below 2 GB (the offset 2 GB itself marks a column without a window), two columns and, but for any_pitch,
+    // rows that share their alignment.
+    FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
+        return (any_pitch || p.pitch % 4 == 0) && size_t(p.pitch) * p.height < 0x7ffffff0ull && p.width >= 2 && p.height >= 1;
     }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
@@ -2071,8 +2074,8 @@ template <class Back> struct Crop {
     static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>();
     FKD_NAME("Crop<" + Back::name() + ">")
-    FKD_HD static bool strip_ok(const Params& p) {
-        if constexpr (requires { Back::strip_ok(p.back); }) return p.w >= 2 && p.h >= 1 && Back::strip_ok(p.back); else return false;
+    FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
+        if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return p.w >= 2 && p.h >= 1 && Back::strip_ok(p.back, any_pitch); else return false;
     }
 #if defined(FKD_EXEC_CODE)
     static constexpr bool kFiniteTaps = finite_taps<Back>();
@@ -2257,8 +2260,8 @@ template <class Back, class... Ops> struct FusedRead {
     static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>() && (finite_map<Ops>() && ...);
     FKD_NAME("FusedRead<" + Back::name() + OpList<Ops...>::names() + ">")
-    FKD_HD static bool strip_ok(const Params& p) {
-        if constexpr (requires { Back::strip_ok(p.back); }) return Back::strip_ok(p.back); else return false;
+    FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
+        if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return Back::strip_ok(p.back, any_pitch); else return false;
     }
 #if defined(FKD_EXEC_CODE)
     static constexpr bool kFiniteTaps = finite_taps<Back>() && (finite_map<Ops>() && ...);
@@ -2350,8 +2353,8 @@ template <int AR, class Back> struct ResizeLinear {
     static constexpr bool kBoundedOut = AR == IGNORE_AR && bounded_out<Back>();   // a letterbox colour is a run-time value
     using BackOp = Back;
     FKD_NAME("ResizeLinear<" + istr(AR) + "," + Back::name() + ">")
-    FKD_HD static bool strip_ok(const Params& p, u32 = 1u) {
-        if constexpr (requires { Back::strip_ok(p.back); }) return Back::strip_ok(p.back); else return false;
+    FKD_HD static bool strip_ok(const Params& p, bool any_pitch, u32 = 1u) {
+        if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return Back::strip_ok(p.back, any_pitch); else return false;
     }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return p.dst_w; }
@@ -2702,9 +2705,9 @@ template <int N, class PlaneOp> struct BatchRead {
     static constexpr int kXGroup = x_group<PlaneOp>();
     static constexpr bool kBoundedOut = bounded_out<PlaneOp>();
     FKD_NAME("BatchRead<" + istr(N) + "," + PlaneOp::name() + ">")
-    FKD_HD static bool strip_ok(const Params& p, u32 planes) {
-        if constexpr (requires { PlaneOp::strip_ok(p.plane[0]); }) {
-            for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::strip_ok(p.plane[z])) return false;
+    FKD_HD static bool strip_ok(const Params& p, bool any_pitch, u32 planes) {
+        if constexpr (requires { PlaneOp::strip_ok(p.plane[0], any_pitch); }) {
+            for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::strip_ok(p.plane[z], any_pitch)) return false;
             return planes <= u32(N);
         } else {
             return false;
@@ -3306,6 +3309,24 @@ template <class I, class P, class O> struct IsSubOp<Sub<I, P, O>> { static const
 template <class T> struct IsDivOp { static constexpr bool value = false; };
 template <class I, class P, class O> struct IsDivOp<Div<I, P, O>> { static constexpr bool value = Div<I, P, O>::kReciprocal; };
 
+#if !defined(FKD_DEVICE_CODE)
+// Which of the two forms of the bilinear kernel a launch takes that the strip form could serve.  us, tile form / strip form, 64
+// crops of a 1280x853 image unless noted (8 crops: four launches):
+//   outputs stored past the last-level cache whose rows are no whole lines: a strip's 128-byte stores then end in partial lines,
+//   which leave the chip one by one: 200x640 23.7 / 45.3, 225x640 34.4 / 74.3 (whole lines: 224x640 23.3 / 19.9, 160x640 22.4 / 15.5);
+//   six steps and more with rows that are no whole 32-byte sectors: 225x200 10.9 / 11.9, 250x200 11.4 / 12.4 (200x200 10.3 / 8.9);
+//   rows that do not share their alignment (width 1279): 160x200 10.3 / 7.0, 224x200 10.5 / 8.4, 224x640 24.2 / 20.2, 8 crops to
+//   100x200 14.9 / 13.3; but with six steps and more and less than a workgroup per compute unit a strip's row is one wave's alone:
+//   8 crops to 200x60 13.7 / 15.6, to 224x60 13.8 / 15.6.
+inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes) {
+    const unsigned long long pixels = (unsigned long long)w * h * planes, workgroups = (unsigned long long)((h + 7u) / 8u) * planes;
+    if (pixels * value_bytes > kStreamOutputBytes && w % 32u != 0u) return false;
+    const bool many_steps = w > 160u, sectors = w % 8u == 0u;
+    if (many_steps && !sectors && pixels >= 1200000u) return false;
+    return !any_pitch || (pixels >= 40000u && (!many_steps || (sectors && workgroups >= 256u)));
+}
+#endif
+
 template <class R, class Ops, class W> struct Chain;
 template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     using Read = R;
@@ -3358,15 +3379,17 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     static void finalize(Params& p) { finalize_from<0>(p); }
     // Host, once read AND write are filled in: bit 0 of `reserved` tells the launcher that every active plane meets what
     // the strip form of the bilinear kernel asks of its source and destination (that form has no other way to decline a
-    // plane).  A parameter block that never came through here keeps the bit clear and gets the tile form.
+    // plane) and that the launch is better off with it (strip_pays).  A parameter block that never came through here keeps the bit clear and gets the tile form.
     // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
     // phase_bound_for).
     static constexpr u32 kStripChecked = 1u;
     static void finalize_write(Params& p) {
         if constexpr (any_x<R>() && has_row_phase<W>())
             p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
-        if constexpr (requires { R::strip_ok(p.read, p.active_z); W::strip_ok(p.write); }) {
-            if (R::strip_ok(p.read, p.active_z) && W::strip_ok(p.write)) p.reserved |= kStripChecked;
+        if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {
+            const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);
+            if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value)) && W::strip_ok(p.write) &&
+                (!any_pitch || R::strip_ok(p.read, true, p.active_z))) p.reserved |= kStripChecked;
         }
     }
 #endif

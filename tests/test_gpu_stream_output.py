@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dst,kernel", [((293, 298), None), ((293, 299), None),      # 67 057 152 and 67 282 176 bytes: ragged rows
-                                        ((251, 348), "strip"), ((251, 349), "strip")])
+                                        ((251, 348), "gather"), ((251, 349), "gather"),
+                                        ((224, 390), "strip"), ((224, 391), "strip")])     # 67 092 480 and 67 264 512 bytes: rows of whole lines
 def test_batches_around_the_limit(dst, kernel):
     import torch
     c = wl.config3(width=640 if kernel else 641, height=359, min_side=2, span=340)      # rows that share their alignment, or not

@@ -1,0 +1,87 @@
+"""The strip form of the bilinear kernel on images whose rows do not share their alignment: bit for bit the oracle's result and the
+tile form's, at every alignment of the image, with enlarging planes (columns clamped to the last one), letterboxes and crops that
+end with the image; and, on the CPU, the bytes its tap windows touch."""
+import numpy as np
+import pytest
+
+import fkl_cases as cases
+import oracle_lib as ol
+import workloads as wl
+
+
+def test_windows_stay_inside_the_dwords_of_the_image():
+    """Read2D<uchar3>, pitch % 4 != 0: window start (column + row bytes) & ~3 from the resource's base, three dwords, those beyond
+    the extent reading zeros; the six bytes of the two taps are always inside it and always inside the window."""
+    for w in (2, 3, 5, 7, 333):
+        for h in (1, 2, 3):
+            for lo in range(4):
+                for pitch in (3 * w, 3 * w + 1, 3 * w + 2):
+                    if pitch % 4 == 0:
+                        continue
+                    extent = (lo + pitch * (h - 1) + 3 * w + 3) & ~3
+                    for y in range(h):
+                        for x1 in range(w - 1):
+                            t = (lo + 3 * x1) + y * pitch
+                            start, drop = t & ~3, t & 3
+                            assert start >= 0 and drop + 6 <= 12 and t + 6 <= extent, (w, h, lo, pitch, x1, y)
+
+
+def _view(img, offset, pad, device):
+    import torch
+    h, w = img.shape[:2]
+    pitch = 3 * w + pad
+    host = np.zeros(offset + pitch * h + 16, np.uint8)
+    np.lib.stride_tricks.as_strided(host[offset:], (h, 3 * w), (pitch, 1))[:] = img.reshape(h, 3 * w)
+    return torch.from_numpy(host).to(device)[offset:].as_strided((h, w, 3), (pitch, 3, 1), offset)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,dst,form", [(64, (224, 224), "strip"), (8, (224, 264), "strip"), (64, (256, 61), "strip"), (8, (97, 130), "strip"),
+                                            (64, (33, 190), "strip"), (8, (160, 32), "strip"), (8, (64, 40), "gather"), (8, (224, 61), "gather"),
+                                            (64, (225, 61), "gather")])
+@pytest.mark.parametrize("w,offset,pad", [(333, 0, 0), (1279, 1, 0), (334, 3, 1), (335, 2, 2), (253, 0, 7)])
+def test_crops(device, batch, dst, form, w, offset, pad):
+    import torch
+    from fusedkernellibrary_amd import last_launch, lib
+    rng = np.random.RandomState(w + batch + dst[0])
+    h = 201
+    img = rng.randint(0, 256, (h, w, 3)).astype(np.uint8)
+    src = _view(img, offset, pad, device)
+    rects = np.zeros((batch, 4), np.int32)
+    for i in range(batch):
+        cw, ch = rng.randint(2, w + 1), rng.randint(1, h + 1)
+        rects[i] = (rng.randint(0, w - cw + 1), rng.randint(0, h - ch + 1), cw, ch)
+    rects[0], rects[1], rects[2] = (0, 0, w, h), (w - 2, h - 2, 2, 2), (w - 40, h - 1, 40, 1)
+    got = []
+    for on in (1, 0):
+        lib().fklhip_strip_form(on)
+        try:
+            out = torch.full((batch, 3, dst[1], dst[0]), -7.0, dtype=torch.float32, device=device)
+            cases.crop_resize_norm_split(src, rects, dst, wl.C3_MEAN, wl.C3_STD, out)
+            torch.cuda.synchronize()
+            assert last_launch()["kernel"] == (form if on else "gather")
+            got.append(out.cpu().numpy())
+        finally:
+            lib().fklhip_strip_form(1)
+    want = ol.oracle_crop_resize_norm_split(img, rects, dst, wl.C3_MEAN, wl.C3_STD)
+    assert got[0].tobytes() == want.tobytes() and got[1].tobytes() == want.tobytes()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,offset", [(321, 0), (322, 1), (323, 2)])
+def test_letterboxes_compiled_on_first_use(device, w, offset):
+    import torch
+    from fusedkernellibrary_amd import last_launch
+    rng = np.random.RandomState(w)
+    img = rng.randint(0, 256, (200, w, 3)).astype(np.uint8)
+    rects = np.array([[10, 20, 300, 60], [40, 0, 50, 200], [w - 120, 80, 120, 120]], np.int32)
+    bg, mul = np.array([0.25, 128.5, 255.0], np.float32), np.array([0.5, 2.0, 1.0 / 255.0], np.float32)
+    dst = (160, 300)
+    out = torch.full((3, 3, dst[1], dst[0]), -7.0, dtype=torch.float32, device=device)
+    cases.uncompiled_letterbox_split_b3(_view(img, offset, 0, device), rects, dst, bg, mul, out)
+    torch.cuda.synchronize()
+    assert last_launch()["kernel"] == "strip_jit"
+    want = np.zeros((3, 3, dst[1], dst[0]), np.float32)
+    reads = [ol.read_2d(img, 3, crop=rects[i], resize=dst, ar=ol.PRESERVE_AR, bg=tuple(bg) + (0.0,)) for i in range(3)]
+    ol.execute(reads, [ol.op(ol.MUL, tuple(mul) + (0.0,))], [ol.write(ol.TENSOR_SPLIT, want, 3, dst[0], dst[1], 3, 3)])
+    assert out.cpu().numpy().tobytes() == want.tobytes()
