@@ -749,8 +749,10 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     const detail::TapImage image = Back::tap_image_bounded(z, q.back);
     // Rows that do not share their alignment: a column's entry then holds the byte offset of its first tap, and where in its
     // dword the window begins is only known together with the row (one more instruction per pixel and line).  Otherwise it
-    // holds the offset of the window.  (wave uniform, as the plane)
-    const bool any_pitch = ((Back::tap_row_offset(1, q.back) - Back::tap_row_offset(0, q.back)) & 3u) != 0u;
+    // holds the offset of the window.  (wave uniform, as the plane.)  For pixels of whole dwords the two are the same: their
+    // windows begin with the first tap, whatever its address.
+    using Window = typename Back::PairBits;
+    const bool any_pitch = Window::kShift && ((Back::tap_row_offset(1, q.back) - Back::tap_row_offset(0, q.back)) & 3u) != 0u;
     const int steps = (aw + kStripStep - 1) / kStripStep;
     if (steps == 0) return;                                             // no columns: nothing to write (the whole workgroup leaves)
 
@@ -794,8 +796,8 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         pa.off = s.e.z + row_a; pa.shift = s.e.w;
         pb.off = s.e.z + row_b; pb.shift = s.e.w;
         if (any) {
-            pa.shift = pa.off; pa.off &= ~3u;
-            pb.shift = pb.off; pb.off &= ~3u;
+            pa = detail::pair_window_at<Window>(pa.off);
+            pb = detail::pair_window_at<Window>(pb.off);
         }
         s.ab = Back::pair_load_prepared(image, 0u, pa, q.back);
         s.cd = Back::pair_load_prepared(image, 0u, pb, q.back);
@@ -822,7 +824,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     {
         bool clamped = false;
         detail::u32x4_t e = column_entry(t, clamped);
-        e.z &= any_pitch ? ~0u : ~3u;
+        if constexpr (Window::kShift) e.z &= any_pitch ? ~0u : ~3u;
         if (t >= steps * kStripStep) { e.z = kNoWindow; clamped = false; }
         column[t] = e;
         const bool any = __builtin_amdgcn_ballot_w64(clamped) != 0ull;

@@ -56,6 +56,26 @@ template <class Op> constexpr bool finite_map() {
 template <class R> constexpr bool bounded_out() {
     if constexpr (requires { R::kBoundedOut; }) return R::kBoundedOut; else return false;
 }
+// The window in which two consecutive elements are fetched (PairWindow): elements of no whole dwords come as whole dwords from
+// the boundary at or below the first one and are shifted into place, elements of whole dwords come from exactly where they begin.
+namespace detail {
+template <class T> struct PairWindowShape {
+    static constexpr int kBytes = 2 * int(sizeof(T));
+    static constexpr bool kShift = sizeof(T) % 4 != 0;
+    static constexpr int kOut = (kBytes + 3) / 4;                          // dwords holding the aligned pair
+    static constexpr int kWords = kShift ? (kBytes + 3 + 3) / 4 : kOut;    // dwords fetched
+    static constexpr bool kSupported = kWords <= 4;
+};
+struct PairPrep { u32 off, shift; };
+// Where the window of a pair begins that starts `at` bytes into an image (counted from a dword boundary), and in bits 0-1 of
+// `shift` the bytes to drop from it (v_alignbyte_b32 looks at no others).
+template <class Shape> FKD_HD PairPrep pair_window_at(u32 at) {
+    if constexpr (Shape::kShift) return PairPrep{at & ~3u, at}; else return PairPrep{at, 0u};
+}
+// The extent, counted from the dword boundary `lo` bytes before an image of `bytes` bytes, that ends with the dword of its last byte.
+FKD_HD u32 tap_extent(size_t bytes, u32 lo) { return (u32(bytes) + lo + 3u) & ~3u; }
+} // namespace detail
+
 // any_x<R>: read R's exec_row may start at any element of the row, not only at a multiple of the run's length.
 template <class R> constexpr bool any_x() {
     if constexpr (requires { R::kAnyX; }) return R::kAnyX; else return false;
@@ -545,14 +565,10 @@ template <int K, class T, int V> FKD_DEV T run_value(const RunBits<T, V>& e) {  
 // below the first element (at most 3 bytes early: same dword, so same page, as a byte that is needed) and the two
 // elements are shifted into place with v_alignbyte_b32 where they are used.  The window may end up to 6 bytes past
 // the second element; the caller guarantees those bytes are inside the allocation.
-template <class T> struct PairWindow {
+// (its measures and where it begins: PairWindowShape, pair_window_at)
+template <class T> struct PairWindow : PairWindowShape<T> {
     static_assert(sizeof(T) == sizeof(base_t<T>) * cn_v<T>, "elements are packed channel arrays");
-    static constexpr int kBytes = 2 * int(sizeof(T));
-    static constexpr bool kShift = sizeof(T) % 4 != 0;
-    static constexpr int kOut = (kBytes + 3) / 4;                          // dwords holding the aligned pair
-    static constexpr int kWords = kShift ? (kBytes + 3 + 3) / 4 : kOut;    // dwords fetched
-    static constexpr bool kSupported = kWords <= 4;
-    u32 w[kWords];
+    u32 w[PairWindowShape<T>::kWords];
     u32 shift;      // bytes between the window start and the first element
 };
 template <class T> FKD_DEV PairWindow<T> load_pair_window(const char* row, u32 off) {
@@ -583,7 +599,6 @@ template <class T> FKD_DEV PairWindow<T> load_pair_window(const char* row, u32 o
 // per-lane one (window start and bytes to drop, prepared once per column because they no longer depend on the row), so
 // a tap costs one buffer_load with no address arithmetic at all.  The resource's size field is left open: staying
 // inside the allocation is the caller's business exactly as for the global-memory loads.
-struct PairPrep { u32 off, shift; };
 template <class B> constexpr bool tap_prepared() {
     if constexpr (requires { B::kTapPrepared; }) return B::kTapPrepared; else return false;
 }
@@ -606,7 +621,7 @@ FKD_DEV TapImage make_tap_image(const void* data) {
 FKD_DEV TapImage make_tap_image(const void* data, size_t bytes) {
     TapImage im;
     im.lo = u32(reinterpret_cast<uintptr_t>(data)) & 3u;
-    const u32 extent = (u32(bytes) + im.lo + 3u) & ~3u;
+    const u32 extent = tap_extent(bytes, im.lo);
     im.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(data)) - im.lo, 0, extent, 0x00020000);
     return im;
 }

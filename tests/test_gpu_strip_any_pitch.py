@@ -7,6 +7,7 @@ import pytest
 import fkl_cases as cases
 import oracle_lib as ol
 import workloads as wl
+from test_gpu_any_alignment import Placed
 
 
 def test_windows_stay_inside_the_dwords_of_the_image():
@@ -85,3 +86,35 @@ def test_letterboxes_compiled_on_first_use(device, w, offset):
     reads = [ol.read_2d(img, 3, crop=rects[i], resize=dst, ar=ol.PRESERVE_AR, bg=tuple(bg) + (0.0,)) for i in range(3)]
     ol.execute(reads, [ol.op(ol.MUL, tuple(mul) + (0.0,))], [ol.write(ol.TENSOR_SPLIT, want, 3, dst[0], dst[1], 3, 3)])
     assert out.cpu().numpy().tobytes() == want.tobytes()
+
+
+# Pixels whose tap pair is shifted into place inside its window (2 and 6 bytes) and pixels of whole dwords, whose pair is fetched
+# from exactly where it begins: every address and pitch that leaves the samples aligned.
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,cn,dtype", [(0, 2, np.uint8), (1, 4, np.uint8), (2, 3, np.uint16)])
+@pytest.mark.parametrize("w,dst,rect", [(201, (160, 256), (3, 1, 190, 90)), (202, (97, 430), (0, 0, 202, 110)),
+                                        (203, (64, 640), (200, 108, 3, 2))])             # the last one enlarges the image's last pixels
+def test_other_pixel_types(device, kind, cn, dtype, w, dst, rect):
+    import torch
+    from fusedkernellibrary_amd import last_launch, lib
+    size, h = np.dtype(dtype).itemsize, 110
+    img = np.random.RandomState(60 + kind).randint(0, 1024 if size == 2 else 256, (h, w, cn)).astype(dtype)
+    want = np.zeros((cn, dst[1], dst[0]), np.float32)
+    ol.execute([ol.read_2d(img, cn, crop=rect, resize=dst, ar=ol.IGNORE_AR)], [ol.op(ol.MUL, (0.5, 0.5, 0.5, 0.5))],
+               [ol.write(ol.TENSOR_SPLIT, want, cn, dst[0], dst[1], 1, cn)])
+    wrong = []
+    for offset in range(0, 4, size):
+        for pad in range(0, 4, size):
+            src = Placed(img.shape, dtype, offset, pad, device, img)
+            for on in (1, 0):
+                old = lib().fklhip_strip_form(on)
+                try:
+                    out = torch.full((cn, dst[1], dst[0]), -7.0, dtype=torch.float32, device=device)
+                    cases.uncompiled_resize_split(kind, src.view(), rect, dst, 0.5, out)
+                    torch.cuda.synchronize()
+                    assert last_launch()["kernel"] == ("strip_jit" if on else "gather_jit")
+                finally:
+                    lib().fklhip_strip_form(old)
+                if out.cpu().numpy().tobytes() != want.tobytes():
+                    wrong.append((offset, src.pitch, on))
+    assert not wrong
