@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52070000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "f1407668cd2db1639747da3edac37c7d380582c442ca71595f08ac621d6b083e"
+TRAFFIC_C3_SOURCES_SHA256 = "505161ae04a392ebcd6308c828773052348a5c1c7d9c5002918334391cba3715"
 
 
 def device_sources_sha256():
