@@ -2550,7 +2550,7 @@ template <int WT, class Back> struct Warp {
 #if defined(FKD_DEVICE_CODE)
     // Images below 4 GB (wave uniform): the two line-pair taps through a buffer resource that ends with the image.
     // Row and column are one 32-bit byte offset per lane (no 64-bit address arithmetic on the vector unit), the
-    // window starts at the dword at or below it, and a window that reaches past the image's last row reads zeros
+    // window starts where pair_window_at says, and a window that reaches past the image's last row reads zeros
     // in bytes nobody uses, so no wave needs the element-wise path.  Lanes whose source point lies outside take
     // the taps of pixel (0, 0) and drop them, so that no load waits behind a branch.  In two halves, so that a thread
     // with several elements has the taps of all of them on their way before it blends the first.
@@ -2573,11 +2573,12 @@ template <int WT, class Back> struct Warp {
         t.edge = x1 >= sw - 1;                        // x1 + 1 is past the line: both taps are the last pixel
         t.xp = t.edge ? sw - 2 : x1;
         const detail::TapImage image = Back::tap_image_bounded(z, p.back);
+        using Window = typename detail::pair_bits_of<Back>::type;
         const detail::PairPrep col = Back::pair_prepare(image, t.xp, p.back);
         const u32 column_bytes = col.off + col.shift;             // from the resource's base
         const u32 ta = column_bytes + Back::tap_row_offset(y1, p.back), tb = column_bytes + Back::tap_row_offset(y2r, p.back);
-        t.wa = Back::pair_load_prepared(image, 0u, detail::PairPrep{ta & ~3u, ta & 3u}, p.back);
-        t.wb = Back::pair_load_prepared(image, 0u, detail::PairPrep{tb & ~3u, tb & 3u}, p.back);
+        t.wa = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(ta), p.back);
+        t.wb = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(tb), p.back);
         return t;
     }
     FKD_DEV static Out bounded_blend(const BoundedTaps& t, const Params& p) {

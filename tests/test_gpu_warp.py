@@ -7,6 +7,7 @@ import pytest
 
 import oracle_lib as ol
 import fkl_cases as cases
+from test_gpu_any_alignment import Placed
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,27 @@ def test_warp_other_pixel_types(device, matrix, persp, dtype, cn):
         torch.cuda.synchronize()
         want = ol.oracle_warp(img, cn, matrix, dst, persp)
         assert out.cpu().numpy().tobytes() == want.tobytes(), dst
+
+
+@pytest.mark.parametrize("dtype,cn", [(np.uint8, 3), (np.uint8, 4), (np.uint16, 3), (np.uint8, 1)])
+@pytest.mark.parametrize("matrix,persp", [(AFFINE, False), (PERSPECTIVE, True)])
+def test_sources_at_every_address(device, matrix, persp, dtype, cn):
+    """Every address and pitch of the source that leaves its samples aligned: windows of pixels of no whole dwords are rounded
+    down to a dword and shifted, those of uchar4 begin exactly at the tap."""
+    import torch
+    size, dst = np.dtype(dtype).itemsize, (131, 90)
+    img = np.random.RandomState(26).randint(0, 1000 if size == 2 else 256, (90, 131, cn) if cn > 1 else (90, 131)).astype(dtype)
+    want = ol.oracle_warp(img, cn, matrix, dst, persp)
+    wrong = []
+    for offset in range(0, 4, size):
+        for pad in range(0, 4, size):
+            src = Placed(img.shape, dtype, offset, pad, device, img)
+            out = torch.full(want.shape, -1.0, dtype=torch.float32, device=device)
+            cases.warp(src.view(), matrix, persp, dst, out, kind=None if (cn, size) == (3, 1) else ol.warp_kind(dtype, cn))
+            torch.cuda.synchronize()
+            if out.cpu().numpy().tobytes() != want.tobytes():
+                wrong.append((offset, src.pitch))
+    assert not wrong
 
 
 def test_lanes_outside_the_source_ignore_what_their_stand_in_pixel_holds(device):
