@@ -190,34 +190,20 @@ FKD_DEV bool none_in_wave(bool flag) { return __builtin_amdgcn_ballot_w64(flag) 
 template <class T> FKD_DEV const FKD_GLOBAL T* gconst(const void* p) { return (const FKD_GLOBAL T*)p; }
 template <class T> FKD_DEV FKD_GLOBAL T* gmut(void* p) { return (FKD_GLOBAL T*)p; }
 
-// Dword vectors that may sit at any dword-aligned address: one global_load/store_dwordx{2,3,4} each.
 typedef u32 u32x2_t __attribute__((ext_vector_type(2)));
 typedef u32 u32x3_t __attribute__((ext_vector_type(3)));
 typedef u32 u32x4_t __attribute__((ext_vector_type(4)));
-typedef u32x2_t u32x2_a4 __attribute__((aligned(4)));
-typedef u32x3_t u32x3_a4 __attribute__((aligned(4)));
-typedef u32x4_t u32x4_a4 __attribute__((aligned(4)));
-// The same at any byte address: the hardware takes global accesses of any width at any byte alignment.
-typedef u16 u16_a1 __attribute__((aligned(1)));
-typedef u32 u32_a1 __attribute__((aligned(1)));
-typedef u32x2_t u32x2_a1 __attribute__((aligned(1)));
-typedef u32x3_t u32x3_a1 __attribute__((aligned(1)));
-typedef u32x4_t u32x4_a1 __attribute__((aligned(1)));
-template <int N, bool ALIGNED> struct DwordsAt;      // N dwords at a dword boundary (ALIGNED) or at any byte
-template <> struct DwordsAt<1, true> { using type = u32; };
-template <> struct DwordsAt<2, true> { using type = u32x2_a4; };
-template <> struct DwordsAt<3, true> { using type = u32x3_a4; };
-template <> struct DwordsAt<4, true> { using type = u32x4_a4; };
-template <> struct DwordsAt<1, false> { using type = u32_a1; };
-template <> struct DwordsAt<2, false> { using type = u32x2_a1; };
-template <> struct DwordsAt<3, false> { using type = u32x3_a1; };
-template <> struct DwordsAt<4, false> { using type = u32x4_a1; };
-template <int N, bool ALIGNED> using dwords_at = typename DwordsAt<N, ALIGNED>::type;
 
-// One whole-dword store (1-4 dwords).  Output is written once and not read again by the kernel, so the stores carry
+// Accesses to dword vectors at dword boundaries or at any byte (the hardware takes global accesses of any width at any byte
+// alignment): ALIGN is what is known about p.  It is declared on a typedef beside the access, because an `aligned` attribute
+// is dropped from a typedef that travels as a template argument.
+// One store of 1-4 whole dwords (or one element).  Output is written once and not read again by the kernel, so the stores carry
 // the non-temporal hint: the L2s then hand the lines on early instead of keeping them dirty until the kernel ends,
 // when all of them would have to be written back at once (a 3840x2160 float copy: 10.6 -> 9.9 us).
-template <class Q> FKD_DEV void gstore(FKD_GLOBAL Q* p, const Q& v) { __builtin_nontemporal_store(v, p); }
+template <int ALIGN, class Q, class P> FKD_DEV void gstore(P* p, const Q& v) {
+    typedef Q At __attribute__((aligned(ALIGN)));
+    __builtin_nontemporal_store(v, (FKD_GLOBAL At*)p);
+}
 // One element of 4 or 8 bytes written through the L2 (a relaxed store at system scope: global_store ... sc0 sc1), for
 // writers whose lanes each store single elements: the planar writer of the bilinear kernel runs configuration 3 in
 // 11.1 us with these, 11.5 us with the non-temporal hint and 12.9 us with plain stores.  Other sizes take gstore.
@@ -227,9 +213,10 @@ template <class B> FKD_DEV void gstore_through(FKD_GLOBAL B* p, const B& v) {
     else *p = v;
 }
 // One whole-dword load of a row run; STREAM marks data that no cache can hold until its next use (see the rows kernel).
-template <bool STREAM, class Q> FKD_DEV Q gload_run(const FKD_GLOBAL Q* p) {
-    if constexpr (STREAM) return __builtin_nontemporal_load(p);
-    else return *p;
+template <class Q, int ALIGN, bool STREAM = false, class P> FKD_DEV Q gload(P* p) {
+    typedef Q At __attribute__((aligned(ALIGN)));
+    if constexpr (STREAM) return __builtin_nontemporal_load((const FKD_GLOBAL At*)p);
+    else return *(const FKD_GLOBAL At*)p;
 }
 template <class T> FKD_DEV T load_elem(const T* p) {
     T v;
@@ -246,7 +233,7 @@ template <class T> FKD_DEV T load_elem(const T* p) {
 }
 template <class T> FKD_DEV void store_elem(T* p, const T& v) {
     if constexpr (cn_v<T> == 1) {
-        if constexpr (sizeof(T) == 4) gstore(gmut<T>(p), v); else *gmut<T>(p) = v;
+        if constexpr (sizeof(T) == 4) gstore<alignof(T)>(p, v); else *gmut<T>(p) = v;
     } else {
         FKD_GLOBAL base_t<T>* b = gmut<base_t<T>>(p);
         b[0] = chan<0>(v);
@@ -257,38 +244,40 @@ template <class T> FKD_DEV void store_elem(T* p, const T& v) {
 }
 
 template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_words(const void* p, u32 (&w)[W]) {
+    constexpr int ALIGN = ALIGNED ? 4 : 1;
     static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
-        w[0] = gload_run<STREAM>(gconst<dwords_at<1, ALIGNED>>(p));
+        w[0] = gload<u32, ALIGN, STREAM>(p);
     } else if constexpr (W == 2) {
-        const u32x2_t v = gload_run<STREAM>(gconst<dwords_at<2, ALIGNED>>(p));
+        const u32x2_t v = gload<u32x2_t, ALIGN, STREAM>(p);
         w[0] = v.x; w[1] = v.y;
     } else if constexpr (W == 3) {
-        const u32x3_t v = gload_run<STREAM>(gconst<dwords_at<3, ALIGNED>>(p));
+        const u32x3_t v = gload<u32x3_t, ALIGN, STREAM>(p);
         w[0] = v.x; w[1] = v.y; w[2] = v.z;
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
-            const u32x4_t v = gload_run<STREAM>(gconst<dwords_at<4, ALIGNED>>(p) + i);
+            const u32x4_t v = gload<u32x4_t, ALIGN, STREAM>(gconst<u32x4_t>(p) + i);
             w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
         }
     }
 }
 template <int W, bool ALIGNED = true> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
+    constexpr int ALIGN = ALIGNED ? 4 : 1;
     static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
-        gstore<dwords_at<1, ALIGNED>>(gmut<dwords_at<1, ALIGNED>>(p), w[0]);
+        gstore<ALIGN>(p, w[0]);
     } else if constexpr (W == 2) {
-        dwords_at<2, ALIGNED> v; v.x = w[0]; v.y = w[1];
-        gstore(gmut<dwords_at<2, ALIGNED>>(p), v);
+        u32x2_t v; v.x = w[0]; v.y = w[1];
+        gstore<ALIGN>(p, v);
     } else if constexpr (W == 3) {
-        dwords_at<3, ALIGNED> v; v.x = w[0]; v.y = w[1]; v.z = w[2];
-        gstore(gmut<dwords_at<3, ALIGNED>>(p), v);
+        u32x3_t v; v.x = w[0]; v.y = w[1]; v.z = w[2];
+        gstore<ALIGN>(p, v);
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
-            dwords_at<4, ALIGNED> v; v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
-            gstore(gmut<dwords_at<4, ALIGNED>>(p) + i, v);
+            u32x4_t v; v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
+            gstore<ALIGN>(gmut<u32x4_t>(p) + i, v);
         }
     }
 }
@@ -394,7 +383,7 @@ template <int W, bool STREAM, bool ALIGNED> FKD_DEV void load_words_wave(const v
     const char* seg = reinterpret_cast<const char*>(p) - size_t(lane) * (W * 4);
     u32x4_t q[W / 4];
 #pragma unroll
-    for (int k = 0; k < W / 4; ++k) q[k] = gload_run<STREAM>(gconst<dwords_at<4, ALIGNED>>(seg + k * 1024 + lane * 16));
+    for (int k = 0; k < W / 4; ++k) q[k] = gload<u32x4_t, ALIGNED ? 4 : 1, STREAM>(seg + k * 1024 + lane * 16);
     wave_exchange_fence();   // the previous exchange's reads come first
 #pragma unroll
     for (int k = 0; k < W / 4; ++k) *reinterpret_cast<u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)) = q[k];
@@ -418,7 +407,7 @@ template <int W, bool ALIGNED> FKD_DEV void store_words_wave(void* p, const u32 
     wave_exchange_fence();
 #pragma unroll
     for (int k = 0; k < W / 4; ++k)
-        gstore<dwords_at<4, ALIGNED>>(gmut<dwords_at<4, ALIGNED>>(seg + k * 1024 + lane * 16), *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
+        gstore<ALIGNED ? 4 : 1>(seg + k * 1024 + lane * 16, *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
 }
 
 template <class T, int V, int MODE_BITS> FKD_DEV void load_run(const T* p, Slot<T> (&out)[V]) {
@@ -494,11 +483,11 @@ template <class T, int V> FKD_DEV void store_run_edge(T* row, int seg, int x, in
         const int f = k * 256 + lane * 4;
         const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(f)));
         if (f >= lo && f + 4 <= hi) {
-            gstore<dwords_at<4, false>>(gmut<dwords_at<4, false>>(base + f * 4), v);
+            gstore<1>(base + f * 4, v);
         } else {
             const u32 d[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) if (f + i >= lo && f + i < hi) gstore<u32_a1>(gmut<u32_a1>(base + (f + i) * 4), d[i]);
+            for (int i = 0; i < 4; ++i) if (f + i >= lo && f + i < hi) gstore<1>(base + (f + i) * 4, d[i]);
         }
     }
 }
@@ -530,20 +519,20 @@ template <class T, int V, bool OVERREAD> FKD_DEV RunBits<T, V> load_bits_at(cons
     if constexpr (n == 1) {
         e.w[0] = u32(*gconst<u8>(a));
     } else if constexpr (n == 2) {
-        e.w[0] = u32(*gconst<u16_a1>(a));
+        e.w[0] = u32(gload<u16, 1>(a));
     } else if constexpr (n > 16 || (overread_bytes<T, V>() > 0 && !OVERREAD)) {
         Slot<T> run[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) run[i].v = load_elem(reinterpret_cast<const T*>(a) + i);
         pack_words<T, V, W>(run, e.w);
     } else if constexpr (W == 1) {
-        e.w[0] = *gconst<u32_a1>(a);
+        e.w[0] = gload<u32, 1>(a);
     } else if constexpr (W == 2) {
-        const u32x2_t v = *gconst<u32x2_a1>(a); e.w[0] = v.x; e.w[1] = v.y;
+        const u32x2_t v = gload<u32x2_t, 1>(a); e.w[0] = v.x; e.w[1] = v.y;
     } else if constexpr (W == 3) {
-        const u32x3_t v = *gconst<u32x3_a1>(a); e.w[0] = v.x; e.w[1] = v.y; e.w[2] = v.z;
+        const u32x3_t v = gload<u32x3_t, 1>(a); e.w[0] = v.x; e.w[1] = v.y; e.w[2] = v.z;
     } else {
-        const u32x4_t v = *gconst<u32x4_a1>(a); e.w[0] = v.x; e.w[1] = v.y; e.w[2] = v.z; e.w[3] = v.w;
+        const u32x4_t v = gload<u32x4_t, 1>(a); e.w[0] = v.x; e.w[1] = v.y; e.w[2] = v.z; e.w[3] = v.w;
     }
     return e;
 }
@@ -586,11 +575,11 @@ template <class T> FKD_DEV PairWindow<T> load_pair_window(const char* row, u32 o
     }
     asm volatile("" : "+v"(off));
     const char* a = base + off;
-    constexpr int W = PW::kWords;
-    if constexpr (W == 1) { p.w[0] = *gconst<u32_a1>(a); }
-    else if constexpr (W == 2) { const u32x2_t v = *gconst<u32x2_a4>(a); p.w[0] = v.x; p.w[1] = v.y; }
-    else if constexpr (W == 3) { const u32x3_t v = *gconst<u32x3_a4>(a); p.w[0] = v.x; p.w[1] = v.y; p.w[2] = v.z; }
-    else { const u32x4_t v = *gconst<u32x4_a4>(a); p.w[0] = v.x; p.w[1] = v.y; p.w[2] = v.z; p.w[3] = v.w; }
+    constexpr int W = PW::kWords, ALIGN = PW::kShift ? 4 : 1;
+    if constexpr (W == 1) { p.w[0] = gload<u32, ALIGN>(a); }
+    else if constexpr (W == 2) { const u32x2_t v = gload<u32x2_t, ALIGN>(a); p.w[0] = v.x; p.w[1] = v.y; }
+    else if constexpr (W == 3) { const u32x3_t v = gload<u32x3_t, ALIGN>(a); p.w[0] = v.x; p.w[1] = v.y; p.w[2] = v.z; }
+    else { const u32x4_t v = gload<u32x4_t, ALIGN>(a); p.w[0] = v.x; p.w[1] = v.y; p.w[2] = v.z; p.w[3] = v.w; }
     return p;
 }
 // The same window through a buffer resource, for images whose rows all start at the same offset inside their dword
@@ -699,13 +688,14 @@ template <class T> FKD_DEV void store_elem_at(char* base, u32 off, const T& v) {
         u32 w[W];
         if constexpr (n == 2) {
             w[0] = to_bits(chan<0>(v)) | (to_bits(chan<1>(v)) << 8);
-            *gmut<u16_a1>(a) = u16(w[0]);
+            typedef u16 At __attribute__((aligned(1)));
+            *(FKD_GLOBAL At*)a = u16(w[0]);
         } else {
             pack_words<T, 1, W>(one, w);
-            if constexpr (W == 1) { gstore(gmut<u32_a1>(a), w[0]); }
-            else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore(gmut<u32x2_a1>(a), q); }
-            else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore(gmut<u32x3_a1>(a), q); }
-            else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore(gmut<u32x4_a1>(a), q); }
+            if constexpr (W == 1) { gstore<1>(a, w[0]); }
+            else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore<1>(a, q); }
+            else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore<1>(a, q); }
+            else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore<1>(a, q); }
         }
     }
 }
@@ -725,10 +715,10 @@ template <class T, int V> FKD_DEV void store_run_at(char* base, u32 off, const S
         }
         asm volatile("" : "+v"(off));
         char* a = base + off;
-        if constexpr (W == 1) { gstore(gmut<u32_a1>(a), w[0]); }
-        else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore(gmut<u32x2_a1>(a), q); }
-        else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore(gmut<u32x3_a1>(a), q); }
-        else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore(gmut<u32x4_a1>(a), q); }
+        if constexpr (W == 1) { gstore<1>(a, w[0]); }
+        else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore<1>(a, q); }
+        else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore<1>(a, q); }
+        else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore<1>(a, q); }
     } else {
 #pragma unroll
         for (int i = 0; i < V; ++i) store_elem_at<T>(base, off + u32(i) * u32(sizeof(T)), v[i].v);
@@ -1891,9 +1881,9 @@ template <bool VU> struct ReadNV {
                     return;
                 }
             }
-            using Dword = detail::dwords_at<1, ALIGNED>;
-            u32 l = *detail::gconst<Dword>(p.data + size_t(y) * p.pitch + x);
-            u32 uv = *detail::gconst<Dword>(p.data + size_t(p.pitch) * p.height + size_t(y >> 1) * p.pitch + x);
+            constexpr int ALIGN = ALIGNED ? 4 : 1;
+            u32 l = detail::gload<u32, ALIGN>(p.data + size_t(y) * p.pitch + x);
+            u32 uv = detail::gload<u32, ALIGN>(p.data + size_t(p.pitch) * p.height + size_t(y >> 1) * p.pitch + x);
             asm("" : "+v"(l), "+v"(uv));     // keep the dwords whole: bytes leave through v_cvt_f32_ubyteN / v_bfe
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -1925,7 +1915,7 @@ template <bool VU> struct ReadNV {
         asm volatile("" : "+v"(xs), "+v"(xc));      // 32-bit lane offsets against scalar row addresses
         TapBits b;
         b.y = u32(*detail::gconst<u8>(r.luma + xs));
-        b.uv = u32(*detail::gconst<detail::u16_a1>(r.chroma + xc));   // (U,V) pair in one access
+        b.uv = u32(detail::gload<u16, 1>(r.chroma + xc));   // (U,V) pair in one access
         return b;
     }
     FKD_DEV static Raw tap_value(const TapBits& b) {
@@ -1944,8 +1934,8 @@ template <bool VU> struct ReadNV {
         u32 xs = u32(r.x0 + x), xc = xs & ~1u;
         asm volatile("" : "+v"(xs), "+v"(xc));
         PairBits b;
-        b.y = u32(*detail::gconst<detail::u16_a1>(r.luma + xs));
-        b.uv = *detail::gconst<detail::u32_a1>(r.chroma + xc);
+        b.y = u32(detail::gload<u16, 1>(r.luma + xs));
+        b.uv = detail::gload<u32, 1>(r.chroma + xc);
         return b;
     }
     FKD_DEV static void pair_values(const PairBits& b, const TapRow& r, int x, Raw& first, Raw& second) {
