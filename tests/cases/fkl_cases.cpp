@@ -295,6 +295,40 @@ int fklcase_copy_f32(void* stream_, const float* in, int w, int h, int pitch, fl
         for (int rep = 0; rep < g_reps; ++rep) executeOperations<TransformDPP<>>(i, o, stream);
     });
 }
+// Tensor of w x h x planes elements -> another one, no compute operation; rows and planes of both are as far apart as the caller says.
+extern "C++" template <typename T>
+void copy_tensor_of(void* stream_, const void* src, int pitch, int plane_pitch, void* out, int out_pitch, int out_plane_pitch, int w, int h, int planes) {
+    Stream stream(stream_);
+    auto view = [&](const void* data, int row, int plane) {
+        Tensor<T> t(reinterpret_cast<T*>(const_cast<void*>(data)), uint(w), uint(h), uint(planes), 1u, MemType::Device, 0);
+        auto v = t.ptr();
+        v.dims.pitch = uint(row);
+        v.dims.plane_pitch = uint(plane);
+        return v;
+    };
+    executeOperations<TransformDPP<>>(stream, Read<TensorRead<T>>{view(src, pitch, plane_pitch)}, Write<TensorWrite<T>>{view(out, out_pitch, out_plane_pitch)});
+}
+int fklcase_copy_tensor(void* stream, int kind, const void* src, int pitch, int plane_pitch, void* out, int out_pitch, int out_plane_pitch,
+                        int w, int h, int planes) {
+    return guarded([&] {
+        auto run = [&](auto tag) { copy_tensor_of<decltype(tag)>(stream, src, pitch, plane_pitch, out, out_pitch, out_plane_pitch, w, h, planes); };
+        switch (kind) {
+        case 0: run(uchar{}); break;
+        case 1: run(uchar2{}); break;
+        case 2: run(uchar3{}); break;
+        case 3: run(uchar4{}); break;
+        case 4: run(ushort3{}); break;
+        case 5: run(ushort4{}); break;
+        case 6: run(float2{}); break;
+        case 7: run(float3{}); break;
+        case 8: run(float4{}); break;
+        case 9: run(double{}); break;
+        case 10: run(double3{}); break;
+        case 11: run(double4{}); break;
+        default: throw std::runtime_error("fklcase_copy_tensor: kind must be 0 to 11");
+        }
+    });
+}
 // Horizontal fusion with fewer live planes than the compiled batch (BatchRead<CONDITIONAL_WITH_DEFAULT>).
 int fklcase_crop_resize_default_norm_split_b8(void* stream_, const uint8_t* src, int w, int h, int pitch, const int32_t* rects,
                                               int dw, int dh, int used_planes, const float* def, const float* sub,

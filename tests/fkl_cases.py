@@ -229,6 +229,18 @@ def uncompiled_resize_split(kind, src, rect, dst, mul, out):
                                                 r.ctypes.data_as(C.c_void_p), int(dst[0]), int(dst[1]), C.c_float(float(mul)), _p(out)))
 
 
+# (base type, channels) of the element kinds of copy_tensor
+TENSOR_KINDS = [(np.uint8, 1), (np.uint8, 2), (np.uint8, 3), (np.uint8, 4), (np.uint16, 3), (np.uint16, 4), (np.float32, 2), (np.float32, 3),
+                (np.float32, 4), (np.float64, 1), (np.float64, 3), (np.float64, 4)]
+
+
+def copy_tensor(kind, src, src_pitches, out, out_pitches, w, h, planes):
+    """Tensor -> tensor of TENSOR_KINDS[kind] elements; src and out are flat cuda byte tensors that begin with the first element,
+    pitches (row, plane) in bytes."""
+    _ok(cases().fklcase_copy_tensor(_stream(), int(kind), _p(src), int(src_pitches[0]), int(src_pitches[1]), _p(out), int(out_pitches[0]),
+                                    int(out_pitches[1]), int(w), int(h), int(planes)))
+
+
 def uncompiled_float4_resize(src, dst, out):
     """(H,W,4) f32 cuda -> bilinear -> out (dh,dw,4) f32 cuda."""
     _ok(cases().fklcase_uncompiled_float4_resize(_stream(), _p(src), src.shape[1], src.shape[0], src.stride(0) * 4, int(dst[0]), int(dst[1]),

@@ -217,3 +217,45 @@ def test_line_aligned_segments_warp(device, w, h, offset):
     cases.warp(torch.from_numpy(img).to(device), m, False, (w, h), out.view())
     torch.cuda.synchronize()
     assert out.read().tobytes() == ol.oracle_warp(img, 3, m, (w, h), False).tobytes()
+
+
+# Whole lines (rows of 2 048 elements: the grid has a column of workgroups more than the row alone needs) and half lines, for every
+# size class of elements, in a tensor whose planes are no whole lines apart, so that each plane's rows have phases of their own
+# (or none: elements of more than one sample whose rows never meet a line boundary in the planes after the first).
+# Element sizes 1, 2, 3, 6 leave a row's ends element by element, 4 as runs, 8 (ushort4, float2), 12 and 16 through the LDS, 8
+# (double), 24 and 32 as runs again.
+@pytest.mark.parametrize("kind", range(len(cases.TENSOR_KINDS)))
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_line_aligned_segments_tensors(device, kind, half, in_place):
+    import torch
+    from fusedkernellibrary_amd import last_launch
+    base, cn = cases.TENSOR_KINDS[kind]
+    size, planes = np.dtype(base).itemsize, 3
+    elem = size * cn
+    unit = elem & -elem                                            # the power of two in an element's size
+    half_line = 128 // unit // 2 - 1                               # elements that a row's first segment begins left of it, at most
+    w = 1024 - half_line if half else 2048                         # four segments with half lines, five with whole ones
+    h = (16000000 if elem % 4 else 24000000) // (w * elem * planes) + 1
+    rng = np.random.RandomState(kind)
+    row, data = w * elem, rng.randint(0, 256, (planes, h, w * elem)).astype(np.uint8)
+
+    def place(offset, pad, plane_pad, fill):
+        pitches = (row + pad, (row + pad) * h + plane_pad)
+        host = np.full(256 + offset + pitches[1] * planes + 256, FILL, np.uint8)
+        at = np.lib.stride_tricks.as_strided(host[256 + offset:], (planes, h, row), (pitches[1], pitches[0], 1))
+        if fill:
+            at[:] = data
+        return host, at, pitches, 256 + offset
+
+    out_host, out_at, out_pitches, out_start = place(3 * unit, unit * (kind % 3 + 1), 5 * size, in_place)
+    out = torch.from_numpy(out_host).to(device)
+    if in_place:
+        cases.copy_tensor(kind, out[out_start:], out_pitches, out[out_start:], out_pitches, w, h, planes)
+    else:
+        src_host, _, src_pitches, src_start = place(size, 0, size, True)
+        cases.copy_tensor(kind, torch.from_numpy(src_host).to(device)[src_start:], src_pitches, out[out_start:], out_pitches, w, h, planes)
+    torch.cuda.synchronize()
+    assert last_launch()["grid"][0] == (4 if half else 9)
+    out_at[:] = data
+    assert np.array_equal(out.cpu().numpy(), out_host)             # the rows are the input's, every byte beside them is as it was
