@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52068000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "cf6b659e4a598266932c70ef838e2f9ab5993a30b1e908616f09555c917faf7b"
+TRAFFIC_C3_SOURCES_SHA256 = "baed8ba30a9f677ac92f7c2ee8530ec9ee0caee079fc37e883192ee674884f51"
 
 
 def device_sources_sha256():

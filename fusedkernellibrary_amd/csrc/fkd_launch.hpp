@@ -43,7 +43,7 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
     if (grid.y > 65535u || grid.z > 65535u) return hipErrorInvalidConfiguration;
-    if constexpr (!rows_any_x<Chain>(V)) {     // (the others take runs at any alignment, one kernel for both)
+    if constexpr (!rows_any_x<Chain>(V)) {
         if (aligned) return launch_by_pointer(&k_rows<Chain, V, ROWS, true>, grid, block, stream, p, g);
     }
     return launch_by_pointer(&k_rows<Chain, V, ROWS, false>, grid, block, stream, p, g);
@@ -52,9 +52,10 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
 template <class Chain>
 hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int V = RowsConfig<Chain>::V, ROWS = RowsConfig<Chain>::ROWS;
-    // Runs move as wide accesses at any alignment; that every row start is dword aligned (checked here, once per launch, on
-    // the host) tells readers of grouped samples that a run starts on a group.
-    const bool aligned = Chain::Read::rows_aligned(p.read, 0) && Chain::Write::rows_aligned(p.write);
+    // Chains whose reads may start anywhere in a row have one kernel for rows at every alignment.  The others have one for rows
+    // that all start on dword boundaries (checked here, once per launch, on the host) and one for the rest.
+    bool aligned = true;
+    if constexpr (!rows_any_x<Chain>(V)) aligned = Chain::Read::rows_aligned(p.read, 0) && Chain::Write::rows_aligned(p.write);
     if constexpr (ROWS > 1) {
         const unsigned long long gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);
         const unsigned long long gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);

@@ -6,7 +6,7 @@
 namespace fkd {
 
 struct LaunchInfo {
-    const char* kernel;   // "rows", "rows_unaligned" or "gather"
+    const char* kernel;   // "rows", "rows_unaligned" (chains with a kernel of its own for such rows), "gather" or "strip"
     unsigned grid[3], block[3];
     unsigned lds_bytes;
 };

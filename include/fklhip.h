@@ -116,7 +116,10 @@ int fklhip_jit_log(const char **log);
 int fklhip_strip_form(int enable);
 
 /* Introspection for tests and benchmarks: what the last fklhip_launch* on this thread launched.
- * kernel receives "rows", "rows_unaligned", "gather", or "rows_jit" / "gather_jit" for chains compiled at run time; grid/block receive 3 values each. */
+ * kernel receives "rows", "gather" or "strip", each with "_jit" behind it for chains compiled at run time, or "rows_unaligned": the
+ * kernel for rows that do not all start on dword boundaries, of the chains compiled ahead of time that have one of its own for
+ * them (padding, deinterlacing, planar and circular reads; the others have one kernel for rows at every alignment).
+ * grid/block receive 3 values each. */
 int fklhip_last_launch(const char **kernel, unsigned grid[3], unsigned block[3], unsigned *lds_bytes);
 
 /* Number of chain signatures compiled into the library and the i-th of them with its parameter block size. */

@@ -117,8 +117,19 @@ def test_uchar3_rows_with_unaligned_pitch(device):
         want = ol.oracle_batch_muladd_sat(srcs_np, mul, add)
         for i in range(4):
             assert np.array_equal(outs[i].cpu().numpy(), want[i]), (w, h, i)
-        expect = "rows" if (w * 3) % 4 == 0 else "rows_unaligned"
-        assert last_launch()["kernel"] == expect
+        assert last_launch()["kernel"] == "rows"               # one kernel for rows at every alignment
+
+
+def test_chains_with_a_kernel_of_their_own_for_unaligned_rows_report_it(device):
+    """Padding reads do not start just anywhere in a row: rows on dword boundaries and others are two kernels."""
+    import torch
+    for w, ow, kernel in ((40, 60, "rows"), (41, 60, "rows_unaligned"), (40, 61, "rows_unaligned")):
+        img = np.random.RandomState(w + ow).randint(0, 256, (30, w, 3)).astype(np.uint8)
+        out = torch.zeros((50, ow, 3), dtype=torch.uint8, device=device)
+        cases.pad(torch.from_numpy(img).to(device), ol.BORDER_REFLECT_101, 8, 8, out)
+        torch.cuda.synchronize()
+        assert last_launch()["kernel"] == kernel
+        assert out.cpu().numpy().tobytes() == ol.oracle_pad(img, ol.BORDER_REFLECT_101, 8, 8, ow, 50).tobytes()
 
 
 def test_repeated_launches_are_idempotent(device):
