@@ -592,6 +592,29 @@ int fklcase_normalise_mode(int kind, const float* sub, const float* div) {
 }
 // How the host would divide by d on the device: 0 generic division, 1 five-instruction sequence, 2 two-instruction
 // sequence proven exact for this divisor (fkd::Div).
+// What the tap windows of the bilinear kernels' strip form and of warps are made of, for pixels of elem_bytes bytes: where the window of a
+// pair that starts `at` bytes into an image begins (out[0]), the bytes dropped from it (out[1]), its length (out[2]); and the
+// extent (out[3]) of an image of image_bytes bytes that begins lo bytes after a dword boundary.
+int fklcase_tap_window(int elem_bytes, unsigned at, unsigned long long image_bytes, unsigned lo, unsigned* out) {
+    auto fill = [&](auto tag) {
+        using Shape = fkd::detail::PairWindowShape<decltype(tag)>;
+        const auto prep = fkd::detail::pair_window_at<Shape>(at);
+        out[0] = prep.off;
+        out[1] = Shape::kShift ? prep.shift & 3u : 0u;
+        out[2] = 4u * Shape::kWords;
+        out[3] = fkd::detail::tap_extent(size_t(image_bytes), lo);
+        return 0;
+    };
+    switch (elem_bytes) {
+    case 1: return fill(fkd::u8{});
+    case 2: return fill(fkd::Vec<fkd::u8, 2>{});
+    case 3: return fill(fkd::Vec<fkd::u8, 3>{});
+    case 4: return fill(fkd::Vec<fkd::u8, 4>{});
+    case 6: return fill(fkd::Vec<fkd::u16, 3>{});
+    case 8: return fill(fkd::Vec<fkd::f32, 2>{});
+    default: return 2;
+    }
+}
 int fklcase_div_mode(float d) { return fkd::Div<float, float, float>::make(d).fast; }
 // The same one-operation chain with the sequence chosen by the caller instead of by the host's proof, through the C
 // ABI with a hand-built parameter block: lets a test compare the proof's verdict with what the device really computes.

@@ -81,10 +81,11 @@ def test_wider_outputs_keep_the_tile_form(device):
     assert got.tobytes() == ol.oracle_crop_resize_norm_split(img, rects, (257, 16), wl.C3_MEAN, wl.C3_STD).tobytes()
 
 
-def test_planes_the_strip_form_cannot_take_are_declined_on_the_host(device):
+def test_launches_that_keep_the_tile_form_are_told_on_the_host(device):
     import torch
     rng = np.random.RandomState(6)
-    # rows that do not share their alignment (pitch 999), and a one-column crop among aligned rows
+    # a launch too small for the strip form to pay on rows that do not share their alignment (pitch 999), and a one-column crop
+    # among aligned rows, which the strip form cannot take
     for w, rects in ((333, np.array([[0, 0, 333, 100]] * 8, np.int32)),
                      (332, np.array([[0, 0, 332, 100]] * 7 + [[5, 7, 1, 50]], np.int32))):
         img = rng.randint(0, 256, (100, w, 3)).astype(np.uint8)

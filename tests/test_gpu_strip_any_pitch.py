@@ -1,6 +1,6 @@
 """The strip form of the bilinear kernel on images whose rows do not share their alignment: bit for bit the oracle's result and the
 tile form's, at every alignment of the image, with enlarging planes (columns clamped to the last one), letterboxes and crops that
-end with the image; and, on the CPU, the bytes its tap windows touch."""
+end with the image.  (The bytes its tap windows touch: test_tap_windows.py.)"""
 import numpy as np
 import pytest
 
@@ -8,23 +8,6 @@ import fkl_cases as cases
 import oracle_lib as ol
 import workloads as wl
 from test_gpu_any_alignment import Placed
-
-
-def test_windows_stay_inside_the_dwords_of_the_image():
-    """Read2D<uchar3>, pitch % 4 != 0: window start (column + row bytes) & ~3 from the resource's base, three dwords, those beyond
-    the extent reading zeros; the six bytes of the two taps are always inside it and always inside the window."""
-    for w in (2, 3, 5, 7, 333):
-        for h in (1, 2, 3):
-            for lo in range(4):
-                for pitch in (3 * w, 3 * w + 1, 3 * w + 2):
-                    if pitch % 4 == 0:
-                        continue
-                    extent = (lo + pitch * (h - 1) + 3 * w + 3) & ~3
-                    for y in range(h):
-                        for x1 in range(w - 1):
-                            t = (lo + 3 * x1) + y * pitch
-                            start, drop = t & ~3, t & 3
-                            assert start >= 0 and drop + 6 <= 12 and t + 6 <= extent, (w, h, lo, pitch, x1, y)
 
 
 def _view(img, offset, pad, device):

@@ -9,9 +9,15 @@ would hide a violation on the GPU, so they are checked here by brute force over 
   take one access per channel instead (Read2D::tap_row / tap_last); every other window must end inside the image;
 * strip form (k_strip): the buffer resource ends with the dword that holds the image's last byte (make_tap_image with a
   size); dwords at or beyond that extent are not fetched (they read as zero).  Every byte a blend USES must lie in a
-  delivered dword, and every delivered dword must start inside the image, so that it lies in a mapped page.
+  delivered dword, and every delivered dword must start inside the image, so that it lies in a mapped page.  Warps fetch the same
+  way.
 """
+import ctypes as C
 import itertools
+
+import pytest
+
+import fkl_cases as cases
 
 ELEM = 3          # bytes per pixel (uchar3)
 WINDOW = 12       # dwords fetched per pair window: 3
@@ -49,19 +55,38 @@ def test_tile_form_windows_stay_inside_the_image():
     assert checked > 5000
 
 
-def test_strip_form_extent_delivers_every_used_byte_and_nothing_unmapped():
-    for w, h, pitch, lo in _cases():
-        if pitch % 4:
-            continue                                            # the strip form is only launched for pitches that are multiples of 4
-        size = _image_bytes(w, h, pitch)
-        extent = (size + lo + 3) & ~3                           # make_tap_image(data, bytes): relative to the dword-aligned base
-        # every delivered dword starts inside the image (so it shares a page with image bytes)
-        assert extent - 4 < lo + size
-        for y in range(h):
-            for x1 in range(w - 1):
-                first_byte = lo + y * pitch + x1 * ELEM         # relative to the resource's base
-                start = first_byte & ~3
-                used = range(first_byte, first_byte + 2 * ELEM)
-                for b in used:
-                    assert (b & ~3) + 4 <= extent, (w, h, pitch, lo, y, x1)     # its dword is inside the extent: delivered
-                assert start + WINDOW <= extent + 8             # at most two dwords of a window are beyond the extent (read as zero)
+# samples of 1, 2 and 4 bytes: an image's rows start and repeat at multiples of their samples' size
+@pytest.mark.parametrize("elem,sample", [(1, 1), (2, 1), (3, 1), (4, 1), (6, 2), (8, 4)])
+def test_strip_form_windows_hold_every_used_byte_and_touch_nothing_unmapped(elem, sample):
+    """The library's own window arithmetic (fkd::detail::pair_window_at, tap_extent), compiled for the host: strip form and warps,
+    images of every address and pitch."""
+    window_of = cases.cases().fklcase_tap_window
+    out = (C.c_uint * 4)()
+    checked = 0
+    for w, h in itertools.product((2, 3, 5, 8, 11), (1, 2, 3, 5)):
+        for pad, lo in itertools.product(range(0, 6, sample), range(0, 4, sample)):
+            pitch = w * elem + pad
+            size = pitch * (h - 1) + w * elem
+            for y, x1 in itertools.product(range(h), range(w - 1)):
+                at = lo + x1 * elem + y * pitch                     # from the dword at or below the image's first byte
+                assert window_of(elem, at, size, lo, out) == 0
+                start, drop, length, extent = out
+                assert extent % 4 == 0 and extent - 4 < lo + size   # every delivered dword starts inside the image: a mapped page
+                assert start + drop == at and drop + 2 * elem <= length         # the pair is where it is looked for
+                assert at + 2 * elem <= extent                      # and all of it is delivered
+                if elem % 4:
+                    assert start % 4 == 0 and drop <= 3 and start <= extent - 4
+                else:
+                    assert drop == 0 and length == 2 * elem
+                checked += 1
+    assert checked > 500
+
+
+def test_columns_without_a_window_touch_no_image():
+    """The strip form marks a column beyond the output with the offset 2 GB; with any row's offset on top it is beyond the extent of
+    the largest image the form takes, and does not wrap."""
+    largest = 0x7ffffff0 - 1
+    out = (C.c_uint * 4)()
+    for elem, row, lo in itertools.product((1, 2, 3, 4, 6, 8), (0, 1, 2, 3, 4097, largest), range(4)):
+        assert cases.cases().fklcase_tap_window(elem, 0x80000000 + row, largest, lo, out) == 0
+        assert out[0] >= 0x80000000 > out[3] and out[0] + out[2] <= 0xffffffff
