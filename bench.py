@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52068000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "baed8ba30a9f677ac92f7c2ee8530ec9ee0caee079fc37e883192ee674884f51"
+TRAFFIC_C3_SOURCES_SHA256 = "8f6d1e6b3c866c6382d49635acc5184a1959f6780b1e7eae5c66a2ad93b148cc"
 
 
 def device_sources_sha256():

@@ -2993,6 +2993,11 @@ template <class T, bool TRANSPOSED = false> struct TensorSplit {
         return G::channel_elements(p) * sizeof(B) * cn_v<T> < size_t(0x7fffffffu) &&
                G::channel_elements(p) * sizeof(B) * (cn_v<T> - 1) + size_t(p.pitch) * p.height < size_t(0x7fffffffu);
     }
+    // The power of two, at most a line, that the addresses of both ends of every row of `w` values are multiples of.
+    FKD_HD static u32 row_grain(const Params& p, u32 w, u32 planes) {
+        const size_t ends = reinterpret_cast<size_t>(p.data) | p.pitch | G::channel_elements(p) * sizeof(B) | (planes > 1u ? G::image_bytes(p) : 0u) | size_t(w) * sizeof(B) | kLineBytes;
+        return u32(ends & (0u - ends));
+    }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static B* at(const Params& p, int x, int y, int z) {
         return reinterpret_cast<B*>(reinterpret_cast<char*>(p.data) + G::image_bytes(p) * z + size_t(y) * p.pitch) + x;
@@ -3327,20 +3332,38 @@ template <class T> struct IsDivOp { static constexpr bool value = false; };
 template <class I, class P, class O> struct IsDivOp<Div<I, P, O>> { static constexpr bool value = Div<I, P, O>::kReciprocal; };
 
 #if !defined(FKD_DEVICE_CODE)
-// Which of the two forms of the bilinear kernel a launch takes that the strip form could serve.  us, tile form / strip form, 64
-// crops of a 1280x853 image unless noted (8 crops: four launches):
-//   outputs stored past the last-level cache whose rows are no whole lines: a strip's 128-byte stores then end in partial lines,
-//   which leave the chip one by one: 200x640 23.7 / 45.3, 225x640 34.4 / 74.3 (whole lines: 224x640 23.3 / 19.9, 160x640 22.4 / 15.5);
-//   six steps and more with rows that are no whole 32-byte sectors: 225x200 10.9 / 11.9, 250x200 11.4 / 12.4 (200x200 10.3 / 8.9);
-//   rows that do not share their alignment (width 1279): 160x200 10.3 / 7.0, 224x200 10.5 / 8.4, 224x640 24.2 / 20.2, 8 crops to
-//   100x200 14.9 / 13.3; but with six steps and more and less than a workgroup per compute unit a strip's row is one wave's alone:
-//   8 crops to 200x60 13.7 / 15.6, to 224x60 13.8 / 15.6.
-inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes) {
+// Which of the two forms of the bilinear kernel a launch takes that the strip form could serve.  row_grain: the power of two (at
+// most a line) that both ends of every output row are multiples of, 4 bytes per channel value.  us, tile form / strip form, 64 crops of
+// a 1280x853 image unless noted, three outputs in turn, launches in a graph:
+//  Outputs stored past the last-level cache: what a strip stores of a line in one step leaves the chip by itself.
+//   Whole lines: the strip form (32 to 224 wide 0.44 to 0.94 of the tile form's time: 160x781 27.9 / 19.5, 224x640 25.1 / 22.6; 256-wide
+//   rows as 224).  With a base 4 bytes off a line 224x640 takes 36.2 / 66.2, which is why the base is asked and not only the width.
+//   Whole half lines: the strip form where the tile form's 128 columns leave more than a quarter of its lanes idle (48x2343
+//   37.7 / 25.3, 80x1406 26.3 / 22.3, 144x781 27.5 / 20.1, 176x639 23.9 / 19.7; 64-wide rows half a line off 30.6 / 21.2), else the tile form
+//   (240x520 21.1 / 23.3, 128x878 half a line off 18.9 / 21.1; 112 and 208 wide within 6 %).
+//   Others: rows of one step the strip form (20x5625 87 / 41, 28x4017 58 / 29), longer ones the tile form (36x5208 75 / 79,
+//   60x1875 32 / 43, 100x1125 27 / 50, 200x625 26 / 45, 225x555 33 / 63).
+//  Smaller outputs, rows of six to eight steps that are no whole 32-byte sectors: from a size on the tile form, later for fewer steps
+//   and for rows of whole 16 bytes.  6 steps, 165 wide: 1.8 M pixels 9.0 / 8.7, 2.5 M 11.3 / 11.4, 3.2 M 13.5 / 14.4; 180 wide: 3.2 M 13.2 / 12.8,
+//   5.2 M 18.4 / 17.8.  7 steps, 197 wide: 1.4 M 7.2 / 6.9, 1.6 M 7.4 / 7.6, 2.4 M 9.8 / 10.7; 220 wide: 2.0 M 8.6 / 8.1, 2.4 M 9.7 / 9.9, 5.2 M 16.8 / 17.6.
+//   8 steps, 250 wide: 1.2 M 6.5 / 6.2, 1.4 M 6.6 / 6.8, 3.2 M 12.0 / 13.6; 236 wide: 1.6 M 7.3 / 7.2, 1.8 M 7.5 / 7.8, 3.2 M 11.3 / 11.8.  Whole
+//   sectors keep the strip form (200x117 6.8 / 6.1, 200x406 17.3 / 15.8).
+//  Images whose rows do not share their alignment (width 1279): 168x64 4.7 / 4.0, 224x64 4.75 / 4.2, 8 crops to 160x62 3.1 / 3.0, to 160x156 3.6 / 3.1;
+//   with six steps and more and less than a workgroup per compute unit a strip's row is one wave's alone: 8 crops to 200x60
+//   3.1 / 3.6, to 256x120 3.2 / 3.7.  Launches below 40 000 pixels and rows of no whole sectors keep the tile form that such images
+//   always had; the strip form would serve some of them better (8 crops to 64x39 3.0 / 2.2, 64 crops to 165x64 4.8 / 4.3, to 250x200 12.2 / 13.5).
+inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes, u32 row_grain) {
     const unsigned long long pixels = (unsigned long long)w * h * planes, workgroups = (unsigned long long)((h + 7u) / 8u) * planes;
-    if (pixels * value_bytes > kStreamOutputBytes && w % 32u != 0u) return false;
-    const bool many_steps = w > 160u, sectors = w % 8u == 0u;
-    if (many_steps && !sectors && pixels >= 1200000u) return false;
-    return !any_pitch || (pixels >= 40000u && (!many_steps || (sectors && workgroups >= 256u)));
+    if (pixels * value_bytes > kStreamOutputBytes) {
+        const bool idle_lanes = w * 4u <= (w + 127u) / 128u * 128u * 3u;
+        if (!(row_grain >= 128u || (row_grain >= 64u && idle_lanes) || w <= 32u)) return false;
+    }
+    const bool many_steps = w > 160u, sectors = w % 8u == 0u, quads = w % 4u == 0u;
+    if (any_pitch) return pixels >= 40000u && (!many_steps || (sectors && workgroups >= 256u));
+    if (!many_steps || sectors) return true;
+    if (w <= 192u) return quads || pixels < 2400000u;
+    if (w <= 224u) return pixels < (quads ? 2400000u : 1600000u);
+    return pixels < (quads ? 1600000u : 1200000u);
 }
 #endif
 
@@ -3405,7 +3428,7 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
             p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
         if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {
             const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);
-            if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value)) && W::strip_ok(p.write) &&
+            if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value), W::row_grain(p.write, p.active_w, p.active_z)) && W::strip_ok(p.write) &&
                 (!any_pitch || R::strip_ok(p.read, true, p.active_z))) p.reserved |= kStripChecked;
         }
     }

@@ -615,6 +615,20 @@ int fklcase_tap_window(int elem_bytes, unsigned at, unsigned long long image_byt
     default: return 2;
     }
 }
+// Whether a launch of the bilinear kernel over `planes` planes of w x h float3 results prefers the strip form (fkd::strip_pays), and the
+// alignment of the ends of its output rows (fkd::TensorSplit::row_grain) for a tightly packed tensor at `address`.
+int fklcase_strip_pays(unsigned w, unsigned h, unsigned planes, int any_pitch, unsigned row_grain) {
+    return fkd::strip_pays(w, h, planes, any_pitch != 0, sizeof(fkd::Vec<fkd::f32, 3>), row_grain) ? 1 : 0;
+}
+unsigned fklcase_row_grain(unsigned long long address, unsigned w, unsigned h, unsigned planes) {
+    Tensor<float> t(reinterpret_cast<float*>(size_t(address)), w, h, planes, 3, MemType::Device, 0);
+    const auto& d = t.ptr().dims;
+    using Split = fkd::TensorSplit<fkd::Vec<fkd::f32, 3>>;
+    Split::Params p{};
+    p.data = t.ptr().data;
+    p.width = d.width; p.height = d.height; p.planes = d.planes; p.color_planes = d.color_planes; p.pitch = d.pitch; p.plane_pitch = d.plane_pitch;
+    return Split::row_grain(p, w, planes);
+}
 int fklcase_div_mode(float d) { return fkd::Div<float, float, float>::make(d).fast; }
 // The same one-operation chain with the sequence chosen by the caller instead of by the host's proof, through the C
 // ABI with a hand-built parameter block: lets a test compare the proof's verdict with what the device really computes.

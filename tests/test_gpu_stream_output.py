@@ -28,6 +28,24 @@ def test_batches_around_the_limit(dst, kernel):
     assert out.cpu().numpy().tobytes() == want.tobytes()
 
 
+@pytest.mark.parametrize("dst,offset,kernel", [((224, 512), 0, "strip"), ((224, 512), 32, "strip"), ((224, 512), 16, "gather"),
+                                               ((224, 512), 1, "gather"), ((48, 2390), 0, "strip"), ((48, 2390), 8, "gather"), ((31, 3700), 0, "strip")])
+def test_outputs_on_and_off_the_lines(dst, offset, kernel):
+    """An output that begins `offset` floats after a line boundary: its rows are whole lines, whole half lines or neither."""
+    import torch
+    c = wl.config3(width=640, height=359, min_side=2, span=340)
+    src = torch.from_numpy(c["src"]).cuda()
+    n = 64 * 3 * dst[0] * dst[1]
+    buf = torch.full((n + 64,), -7.0, dtype=torch.float32, device="cuda")
+    assert buf.data_ptr() % 128 == 0
+    cases.crop_resize_norm_split(src, c["rects"], dst, c["sub"], c["div"], buf[offset:offset + n].view(64, 3, dst[1], dst[0]))
+    torch.cuda.synchronize()
+    assert last_launch()["kernel"] == kernel
+    got = buf.cpu().numpy()
+    assert (got[:offset] == -7.0).all() and (got[offset + n:] == -7.0).all()
+    assert got[offset:offset + n].tobytes() == ol.oracle_crop_resize_norm_split(c["src"], c["rects"], dst, c["sub"], c["div"]).tobytes()
+
+
 @pytest.mark.parametrize("dst", [(1365, 1365), (1366, 1366), (201, 9275)])           # 67 076 100, 67 174 416 and 67 113 900 bytes
 def test_a_chain_compiled_on_first_use(dst):
     import torch
