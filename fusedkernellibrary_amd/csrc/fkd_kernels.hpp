@@ -704,7 +704,8 @@ template <class Chain> constexpr bool strip_capable() {
     }
 }
 
-template <class Chain, bool STREAM>
+// ANY_PITCH: some image of the launch has rows that do not share their alignment (Chain::kStripAnyPitch).
+template <class Chain, bool STREAM, bool ANY_PITCH>
 __device__ __forceinline__ void strip_body(const typename Chain::Params& p, const u32 first_late_workgroup) {
     using Root = ResizeRoot<typename Chain::Read>;
     using RZ = typename Root::Resize;
@@ -749,10 +750,12 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     const detail::TapImage image = Back::tap_image_bounded(z, q.back);
     // Rows that do not share their alignment: a column's entry then holds the byte offset of its first tap, and where in its
     // dword the window begins is only known together with the row (one more instruction per pixel and line).  Otherwise it
-    // holds the offset of the window.  (wave uniform, as the plane.)  For pixels of whole dwords the two are the same: their
-    // windows begin with the first tap, whatever its address.
+    // holds the offset of the window.  For pixels of whole dwords the two are the same: their windows begin with the first tap,
+    // whatever its address.
     using Window = typename Back::PairBits;
-    const bool any_pitch = Window::kShift && ((Back::tap_row_offset(1, q.back) - Back::tap_row_offset(0, q.back)) & 3u) != 0u;
+    // Each kind has a kernel of its own: with both in one, its code half as long again, launches of more than one workgroup per
+    // compute unit were 2 to 7 % slower, of either kind (8 crops to 128x640 3.31 -> 3.51 us).
+    constexpr bool kAnyPitch = Window::kShift && ANY_PITCH;
     const int steps = (aw + kStripStep - 1) / kStripStep;
     if (steps == 0) return;                                             // no columns: nothing to write (the whole workgroup leaves)
 
@@ -770,7 +773,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         u32 flags = pp.shift | (clamped ? kClamped : 0u);
         if constexpr (RZ::kAR != IGNORE_AR) flags |= (x >= q.x1 && x <= q.x2) ? 0u : kOutsideX;
         detail::u32x4_t e;
-        e.x = __builtin_bit_cast(u32, ax); e.y = __builtin_bit_cast(u32, bx); e.z = pp.off + pp.shift; e.w = flags;
+        e.x = __builtin_bit_cast(u32, ax); e.y = __builtin_bit_cast(u32, bx); e.z = kAnyPitch ? pp.off + pp.shift : pp.off; e.w = flags;
         return e;
     };
 
@@ -790,21 +793,21 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     if constexpr (RZ::kAR != IGNORE_AR) yin = yc >= q.y1 && yc <= q.y2;
 
     struct StepTaps { detail::u32x4_t e; typename Back::PairBits ab, cd; };
-    auto fetch = [&](StepTaps& s, bool any) {
+    auto fetch = [&](StepTaps& s) {
         // (v_alignbyte_b32 takes the bytes to drop from bits 0-1 of its operand, so the flags may ride along)
         detail::PairPrep pa, pb;
         pa.off = s.e.z + row_a; pa.shift = s.e.w;
         pb.off = s.e.z + row_b; pb.shift = s.e.w;
-        if (any) {
+        if constexpr (kAnyPitch) {
             pa = detail::pair_window_at<Window>(pa.off);
             pb = detail::pair_window_at<Window>(pb.off);
         }
         s.ab = Back::pair_load_prepared(image, 0u, pa, q.back);
         s.cd = Back::pair_load_prepared(image, 0u, pb, q.back);
     };
-    auto request = [&](int k, StepTaps& s, bool any) {
+    auto request = [&](int k, StepTaps& s) {
         s.e = column[g + kStripStep * k];
-        fetch(s, any);
+        fetch(s);
         __builtin_amdgcn_sched_barrier(0);      // the next step's taps leave before anything waits for this step's
     };
     // The taps of step 0 are requested before the table exists, from the lane's own working out of its first column:
@@ -813,7 +816,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     {
         bool unused;
         first.e = column_entry(g, unused);
-        fetch(first, true);                         // (the general form serves both)
+        fetch(first);
     }
 
     // ---- the column table: one column per thread (the workgroup has as many threads as the form has columns).  Columns
@@ -824,7 +827,6 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     {
         bool clamped = false;
         detail::u32x4_t e = column_entry(t, clamped);
-        if constexpr (Window::kShift) e.z &= any_pitch ? ~0u : ~3u;
         if (t >= steps * kStripStep) { e.z = kNoWindow; clamped = false; }
         column[t] = e;
         const bool any = __builtin_amdgcn_ballot_w64(clamped) != 0ull;
@@ -841,10 +843,9 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     const u32 out0 = yvalid ? WP::row_offset(y, oplane) + WP::lane_offset(g, true) : WP::kMaskedOut;
     const bool partial = (aw & (kStripStep - 1)) != 0;             // the last step has columns beyond the output
 
-    auto run = [&](auto static_tag, auto clamp_tag, auto pitch_tag) {
+    auto run = [&](auto static_tag, auto clamp_tag) {
         constexpr bool STATIC = decltype(static_tag)::value != 0;
         constexpr bool CLAMP = decltype(clamp_tag)::value != 0;
-        constexpr bool ANY = decltype(pitch_tag)::value != 0;
         auto produce = [&](int k, const StepTaps& s) {
             // (k is known where the steps are written out: one comparison in four of the steps)
             if ((k == 3 || k == 4) && k == falls[0]) __builtin_amdgcn_s_setprio(2);
@@ -882,21 +883,20 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         // in the instruction's immediate offset, and there is no loop bookkeeping.  The request behind the last step meets
         // a column without a window.
         StepTaps sa = first, sb;
-        request(1, sb, ANY);
+        request(1, sb);
 #pragma unroll
         for (int k = 0; k < kStripMaxSteps; k += 2) {
-            if (k > 0) request(k + 1, sb, ANY);
+            if (k > 0) request(k + 1, sb);
             produce(k, sa);
             if (k + 1 >= steps) return;
-            if (k + 2 < kStripMaxSteps) request(k + 2, sa, ANY);
+            if (k + 2 < kStripMaxSteps) request(k + 2, sa);
             produce(k + 1, sb);
             if (k + 2 >= steps) return;
         }
     };
     auto run_static = [&](auto static_tag) {
-        if (any_pitch) run(static_tag, IntTag<1>{}, IntTag<1>{});
-        else if (some_clamped) run(static_tag, IntTag<1>{}, IntTag<0>{});
-        else run(static_tag, IntTag<0>{}, IntTag<0>{});
+        if (kAnyPitch || some_clamped) run(static_tag, IntTag<1>{});
+        else run(static_tag, IntTag<0>{});
     };
     if constexpr (Chain::kQuick) {
         if (Chain::ops_static(ops)) { run_static(IntTag<1>{}); return; }
@@ -904,9 +904,9 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     run_static(IntTag<0>{});
 }
 
-template <class Chain, bool STREAM>
+template <class Chain, bool STREAM, bool ANY_PITCH>
 __global__ __launch_bounds__(kStripThreads) void k_strip(const typename Chain::Params p, const u32 first_late_workgroup) {
-    if constexpr (strip_capable<Chain>()) strip_body<Chain, STREAM>(p, first_late_workgroup);
+    if constexpr (strip_capable<Chain>()) strip_body<Chain, STREAM, ANY_PITCH>(p, first_late_workgroup);
 }
 
 template <class Chain, int XI, int YI, bool STREAM>
@@ -998,8 +998,14 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
         const bool streamed = (g.n_tiles & kStreamFlag) != 0u;
         if constexpr (strip_capable<Chain>()) {
             if (g.tiles_x == 0u) {                       // wave uniform: the launcher chose the strip form
-                if (streamed) strip_body<Chain, true>(p, g.n_tiles & ~kStreamFlag);
-                else strip_body<Chain, false>(p, g.n_tiles);
+                const u32 first_late = g.n_tiles & ~(kStreamFlag | kAnyPitchFlag);
+                if ((g.n_tiles & kAnyPitchFlag) != 0u) {
+                    if (streamed) strip_body<Chain, true, true>(p, first_late);
+                    else strip_body<Chain, false, true>(p, first_late);
+                } else {
+                    if (streamed) strip_body<Chain, true, false>(p, first_late);
+                    else strip_body<Chain, false, false>(p, first_late);
+                }
                 return;
             }
         }

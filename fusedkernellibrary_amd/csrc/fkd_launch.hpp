@@ -79,8 +79,12 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
             if (grid.x == 0 || grid.z == 0) return hipSuccess;
             if (grid.z > 65535u) return hipErrorInvalidConfiguration;
             const unsigned first_late = strip_first_late_workgroup((unsigned long long)grid.x * grid.z);
-            if (streamed) return launch_by_pointer(&k_strip<Chain, kStreams>, grid, block, stream, p, first_late);
-            return launch_by_pointer(&k_strip<Chain, false>, grid, block, stream, p, first_late);
+            if ((p.reserved & Chain::kStripAnyPitch) != 0u) {
+                if (streamed) return launch_by_pointer(&k_strip<Chain, kStreams, true>, grid, block, stream, p, first_late);
+                return launch_by_pointer(&k_strip<Chain, false, true>, grid, block, stream, p, first_late);
+            }
+            if (streamed) return launch_by_pointer(&k_strip<Chain, kStreams, false>, grid, block, stream, p, first_late);
+            return launch_by_pointer(&k_strip<Chain, false, false>, grid, block, stream, p, first_late);
         }
     }
     TileGeom g;

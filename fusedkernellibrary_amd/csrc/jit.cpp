@@ -40,6 +40,7 @@ using fkd::JitMeta;
 using fkd::TileGeom;
 using fkd::division_magic;
 using fkd::kRowsBandBlocks;
+using fkd::kAnyPitchFlag;
 using fkd::kStreamFlag;
 using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
@@ -204,7 +205,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     if (!blob) return FKLHIP_EINVAL;
     if (bytes != k->meta.params_bytes) return FKLHIP_EBLOB_SIZE;
     unsigned active[4];
-    memcpy(active, blob, sizeof(active));   // Chain::Params starts with active_w, active_h, active_z, reserved (bit 0: strip form allowed)
+    memcpy(active, blob, sizeof(active));   // Chain::Params starts with active_w, active_h, active_z, reserved (bit 0: strip form allowed, bit 1: for rows at any pitch)
     const JitMeta& m = k->meta;
     TileGeom g{0, 0, 0, 0};
     const bool streamed = m.gather && (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes;
@@ -218,7 +219,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[1] = 1;
         grid[2] = active[2];
         block[1] = m.by;
-        g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]) | (streamed ? kStreamFlag : 0u);
+        g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]) | (streamed ? kStreamFlag : 0u) | ((active[3] & 2u) != 0 ? kAnyPitchFlag : 0u);
     } else if (m.gather) {
         const unsigned tw = 64 * m.xi, th = m.by * m.yi;
         g.tiles_x = (active[0] + tw - 1) / tw;

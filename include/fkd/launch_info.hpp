@@ -18,7 +18,8 @@ struct LaunchInfo {
 // kStreamFlag in n_tiles: the output of the run-time compiled bilinear kernel is streamed past the last-level cache (the
 // ahead-of-time kernels are told by their type).
 // (Four words: with a fifth, launches of few waves took 0.15 us longer, 8 crops to 224x224 3.96 instead of 3.80 us each.)
-constexpr unsigned kStreamFlag = 0x80000000u;
+// kAnyPitchFlag beside it: a launch of the strip form whose source rows do not share their alignment.
+constexpr unsigned kStreamFlag = 0x80000000u, kAnyPitchFlag = 0x40000000u;
 struct TileGeom {
     unsigned tiles_x, tiles_y, n_tiles;
     // floor(2^32 / tiles_x) + 1 when (t * magic) >> 32 == t / tiles_x for every tile number t of a plane, else 0: the

@@ -3379,6 +3379,8 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
         typename W::Params write;
     };
     FKD_NAME("Chain<" + R::name() + ",OpList<" + (sizeof...(Ops) ? OpList<Ops...>::names().substr(1) : std::string()) + ">," + W::name() + ">")
+    // Bits of Params::reserved, set by finalize_write.
+    static constexpr u32 kStripChecked = 1u, kStripAnyPitch = 2u;
 #if !defined(FKD_DEVICE_CODE)
     // Host, once the parameter block is filled: what only the whole chain knows about the values an operation receives.
     //
@@ -3419,17 +3421,17 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     static void finalize(Params& p) { finalize_from<0>(p); }
     // Host, once read AND write are filled in: bit 0 of `reserved` tells the launcher that every active plane meets what
     // the strip form of the bilinear kernel asks of its source and destination (that form has no other way to decline a
-    // plane) and that the launch is better off with it (strip_pays).  A parameter block that never came through here keeps the bit clear and gets the tile form.
+    // plane) and that the launch is better off with it (strip_pays); bit 1 that some plane's source rows do not share their
+    // alignment.  A parameter block that never came through here keeps the bits clear and gets the tile form.
     // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
     // phase_bound_for).
-    static constexpr u32 kStripChecked = 1u;
     static void finalize_write(Params& p) {
         if constexpr (any_x<R>() && has_row_phase<W>())
             p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
         if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {
             const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);
             if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value), W::row_grain(p.write, p.active_w, p.active_z)) && W::strip_ok(p.write) &&
-                (!any_pitch || R::strip_ok(p.read, true, p.active_z))) p.reserved |= kStripChecked;
+                (!any_pitch || R::strip_ok(p.read, true, p.active_z))) p.reserved |= kStripChecked | (any_pitch ? kStripAnyPitch : 0u);
         }
     }
 #endif
