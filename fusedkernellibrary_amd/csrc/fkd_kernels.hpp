@@ -90,7 +90,6 @@ template <class Chain> constexpr bool writer_streams() {
 
 constexpr int kRowsBX = 64;   // lanes along x: one wave per row segment
 constexpr int kRowsBY = 4;    // waves per workgroup
-constexpr unsigned long long kStreamElements = 1ull << 26;   // launches over more elements stream their input
 
 // For the test of what run-time compilation does with a chain whose per-thread array cannot stay in registers: with
 // FKD_TEST_UNRESOLVED_INDEX defined, the rows kernel indexes its values with an offset that is zero when the kernel runs
@@ -102,13 +101,13 @@ constexpr unsigned long long kStreamElements = 1ull << 26;   // launches over mo
 #endif
 
 // One wave's part of the rows kernel: V elements of each of ROWS rows per lane, row r from element x[r] on.  MODE as in
-// detail::load_run.  EDGE: the wave's segment of 64 * V elements, which begins at seg[r], reaches past the end of the row
+// detail::load_run for the loads; PLAIN: stores without the non-temporal hint.  EDGE: the wave's segment of 64 * V elements, which begins at seg[r], reaches past the end of the row
 // (kRowEnd: lanes that have no element inside are not here) or past either end (kRowEnds: all lanes of the wave are here).  A
 // lane that has fewer than V of its elements inside, or none, then works on the first or last V elements of the row, and only
 // the elements of the segment are stored; what a lane reads beside its own is not used or its neighbour's in the same wave,
 // so a chain that works in place is none the wiser.
 constexpr int kRowEnd = 1, kRowEnds = 2;
-template <class Chain, int V, int ROWS, int MODE, int EDGE = 0>
+template <class Chain, int V, int ROWS, int MODE, bool PLAIN, int EDGE = 0>
 __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 kernarg_offset, const int (&seg)[ROWS], const int (&x)[ROWS],
                                           int ybase, int z, int aw, int ah) {
     using R = typename Chain::Read;
@@ -133,6 +132,7 @@ __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 k
     Slot<typename Chain::Value> out[ROWS * V];
     if constexpr (Chain::kLongChain) Chain::template compute_run_kernarg<ROWS * V>(in, out, (const FKD_CONSTANT char*)__builtin_amdgcn_kernarg_segment_ptr() + kernarg_offset);
     else Chain::template compute_run<ROWS * V>(in, out, p.ops);
+    constexpr int STORE = MODE | (PLAIN ? detail::kPlainStores : 0);
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
         const int y = ybase + r;
@@ -144,7 +144,7 @@ __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 k
             W::template exec_edge<V>(seg[r], x0[r], aw, y, z, row, p.write);
         } else if constexpr (EDGE != 0) {
             if (x0[r] == x[r]) {
-                W::template exec_row<V, MODE>(x0[r], y, z, row, p.write);
+                W::template exec_row<V, STORE>(x0[r], y, z, row, p.write);
             } else if (EDGE == kRowEnd || (x[r] > -V && x[r] < aw)) {
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
@@ -153,7 +153,7 @@ __device__ __forceinline__ void rows_full(const typename Chain::Params& p, u32 k
                 }
             }
         } else {
-            W::template exec_row<V, MODE>(x0[r], y, z, row, p.write);
+            W::template exec_row<V, STORE>(x0[r], y, z, row, p.write);
         }
     }
 }
@@ -178,8 +178,13 @@ template <class Chain> constexpr bool rows_in_bands() {
 // `kernarg_offset`: where p sits inside the kernel-argument segment (0 when the chain's parameter block is the
 // kernel's first argument); long chains fetch their operations' parameters from there.  BANDS: the launch has the bands
 // form of grid (see rows_band_chunk).
-// SHIFT: the launch's grid has room for segments that begin left of a row (Chain::row_phase_bound).
-template <class Chain, int V, int ROWS, bool ALIGNED, bool BANDS = false, bool SHIFT = false>
+// FORM: the form of the launch (rows_form); kRowsOpen also for the chains of a divergent launch, whose forms are not known when the
+// kernel is compiled.  The forms are kernels of their own: in one for all of them, three to five times as long, small launches took 2 to
+// 5 % longer (30 operations on 1544x90 floats 2.31 us instead of 2.20), and without a form for small outputs 15 % (see kSmallOutputBytes).
+template <class Chain> constexpr bool rows_may_stream(int v) {
+    return !Chain::kLongChain && !detail::wave_exchange_ok<typename Chain::Read::Out>(v) && !detail::wave_exchange_ok<typename Chain::Write::In>(v);
+}
+template <class Chain, int V, int ROWS, bool ALIGNED, bool BANDS = false, int FORM = kRowsOpen>
 __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     using R = typename Chain::Read;
     using W = typename Chain::Write;
@@ -199,16 +204,15 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     }
     // Wave-cooperative accesses (mode 2 of load_run / store_run) need every lane of the wave on a full run.
     constexpr bool kExchange = (detail::wave_exchange_ok<typename R::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
-    // A launch over more elements than the last-level cache could hold between two launches reads them with the
-    // non-temporal hint (100 images of 1920x1080 uchar3: 225 -> 209 us); smaller inputs are left to the caches, where a
-    // pipeline's previous stage may have put them (the hint costs 15 % on a 33 MB image that is still cached).
-    constexpr bool kMayStream = !Chain::kLongChain && !kExchange;
+    constexpr int KIND = FORM & 7;
+    constexpr bool kOpen = KIND == kRowsOpen, kStream = (FORM & kRowsStream) != 0, kPlain = (FORM & kRowsPlain) != 0;
+    constexpr bool kMayStream = kOpen && !kPlain && rows_may_stream<Chain>(V);
     const bool stream = kMayStream && (unsigned long long)(u32(aw)) * u32(ah) * gridDim.z > kStreamElements;
-    if constexpr (rows_any_x<Chain>(V)) {
+    if constexpr (rows_any_x<Chain>(V) && KIND != kRowsNarrow) {
         // A wave owns a segment of 64 * V elements of a row.  Segments are counted from the row's start or, in launches with
         // room for it (row_phase_bound), from the last line boundary before it, so that every wave but the two at a row's ends
         // stores whole lines: a line shared by two waves leaves the chip as two partial writes.
-        if (aw >= V) {
+        if (!kOpen || aw >= V) {
             const int yw = (block_y * kRowsBY + __builtin_amdgcn_readfirstlane(int(threadIdx.y))) * ROWS;
             if (yw >= ah) return;
             constexpr int kWhole = kExchange ? 2 | detail::kAnyAlign : 0;
@@ -217,26 +221,24 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
             auto go = [&](auto edge_tag) {
                 constexpr int EDGE = decltype(edge_tag)::value;
                 if constexpr (kMayStream) {
-                    if (stream) { rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | 4, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
+                    if (stream) { rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | 4, false, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
                 }
-                rows_full<Chain, V, ROWS, EDGE ? 0 : kWhole, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah);
+                rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | (kStream ? 4 : 0), kPlain, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah);
             };
-            if constexpr (SHIFT && has_row_phase<W>()) {
+            if constexpr (KIND == kRowsLines && has_row_phase<W>()) {
                 const u32 bound = Chain::row_phase_bound(p.reserved);
-                if (bound != 0u) {
-                    bool outside = true;
+                bool outside = true;
 #pragma unroll
-                    for (int r = 0; r < ROWS; ++r) {
-                        const int phase = W::row_phase(yw + r < ah ? yw + r : ah - 1, z, p.write) & int(bound);
-                        seg[r] = int(block_x) * kRowsBX * V - (phase % x_group<R>() == 0 ? phase : 0);
-                        whole = whole && seg[r] >= 0 && seg[r] + kRowsBX * V <= aw;
-                        outside = outside && seg[r] >= aw;
-                        x[r] = seg[r] + int(threadIdx.x) * V;
-                    }
-                    if (outside) return;                                   // (wave uniform, as `whole`)
-                    if (whole) go(IntTag<0>{}); else go(IntTag<kRowEnds>{});
-                    return;
+                for (int r = 0; r < ROWS; ++r) {
+                    const int phase = W::row_phase(yw + r < ah ? yw + r : ah - 1, z, p.write) & int(bound);
+                    seg[r] = int(block_x) * kRowsBX * V - (phase % x_group<R>() == 0 ? phase : 0);
+                    whole = whole && seg[r] >= 0 && seg[r] + kRowsBX * V <= aw;
+                    outside = outside && seg[r] >= aw;
+                    x[r] = seg[r] + int(threadIdx.x) * V;
                 }
+                if (outside) return;                                       // (wave uniform, as `whole`)
+                if (whole) go(IntTag<0>{}); else go(IntTag<kRowEnds>{});
+                return;
             }
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) { seg[r] = int(block_x) * kRowsBX * V; x[r] = seg[r] + int(threadIdx.x) * V; }
@@ -257,14 +259,14 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
         if constexpr (!rows_any_x<Chain>(V)) {
             if constexpr (kExchange) {
                 if (int(block_x * kRowsBX + kRowsBX) * V <= aw) {
-                    rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign>(p, kernarg_offset, same, same, ybase, z, aw, ah);
+                    rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign, kPlain>(p, kernarg_offset, same, same, ybase, z, aw, ah);
                     return;
                 }
             }
             if constexpr (kMayStream) {
-                if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4>(p, kernarg_offset, same, same, ybase, z, aw, ah); return; }
+                if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4, false>(p, kernarg_offset, same, same, ybase, z, aw, ah); return; }
             }
-            rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0>(p, kernarg_offset, same, same, ybase, z, aw, ah);
+            rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0, kPlain>(p, kernarg_offset, same, same, ybase, z, aw, ah);
         }
     } else {
         for (int r = 0; r < ROWS; ++r) {
@@ -282,9 +284,9 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     }
 }
 
-template <class Chain, int V, int ROWS, bool ALIGNED>
+template <class Chain, int V, int ROWS, bool ALIGNED, int FORM>
 __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_rows(const typename Chain::Params p, const TileGeom g) {
-    rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), true>(p, 0u, &g);
+    rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
 }
 
 // Whether the rows of plane z of the read and of the write all start on dword boundaries, decided on the device
@@ -298,13 +300,13 @@ template <class Op, class P> FKD_DEV bool write_plane_aligned(const P& p, int z)
     if constexpr (requires { Op::plane_rows_aligned(p, z); }) return Op::plane_rows_aligned(p, z);
     else return Op::rows_aligned(p);
 }
-template <class Chain, int V, int ROWS, bool BANDS = false, bool SHIFT = false>
+template <class Chain, int V, int ROWS, bool BANDS = false, int FORM = kRowsOpen>
 __device__ __forceinline__ void rows_auto_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     const int z = blockIdx.z;
-    if constexpr (rows_any_x<Chain>(V)) { rows_body<Chain, V, ROWS, false, BANDS, SHIFT>(p, kernarg_offset, bands); return; }
+    if constexpr (rows_any_x<Chain>(V)) { rows_body<Chain, V, ROWS, false, BANDS, FORM>(p, kernarg_offset, bands); return; }
     const bool aligned = read_plane_aligned<typename Chain::Read>(p.read, z) && write_plane_aligned<typename Chain::Write>(p.write, z);
-    if (aligned) rows_body<Chain, V, ROWS, true, BANDS>(p, kernarg_offset, bands);
-    else rows_body<Chain, V, ROWS, false, BANDS>(p, kernarg_offset, bands);
+    if (aligned) rows_body<Chain, V, ROWS, true, BANDS, FORM>(p, kernarg_offset, bands);
+    else rows_body<Chain, V, ROWS, false, BANDS, FORM>(p, kernarg_offset, bands);
 }
 
 // ---- gather bilinear kernel ----------------------------------------------------------------------------
@@ -981,15 +983,29 @@ template <class D> __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_diverg
 
 // The one kernel of a chain compiled at run time, and what its launcher needs to know about it.  A launcher that
 // only has the parameter block as bytes reads the active grid from its first three words.
+// Which kernels the chain has for the forms of a launch of the rows kernel, 0 when it has one for all launches.
+template <class Chain> constexpr u32 rows_forms() {
+    if constexpr (IsDivergent<Chain>::value) return 0u;
+    else if constexpr (is_gather_chain<Chain>()) return 0u;
+    else if constexpr (!rows_any_x<Chain>(RowsConfig<Chain>::V)) return kRowsForms;
+    else return kRowsForms | kRowsAnyX | (has_row_phase<typename Chain::Write>() ? kRowsHasLines : 0u) | (rows_may_stream<Chain>(RowsConfig<Chain>::V) ? kRowsMayStream : 0u);
+}
+// Whether form FORM is one of them.
+template <class Chain, int FORM> constexpr bool rows_has_form() {
+    constexpr u32 forms = rows_forms<Chain>();
+    if constexpr ((forms & kRowsForms) == 0u) return false;
+    else if constexpr ((forms & kRowsAnyX) == 0u) return (FORM & 7) == kRowsOpen;
+    else return (FORM & 7) != kRowsOpen && ((FORM & kRowsStream) == 0 || (forms & kRowsMayStream) != 0u) && ((FORM & 7) != kRowsLines || (forms & kRowsHasLines) != 0u);
+}
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
-                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u,
+                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u, rows_forms<Chain>(),
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
@@ -1014,7 +1030,10 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
         }
         gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, false>(p, g);
     }
-    else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), true>(p, 0u, &g);
+}
+// The kernel of one form of the rows kernel (nothing for chains that do not have it).
+template <class Chain, int FORM> __device__ __forceinline__ void jit_rows_body(const typename Chain::Params& p, const TileGeom& g) {
+    if constexpr (rows_has_form<Chain, FORM>()) rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
 }
 
 } // namespace fkd

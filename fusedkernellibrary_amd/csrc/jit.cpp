@@ -27,6 +27,7 @@
 #include <sys/stat.h>
 #include <unistd.h>
 
+#include <array>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -46,12 +47,22 @@ using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
+// A module's kernels: the chain's own (bilinear and divergent launches) and one for each form of the rows kernel; a chain has the one
+// or some of the others (JitMeta::rows_forms), the rest are empty.
+struct JitForm { int form; const char* suffix; };
+constexpr JitForm kJitForms[] = {{-1, ""}, {fkd::kRowsRuns, "_runs"}, {fkd::kRowsRuns | fkd::kRowsPlain, "_runs_plain"}, {fkd::kRowsLines, "_lines"},
+                                 {fkd::kRowsNarrow, "_narrow"}, {fkd::kRowsRuns | fkd::kRowsStream, "_runs_stream"},
+                                 {fkd::kRowsLines | fkd::kRowsStream, "_lines_stream"}, {fkd::kRowsOpen, "_open"},
+                                 {fkd::kRowsOpen | fkd::kRowsPlain, "_open_plain"}};
+constexpr size_t kJitFormCount = sizeof(kJitForms) / sizeof(kJitForms[0]);
+using JitFunctions = std::array<hipFunction_t, kJitFormCount>;
+
 struct JitKernel {
     std::string signature;
     std::vector<char> code;
     JitMeta meta{};
     std::mutex mu;
-    std::unordered_map<int, hipFunction_t> per_device;   // a module is loaded once per device that launches it
+    std::unordered_map<int, JitFunctions> per_device;    // a module is loaded once per device that launches it
 };
 
 thread_local std::string g_log;
@@ -184,19 +195,31 @@ void write_file(const std::string& path, const std::vector<char>& data) {
     if (close(fd) != 0 || !ok || rename(tmp.c_str(), path.c_str()) != 0) unlink(tmp.c_str());
 }
 
-int get_function(JitKernel* k, hipFunction_t* fn) {
+hipError_t get_functions(hipModule_t mod, const std::string& signature, JitFunctions* fns) {
+    const std::string name = kernel_symbol(signature);
+    for (size_t i = 0; i < kJitFormCount; ++i) {
+        const hipError_t e = hipModuleGetFunction(&(*fns)[i], mod, (name + kJitForms[i].suffix).c_str());
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+int get_function(JitKernel* k, int form, hipFunction_t* fn) {
+    size_t index = 0;
+    while (index < kJitFormCount && kJitForms[index].form != form) ++index;
+    if (index == kJitFormCount) return int(hipErrorInvalidValue);
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return int(e);
     std::lock_guard<std::mutex> lock(k->mu);
     const auto it = k->per_device.find(dev);
-    if (it != k->per_device.end()) { *fn = it->second; return FKLHIP_OK; }
+    if (it != k->per_device.end()) { *fn = it->second[index]; return FKLHIP_OK; }
     hipModule_t mod = nullptr;
     if ((e = hipModuleLoadData(&mod, k->code.data())) != hipSuccess) return int(e);
-    hipFunction_t f = nullptr;
-    if ((e = hipModuleGetFunction(&f, mod, kernel_symbol(k->signature).c_str())) != hipSuccess) return int(e);
-    k->per_device.emplace(dev, f);   // the module stays loaded for the life of the process
-    *fn = f;
+    JitFunctions fns{};
+    if ((e = get_functions(mod, k->signature, &fns)) != hipSuccess) return int(e);
+    k->per_device.emplace(dev, fns);   // the module stays loaded for the life of the process
+    *fn = fns[index];
     return FKLHIP_OK;
 }
 
@@ -250,7 +273,8 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     if (grid[1] > 65535u || grid[2] > 65535u) return int(hipErrorInvalidConfiguration);
     if (m.max_planes != 0 && grid[2] > m.max_planes) return int(hipErrorInvalidConfiguration);   // as launch_divergent
     hipFunction_t fn = nullptr;
-    const int rc = get_function(k, &fn);
+    const int form = m.rows_forms != 0u ? fkd::rows_form(active[0], active[1], active[2], active[3], m.v, m.rows_forms) : -1;
+    const int rc = get_function(k, form, &fn);
     if (rc != FKLHIP_OK) return rc;
     // Kernel-argument segment: the parameter block, then the TileGeom at the next 4-byte boundary.  The runtime
     // copies the buffer during the call, so the caller's block may go away as soon as we return.
@@ -287,6 +311,10 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
         src += "(const JitChain::Params p, const TileGeom g) {\n"
                "    jit_body<JitChain>(p, g);\n"
                "}\n";
+        for (size_t i = 1; i < kJitFormCount; ++i) {
+            src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitForms[i].suffix +
+                   "(const JitChain::Params p, const TileGeom g) { jit_rows_body<JitChain, " + std::to_string(kJitForms[i].form) + ">(p, g); }\n";
+        }
         hiprtcProgram prog = nullptr;
         hiprtcResult r = hiprtcCreateProgram(&prog, src.c_str(), "fkd_jit_chain.hip", kJitHeaderCount, kJitHeaderTexts, kJitHeaderNames);
         if (r != HIPRTC_SUCCESS) { g_log = hiprtcGetErrorString(r); delete k; return FKLHIP_EUNKNOWN_SIGNATURE; }
@@ -326,8 +354,8 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
     if (e == hipSuccess) e = hipModuleGetGlobal(&meta_ptr, &meta_bytes, mod, "fkd_jit_meta");
     if (e == hipSuccess && meta_bytes != sizeof(JitMeta)) e = hipErrorInvalidValue;
     if (e == hipSuccess) e = hipMemcpyDtoH(&k->meta, meta_ptr, sizeof(JitMeta));
-    hipFunction_t fn = nullptr;
-    if (e == hipSuccess) e = hipModuleGetFunction(&fn, mod, kernel_symbol(k->signature).c_str());
+    JitFunctions fns{};
+    if (e == hipSuccess) e = get_functions(mod, k->signature, &fns);
     if (e != hipSuccess) {
         if (mod) hipModuleUnload(mod);
         delete k;
@@ -352,7 +380,10 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
     // once more with such arrays moved to LDS, which is the faster of the two homes, and the note goes into the log; with
     // FKLHIP_JIT_STRICT=1 it is refused like there.
     int scratch_bytes = 0;
-    if (hipFuncGetAttribute(&scratch_bytes, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, fn) != hipSuccess) scratch_bytes = 0;
+    for (hipFunction_t fn : fns) {
+        int needs = 0;
+        if (hipFuncGetAttribute(&needs, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, fn) == hipSuccess && needs > scratch_bytes) scratch_bytes = needs;
+    }
     if (scratch_bytes > 0) {
         const char* strict = getenv("FKLHIP_JIT_STRICT");
         const std::string note = "the compiled chain needs " + std::to_string(scratch_bytes) + " bytes of scratch memory per lane";
@@ -378,7 +409,7 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
     if (!from_cache && !cached.empty() && !arrays_to_lds) write_file(cached, k->code);
     int dev = 0;
     hipGetDevice(&dev);
-    k->per_device.emplace(dev, fn);
+    k->per_device.emplace(dev, fns);
     register_chain(k->signature.c_str(), k->meta.params_bytes, &jit_launch, k);
     return FKLHIP_OK;
 }

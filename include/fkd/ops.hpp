@@ -37,8 +37,9 @@ namespace detail {
 // How a run of elements is accessed (the mode of exec_row, load_run and store_run; p is the run's address).  Low two bits: 0:
 // nothing is known about p.  1: p is dword aligned.  2: all 64 lanes of the wave are in this
 // call with consecutive runs (lane i at p0 + i * V elements), and p is dword aligned unless kAnyAlign is set.  Bit 2 (value
-// 4): the launch reads more than the caches hold, loads carry the non-temporal hint.
-constexpr int kAnyAlign = 16;
+// 4): the launch reads more than the caches hold, loads carry the non-temporal hint.  kPlainStores: the launch writes little
+// (kSmallOutputBytes), stores carry no hint.
+constexpr int kAnyAlign = 16, kPlainStores = 32;
 constexpr bool aligned_mode(int mode) { return (mode & 3) != 0 && (mode & kAnyAlign) == 0; }
 } // namespace detail
 
@@ -200,9 +201,11 @@ typedef u32 u32x4_t __attribute__((ext_vector_type(4)));
 // One store of 1-4 whole dwords (or one element).  Output is written once and not read again by the kernel, so the stores carry
 // the non-temporal hint: the L2s then hand the lines on early instead of keeping them dirty until the kernel ends,
 // when all of them would have to be written back at once (a 3840x2160 float copy: 10.6 -> 9.9 us).
-template <int ALIGN, class Q, class P> FKD_DEV void gstore(P* p, const Q& v) {
+// Not in launches that write little (PLAIN, see kSmallOutputBytes): they end sooner with their lines left in the L2s.
+template <int ALIGN, bool PLAIN = false, class Q, class P> FKD_DEV void gstore(P* p, const Q& v) {
     typedef Q At __attribute__((aligned(ALIGN)));
-    __builtin_nontemporal_store(v, (FKD_GLOBAL At*)p);
+    if constexpr (PLAIN) *(FKD_GLOBAL At*)p = v;
+    else __builtin_nontemporal_store(v, (FKD_GLOBAL At*)p);
 }
 // One element of 4 or 8 bytes written through the L2 (a relaxed store at system scope: global_store ... sc0 sc1), for
 // writers whose lanes each store single elements: the planar writer of the bilinear kernel runs configuration 3 in
@@ -262,22 +265,22 @@ template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_wor
         }
     }
 }
-template <int W, bool ALIGNED = true> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
+template <int W, bool ALIGNED = true, bool PLAIN = false> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
     constexpr int ALIGN = ALIGNED ? 4 : 1;
     static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
-        gstore<ALIGN>(p, w[0]);
+        gstore<ALIGN, PLAIN>(p, w[0]);
     } else if constexpr (W == 2) {
         u32x2_t v; v.x = w[0]; v.y = w[1];
-        gstore<ALIGN>(p, v);
+        gstore<ALIGN, PLAIN>(p, v);
     } else if constexpr (W == 3) {
         u32x3_t v; v.x = w[0]; v.y = w[1]; v.z = w[2];
-        gstore<ALIGN>(p, v);
+        gstore<ALIGN, PLAIN>(p, v);
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
             u32x4_t v; v.x = w[4 * i]; v.y = w[4 * i + 1]; v.z = w[4 * i + 2]; v.w = w[4 * i + 3];
-            gstore<ALIGN>(gmut<u32x4_t>(p) + i, v);
+            gstore<ALIGN, PLAIN>(gmut<u32x4_t>(p) + i, v);
         }
     }
 }
@@ -394,7 +397,7 @@ template <int W, bool STREAM, bool ALIGNED> FKD_DEV void load_words_wave(const v
         w[4 * j] = v.x; w[4 * j + 1] = v.y; w[4 * j + 2] = v.z; w[4 * j + 3] = v.w;
     }
 }
-template <int W, bool ALIGNED> FKD_DEV void store_words_wave(void* p, const u32 (&w)[W]) {
+template <int W, bool ALIGNED, bool PLAIN = false> FKD_DEV void store_words_wave(void* p, const u32 (&w)[W]) {
     const u32 lane = threadIdx.x;
     u32* stage = wave_stage();
     char* seg = reinterpret_cast<char*>(p) - size_t(lane) * (W * 4);
@@ -407,7 +410,7 @@ template <int W, bool ALIGNED> FKD_DEV void store_words_wave(void* p, const u32 
     wave_exchange_fence();
 #pragma unroll
     for (int k = 0; k < W / 4; ++k)
-        gstore<ALIGNED ? 4 : 1>(seg + k * 1024 + lane * 16, *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
+        gstore<ALIGNED ? 4 : 1, PLAIN>(seg + k * 1024 + lane * 16, *reinterpret_cast<const u32x4_t*>(stage + stage_at<W>(u32(k) * 256u + lane * 4u)));
 }
 
 template <class T, int V, int MODE_BITS> FKD_DEV void load_run(const T* p, Slot<T> (&out)[V]) {
@@ -437,12 +440,12 @@ template <class T, int V, int MODE_BITS> FKD_DEV void load_run(const T* p, Slot<
 }
 template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot<T> (&in)[V]) {
     constexpr int MODE = MODE_BITS & 3;
-    constexpr bool ALIGNED = aligned_mode(MODE_BITS);
+    constexpr bool ALIGNED = aligned_mode(MODE_BITS), PLAIN = (MODE_BITS & kPlainStores) != 0;
     if constexpr (MODE == 2 && wave_exchange_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
         pack_words<T, V, W>(in, w);
-        store_words_wave<W, ALIGNED>(p, w);
+        store_words_wave<W, ALIGNED, PLAIN>(p, w);
     } else if constexpr (wide_ok<T>(V)) {
         constexpr int W = int(sizeof(T)) * V / 4;
         u32 w[W];
@@ -453,7 +456,7 @@ template <class T, int V, int MODE_BITS> FKD_DEV void store_run(T* p, const Slot
 #pragma unroll
             for (int i = 0; i < W; ++i) asm("" : "+v"(w[i]));
         }
-        store_words<W, ALIGNED>(p, w);
+        store_words<W, ALIGNED, PLAIN>(p, w);
     } else {
 #pragma unroll
         for (int i = 0; i < V; ++i) store_elem(p + i, in[i].v);
@@ -3178,7 +3181,7 @@ template <int PF> struct WriteYUV {
                 Slot<B> luma[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) luma[i].v = v[i].v.x;
-                detail::store_run<B, 4, 0>(reinterpret_cast<B*>(r.row) + x, luma);
+                detail::store_run<B, 4, A & detail::kPlainStores>(reinterpret_cast<B*>(r.row) + x, luma);
                 if (r.chroma_row) {
                     Slot<B> pairs[4];
 #pragma unroll
@@ -3187,7 +3190,7 @@ template <int PF> struct WriteYUV {
                         pairs[2 * k].v = L::kSwapUV ? from.z : from.y;
                         pairs[2 * k + 1].v = L::kSwapUV ? from.y : from.z;
                     }
-                    detail::store_run<B, 4, 0>(reinterpret_cast<B*>(r.crow) + x, pairs);
+                    detail::store_run<B, 4, A & detail::kPlainStores>(reinterpret_cast<B*>(r.crow) + x, pairs);
                 }
             } else {
                 u32 g[2 * S];
@@ -3204,7 +3207,7 @@ template <int PF> struct WriteYUV {
 #pragma unroll
                     for (int i = 0; i < S; ++i) { asm("" : "+v"(w[i])); g[k * S + i] = w[i]; }
                 }
-                detail::store_words<2 * S, false>(r.row + size_t(x) * 2 * S, g);
+                detail::store_words<2 * S, false, (A & detail::kPlainStores) != 0>(r.row + size_t(x) * 2 * S, g);
             }
         } else {
             put_run<V>(r, x, v);
@@ -3425,7 +3428,9 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     // alignment.  A parameter block that never came through here keeps the bits clear and gets the tile form.
     // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
     // phase_bound_for).
+    // Bit 2: the launch writes no more than kSmallOutputBytes.
     static void finalize_write(Params& p) {
+        if ((unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value) <= kSmallOutputBytes) p.reserved |= kSmallOutputBit;
         if constexpr (any_x<R>() && has_row_phase<W>())
             p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
         if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {

@@ -259,3 +259,65 @@ def test_line_aligned_segments_tensors(device, kind, half, in_place):
     assert last_launch()["grid"][0] == (4 if half else 9)
     out_at[:] = data
     assert np.array_equal(out.cpu().numpy(), out_host)             # the rows are the input's, every byte beside them is as it was
+
+
+# Launches that write up to 4 MiB (as the chain's values count) store without the non-temporal hint, larger ones with it: both sides of
+# the line, in widths below those of line-aligned segments, whole runs and remainders.
+@pytest.mark.parametrize("w,h", [(300, 1165), (300, 1166), (299, 1168), (299, 1170), (301, 1161), (301, 1162)])
+def test_small_and_larger_outputs(device, w, h):
+    import torch
+    rng = np.random.RandomState(w + h)
+    mul, add = rng.uniform(0.5, 2.0, (4, 3)).astype(np.float32), rng.uniform(-64, 64, (4, 3)).astype(np.float32)
+    imgs = [rng.randint(0, 256, (h, w, 3)).astype(np.uint8) for _ in range(4)]                   # 4 194 000 ... 4 197 600 bytes
+    srcs = [Placed((h, w, 3), np.uint8, 0, 0, device, a) for a in imgs]
+    outs = [Placed((h, w, 3), np.uint8, 0, 0, device) for _ in imgs]
+    cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [o.view() for o in outs])
+    fh = 3 * h                                                                                 # as many bytes of floats
+    img = rng.uniform(-1, 1, (fh, w)).astype(np.float32)
+    src, out = Placed((fh, w), np.float32, 4, 0, device, img), Placed((fh, w), np.float32, 8, 0, device)
+    cases.add_mul_chain(src.view(), 3, 0.5, 1.0001, out.view())
+    padded = torch.zeros((4 * h, w, 3), dtype=torch.uint8, device=device)                      # a kernel for whole runs only
+    cases.pad(srcs[0].view(), ol.BORDER_REFLECT_101, 8, 8, padded)
+    torch.cuda.synchronize()
+    for b, c in zip(outs, ol.oracle_batch_muladd_sat(imgs, mul, add)):
+        assert np.array_equal(b.read(), c)
+    assert out.read().tobytes() == ol.oracle_add_mul_chain(img, 3, np.float32(0.5), np.float32(1.0001)).tobytes()
+    assert padded.cpu().numpy().tobytes() == ol.oracle_pad(imgs[0], ol.BORDER_REFLECT_101, 8, 8, w, 4 * h).tobytes()
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_P010, 0, 2), (ol.PF_UYVY, 1, 1)])
+@pytest.mark.parametrize("w,h", [(300, 1164), (300, 1166), (254, 1376), (258, 1356)])
+def test_small_and_larger_video_frames(device, pf, cr, cp, w, h):
+    """Decoded to float3 (12 bytes a pixel) and encoded from RGB (3 or 6 bytes a pixel): chains compiled ahead of time and on first use."""
+    import torch
+    dt, size = (np.uint16, 2) if ol.PF_WIDE[pf] else (np.uint8, 1)
+    rng = np.random.RandomState(w + pf)
+    rows, cols = ol.frame_shape(pf, w, h)
+    buf = rng.randint(0, 1024 if size == 2 else 256, (rows, cols)).astype(dt)
+    frame, out = Placed((rows, cols), dt, 0, 0, device, buf), Placed((h, w, 3), np.float32, 4, 0, device)
+    cases.yuv_to_rgb(pf, cr, cp, frame.view(), w, h, out.view())
+    eh = 4 * h // size                                                                         # as many bytes of samples
+    rgb = rng.randint(0, 1024 if size == 2 else 256, (eh, w, 3)).astype(dt)
+    rows, cols = ol.frame_shape(pf, w, eh)
+    start = np.full((rows, cols), 9, dt)
+    encoded, src = Placed((rows, cols), dt, 0, 0, device, start), Placed((eh, w, 3), dt, 0, 0, device, rgb)
+    cases.rgb_to_yuv(pf, cr, {ol.PF_UYVY: 2}.get(pf, cp), src.view(), encoded.view())
+    torch.cuda.synchronize()
+    assert out.read().tobytes() == ol.oracle_yuv_to_rgb(pf, cr, cp, buf, w, h).tobytes()
+    assert np.array_equal(encoded.read(), ol.oracle_rgb_to_yuv(pf, cr, {ol.PF_UYVY: 2}.get(pf, cp), rgb, start))
+
+
+@pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_NV21, 0, 0), (ol.PF_P010, 0, 2)])
+def test_video_frames_of_odd_width_to_rgb(device, pf, cr, cp):
+    """The last four pixels of a row of odd width begin inside a chroma pair."""
+    import torch
+    dt = np.uint16 if ol.PF_WIDE[pf] else np.uint8
+    rng = np.random.RandomState(170 + pf)
+    for n, w in enumerate((1, 3, 5, 7, 9, 255, 257, 259, 511, 515, 1021)):
+        h = (2, 6, 12)[n % 3]
+        rows, cols = ol.frame_shape(pf, w + 1, h)
+        buf = rng.randint(0, 1024 if ol.PF_WIDE[pf] else 256, (rows, cols)).astype(dt)
+        frame, out = Placed((rows, cols), dt, 0, 0, device, buf), Placed((h, w, 3), np.float32, 4, 4, device)
+        cases.yuv_to_rgb(pf, cr, cp, frame.view(), w, h, out.view())
+        torch.cuda.synchronize()
+        assert out.read().tobytes() == ol.oracle_yuv_to_rgb(pf, cr, cp, buf, w + 1, h)[:, :w].tobytes(), (w, h)
