@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52051000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "a3274910807c8743629e353cfdea6215e91a157008f51330b52800c0e74b67ca"
+TRAFFIC_C3_SOURCES_SHA256 = "bb166f45573af32b364382b208441838b06432425639e0e2d5620ea31ac8edac"
 
 
 def device_sources_sha256():
