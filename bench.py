@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52051000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "bb166f45573af32b364382b208441838b06432425639e0e2d5620ea31ac8edac"
+TRAFFIC_C3_SOURCES_SHA256 = "b74e3d4283c34466eb88eea64e0e622a185ac91e98107a5431e709de48697b13"
 
 
 def device_sources_sha256():

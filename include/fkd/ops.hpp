@@ -3347,9 +3347,10 @@ template <class I, class P, class O> struct IsDivOp<Div<I, P, O>> { static const
 //   Others: rows of one step the strip form (20x5625 87 / 41, 28x4017 58 / 29), longer ones the tile form (36x5208 75 / 79,
 //   60x1875 32 / 43, 100x1125 27 / 50, 200x625 26 / 45, 225x555 33 / 63).
 //  Smaller outputs, rows of six to eight steps that are no whole 32-byte sectors: from a size on the tile form, later for fewer steps
-//   and for rows of whole 16 bytes.  6 steps, 165 wide: 1.8 M pixels 9.0 / 8.7, 2.5 M 11.3 / 11.4, 3.2 M 13.5 / 14.4; 180 wide: 3.2 M 13.2 / 12.8,
-//   5.2 M 18.4 / 17.8.  7 steps, 197 wide: 1.4 M 7.2 / 6.9, 1.6 M 7.4 / 7.6, 2.4 M 9.8 / 10.7; 220 wide: 2.0 M 8.6 / 8.1, 2.4 M 9.7 / 9.9, 5.2 M 16.8 / 17.6.
-//   8 steps, 250 wide: 1.2 M 6.5 / 6.2, 1.4 M 6.6 / 6.8, 3.2 M 12.0 / 13.6; 236 wide: 1.6 M 7.3 / 7.2, 1.8 M 7.5 / 7.8, 3.2 M 11.3 / 11.8.  Whole
+//   and for rows of whole 16 bytes.  6 steps, 165 wide: 1.8 M pixels 9.1 / 8.7, 2.5 M 11.3 / 11.4, 3.2 M 13.2 / 14.1; 180 wide: 2.3 M 10.2 / 9.5,
+//   2.5 M 10.1 / 10.1, 3.2 M 12.2 / 12.7.  7 steps, 197 wide: 1.4 M 7.2 / 6.9, 1.6 M 7.4 / 7.5, 2.4 M 9.6 / 10.6; 204 wide: 1.8 M 8.3 / 7.8, 2.4 M
+//   9.6 / 9.7, 3.2 M 11.6 / 12.4.  8 steps, 250 wide: 1.2 M 6.5 / 6.2, 1.4 M 6.5 / 6.8, 3.2 M 11.9 / 13.6; 236 wide: 1.6 M 7.3 / 7.1, 1.8 M 7.5 / 7.7,
+//   2.4 M 8.7 / 9.6.  8 crops each cross earlier by up to a quarter (236 wide: 1.2 M 5.5 / 5.6, 1.6 M 6.4 / 6.9).  Whole
 //   sectors keep the strip form (200x117 6.8 / 6.1, 200x406 17.3 / 15.8).
 //  Images whose rows do not share their alignment (width 1279): 168x64 4.7 / 4.0, 224x64 4.75 / 4.2, 8 crops to 160x62 3.1 / 3.0, to 160x156 3.6 / 3.1;
 //   with six steps and more and less than a workgroup per compute unit a strip's row is one wave's alone: 8 crops to 200x60
@@ -3364,7 +3365,7 @@ inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes
     const bool many_steps = w > 160u, sectors = w % 8u == 0u, quads = w % 4u == 0u;
     if (any_pitch) return pixels >= 40000u && (!many_steps || (sectors && workgroups >= 256u));
     if (!many_steps || sectors) return true;
-    if (w <= 192u) return quads || pixels < 2400000u;
+    if (w <= 192u) return pixels < (quads ? 2800000u : 2400000u);
     if (w <= 224u) return pixels < (quads ? 2400000u : 1600000u);
     return pixels < (quads ? 1600000u : 1200000u);
 }

@@ -23,7 +23,7 @@ def test_alignment_of_output_rows(address, w, h, planes, grain):
     (200, 1092, 64, False, 32, False), (225, 1274, 64, True, 4, False),
     # smaller ones: images whose rows share their alignment
     (224, 224, 64, False, 128, True), (100, 200, 64, False, 16, True), (200, 406, 64, False, 32, True), (165, 170, 64, False, 4, True),
-    (165, 378, 64, False, 4, False), (180, 277, 64, False, 16, True), (197, 79, 64, False, 4, True), (197, 253, 64, False, 4, False),
+    (165, 378, 64, False, 4, False), (180, 156, 64, False, 16, True), (180, 277, 64, False, 16, False), (197, 79, 64, False, 4, True), (197, 253, 64, False, 4, False),
     (212, 132, 64, False, 16, True), (212, 383, 64, False, 16, False), (225, 83, 64, False, 4, True), (225, 222, 64, False, 4, False),
     (252, 86, 64, False, 16, True), (236, 211, 64, False, 16, False), (250, 800, 8, False, 8, False),
     # ... and images whose rows do not
