@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52051000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "b74e3d4283c34466eb88eea64e0e622a185ac91e98107a5431e709de48697b13"
+TRAFFIC_C3_SOURCES_SHA256 = "6e2e92cbaa314e895347ebc20b62830e0e6f48b26ba8a18cc0d42c94e53ec715"
 
 
 def device_sources_sha256():

@@ -30,10 +30,16 @@ struct TileGeom {
 // L2 they are kept by the 256 MB last-level cache, which pushes the source images out of it; every tap line then comes from
 // HBM between the writes, one isolated read at a time, and each costs the channel a turn from writing to reading and back.
 // 64 crops of a 3840x2160 image to 640x640 (314 MB out, 25 MB of source): 77 us written through, 60 us non-temporal, although
-// the stores alone take 55 us either way.  The line lies where the two cross (64 crops of a 1920x1080 image; written through /
-// non-temporal): 224x224, 38 MB 9.8 / 10.2 us; 288x288, 64 MB 14.4 / 14.6; 320x320, 79 MB 17.2 / 16.4; 384x384, 113 MB 26.9 /
-// 21.6; 512x512, 201 MB 48.8 / 35.1.
-constexpr unsigned long long kStreamOutputBytes = 64ull << 20;
+// the stores alone take 55 us either way.
+// The line lies where a program that fills three such outputs in turn crosses it: at a third of that cache.  64 crops of a 1280x853
+// image, written through / non-temporal: 224x457 (75 MiB) 15.8 / 16.1 us, 224x512 (84) 19.3 / 16.9, 224x670 (110) 26.3 / 21.4; rows of no
+// whole lines, whose partial lines cost more without the cache to gather them: 225x455 (75) 19.3 / 26.1, 225x509 (84) 30.2 / 28.2, 225x667
+// (110) 50 / 38, 36x2503 (66) 25.8 / 35.6.
+// What it costs: a program with one output buffer, which would have stayed in the cache up to twice that size, writes slower and finds
+// its output in HBM.  One buffer, launch alone: 224x670 19.6 / 21.2, 225x667 23.8 / 38.5; with a reader of the output (a conversion to
+// bfloat16) behind each launch: 224x670 49.4 / 50.8, 225x667 53.0 / 57.6, 500x436 (160) 71 / 80; from 190 MiB on even these gain (224x1401,
+// 230 MiB 110 / 97).  Three buffers with a reader: 225x667 67 / 64, 500x518 (190) 123 / 106.
+constexpr unsigned long long kStreamOutputBytes = 80ull << 20;
 // Launches of the rows kernel that write no more than this (as the chain's values count) store without the non-temporal hint: with it
 // a launch is not over before its last lines have left the chip.  us per launch, with the hint / without: 4 uchar3 images of 225x165
 // (0.4 MB) 2.32 / 2.01, of 943x179 (2.0 MB) 2.93 / 2.68, of 886x260 (2.8 MB) 3.21 / 2.97; 30 operations on 1544x90 floats (0.6 MB)
