@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52051000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "6e2e92cbaa314e895347ebc20b62830e0e6f48b26ba8a18cc0d42c94e53ec715"
+TRAFFIC_C3_SOURCES_SHA256 = "26987c59810a6ef57d35a3585dc564b54a5f83d81e13b0c267bcd60b2274192a"
 
 
 def device_sources_sha256():

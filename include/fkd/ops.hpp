@@ -3354,7 +3354,8 @@ template <class I, class P, class O> struct IsDivOp<Div<I, P, O>> { static const
 //   sectors keep the strip form (200x117 6.8 / 6.1, 200x406 17.3 / 15.8).
 //  Images whose rows do not share their alignment (width 1279): 168x64 4.7 / 4.0, 224x64 4.75 / 4.2, 8 crops to 160x62 3.1 / 3.0, to 160x156 3.6 / 3.1;
 //   with six steps and more and less than a workgroup per compute unit a strip's row is one wave's alone: 8 crops to 200x60
-//   3.1 / 3.6, to 256x120 3.2 / 3.7.  Launches below 40 000 pixels and rows of no whole sectors keep the tile form that such images
+//   3.1 / 3.6, to 256x120 3.2 / 3.7; and rows of no whole sectors that nearly fill the tile form's 128 columns are its own from a size
+//   on: 105x193 (1.3 M pixels) 8.1 / 7.6, 105x297 (2.0 M) 9.0 / 10.3, 125x437 12.5 / 15.0 (112x279 8.5 / 7.7, 95x328 9.9 / 9.7, 130x300 13.2 / 11.6).  Launches below 40 000 pixels and rows of no whole sectors keep the tile form that such images
 //   always had; the strip form would serve some of them better (8 crops to 64x39 3.0 / 2.2, 64 crops to 165x64 4.8 / 4.3, to 250x200 12.2 / 13.5).
 inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes, u32 row_grain) {
     const unsigned long long pixels = (unsigned long long)w * h * planes, workgroups = (unsigned long long)((h + 7u) / 8u) * planes;
@@ -3363,7 +3364,7 @@ inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes
         if (!(row_grain >= 128u || (row_grain >= 64u && idle_lanes) || w <= 32u)) return false;
     }
     const bool many_steps = w > 160u, sectors = w % 8u == 0u, quads = w % 4u == 0u;
-    if (any_pitch) return pixels >= 40000u && (!many_steps || (sectors && workgroups >= 256u));
+    if (any_pitch) return pixels >= 40000u && (many_steps ? sectors && workgroups >= 256u : sectors || w <= 96u || w > 128u || pixels < 1600000u);
     if (!many_steps || sectors) return true;
     if (w <= 192u) return pixels < (quads ? 2800000u : 2400000u);
     if (w <= 224u) return pixels < (quads ? 2400000u : 1600000u);

@@ -28,6 +28,7 @@ def test_alignment_of_output_rows(address, w, h, planes, grain):
     (252, 86, 64, False, 16, True), (236, 211, 64, False, 16, False), (250, 800, 8, False, 8, False),
     # ... and images whose rows do not
     (160, 200, 64, True, 128, True), (224, 224, 64, True, 128, True), (200, 60, 8, True, 32, False), (225, 60, 64, True, 4, False),
+    (105, 119, 64, True, 4, True), (125, 437, 64, True, 4, False), (112, 279, 64, True, 64, True), (130, 300, 64, True, 8, True),
     (64, 39, 8, True, 128, False), (64, 156, 8, True, 128, True)])
 def test_form_of_measured_launches(w, h, planes, any_pitch, grain, strip):
     assert cases.cases().fklcase_strip_pays(w, h, planes, int(any_pitch), grain) == int(strip)
