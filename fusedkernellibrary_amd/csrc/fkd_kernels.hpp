@@ -90,6 +90,7 @@ template <class Chain> constexpr bool writer_streams() {
 
 constexpr int kRowsBX = 64;   // lanes along x: one wave per row segment
 constexpr int kRowsBY = 4;    // waves per workgroup
+constexpr unsigned long long kStreamElements = 1ull << 26;   // launches over more elements stream their input
 
 // For the test of what run-time compilation does with a chain whose per-thread array cannot stay in registers: with
 // FKD_TEST_UNRESOLVED_INDEX defined, the rows kernel indexes its values with an offset that is zero when the kernel runs
@@ -101,7 +102,8 @@ constexpr int kRowsBY = 4;    // waves per workgroup
 #endif
 
 // One wave's part of the rows kernel: V elements of each of ROWS rows per lane, row r from element x[r] on.  MODE as in
-// detail::load_run for the loads; PLAIN: stores without the non-temporal hint.  EDGE: the wave's segment of 64 * V elements, which begins at seg[r], reaches past the end of the row
+// detail::load_run for the loads; PLAIN: stores without the non-temporal hint.
+// EDGE: the wave's segment of 64 * V elements, which begins at seg[r], reaches past the end of the row
 // (kRowEnd: lanes that have no element inside are not here) or past either end (kRowEnds: all lanes of the wave are here).  A
 // lane that has fewer than V of its elements inside, or none, then works on the first or last V elements of the row, and only
 // the elements of the segment are stored; what a lane reads beside its own is not used or its neighbour's in the same wave,
@@ -184,12 +186,12 @@ template <class Chain> constexpr bool rows_in_bands() {
 // `kernarg_offset`: where p sits inside the kernel-argument segment (0 when the chain's parameter block is the
 // kernel's first argument); long chains fetch their operations' parameters from there.  BANDS: the launch has the bands
 // form of grid (see rows_band_chunk).
-// FORM: the form of the launch (rows_form); kRowsOpen also for the chains of a divergent launch, whose forms are not known when the
-// kernel is compiled.  The forms are kernels of their own: in one for all of them, three to five times as long, small launches took 2 to
-// 5 % longer (30 operations on 1544x90 floats 2.31 us instead of 2.20), and without a form for small outputs 15 % (see kSmallOutputBytes).
-template <class Chain> constexpr bool rows_may_stream(int v) {
-    return !Chain::kLongChain && !detail::wave_exchange_ok<typename Chain::Read::Out>(v) && !detail::wave_exchange_ok<typename Chain::Write::In>(v);
-}
+// FORM: kRowsOpen serves every launch; kRowsLines as well, one whose grid has room for segments that begin left of a row
+// (Chain::row_phase_bound); kRowsSmall those of rows_small.  The latter is a kernel of its own, a third to a fifth as long: besides the
+// stores' hint (see kSmallOutputBytes) small launches lost 2 to 5 % to the length of the other one (30 operations on 1544x90 floats
+// 2.31 us instead of 2.20).  Larger launches gain nothing from shorter kernels of their own (50 operations at 3840x2160 12.1 -> 12.3 us, RGB
+// to NV12 6.9 -> 7.0).
+constexpr int kRowsOpen = 0, kRowsLines = 1, kRowsSmall = 2;
 template <class Chain, int V, int ROWS, bool ALIGNED, bool BANDS = false, int FORM = kRowsOpen>
 __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     using R = typename Chain::Read;
@@ -210,15 +212,17 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     }
     // Wave-cooperative accesses (mode 2 of load_run / store_run) need every lane of the wave on a full run.
     constexpr bool kExchange = (detail::wave_exchange_ok<typename R::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
-    constexpr int KIND = FORM & 7;
-    constexpr bool kOpen = KIND == kRowsOpen, kStream = (FORM & kRowsStream) != 0, kPlain = (FORM & kRowsPlain) != 0;
-    constexpr bool kMayStream = kOpen && !kPlain && rows_may_stream<Chain>(V);
+    // A launch over more elements than the last-level cache could hold between two launches reads them with the
+    // non-temporal hint (100 images of 1920x1080 uchar3: 225 -> 209 us); smaller inputs are left to the caches, where a
+    // pipeline's previous stage may have put them (the hint costs 15 % on a 33 MB image that is still cached).
+    constexpr bool kSmall = FORM == kRowsSmall;
+    constexpr bool kMayStream = !kSmall && !Chain::kLongChain && !kExchange;
     const bool stream = kMayStream && (unsigned long long)(u32(aw)) * u32(ah) * gridDim.z > kStreamElements;
-    if constexpr (rows_any_x<Chain>(V) && KIND != kRowsNarrow) {
+    if constexpr (rows_any_x<Chain>(V)) {
         // A wave owns a segment of 64 * V elements of a row.  Segments are counted from the row's start or, in launches with
         // room for it (row_phase_bound), from the last line boundary before it, so that every wave but the two at a row's ends
         // stores whole lines: a line shared by two waves leaves the chip as two partial writes.
-        if (!kOpen || aw >= V) {
+        if (kSmall || aw >= V) {
             const int yw = (block_y * kRowsBY + __builtin_amdgcn_readfirstlane(int(threadIdx.y))) * ROWS;
             if (yw >= ah) return;
             constexpr int kWhole = kExchange ? 2 | detail::kAnyAlign : 0;
@@ -229,25 +233,27 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
                 if constexpr (kMayStream) {
                     if (stream) { rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | 4, false, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
                 }
-                if constexpr (EDGE != 0 && !kOpen && x_group<R>() == 2 && V % 2 == 0) {
-                    if ((aw & 1) == 0) { rows_full<Chain, V, ROWS, kStream ? 4 : 0, kPlain, EDGE | kEvenWidth>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
+                if constexpr (EDGE != 0 && x_group<R>() == 2 && V % 2 == 0) {
+                    if ((aw & 1) == 0) { rows_full<Chain, V, ROWS, 0, kSmall, EDGE | kEvenWidth>(p, kernarg_offset, seg, x, yw, z, aw, ah); return; }
                 }
-                rows_full<Chain, V, ROWS, (EDGE ? 0 : kWhole) | (kStream ? 4 : 0), kPlain, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah);
+                rows_full<Chain, V, ROWS, EDGE ? 0 : kWhole, kSmall, EDGE>(p, kernarg_offset, seg, x, yw, z, aw, ah);
             };
-            if constexpr (KIND == kRowsLines && has_row_phase<W>()) {
+            if constexpr (FORM == kRowsLines && has_row_phase<W>()) {
                 const u32 bound = Chain::row_phase_bound(p.reserved);
-                bool outside = true;
+                if (bound != 0u) {
+                    bool outside = true;
 #pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    const int phase = W::row_phase(yw + r < ah ? yw + r : ah - 1, z, p.write) & int(bound);
-                    seg[r] = int(block_x) * kRowsBX * V - (phase % x_group<R>() == 0 ? phase : 0);
-                    whole = whole && seg[r] >= 0 && seg[r] + kRowsBX * V <= aw;
-                    outside = outside && seg[r] >= aw;
-                    x[r] = seg[r] + int(threadIdx.x) * V;
+                    for (int r = 0; r < ROWS; ++r) {
+                        const int phase = W::row_phase(yw + r < ah ? yw + r : ah - 1, z, p.write) & int(bound);
+                        seg[r] = int(block_x) * kRowsBX * V - (phase % x_group<R>() == 0 ? phase : 0);
+                        whole = whole && seg[r] >= 0 && seg[r] + kRowsBX * V <= aw;
+                        outside = outside && seg[r] >= aw;
+                        x[r] = seg[r] + int(threadIdx.x) * V;
+                    }
+                    if (outside) return;                                   // (wave uniform, as `whole`)
+                    if (whole) go(IntTag<0>{}); else go(IntTag<kRowEnds>{});
+                    return;
                 }
-                if (outside) return;                                       // (wave uniform, as `whole`)
-                if (whole) go(IntTag<0>{}); else go(IntTag<kRowEnds>{});
-                return;
             }
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) { seg[r] = int(block_x) * kRowsBX * V; x[r] = seg[r] + int(threadIdx.x) * V; }
@@ -268,14 +274,14 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
         if constexpr (!rows_any_x<Chain>(V)) {
             if constexpr (kExchange) {
                 if (int(block_x * kRowsBX + kRowsBX) * V <= aw) {
-                    rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign, kPlain>(p, kernarg_offset, same, same, ybase, z, aw, ah);
+                    rows_full<Chain, V, ROWS, ALIGNED ? 2 : 2 | detail::kAnyAlign, kSmall>(p, kernarg_offset, same, same, ybase, z, aw, ah);
                     return;
                 }
             }
             if constexpr (kMayStream) {
                 if (stream) { rows_full<Chain, V, ROWS, (ALIGNED ? 1 : 0) | 4, false>(p, kernarg_offset, same, same, ybase, z, aw, ah); return; }
             }
-            rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0, kPlain>(p, kernarg_offset, same, same, ybase, z, aw, ah);
+            rows_full<Chain, V, ROWS, ALIGNED ? 1 : 0, kSmall>(p, kernarg_offset, same, same, ybase, z, aw, ah);
         }
     } else {
         for (int r = 0; r < ROWS; ++r) {
@@ -992,19 +998,9 @@ template <class D> __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_diverg
 
 // The one kernel of a chain compiled at run time, and what its launcher needs to know about it.  A launcher that
 // only has the parameter block as bytes reads the active grid from its first three words.
-// Which kernels the chain has for the forms of a launch of the rows kernel, 0 when it has one for all launches.
-template <class Chain> constexpr u32 rows_forms() {
-    if constexpr (IsDivergent<Chain>::value) return 0u;
-    else if constexpr (is_gather_chain<Chain>()) return 0u;
-    else if constexpr (!rows_any_x<Chain>(RowsConfig<Chain>::V)) return kRowsForms;
-    else return kRowsForms | kRowsAnyX | (has_row_phase<typename Chain::Write>() ? kRowsHasLines : 0u) | (rows_may_stream<Chain>(RowsConfig<Chain>::V) ? kRowsMayStream : 0u);
-}
-// Whether form FORM is one of them.
-template <class Chain, int FORM> constexpr bool rows_has_form() {
-    constexpr u32 forms = rows_forms<Chain>();
-    if constexpr ((forms & kRowsForms) == 0u) return false;
-    else if constexpr ((forms & kRowsAnyX) == 0u) return (FORM & 7) == kRowsOpen;
-    else return (FORM & 7) != kRowsOpen && ((FORM & kRowsStream) == 0 || (forms & kRowsMayStream) != 0u) && ((FORM & 7) != kRowsLines || (forms & kRowsHasLines) != 0u);
+// Whether the chain has a kernel for small outputs.
+template <class Chain> constexpr bool rows_have_small() {
+    if constexpr (IsDivergent<Chain>::value) return false; else return !is_gather_chain<Chain>();
 }
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
@@ -1014,7 +1010,7 @@ template <class Chain> constexpr JitMeta jit_meta() {
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
-                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u, rows_forms<Chain>(),
+                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u, rows_have_small<Chain>() ? 1u : 0u,
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
@@ -1039,10 +1035,11 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
         }
         gather_body<Chain, FKD_GATHER_XI, FKD_GATHER_YI, false>(p, g);
     }
+    else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsLines>(p, 0u, &g);
 }
-// The kernel of one form of the rows kernel (nothing for chains that do not have it).
-template <class Chain, int FORM> __device__ __forceinline__ void jit_rows_body(const typename Chain::Params& p, const TileGeom& g) {
-    if constexpr (rows_has_form<Chain, FORM>()) rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
+// The kernel for small outputs (nothing for chains that have none).
+template <class Chain> __device__ __forceinline__ void jit_small_body(const typename Chain::Params& p, const TileGeom& g) {
+    if constexpr (rows_have_small<Chain>()) rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
 }
 
 } // namespace fkd

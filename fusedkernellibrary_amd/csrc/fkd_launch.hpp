@@ -43,22 +43,15 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
     if (grid.y > 65535u || grid.z > 65535u) return hipErrorInvalidConfiguration;
-    const int form = rows_form(p.active_w, p.active_h, p.active_z, p.reserved, V, rows_forms<Chain>());
-    hipError_t e = hipErrorInvalidValue;
-    auto launch_if = [&](auto form_tag) {
-        constexpr int FORM = decltype(form_tag)::value;
-        if constexpr (rows_has_form<Chain, FORM>()) {
-            if (form != FORM) return;
-            if constexpr (!rows_any_x<Chain>(V)) {
-                if (aligned) { e = launch_by_pointer(&k_rows<Chain, V, ROWS, true, FORM>, grid, block, stream, p, g); return; }
-            }
-            e = launch_by_pointer(&k_rows<Chain, V, ROWS, false, FORM>, grid, block, stream, p, g);
+    const bool small = rows_small(p.active_w, V, p.reserved);
+    if constexpr (!rows_any_x<Chain>(V)) {
+        if (aligned) {
+            if (small) return launch_by_pointer(&k_rows<Chain, V, ROWS, true, kRowsSmall>, grid, block, stream, p, g);
+            return launch_by_pointer(&k_rows<Chain, V, ROWS, true, kRowsLines>, grid, block, stream, p, g);
         }
-    };
-    launch_if(IntTag<kRowsRuns>{}); launch_if(IntTag<kRowsRuns | kRowsPlain>{}); launch_if(IntTag<kRowsLines>{}); launch_if(IntTag<kRowsNarrow>{});
-    launch_if(IntTag<kRowsRuns | kRowsStream>{}); launch_if(IntTag<kRowsLines | kRowsStream>{});
-    launch_if(IntTag<kRowsOpen>{}); launch_if(IntTag<kRowsOpen | kRowsPlain>{});
-    return e;
+    }
+    if (small) return launch_by_pointer(&k_rows<Chain, V, ROWS, false, kRowsSmall>, grid, block, stream, p, g);
+    return launch_by_pointer(&k_rows<Chain, V, ROWS, false, kRowsLines>, grid, block, stream, p, g);
 }
 
 template <class Chain>

@@ -47,15 +47,9 @@ using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
-// A module's kernels: the chain's own (bilinear and divergent launches) and one for each form of the rows kernel; a chain has the one
-// or some of the others (JitMeta::rows_forms), the rest are empty.
-struct JitForm { int form; const char* suffix; };
-constexpr JitForm kJitForms[] = {{-1, ""}, {fkd::kRowsRuns, "_runs"}, {fkd::kRowsRuns | fkd::kRowsPlain, "_runs_plain"}, {fkd::kRowsLines, "_lines"},
-                                 {fkd::kRowsNarrow, "_narrow"}, {fkd::kRowsRuns | fkd::kRowsStream, "_runs_stream"},
-                                 {fkd::kRowsLines | fkd::kRowsStream, "_lines_stream"}, {fkd::kRowsOpen, "_open"},
-                                 {fkd::kRowsOpen | fkd::kRowsPlain, "_open_plain"}};
-constexpr size_t kJitFormCount = sizeof(kJitForms) / sizeof(kJitForms[0]);
-using JitFunctions = std::array<hipFunction_t, kJitFormCount>;
+// A module's kernels: the chain's own and the one for small outputs (empty where JitMeta::has_small is 0).
+constexpr const char* kJitSuffix[2] = {"", "_small"};
+using JitFunctions = std::array<hipFunction_t, 2>;
 
 struct JitKernel {
     std::string signature;
@@ -197,29 +191,26 @@ void write_file(const std::string& path, const std::vector<char>& data) {
 
 hipError_t get_functions(hipModule_t mod, const std::string& signature, JitFunctions* fns) {
     const std::string name = kernel_symbol(signature);
-    for (size_t i = 0; i < kJitFormCount; ++i) {
-        const hipError_t e = hipModuleGetFunction(&(*fns)[i], mod, (name + kJitForms[i].suffix).c_str());
+    for (size_t i = 0; i < fns->size(); ++i) {
+        const hipError_t e = hipModuleGetFunction(&(*fns)[i], mod, (name + kJitSuffix[i]).c_str());
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
-int get_function(JitKernel* k, int form, hipFunction_t* fn) {
-    size_t index = 0;
-    while (index < kJitFormCount && kJitForms[index].form != form) ++index;
-    if (index == kJitFormCount) return int(hipErrorInvalidValue);
+int get_function(JitKernel* k, bool small, hipFunction_t* fn) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return int(e);
     std::lock_guard<std::mutex> lock(k->mu);
     const auto it = k->per_device.find(dev);
-    if (it != k->per_device.end()) { *fn = it->second[index]; return FKLHIP_OK; }
+    if (it != k->per_device.end()) { *fn = it->second[small ? 1 : 0]; return FKLHIP_OK; }
     hipModule_t mod = nullptr;
     if ((e = hipModuleLoadData(&mod, k->code.data())) != hipSuccess) return int(e);
     JitFunctions fns{};
     if ((e = get_functions(mod, k->signature, &fns)) != hipSuccess) return int(e);
     k->per_device.emplace(dev, fns);   // the module stays loaded for the life of the process
-    *fn = fns[index];
+    *fn = fns[small ? 1 : 0];
     return FKLHIP_OK;
 }
 
@@ -273,8 +264,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     if (grid[1] > 65535u || grid[2] > 65535u) return int(hipErrorInvalidConfiguration);
     if (m.max_planes != 0 && grid[2] > m.max_planes) return int(hipErrorInvalidConfiguration);   // as launch_divergent
     hipFunction_t fn = nullptr;
-    const int form = m.rows_forms != 0u ? fkd::rows_form(active[0], active[1], active[2], active[3], m.v, m.rows_forms) : -1;
-    const int rc = get_function(k, form, &fn);
+    const int rc = get_function(k, m.has_small != 0u && fkd::rows_small(active[0], m.v, active[3]), &fn);
     if (rc != FKLHIP_OK) return rc;
     // Kernel-argument segment: the parameter block, then the TileGeom at the next 4-byte boundary.  The runtime
     // copies the buffer during the call, so the caller's block may go away as soon as we return.
@@ -311,10 +301,10 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
         src += "(const JitChain::Params p, const TileGeom g) {\n"
                "    jit_body<JitChain>(p, g);\n"
                "}\n";
-        for (size_t i = 1; i < kJitFormCount; ++i) {
-            src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitForms[i].suffix +
-                   "(const JitChain::Params p, const TileGeom g) { jit_rows_body<JitChain, " + std::to_string(kJitForms[i].form) + ">(p, g); }\n";
-        }
+        src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitSuffix[1] +
+               "(const JitChain::Params p, const TileGeom g) {\n"
+               "    jit_small_body<JitChain>(p, g);\n"
+               "}\n";
         hiprtcProgram prog = nullptr;
         hiprtcResult r = hiprtcCreateProgram(&prog, src.c_str(), "fkd_jit_chain.hip", kJitHeaderCount, kJitHeaderTexts, kJitHeaderNames);
         if (r != HIPRTC_SUCCESS) { g_log = hiprtcGetErrorString(r); delete k; return FKLHIP_EUNKNOWN_SIGNATURE; }

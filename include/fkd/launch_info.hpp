@@ -40,11 +40,11 @@ struct TileGeom {
 // bfloat16) behind each launch: 224x670 49.4 / 50.8, 225x667 53.0 / 57.6, 500x436 (160) 71 / 80; from 190 MiB on even these gain (224x1401,
 // 230 MiB 110 / 97).  Three buffers with a reader: 225x667 67 / 64, 500x518 (190) 123 / 106.
 constexpr unsigned long long kStreamOutputBytes = 80ull << 20;
-// Launches of the rows kernel that write no more than this (as the chain's values count) store without the non-temporal hint: with it
+// Launches of the rows kernel that write no more than this store without the non-temporal hint: with it
 // a launch is not over before its last lines have left the chip.  us per launch, with the hint / without: 4 uchar3 images of 225x165
 // (0.4 MB) 2.32 / 2.01, of 943x179 (2.0 MB) 2.93 / 2.68, of 886x260 (2.8 MB) 3.21 / 2.97; 30 operations on 1544x90 floats (0.6 MB)
-// 2.20 / 1.91; P010 to float3 at 404x862 (4.2 MB) 3.07 / 2.93; UYVY to float3 at 1552x284 (5.3 MB) 2.44 / 2.67; RGB to UYVY at 3638x632 (6.9
-// MB) 4.09 / 4.32; 100 images of 75x200 (4.5 MB) 6.5 / 6.1, of 228x113 (7.7 MB) 4.4 / 4.8, of 361x467 (51 MB) 20.9 / 25.9.
+// 2.20 / 1.91; P010 to float3 at 404x862 (4.2 MB) 3.07 / 2.93; UYVY to float3 at 1552x284 (5.3 MB) 2.44 / 2.67; RGB to UYVY at 2460x714 (3.5
+// MB) 3.80 / 3.56, at 3638x632 (4.6 MB) 4.09 / 4.32; 100 images of 75x200 (4.5 MB) 6.5 / 6.1, of 228x113 (7.7 MB) 4.4 / 4.8, of 361x467 (51 MB) 20.9 / 25.9.
 constexpr unsigned long long kSmallOutputBytes = 4ull << 20;
 // The magic for dividing numbers below `limit` by d, or 0 when there is none.
 inline unsigned division_magic(unsigned d, unsigned limit) {
@@ -70,30 +70,11 @@ inline unsigned strip_first_late_workgroup(unsigned long long workgroups) {
     return workgroups <= kStripOneRoundWorkgroups ? kStripLateWorkgroup * kComputeUnits : 0u;
 }
 
-// The forms of the rows kernel; each is a kernel of its own (see the kernels' header for why).  For chains whose waves may take runs
-// that start anywhere in a row (kRowsAnyX) one of
-//   kRowsNarrow  rows shorter than a run
-//   kRowsRuns    segments counted from the row's start
-//   kRowsLines   segments that begin at line boundaries (the grid has room for them: rows_phase_bound)
-// and for the others kRowsOpen.  kRowsStream: loads carry the non-temporal hint.  kRowsPlain: stores carry none.
-constexpr int kRowsRuns = 0, kRowsLines = 1, kRowsNarrow = 2, kRowsOpen = 3, kRowsStream = 8, kRowsPlain = 16;
-constexpr unsigned kRowsForms = 1u, kRowsAnyX = 2u, kRowsHasLines = 4u, kRowsMayStream = 8u;
-// A launch over more elements than this reads them with the non-temporal hint: more than the last-level cache could hold between two
-// launches (100 images of 1920x1080 uchar3: 225 -> 209 us); smaller inputs are left to the caches, where a pipeline's previous stage may
-// have put them (the hint costs 15 % on a 33 MB image that is still cached).
-constexpr unsigned long long kStreamElements = 1ull << 26;
-// Bit 2 of a chain's Params::reserved: the launch writes no more than kSmallOutputBytes.
+// Bit 2 of a chain's Params::reserved: the launch writes no more than kSmallOutputBytes (and has no segments that begin left of a row).
 constexpr unsigned kSmallOutputBit = 4u;
-// Which form a launch over w x h x planes elements takes; reserved: the parameter block's flags, run: elements a thread handles in a
-// row, forms: what the chain has (JitMeta::rows_forms).
-inline int rows_form(unsigned w, unsigned h, unsigned planes, unsigned reserved, unsigned run, unsigned forms) {
-    const bool small_output = (reserved & kSmallOutputBit) != 0u;
-    if ((forms & kRowsAnyX) == 0u) return kRowsOpen | (small_output ? kRowsPlain : 0);
-    if (w < run) return kRowsNarrow;
-    if (small_output) return kRowsRuns | kRowsPlain;
-    const int stream = (forms & kRowsMayStream) != 0u && (unsigned long long)w * h * planes > kStreamElements ? kRowsStream : 0;
-    return ((forms & kRowsHasLines) != 0u && rows_phase_bound(reserved) != 0u ? kRowsLines : kRowsRuns) | stream;
-}
+// Whether a launch of the rows kernel takes the kernel for small outputs; run: elements a thread handles in a row (rows shorter than
+// that, of which such a kernel knows nothing, are left to the other one), reserved: the parameter block's flags.
+inline bool rows_small(unsigned w, unsigned run, unsigned reserved) { return (reserved & kSmallOutputBit) != 0u && w >= run; }
 
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
@@ -104,7 +85,7 @@ struct JitMeta {
     unsigned max_planes;      // most planes (grid z) a launch may have, 0: no limit of the kernel's own
     unsigned strip_width;     // gather kernel: outputs up to this width are launched in strip form (TileGeom::tiles_x == 0), 0: never
     unsigned bands;           // rows kernel: 1 when launches of kRowsBandBlocks blocks per plane or more take the bands form of grid
-    unsigned rows_forms;      // rows kernel: which kernels the chain has for the forms of a launch (see rows_form), 0: one for all launches
+    unsigned has_small;       // rows kernel: 1 when the module has a kernel for small outputs (see rows_small)
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
 };
 

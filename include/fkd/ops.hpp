@@ -3124,6 +3124,7 @@ template <int PF> struct WriteYUV {
     using Group = Vec<B, L::kSemiPlanar ? 2 : 4>;
     static constexpr bool kRowPhase = true;
     static constexpr unsigned long long kPhaseMin = phase_min_bytes<u32>();
+    FKD_HD static unsigned long long stored_bytes(unsigned long long pixels) { return pixels * sizeof(B) * (L::k420 ? 3u : 4u) / 2u; }
     FKD_HD static u32 row_phase_bound(const Params& p) {
         const u32 groups = row_phase_bound_of<Group>(p.data, p.pitch);
         return groups != 0u ? 2u * groups : 0u;
@@ -3430,11 +3431,13 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     // alignment.  A parameter block that never came through here keeps the bits clear and gets the tile form.
     // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
     // phase_bound_for).
-    // Bit 2: the launch writes no more than kSmallOutputBytes.
+    // Bit 2: the launch writes no more than kSmallOutputBytes and its segments begin at the row's start.
     static void finalize_write(Params& p) {
-        if ((unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value) <= kSmallOutputBytes) p.reserved |= kSmallOutputBit;
-        if constexpr (any_x<R>() && has_row_phase<W>())
-            p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(Value), W::kPhaseMin) << 8;
+        const unsigned long long elements = (unsigned long long)p.active_w * p.active_h * p.active_z;
+        if constexpr (any_x<R>() && has_row_phase<W>()) p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, elements * sizeof(Value), W::kPhaseMin) << 8;
+        unsigned long long stored = elements * sizeof(Value);
+        if constexpr (requires { W::stored_bytes(elements); }) stored = W::stored_bytes(elements);
+        if (row_phase_bound(p.reserved) == 0u && stored <= kSmallOutputBytes) p.reserved |= kSmallOutputBit;
         if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {
             const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);
             if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value), W::row_grain(p.write, p.active_w, p.active_z)) && W::strip_ok(p.write) &&

@@ -261,7 +261,7 @@ def test_line_aligned_segments_tensors(device, kind, half, in_place):
     assert np.array_equal(out.cpu().numpy(), out_host)             # the rows are the input's, every byte beside them is as it was
 
 
-# Launches that write up to 4 MiB (as the chain's values count) store without the non-temporal hint, larger ones with it: both sides of
+# Launches that write up to 4 MiB store without the non-temporal hint, larger ones with it: both sides of
 # the line, in widths below those of line-aligned segments, whole runs and remainders.
 @pytest.mark.parametrize("w,h", [(300, 1165), (300, 1166), (299, 1168), (299, 1170), (301, 1161), (301, 1162)])
 def test_small_and_larger_outputs(device, w, h):
@@ -288,7 +288,7 @@ def test_small_and_larger_outputs(device, w, h):
 @pytest.mark.parametrize("pf,cr,cp", [(ol.PF_NV12, 0, 1), (ol.PF_P010, 0, 2), (ol.PF_UYVY, 1, 1)])
 @pytest.mark.parametrize("w,h", [(300, 1164), (300, 1166), (254, 1376), (258, 1356)])
 def test_small_and_larger_video_frames(device, pf, cr, cp, w, h):
-    """Decoded to float3 (12 bytes a pixel) and encoded from RGB (3 or 6 bytes a pixel): chains compiled ahead of time and on first use."""
+    """Decoded to float3 and encoded from RGB, as many bytes stored: chains compiled ahead of time and on first use."""
     import torch
     dt, size = (np.uint16, 2) if ol.PF_WIDE[pf] else (np.uint8, 1)
     rng = np.random.RandomState(w + pf)
@@ -296,7 +296,7 @@ def test_small_and_larger_video_frames(device, pf, cr, cp, w, h):
     buf = rng.randint(0, 1024 if size == 2 else 256, (rows, cols)).astype(dt)
     frame, out = Placed((rows, cols), dt, 0, 0, device, buf), Placed((h, w, 3), np.float32, 4, 0, device)
     cases.yuv_to_rgb(pf, cr, cp, frame.view(), w, h, out.view())
-    eh = 4 * h // size                                                                         # as many bytes of samples
+    eh = {ol.PF_NV12: 8, ol.PF_P010: 4, ol.PF_UYVY: 6}[pf] * h                                 # 1.5, 3 and 2 bytes a pixel instead of 12
     rgb = rng.randint(0, 1024 if size == 2 else 256, (eh, w, 3)).astype(dt)
     rows, cols = ol.frame_shape(pf, w, eh)
     start = np.full((rows, cols), 9, dt)
