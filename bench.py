@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52054000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "c29170ae4bdd280290c7cda102c8d15c79e0e4c717d193c302b60618d3fe94de"
+TRAFFIC_C3_SOURCES_SHA256 = "e1713470c473d705ccd5c436a883bc66284f38a14d8b7613db1df01ddb924950"
 
 
 def device_sources_sha256():

@@ -56,7 +56,7 @@ template <int N, int AR, class Back> struct ResizeRoot<BatchReadDefault<N, Resiz
 template <class R> struct HasDefaultPlanes { static constexpr bool value = false; };
 template <int N, class PlaneOp> struct HasDefaultPlanes<BatchReadDefault<N, PlaneOp>> { static constexpr bool value = true; };
 
-// Reads whose taps are scattered gathers (warps): the rows kernel then keeps one element per thread.
+// Reads whose taps are scattered gathers (warps).
 template <class R> constexpr bool is_scattered_read() {
     if constexpr (requires { R::kGatherRead; }) return R::kGatherRead;
     else if constexpr (requires { typename R::Plane; }) return is_scattered_read<typename R::Plane>();

@@ -2532,7 +2532,7 @@ template <int WT, class Back> struct Warp {
     };
     static constexpr bool kTapCursor = false;
     static constexpr bool kAnyX = true;
-    static constexpr bool kGatherRead = true;     // taps are scattered: one element per thread
+    static constexpr bool kGatherRead = true;     // taps are scattered: the source is read where the coordinates send it
     static constexpr bool kPairTaps = [] {
         if constexpr (requires { Back::kTapPair; }) return Back::kTapCursor && Back::kTapPair; else return false;
     }();
@@ -3169,7 +3169,7 @@ template <int PF> struct WriteYUV {
 #pragma unroll
         for (int i = 0; i < V; ++i) put(r, x + i, v[i].v);
     }
-    // Four pixels (x is a multiple of four here) leave as whole dwords at any alignment: their luma samples and, on rows that
+    // Four pixels (x is even here: a multiple of four unless segments begin at line boundaries) leave as whole dwords at any alignment: their luma samples and, on rows that
     // store chroma, their two pairs, or the two groups of four samples of a packed format.  Sample by sample a frame was
     // bound by the number of stores (3840x2160: to NV12 8.6 -> 7.2 us (6.9 with rows on the scalar unit), P010 16.6 -> 13.0, UYVY 8.6 ->
     // 7.8; 3838x2160 to NV12 10.6 -> 8.8).  Which pixels of a run store chroma is known at compile time, and so is the row where a thread has two of
