@@ -299,9 +299,99 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     }
 }
 
+// ---- rows kernel, scattered reads ----
+//
+// A warp's taps lie along a slanted line of the source, so what one instruction of a wave touches is decided by how far its
+// lanes are apart in the output: with four adjacent outputs per lane, 64 lanes span 256 columns, which a turn by 7 degrees
+// spreads over 31 source rows, nearly a cache line per lane and tap.  Here a wave owns 64 columns of the block's 256 and each
+// lane one column of its four rows: an instruction spans 64 columns (8 rows at 7 degrees), its stores are 64 whole pixels
+// side by side without an exchange through LDS, and what depends on the column serves four pixels.  What is left is bound by the
+// lines the taps touch and the stores.  Four adjacent outputs per lane / one column of four rows, three sources and
+// outputs in turn, us: 3840x2160 by 7 degrees 28.0 / 22.5, 2709x1462 by -18 degrees 19.8 / 14.5, perspective 1474x2063 by 29
+// degrees 17.7 / 13.7, 4 of 811x319 13.9 / 12.1, 4 of 200x79 9.7 / 9.3.  (Lanes as 32 columns of two rows serve steep angles a little better,
+// 13.1 for the 13.7, and everything else worse by 3 to 6 %: the stores' addresses are then the lanes' own.)
+//
+// The kernel's arguments are requested together and waited for once: a trip to the kernel-argument segment is 0.1 us of a
+// launch of 2.3.
+// For writers that store an element as one wide access; planar writers and elements of 1 to 3 bytes keep four outputs
+// of a row per lane, which they store as one access.
+template <class R> struct PointsRoot { using Op = R; static constexpr bool batched = false; };
+template <int N, class PlaneOp> struct PointsRoot<BatchRead<N, PlaneOp>> { using Op = PlaneOp; static constexpr bool batched = true; };
+template <class Op> constexpr bool reads_points() {
+    if constexpr (requires { Op::kPoints; }) return Op::kPoints; else return false;
+}
+template <class Chain, int V, int ROWS> constexpr bool rows_by_points() {
+    return V == kRowsBY && ROWS == 1 && reads_points<typename PointsRoot<typename Chain::Read>::Op>() && puts_whole<typename Chain::Write>();
+}
+template <class Chain, int V, int FORM>
+__device__ __forceinline__ void points_body(const typename Chain::Params& p, const TileGeom& bands) {
+    using Root = PointsRoot<typename Chain::Read>;
+    using Op = typename Root::Op;
+    using W = typename Chain::Write;
+    using WP = typename W::Plane;
+    constexpr bool kPhases = FORM == kRowsLines && has_row_phase<WP>();
+    const int z = int(blockIdx.z);
+    const typename Op::Params* rp;
+    if constexpr (Root::batched) rp = &p.read.plane[z]; else rp = &p.read;
+    TileGeom g = bands;
+    typename Op::Params q = *rp;
+    typename WP::Params wpar = W::plane_params(p.write, z);
+    u32 head[3] = {p.active_w, p.active_h, p.reserved};
+    detail::pin_scalars(g);
+    detail::pin_scalars(q);
+    detail::pin_scalars(wpar);
+    detail::pin_scalars(head);
+    const int aw = int(head[0]), ah = int(head[1]);
+    u32 block_x = blockIdx.x, block_y = blockIdx.y;
+    if (g.tiles_x != 0u) {
+        // one band of the plane's blocks per XCD (see rows_in_bands); a two-dimensional grid holds exactly the plane's blocks
+        const u32 gx = g.tiles_x, blocks = gx * g.tiles_y;
+        u32 tin;
+        if (g.n_tiles != 0u) {
+            tin = (blockIdx.x % 8u) * rows_band_chunk(blocks) + blockIdx.x / 8u;
+            if (tin >= blocks) return;
+        } else {
+            const u32 number = block_y * gx + block_x, k = number % 8u, rest = blocks % 8u;
+            tin = k * (blocks / 8u) + (k < rest ? k : rest) + number / 8u;
+        }
+        block_y = g.tiles_x_magic ? u32(((unsigned long long)tin * g.tiles_x_magic) >> 32) : tin / gx;
+        block_x = tin - block_y * gx;
+    }
+    const int lane = int(threadIdx.x), wave = __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+    const int left = int(block_x) * kRowsBX * V + wave * kRowsBX, top = int(block_y) * kRowsBY;
+    u32 bound = 0;
+    if constexpr (kPhases) bound = Chain::row_phase_bound(head[2]);
+    if (left - int(bound) >= aw || top >= ah) return;
+    int seg[V], x[V], y[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) { seg[i] = left; x[i] = left + lane; y[i] = top + i; }
+    if constexpr (kPhases) {
+        if (bound != 0u) {                              // (segments of 64 columns begin where a line does, see row_phase_bound)
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                seg[i] = left - (WP::row_phase(y[i] < ah ? y[i] : ah - 1, z, wpar) & int(bound));
+                x[i] = seg[i] + lane;
+            }
+        }
+    }
+    Slot<typename Chain::Read::Out> in[V];
+    Slot<typename Chain::Value> out[V];
+    // (a second copy of the work for waves that are inside throughout costs launches of few waves more than it gives)
+    Op::template exec_points<V, FORM == kRowsLines>(x, y, z, q, in, g.n_tiles != 0u);
+    if constexpr (Chain::kLongChain) Chain::template compute_run_kernarg<V>(in, out, (const FKD_CONSTANT char*)__builtin_amdgcn_kernarg_segment_ptr());
+    else Chain::template compute_run<V>(in, out, p.ops);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        typename WP::RowRef row = WP::row(y[i], z, wpar);
+        row.p += seg[i];
+        if (y[i] < ah && x[i] >= 0 && x[i] < aw) WP::template put<FORM == kRowsSmall>(row, lane, out[i].v);
+    }
+}
+
 template <class Chain, int V, int ROWS, bool ALIGNED, int FORM>
-__global__ __launch_bounds__(kRowsBX * kRowsBY) void k_rows(const typename Chain::Params p, const TileGeom g) {
-    rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
+__global__ __launch_bounds__(kRowsBX * kRowsBY, (rows_by_points<Chain, V, ROWS>() ? 8 : 1)) void k_rows(const typename Chain::Params p, const TileGeom g) {
+    if constexpr (rows_by_points<Chain, V, ROWS>()) points_body<Chain, V, FORM>(p, g);
+    else rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
 }
 
 // Whether the rows of plane z of the read and of the write all start on dword boundaries, decided on the device
@@ -318,6 +408,7 @@ template <class Op, class P> FKD_DEV bool write_plane_aligned(const P& p, int z)
 template <class Chain, int V, int ROWS, bool BANDS = false, int FORM = kRowsOpen>
 __device__ __forceinline__ void rows_auto_body(const typename Chain::Params& p, u32 kernarg_offset = 0, const TileGeom* bands = nullptr) {
     const int z = blockIdx.z;
+    if constexpr (BANDS && rows_by_points<Chain, V, ROWS>()) { points_body<Chain, V, FORM>(p, *bands); return; }
     if constexpr (rows_any_x<Chain>(V)) { rows_body<Chain, V, ROWS, false, BANDS, FORM>(p, kernarg_offset, bands); return; }
     const bool aligned = read_plane_aligned<typename Chain::Read>(p.read, z) && write_plane_aligned<typename Chain::Write>(p.write, z);
     if (aligned) rows_body<Chain, V, ROWS, true, BANDS, FORM>(p, kernarg_offset, bands);
@@ -935,8 +1026,7 @@ __global__ __launch_bounds__(kGatherBX * kGatherBY) void k_gather(const typename
 
 template <class Chain> struct RowsConfig {
     // Four elements per thread; a bilinear resize without a tap cursor keeps one element per thread.  (Warps take four
-    // as well: their taps are gathers either way, and four float3 results per lane leave as dense wave-wide stores:
-    // 1080p 9.06 -> 8.83 us, 2160p in bands 27.1 -> 25.1 us.)
+    // as well, of one column: points_body.)
     static constexpr bool kScattered = ResizeRoot<typename Chain::Read>::value;
 #ifndef FKD_ROWS
 #define FKD_ROWS 2
@@ -1010,7 +1100,7 @@ template <class Chain> constexpr JitMeta jit_meta() {
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
-                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? 1u : 0u, rows_have_small<Chain>() ? 1u : 0u,
+                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u,
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {

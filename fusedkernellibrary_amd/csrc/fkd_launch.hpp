@@ -38,6 +38,8 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
         if (gx * gy >= kRowsBandBlocks) {
             grid = dim3(rows_band_chunk(gx * gy) * 8u, 1, p.active_z);
             g = TileGeom{gx, gy, gx * gy * p.active_z, division_magic(gx, gx * gy)};
+        } else if (rows_by_points<Chain, V, ROWS>() && rows_bands_2d(gx, gy)) {
+            g = TileGeom{gx, gy, 0u, division_magic(gx, gx * gy)};
         }
     }
     if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};

@@ -257,6 +257,10 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
             g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
             grid[0] = (grid[0] * grid[1] + 7u) / 8u * 8u;
             grid[1] = 1;
+        } else if (m.bands > 1u && fkd::rows_bands_2d(grid[0], grid[1])) {
+            g.tiles_x = grid[0];
+            g.tiles_y = grid[1];
+            g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
         }
     }
     if (info) *info = fkd::LaunchInfo{kind, {grid[0], grid[1], grid[2]}, {block[0], block[1], 1}, 0};

@@ -58,6 +58,14 @@ inline unsigned division_magic(unsigned d, unsigned limit) {
 inline constexpr unsigned rows_band_chunk(unsigned blocks) { return (blocks + 7u) / 8u; }
 constexpr unsigned kRowsBandBlocks = 4096;
 
+// Scattered reads (points_body in the kernels' header): smaller launches keep the two-dimensional grid, whose workgroups are renumbered
+// into bands as well (TileGeom::n_tiles == 0).  us without / with: 3 launches in turn each, perspective 686x1247 (4 of them) 26.4 / 20.9, 4 of
+// 811x319 (320 blocks) 13.7 / 12.1, 4 of 336x905 (454) 14.5 / 12.0.  Not with a few blocks, whose launches are over before a second
+// XCD asks for the same line (4 of 141x351, 88 blocks 9.4 / 9.6), nor where one block spans the row (4 of 187x1511 11.6 / 11.75).
+inline bool rows_bands_2d(unsigned gx, unsigned gy) {
+    return gx >= 2u && (unsigned long long)gx * gy >= 256u && division_magic(gx, gx * gy) != 0u;
+}
+
 // Bits 8 to 15 of a chain's Params::reserved: by how many elements at most the rows kernel's waves begin left of a row so
 // that they store whole lines (Chain::finalize_write); the grid has to reach that much further.
 inline constexpr unsigned rows_phase_bound(unsigned reserved) { return (reserved >> 8) & 0xffu; }
@@ -84,7 +92,7 @@ struct JitMeta {
     unsigned xi, yi, by;      // gather kernel: pixels per lane along x, rows per wave, waves per workgroup
     unsigned max_planes;      // most planes (grid z) a launch may have, 0: no limit of the kernel's own
     unsigned strip_width;     // gather kernel: outputs up to this width are launched in strip form (TileGeom::tiles_x == 0), 0: never
-    unsigned bands;           // rows kernel: 1 when launches of kRowsBandBlocks blocks per plane or more take the bands form of grid
+    unsigned bands;           // rows kernel: 1 when launches of kRowsBandBlocks blocks per plane or more take the bands form of grid, 2 when smaller ones may as well (rows_bands_2d)
     unsigned has_small;       // rows kernel: 1 when the module has a kernel for small outputs (see rows_small)
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
 };

@@ -140,6 +140,10 @@ inline u32 phase_bound_for(u32 full, u32 width, unsigned long long bytes, unsign
 template <class W> constexpr bool has_row_phase() {
     if constexpr (requires { W::kRowPhase; }) return W::kRowPhase; else return false;
 }
+// puts_whole<W>: write W stores one element as one wide access, told whether to carry the non-temporal hint.
+template <class W> constexpr bool puts_whole() {
+    if constexpr (requires { W::kPutWhole; }) return W::kPutWhole; else return false;
+}
 template <class T> constexpr bool small_integer_base() {
     return !(__is_same(base_t<T>, f32) || __is_same(base_t<T>, f64)) && sizeof(base_t<T>) <= 2;
 }
@@ -181,6 +185,7 @@ inline bool none_in_wave(bool) { return false; }     // never reached: host code
 #if defined(FKD_DEVICE_CODE)
 namespace detail {
 
+template <bool B> struct BoolTag { static constexpr bool value = B; };
 // True when no lane of the wave holds `flag`.
 FKD_DEV bool none_in_wave(bool flag) { return __builtin_amdgcn_ballot_w64(flag) == 0; }
 
@@ -677,12 +682,14 @@ template <bool DUP = false, class T> FKD_DEV void pair_window_values(const PairW
 }
 
 // Store counterpart of load_bits_at: element sizes 2 and multiples of 4 (up to 16) leave as one access.
-template <class T> FKD_DEV void store_elem_at(char* base, u32 off, const T& v) {
+template <class T, bool PLAIN = false> FKD_DEV void store_elem_at(char* base, u32 off, const T& v) {
     constexpr int n = int(sizeof(T));
     constexpr bool packed = sizeof(T) == sizeof(base_t<T>) * cn_v<T>;
     asm volatile("" : "+v"(off));   // as in load_bits_at: keep the scalar-base addressing form
     char* a = base + off;
-    if constexpr (!packed || n > 16 || (n % 4 != 0 && n != 2) || cn_v<T> == 1) {
+    if constexpr (packed && n == 4 && cn_v<T> == 1) {
+        gstore<alignof(T), PLAIN>(reinterpret_cast<T*>(a), v);
+    } else if constexpr (!packed || n > 16 || (n % 4 != 0 && n != 2) || cn_v<T> == 1) {
         store_elem(reinterpret_cast<T*>(a), v);
     } else {
         Slot<T> one[1];
@@ -695,10 +702,10 @@ template <class T> FKD_DEV void store_elem_at(char* base, u32 off, const T& v) {
             *(FKD_GLOBAL At*)a = u16(w[0]);
         } else {
             pack_words<T, 1, W>(one, w);
-            if constexpr (W == 1) { gstore<1>(a, w[0]); }
-            else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore<1>(a, q); }
-            else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore<1>(a, q); }
-            else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore<1>(a, q); }
+            if constexpr (W == 1) { gstore<1, PLAIN>(a, w[0]); }
+            else if constexpr (W == 2) { u32x2_t q; q.x = w[0]; q.y = w[1]; gstore<1, PLAIN>(a, q); }
+            else if constexpr (W == 3) { u32x3_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; gstore<1, PLAIN>(a, q); }
+            else { u32x4_t q; q.x = w[0]; q.y = w[1]; q.z = w[2]; q.w = w[3]; gstore<1, PLAIN>(a, q); }
         }
     }
 }
@@ -2533,6 +2540,7 @@ template <int WT, class Back> struct Warp {
     static constexpr bool kTapCursor = false;
     static constexpr bool kAnyX = true;
     static constexpr bool kGatherRead = true;     // taps are scattered: the source is read where the coordinates send it
+    static constexpr bool kPoints = true;         // exec_points: several output pixels from anywhere at once
     static constexpr bool kPairTaps = [] {
         if constexpr (requires { Back::kTapPair; }) return Back::kTapCursor && Back::kTapPair; else return false;
     }();
@@ -2553,38 +2561,48 @@ template <int WT, class Back> struct Warp {
         int xp;
         bool inside, edge;
     };
-    // Whether the bounded form serves this image (wave uniform): at least two columns, every byte offset within 32 bits.
-    // (Offsets by two 24-bit multiplications instead of the 32-bit ones the compiler picks were measured and are slower.)
-    FKD_DEV static bool bounded_ok(int sw, const Params& p) { return sw >= 2 && Back::tap_offsets_fit(p.back); }
-    FKD_DEV static BoundedTaps bounded_request(f32 sx, f32 sy, int sw, int sh, int z, const Params& p) {
+    // Whether the bounded form serves this image (wave uniform): at least two columns, every byte offset within 32 bits, and rows
+    // and pitch within 24 bits, so that an offset costs one multiplication that does not widen (the compiler's own choice is a
+    // 64-bit multiply-add, four times as long).
+    FKD_DEV static bool bounded_ok(int sw, int sh, const Params& p) {
+        return sw >= 2 && Back::tap_offsets_fit(p.back) && u32(sh) < (1u << 24) && Back::tap_row_offset(1, p.back) < (1u << 24);
+    }
+    // 0 <= s < limit for a limit above zero, as one comparison of the bit patterns: those of negative numbers and of NaNs are above
+    // every finite positive one's, and -0, which is inside, becomes +0 first.
+    FKD_DEV static bool within(f32 s, f32 limit) { return __builtin_bit_cast(u32, s + 0.0f) < __builtin_bit_cast(u32, limit); }
+    // INTERIOR: the source point lies inside, in neither the last column nor the last row.
+    template <bool INTERIOR> FKD_DEV static BoundedTaps bounded_request(f32 sx, f32 sy, int sw, int sh, const detail::TapImage& image, const Params& p) {
         BoundedTaps t;
-        t.inside = sx >= 0.f && sx < f32(sw) && sy >= 0.f && sy < f32(sh);
+        t.inside = INTERIOR || (within(sx, f32(sw)) & within(sy, f32(sh)));
         t.cx = t.inside ? sx : 0.f; t.cy = t.inside ? sy : 0.f;
         t.fx1 = __builtin_floorf(t.cx); t.fy1 = __builtin_floorf(t.cy);
-        const int x1 = int(t.fx1), y1 = int(t.fy1);
-        const int y2r = y1 + 1 < sh - 1 ? y1 + 1 : sh - 1;
-        t.edge = x1 >= sw - 1;                        // x1 + 1 is past the line: both taps are the last pixel
+        const int x1 = int(t.fx1);
+        const u32 y1 = u32(int(t.fy1)) & 0xffffffu;
+        t.edge = !INTERIOR && x1 >= sw - 1;           // x1 + 1 is past the line: both taps are the last pixel
         t.xp = t.edge ? sw - 2 : x1;
-        const detail::TapImage image = Back::tap_image_bounded(z, p.back);
         using Window = typename detail::pair_bits_of<Back>::type;
         const detail::PairPrep col = Back::pair_prepare(image, t.xp, p.back);
-        const u32 column_bytes = col.off + col.shift;             // from the resource's base
-        const u32 ta = column_bytes + Back::tap_row_offset(y1, p.back), tb = column_bytes + Back::tap_row_offset(y2r, p.back);
+        const u32 pitch = Back::tap_row_offset(1, p.back) & 0xffffffu;
+        const u32 ta = col.off + col.shift + y1 * pitch;          // from the resource's base
+        const u32 tb = ta + (INTERIOR || int(y1) < sh - 1 ? pitch : 0u);
         t.wa = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(ta), p.back);
         t.wb = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(tb), p.back);
         return t;
     }
-    FKD_DEV static Out bounded_blend(const BoundedTaps& t, const Params& p) {
+    template <bool INTERIOR> FKD_DEV static Out bounded_blend(const BoundedTaps& t, const Params& p) {
         // (x1 and x1 + 1 as floats are the floor and the floor plus one: coordinates are below 2^24.  Where the taps are
         // finite and not negative whatever the image holds, a lane outside gets horizontal weights of +0, hence four weights
         // of +0 and a result of +0 in every channel; otherwise its channels are replaced one by one)
         constexpr bool kZeroWeights = finite_taps<Back>() && is_integer_v<base_t<Src>> && base_t<Src>(-1) > base_t<Src>(0);
         f32 ax = (t.fx1 + 1.0f) - t.cx, bx = t.cx - t.fx1;
         const f32 ay = (t.fy1 + 1.0f) - t.cy, by = t.cy - t.fy1;
-        if constexpr (kZeroWeights) { if (!t.inside) { ax = 0.f; bx = 0.f; } }
+        if constexpr (kZeroWeights && !INTERIOR) { if (!t.inside) { ax = 0.f; bx = 0.f; } }
         const f32 w00 = ax * ay, w10 = bx * ay, w01 = ax * by, w11 = bx * by;
         typename Back::Raw a0, a1, b0, b1;
-        if constexpr (requires { Back::pair_values_dup(t.wa, t.edge, a0, a1); }) {
+        if constexpr (INTERIOR) {
+            Back::pair_values(t.wa, typename Back::TapRow{}, t.xp, a0, a1);
+            Back::pair_values(t.wb, typename Back::TapRow{}, t.xp, b0, b1);
+        } else if constexpr (requires { Back::pair_values_dup(t.wa, t.edge, a0, a1); }) {
             // (at the edge the left tap is the right one again: chosen inside the window, before the bytes are taken apart)
             Back::pair_values_dup(t.wa, t.edge, a0, a1);
             Back::pair_values_dup(t.wb, t.edge, b0, b1);
@@ -2598,7 +2616,7 @@ template <int WT, class Back> struct Warp {
         const bool inside = t.inside;
         auto one = [&](auto pa, auto pb, auto pc, auto pd) {
             const f32 v = ((f32(pa) * w00 + f32(pb) * w10) + f32(pc) * w01) + f32(pd) * w11;
-            if constexpr (kZeroWeights) return v; else return inside ? v : 0.f;
+            if constexpr (kZeroWeights || INTERIOR) return v; else return inside ? v : 0.f;
         };
         Out o;
         chan<0>(o) = one(chan<0>(a), chan<0>(b), chan<0>(c), chan<0>(d));
@@ -2623,12 +2641,17 @@ template <int WT, class Back> struct Warp {
         f32 sx, sy;
         source_point(x, y, p, sx, sy);
         const int sw = Back::width(p.back), sh = Back::height(p.back);
-        Out o;
 #if defined(FKD_DEVICE_CODE)
         if constexpr (kPairTaps && detail::tap_prepared<Back>()) {
-            if (bounded_ok(sw, p)) return bounded_blend(bounded_request(sx, sy, sw, sh, z, p), p);
+            if (bounded_ok(sw, sh, p)) return bounded_blend<false>(bounded_request<false>(sx, sy, sw, sh, Back::tap_image_bounded(z, p.back), p), p);
         }
 #endif
+        return value_at(sx, sy, sw, sh, z, p);
+    }
+    // The value at a source point of any image.
+    FKD_DEV static Out value_at(f32 sx, f32 sy, int sw, int sh, int z, const Params& p) {
+        Out o;
+#if defined(FKD_DEVICE_CODE)
         if constexpr (kPairTaps) {
             // Taps x1 and x1 + 1 of a source line in one access each, issued by every lane (lanes whose source point
             // lies outside take the taps of pixel (0, 0) and drop them), so that no load waits behind a branch.  A wave
@@ -2662,6 +2685,7 @@ template <int WT, class Back> struct Warp {
                 return o;
             }
         }
+#endif
         if (sx >= 0.f && sx < f32(sw) && sy >= 0.f && sy < f32(sh)) {
             const f32 f1x = __builtin_floorf(sx), f1y = __builtin_floorf(sy);
             const int x1 = int(f1x), y1 = int(f1y);
@@ -2689,25 +2713,44 @@ template <int WT, class Back> struct Warp {
 #endif
 #if defined(FKD_DEVICE_CODE)
     template <int V, int A> FKD_DEV static void exec_row(int x, int y, int z, const Params& p, Slot<Out> (&out)[V]) {
+        int xs[V], ys[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) { xs[i] = x + i; ys[i] = y; }
+        exec_points<V, false>(xs, ys, z, p, out, false);
+    }
+    // V output pixels from wherever they are.  MAY_SPLIT and `split`: waves whose source points all lie inside, off the last column
+    // and row, go without the tests and selects that only the others need (3840x2160 25.7 -> 22.8 us; 2304x589
+    // takes 5.7 us with the split and 5.4 without: all four points are then worked out before the first tap leaves).
+    template <int V, bool MAY_SPLIT> FKD_DEV static void exec_points(const int (&x)[V], const int (&y)[V], int z, const Params& p, Slot<Out> (&out)[V], bool split) {
+        const int sw = Back::width(p.back), sh = Back::height(p.back);
+        f32 sx[V], sy[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) source_point(x[i], y[i], p, sx[i], sy[i]);
         if constexpr (kPairTaps && detail::tap_prepared<Back>()) {
-            const int sw = Back::width(p.back), sh = Back::height(p.back);
-            if (bounded_ok(sw, p)) {
-                BoundedTaps taps[V];
+            if (bounded_ok(sw, sh, p)) {
+                const detail::TapImage image = Back::tap_image_bounded(z, p.back);
+                auto points = [&](auto tag) {
+                    constexpr bool INTERIOR = decltype(tag)::value;
+                    BoundedTaps taps[V];
 #pragma unroll
-                for (int i = 0; i < V; ++i) {
-                    f32 sx, sy;
-                    source_point(x + i, y, p, sx, sy);
-                    taps[i] = bounded_request(sx, sy, sw, sh, z, p);
+                    for (int i = 0; i < V; ++i) taps[i] = bounded_request<INTERIOR>(sx[i], sy[i], sw, sh, image, p);
+#pragma unroll
+                    for (int i = 0; i < V; ++i) out[i].v = bounded_blend<INTERIOR>(taps[i], p);
+                };
+                if constexpr (MAY_SPLIT) {
+                    if (split && sh > 1) {
+                        bool interior = true;
+#pragma unroll
+                        for (int i = 0; i < V; ++i) interior = interior & within(sx[i], f32(sw - 1)) & within(sy[i], f32(sh - 1));
+                        if (detail::none_in_wave(!interior)) { points(detail::BoolTag<true>{}); return; }
+                    }
                 }
-                // (a variant without the selects for waves that have every source point inside and none on the last column
-                // was measured: 1 % slower at 1080p, 1 % faster at 2160p, eleven registers more)
-#pragma unroll
-                for (int i = 0; i < V; ++i) out[i].v = bounded_blend(taps[i], p);
+                points(detail::BoolTag<false>{});
                 return;
             }
         }
 #pragma unroll
-        for (int i = 0; i < V; ++i) out[i].v = exec(x + i, y, z, p);
+        for (int i = 0; i < V; ++i) out[i].v = value_at(sx[i], sy[i], sw, sh, z, p);
     }
     FKD_HD static bool rows_aligned(const Params&, int) { return true; }
 #endif
@@ -2837,9 +2880,10 @@ template <class T> struct Write2D {
     struct RowRef { T* p; };
     FKD_DEV static RowRef row(int y, int, const Params& p) { return RowRef{detail::row_ptr(p.data, p.pitch, 0, y)}; }
     // wave-uniform row address + 32-bit byte offset of the lane: the address form that needs no per-lane 64-bit add
-    FKD_DEV static void put(const RowRef& r, int x, const T& v) {
-        detail::store_elem_at<T>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
+    template <bool PLAIN = false> FKD_DEV static void put(const RowRef& r, int x, const T& v) {
+        detail::store_elem_at<T, PLAIN>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
     }
+    static constexpr bool kPutWhole = sizeof(T) % 4 == 0 && sizeof(T) == sizeof(base_t<T>) * cn_v<T> && sizeof(T) <= 16 && sizeof(base_t<T>) <= 4;
     template <int V> FKD_DEV static void put_run(const RowRef& r, int x, const Slot<T> (&v)[V]) {
         detail::store_run_at<T, V>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
     }
@@ -2973,9 +3017,10 @@ template <class T> struct TensorWrite {
     FKD_DEV static const Params& plane_params(const Params& p, int) { return p; }
     struct RowRef { T* p; };
     FKD_DEV static RowRef row(int y, int z, const Params& p) { return RowRef{detail::row_ptr(plane(p, z), p.pitch, 0, y)}; }
-    FKD_DEV static void put(const RowRef& r, int x, const T& v) {
-        detail::store_elem_at<T>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
+    template <bool PLAIN = false> FKD_DEV static void put(const RowRef& r, int x, const T& v) {
+        detail::store_elem_at<T, PLAIN>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
     }
+    static constexpr bool kPutWhole = sizeof(T) % 4 == 0 && sizeof(T) == sizeof(base_t<T>) * cn_v<T> && sizeof(T) <= 16 && sizeof(base_t<T>) <= 4;
     template <int V> FKD_DEV static void put_run(const RowRef& r, int x, const Slot<T> (&v)[V]) {
         detail::store_run_at<T, V>(reinterpret_cast<char*>(r.p), u32(x) * u32(sizeof(T)), v);
     }
@@ -3257,7 +3302,10 @@ template <int N, class W> struct BatchWrite {
     FKD_DEV static const typename W::Params& plane_params(const Params& p, int z) { return p.plane[z]; }
     using RowRef = typename W::RowRef;
     FKD_DEV static RowRef row(int y, int z, const Params& p) { return W::row(y, z, p.plane[z]); }
-    FKD_DEV static void put(const RowRef& r, int x, const In& v) { W::put(r, x, v); }
+    template <bool PLAIN = false> FKD_DEV static void put(const RowRef& r, int x, const In& v) {
+        if constexpr (puts_whole<W>()) W::template put<PLAIN>(r, x, v); else W::put(r, x, v);
+    }
+    static constexpr bool kPutWhole = puts_whole<W>();
     template <int V> FKD_DEV static void put_run(const RowRef& r, int x, const Slot<In> (&v)[V]) { W::template put_run<V>(r, x, v); }
 #endif
 };

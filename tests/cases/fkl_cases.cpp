@@ -530,6 +530,24 @@ int fklcase_warp_f32(void* stream, const float* src, int w, int h, int pitch, co
     });
 }
 
+// Three images of one size, each through a matrix of its own (m: three times nine values), into a tensor; compiled on first use.
+int fklcase_warp_batch_u8x3(void* stream_, const uint8_t* const* srcs, int w, int h, int pitch, const float* m, int dw, int dh, float* out) {
+    return guarded([&] {
+        constexpr size_t B = 3;
+        Stream stream(stream_);
+        auto plane = [&](size_t i) {
+            WarpingParameters<WarpType::Affine> params{};
+            for (int r = 0; r < 2; ++r)
+                for (int c = 0; c < 3; ++c) params.transformMatrix.data[r][c] = m[i * 9 + r * 3 + c];
+            params.dstSize = Size(dw, dh);
+            return PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(srcs[i], w, h, pitch).ptr()).then(Warping<WarpType::Affine>::build(params));
+        };
+        const std::array<decltype(plane(0)), B> planes{plane(0), plane(1), plane(2)};
+        Tensor<float3> o(reinterpret_cast<float3*>(out), uint(dw), uint(dh), uint(B), 1, MemType::Device, 0);
+        executeOperations<TransformDPP<>>(stream, BatchRead<PlanePolicy::PROCESS_ALL>::build(planes), TensorWrite<float3>::build(o.ptr()));
+    });
+}
+
 // Other pixel types (compiled on first use): kind 2 uchar4 -> float4, 3 ushort3 -> float3, 4 uchar -> float.
 int fklcase_warp_kind(void* stream, int kind, const void* src, int w, int h, int pitch, const float* m, int perspective, int dw, int dh,
                       float* out, int out_pitch) {

@@ -263,6 +263,15 @@ def warp(src, matrix, perspective, dst, out, kind=None):
            int(dst[0]), int(dst[1]), _p(out), out.stride(0) * 4))
 
 
+def warp_batch(srcs, matrices, dst, out):
+    """Three (H,W,3) u8 cuda images of one shape; matrices 3 times 2x3; out (3,dh,dw,3) f32 cuda."""
+    m = np.zeros((3, 9), np.float32)
+    m[:, :6] = np.asarray(matrices, np.float32).reshape(3, 6)
+    ptrs = (C.c_void_p * 3)(*[s.data_ptr() for s in srcs])
+    _ok(cases().fklcase_warp_batch_u8x3(_stream(), ptrs, srcs[0].shape[1], srcs[0].shape[0], srcs[0].stride(0), m.ctypes.data_as(C.c_void_p),
+                                        int(dst[0]), int(dst[1]), _p(out)))
+
+
 def deinterlace(src, mode, out):
     """src (H,W,3) u8 or (H,W) f32 cuda; mode 1 BLEND, 2 INTER_LINEAR keeping even lines, 3 keeping odd; out f32 same shape."""
     is_u8 = src.element_size() == 1
