@@ -299,6 +299,109 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
     }
 }
 
+// What one plane of a read is, and its parameters.
+template <class R> struct ReadRoot { using Op = R; static constexpr bool batched = false; };
+template <int N, class PlaneOp> struct ReadRoot<BatchRead<N, PlaneOp>> { using Op = PlaneOp; static constexpr bool batched = true; };
+
+// ---- rows kernel, planes without gaps ----
+//
+// Images as decoders hand them over have no padding between their rows, so a plane is one row of w * h elements: segments of 256
+// elements that begin where a line does follow each other through the whole plane, with no segment per row that is partly empty and no
+// line that two waves share, and the kernel has no rows to work out.  A wave takes ROWS segments one after the other.  Bound by the memory
+// (100 uchar3 images of 1527x794: 119 us for 728 MB) or, below 20 MB, by the launch and one trip to the memory.  us, rows / so:
+// 4 uchar3 images of 1279x719 6.1 / 4.5, 100 of 103x243 7.9 / 4.0, of 439x918 55 / 41, of 1920x1080 208 / 204; floats 4 times 1861x714 through
+// 30 operations 16.5 / 13.4, 4 of 317x63 through 100 20.6 / 11.9, 3840x2160 through 50 14.0 / 12.6.  Nothing measured got slower.
+// The arguments that every wave needs are requested together and waited for once, and what is left of an address after the wave's own
+// part is a lane's small offset.
+template <class Chain> constexpr bool rows_flat() { return flat_capable<typename Chain::Read, typename Chain::Write>(); }
+template <class Chain, int V, int ROWS, int MODE, bool PLAIN, bool EDGE, class Q, class WQ, class OPS>
+__device__ __forceinline__ void flat_run(const Q& q, const WQ& wpar, const OPS& ops, int first, int total, int z) {
+    using Op = typename ReadRoot<typename Chain::Read>::Op;
+    using WP = typename Chain::Write::Plane;
+    constexpr int kSegment = kRowsBX * V;
+    const int lane = int(threadIdx.x);
+    int x[ROWS], x0[ROWS];
+    Slot<typename Op::Out> in[ROWS * V];
+    // EDGE: some segment reaches past an end of the plane: lanes work on the first or last V elements instead and store the segment's own,
+    // as in rows_full.
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        x0[r] = x[r] = (EDGE ? first : 0) + r * kSegment + lane * V;
+        if constexpr (EDGE) x0[r] = x[r] < 0 ? 0 : (x[r] < total - V ? x[r] : total - V);
+        Slot<typename Op::Out> row[V];
+        Op::template exec_row<V, MODE>(x0[r], 0, z, q, row);
+#pragma unroll
+        for (int i = 0; i < V; ++i) in[r * V + i].v = row[i].v;
+    }
+    Slot<typename Chain::Value> out[ROWS * V];
+    if constexpr (Chain::kLongChain) Chain::template compute_run_kernarg<ROWS * V>(in, out, (const FKD_CONSTANT char*)__builtin_amdgcn_kernarg_segment_ptr());
+    else Chain::template compute_run<ROWS * V>(in, out, ops);
+    constexpr int STORE = MODE | (PLAIN ? detail::kPlainStores : 0);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        Slot<typename Chain::Value> row[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) row[i].v = out[r * V + i].v;
+        if constexpr (!EDGE) {
+            WP::template exec_row<V, STORE>(x0[r], 0, z, row, wpar);
+        } else if constexpr (has_edge_store<WP, V>()) {
+            if (first + r * kSegment < total) WP::template exec_edge<V>(first + r * kSegment, x0[r], total, 0, z, row, wpar);
+        } else {
+            if (x0[r] == x[r]) {
+                WP::template exec_row<V, STORE>(x0[r], 0, z, row, wpar);
+            } else if (x[r] > -V && x[r] < total) {
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    if (x0[r] + i >= x[r] && x0[r] + i < x[r] + V) WP::exec(x0[r] + i, 0, z, row[i].v, wpar);
+            }
+        }
+    }
+}
+template <class Chain, int V, int ROWS, bool SMALL>
+__device__ __forceinline__ void flat_body(const typename Chain::Params& p) {
+    using Root = ReadRoot<typename Chain::Read>;
+    using Op = typename Root::Op;
+    using W = typename Chain::Write;
+    using WP = typename W::Plane;
+    static_assert(V == int(kFlatRun) && kRowsBX == 64 && kRowsBY == 4, "flat_blocks lays out the grid");
+    constexpr int kSegment = kRowsBX * V;
+    const int z = int(blockIdx.z);
+    const typename Op::Params* rp;
+    if constexpr (Root::batched) rp = &p.read.plane[z]; else rp = &p.read;
+    typename Op::Params q = *rp;
+    typename WP::Params wpar = W::plane_params(p.write, z);
+    u32 head[4] = {p.active_w, p.active_h, p.reserved, gridDim.z};
+    detail::pin_scalars(q);
+    detail::pin_scalars(wpar);
+    detail::pin_scalars(head);
+    const int total = int(head[0] * head[1]);
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.y));
+    int first = (int(blockIdx.x) * kRowsBY + wave) * ROWS * kSegment;
+    if constexpr (!SMALL && has_row_phase<WP>()) {
+        const int phase = WP::row_phase(0, z, wpar) & int(Chain::row_phase_bound(head[2]));
+        first -= phase % x_group<Op>() == 0 ? phase : 0;
+    }
+    if (first >= total) return;
+    constexpr bool kExchange = (detail::wave_exchange_ok<typename Op::Out>(V) || detail::wave_exchange_ok<typename W::In>(V));
+    constexpr bool kMayStream = !SMALL && !Chain::kLongChain && !kExchange;
+    constexpr int kWhole = kExchange ? 2 | detail::kAnyAlign : 0;
+    if (first >= 0 && first + ROWS * kSegment <= total) {
+        // the wave's own part as base addresses: what is left of an address is the lane's small offset
+        Op::advance(q, first);
+        WP::advance(wpar, first);
+        if constexpr (kMayStream) {
+            if ((unsigned long long)u32(total) * head[3] > kStreamElements) { flat_run<Chain, V, ROWS, kWhole | 4, SMALL, false>(q, wpar, p.ops, first, total, z); return; }
+        }
+        flat_run<Chain, V, ROWS, kWhole, SMALL, false>(q, wpar, p.ops, first, total, z);
+    } else {
+        flat_run<Chain, V, ROWS, 0, SMALL, true>(q, wpar, p.ops, first, total, z);
+    }
+}
+template <class Chain, int V, int ROWS, bool SMALL>
+__global__ __launch_bounds__(kRowsBX * kRowsBY) void k_flat(const typename Chain::Params p) {
+    if constexpr (rows_flat<Chain>()) flat_body<Chain, V, ROWS, SMALL>(p);
+}
+
 // ---- rows kernel, scattered reads ----
 //
 // A warp's taps lie along a slanted line of the source, so what one instruction of a wave touches is decided by how far its
@@ -315,17 +418,15 @@ __device__ __forceinline__ void rows_body(const typename Chain::Params& p, u32 k
 // launch of 2.3.
 // For writers that store an element as one wide access; planar writers and elements of 1 to 3 bytes keep four outputs
 // of a row per lane, which they store as one access.
-template <class R> struct PointsRoot { using Op = R; static constexpr bool batched = false; };
-template <int N, class PlaneOp> struct PointsRoot<BatchRead<N, PlaneOp>> { using Op = PlaneOp; static constexpr bool batched = true; };
 template <class Op> constexpr bool reads_points() {
     if constexpr (requires { Op::kPoints; }) return Op::kPoints; else return false;
 }
 template <class Chain, int V, int ROWS> constexpr bool rows_by_points() {
-    return V == kRowsBY && ROWS == 1 && reads_points<typename PointsRoot<typename Chain::Read>::Op>() && puts_whole<typename Chain::Write>();
+    return V == kRowsBY && ROWS == 1 && reads_points<typename ReadRoot<typename Chain::Read>::Op>() && puts_whole<typename Chain::Write>();
 }
 template <class Chain, int V, int FORM>
 __device__ __forceinline__ void points_body(const typename Chain::Params& p, const TileGeom& bands) {
-    using Root = PointsRoot<typename Chain::Read>;
+    using Root = ReadRoot<typename Chain::Read>;
     using Op = typename Root::Op;
     using W = typename Chain::Write;
     using WP = typename W::Plane;
@@ -1092,15 +1193,19 @@ template <class D> __global__ __launch_bounds__(kRowsBX * kRowsBY) void k_diverg
 template <class Chain> constexpr bool rows_have_small() {
     if constexpr (IsDivergent<Chain>::value) return false; else return !is_gather_chain<Chain>();
 }
+// ... and kernels for planes without gaps.
+template <class Chain> constexpr bool rows_have_flat() {
+    if constexpr (IsDivergent<Chain>::value) return false; else return !is_gather_chain<Chain>() && rows_flat<Chain>();
+}
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
-                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u,
+                       !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u, rows_have_flat<Chain>() ? 1u : 0u,
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
@@ -1130,6 +1235,10 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
 // The kernel for small outputs (nothing for chains that have none).
 template <class Chain> __device__ __forceinline__ void jit_small_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (rows_have_small<Chain>()) rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
+}
+// The kernels for planes without gaps, likewise.
+template <class Chain, bool SMALL> __device__ __forceinline__ void jit_flat_body(const typename Chain::Params& p) {
+    if constexpr (rows_have_flat<Chain>()) flat_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, SMALL>(p);
 }
 
 } // namespace fkd

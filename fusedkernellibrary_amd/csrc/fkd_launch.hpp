@@ -56,9 +56,31 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     return launch_by_pointer(&k_rows<Chain, V, ROWS, false, kRowsLines>, grid, block, stream, p, g);
 }
 
+// Planes without gaps (kFlatBit): a one-dimensional grid per plane.  Below four workgroups per compute unit a wave takes half the
+// segments.  us with the line at 768 / 1024 / 2048 workgroups: 4 uchar3 images of 1279x719 (1 800) 4.5 / 4.5 / 4.9, 4 of 1209x263 (624; 4
+// launches) 12.4 / 12.4 / 12.4 (at 512: 13.05), 4 of 849x880 (1 460; 4 launches) 16.2 / 16.2 / 17.9, 50 operations on 3840x2160 floats (2 025) 12.6 / 12.6 /
+// 13.6, on 3384x77 (64) 9.2 to 10.6 from run to run.
+constexpr unsigned kFlatFewBlocks = 1024;
+template <class Chain, int V, int ROWS>
+hipError_t launch_flat(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
+    const unsigned blocks = flat_blocks(p.active_w, p.active_h, p.reserved, ROWS);
+    if constexpr (ROWS > 1) {
+        if ((unsigned long long)blocks * p.active_z < kFlatFewBlocks) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
+    }
+    const dim3 grid(blocks, 1, p.active_z), block(kRowsBX, kRowsBY, 1);
+    if (info) *info = LaunchInfo{"rows", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
+    if (grid.z == 0) return hipSuccess;
+    if (grid.z > 65535u) return hipErrorInvalidConfiguration;
+    if ((p.reserved & kSmallOutputBit) != 0u) return launch_by_pointer(&k_flat<Chain, V, ROWS, true>, grid, block, stream, p);
+    return launch_by_pointer(&k_flat<Chain, V, ROWS, false>, grid, block, stream, p);
+}
+
 template <class Chain>
 hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int V = RowsConfig<Chain>::V, ROWS = RowsConfig<Chain>::ROWS;
+    if constexpr (rows_flat<Chain>()) {
+        if ((p.reserved & kFlatBit) != 0u) return launch_flat<Chain, V, ROWS>(p, stream, info);
+    }
     // Chains whose reads may start anywhere in a row have one kernel for rows at every alignment.  The others have one for rows
     // that all start on dword boundaries (checked here, once per launch, on the host) and one for the rest.
     bool aligned = true;

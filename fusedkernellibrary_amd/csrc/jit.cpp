@@ -47,9 +47,10 @@ using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
-// A module's kernels: the chain's own and the one for small outputs (empty where JitMeta::has_small is 0).
-constexpr const char* kJitSuffix[2] = {"", "_small"};
-using JitFunctions = std::array<hipFunction_t, 2>;
+// A module's kernels: the chain's own, the one for small outputs (empty where JitMeta::has_small is 0), and the two for planes without gaps
+// (empty where JitMeta::has_flat is 0).
+constexpr const char* kJitSuffix[4] = {"", "_small", "_flat", "_flat_small"};
+using JitFunctions = std::array<hipFunction_t, 4>;
 
 struct JitKernel {
     std::string signature;
@@ -198,19 +199,19 @@ hipError_t get_functions(hipModule_t mod, const std::string& signature, JitFunct
     return hipSuccess;
 }
 
-int get_function(JitKernel* k, bool small, hipFunction_t* fn) {
+int get_function(JitKernel* k, unsigned which, hipFunction_t* fn) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return int(e);
     std::lock_guard<std::mutex> lock(k->mu);
     const auto it = k->per_device.find(dev);
-    if (it != k->per_device.end()) { *fn = it->second[small ? 1 : 0]; return FKLHIP_OK; }
+    if (it != k->per_device.end()) { *fn = it->second[which]; return FKLHIP_OK; }
     hipModule_t mod = nullptr;
     if ((e = hipModuleLoadData(&mod, k->code.data())) != hipSuccess) return int(e);
     JitFunctions fns{};
     if ((e = get_functions(mod, k->signature, &fns)) != hipSuccess) return int(e);
     k->per_device.emplace(dev, fns);   // the module stays loaded for the life of the process
-    *fn = fns[small ? 1 : 0];
+    *fn = fns[which];
     return FKLHIP_OK;
 }
 
@@ -225,6 +226,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     const bool streamed = m.gather && (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes;
     unsigned grid[3], block[3] = {64, 4, 1};
     const char* kind = m.gather ? "gather_jit" : "rows_jit";
+    unsigned which = 0;                      // of kJitSuffix
     if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {
         // strip form: one workgroup per m.by * m.yi output rows of a plane; tiles_x == 0 tells the kernel, and n_tiles
         // carries the launch's priority schedule
@@ -244,7 +246,13 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[1] = 1;
         grid[2] = active[2];
         block[1] = m.by;
+    } else if (m.has_flat != 0u && (active[3] & fkd::kFlatBit) != 0u) {
+        which = (active[3] & fkd::kSmallOutputBit) != 0u ? 3u : 2u;
+        grid[0] = fkd::flat_blocks(active[0], active[1], active[3], m.rows);
+        grid[1] = 1;
+        grid[2] = active[2];
     } else {
+        if (m.has_small != 0u && fkd::rows_small(active[0], m.v, active[3])) which = 1u;
         grid[0] = (active[0] + (m.max_planes != 0 ? 0u : rows_phase_bound(active[3])) + 64 * m.v - 1) / (64 * m.v);
         grid[1] = (active[1] + 4 * m.rows - 1) / (4 * m.rows);
         grid[2] = active[2];
@@ -268,7 +276,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     if (grid[1] > 65535u || grid[2] > 65535u) return int(hipErrorInvalidConfiguration);
     if (m.max_planes != 0 && grid[2] > m.max_planes) return int(hipErrorInvalidConfiguration);   // as launch_divergent
     hipFunction_t fn = nullptr;
-    const int rc = get_function(k, m.has_small != 0u && fkd::rows_small(active[0], m.v, active[3]), &fn);
+    const int rc = get_function(k, which, &fn);
     if (rc != FKLHIP_OK) return rc;
     // Kernel-argument segment: the parameter block, then the TileGeom at the next 4-byte boundary.  The runtime
     // copies the buffer during the call, so the caller's block may go away as soon as we return.
@@ -309,6 +317,11 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
                "(const JitChain::Params p, const TileGeom g) {\n"
                "    jit_small_body<JitChain>(p, g);\n"
                "}\n";
+        for (int i = 2; i < 4; ++i)
+            src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitSuffix[i] +
+                   "(const JitChain::Params p, const TileGeom) {\n"
+                   "    jit_flat_body<JitChain, " + (i == 3 ? "true" : "false") + ">(p);\n"
+                   "}\n";
         hiprtcProgram prog = nullptr;
         hiprtcResult r = hiprtcCreateProgram(&prog, src.c_str(), "fkd_jit_chain.hip", kJitHeaderCount, kJitHeaderTexts, kJitHeaderNames);
         if (r != HIPRTC_SUCCESS) { g_log = hiprtcGetErrorString(r); delete k; return FKLHIP_EUNKNOWN_SIGNATURE; }

@@ -84,6 +84,20 @@ constexpr unsigned kSmallOutputBit = 4u;
 // that, of which such a kernel knows nothing, are left to the other one), reserved: the parameter block's flags.
 inline bool rows_small(unsigned w, unsigned run, unsigned reserved) { return (reserved & kSmallOutputBit) != 0u && w >= run; }
 
+// Bit 3 of a chain's Params::reserved: the rows of every plane, read and written, follow each other without gaps, so the launch takes
+// a plane as one row of w * h elements.
+constexpr unsigned kFlatBit = 8u;
+constexpr unsigned kFlatRun = 4;             // elements of a thread's run in such a launch
+inline bool flat_fits(unsigned w, unsigned h) {
+    const unsigned long long n = (unsigned long long)w * h;
+    return n >= kFlatRun && n <= 0x7fff0000ull;
+}
+// The workgroups of a plane of such a launch; `rows`: segments of 64 runs per wave, of which a workgroup has four.
+inline unsigned flat_blocks(unsigned w, unsigned h, unsigned reserved, unsigned rows) {
+    const unsigned per_block = 64u * kFlatRun * 4u * rows;
+    return unsigned(((unsigned long long)w * h + rows_phase_bound(reserved) + per_block - 1u) / per_block);
+}
+
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
     unsigned gather;          // 1: gather kernel geometry, 0: rows kernel geometry
@@ -94,6 +108,7 @@ struct JitMeta {
     unsigned strip_width;     // gather kernel: outputs up to this width are launched in strip form (TileGeom::tiles_x == 0), 0: never
     unsigned bands;           // rows kernel: 1 when launches of kRowsBandBlocks blocks per plane or more take the bands form of grid, 2 when smaller ones may as well (rows_bands_2d)
     unsigned has_small;       // rows kernel: 1 when the module has a kernel for small outputs (see rows_small)
+    unsigned has_flat;        // rows kernel: 1 when the module has kernels for planes taken as one row (kFlatBit)
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
 };
 

@@ -140,6 +140,12 @@ inline u32 phase_bound_for(u32 full, u32 width, unsigned long long bytes, unsign
 template <class W> constexpr bool has_row_phase() {
     if constexpr (requires { W::kRowPhase; }) return W::kRowPhase; else return false;
 }
+// knows_dense<Op>: read or write Op can tell (dense) whether the elements of a plane w elements wide follow each other without gaps
+// from the first row to the last, so that element (x, y) is element y * w + x of its first row, and its parameters can be moved on
+// by n elements (advance).
+template <class Op> constexpr bool knows_dense() {
+    return requires(const typename Op::Params& p) { Op::dense(p, 1u, 1u); };
+}
 // puts_whole<W>: write W stores one element as one wide access, told whether to carry the non-temporal hint.
 template <class W> constexpr bool puts_whole() {
     if constexpr (requires { W::kPutWhole; }) return W::kPutWhole; else return false;
@@ -1613,6 +1619,8 @@ template <class T> struct Read2D {
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
         return (any_pitch || p.pitch % 4 == 0) && size_t(p.pitch) * p.height < 0x7ffffff0ull && p.width >= 2 && p.height >= 1;
     }
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(T); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
     FKD_DEV static int height(const Params& p) { return int(p.height); }
@@ -1696,6 +1704,8 @@ template <class T> struct Read3D {
     static constexpr bool kAnyX = true;
     static constexpr bool kBoundedOut = small_integer_base<T>();
     FKD_NAME("Read3D<" + type_name<T>() + ">")
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(T); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
     FKD_DEV static int height(const Params& p) { return int(p.height); }
@@ -1990,6 +2000,9 @@ template <int PF> struct ReadYUV {
     static constexpr bool kAnyX = true;
     static constexpr bool kTapCursor = false;
     FKD_NAME("ReadYUV<" + istr(PF) + ">")
+    // (packed formats: two samples per pixel; the planes of the others are two images)
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return !L::kSemiPlanar && w % 2 == 0 && p.pitch == size_t(w) * 2 * sizeof(B); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n * 2 * ptrdiff_t(sizeof(B)); }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
     FKD_DEV static int height(const Params& p) { return int(p.height); }
@@ -2286,6 +2299,8 @@ template <class Back, class... Ops> struct FusedRead {
     static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>() && (finite_map<Ops>() && ...);
     FKD_NAME("FusedRead<" + Back::name() + OpList<Ops...>::names() + ">")
+    FKD_HD static bool dense(const Params& p, u32 w, u32 planes) requires (knows_dense<Back>()) { return Back::dense(p.back, w, planes); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) requires (knows_dense<Back>()) { Back::advance(p.back, n); }
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
         if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return Back::strip_ok(p.back, any_pitch); else return false;
     }
@@ -2768,6 +2783,11 @@ template <int N, class PlaneOp> struct BatchRead {
     static constexpr int kXGroup = x_group<PlaneOp>();
     static constexpr bool kBoundedOut = bounded_out<PlaneOp>();
     FKD_NAME("BatchRead<" + istr(N) + "," + PlaneOp::name() + ">")
+    FKD_HD static bool dense(const Params& p, u32 w, u32 planes) requires (knows_dense<PlaneOp>()) {
+        for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::dense(p.plane[z], w, 1u)) return false;
+        return planes <= u32(N);
+    }
+    static constexpr bool kPlanes = true;      // plane z is plane[z], a PlaneOp of its own
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch, u32 planes) {
         if constexpr (requires { PlaneOp::strip_ok(p.plane[0], any_pitch); }) {
             for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::strip_ok(p.plane[z], any_pitch)) return false;
@@ -2858,6 +2878,9 @@ template <class T> struct Write2D {
     static constexpr bool kRowPhase = true;
     static constexpr unsigned long long kPhaseMin = phase_min_bytes<T>();
     FKD_HD static u32 row_phase_bound(const Params& p) { return row_phase_bound_of<T>(p.data, p.pitch); }
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(T); }
+    FKD_HD static u32 dense_phase_bound(const Params& p) { return row_phase_bound_of<T>(p.data, 0); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static void exec(int x, int y, int, const T& v, const Params& p) {
         detail::store_elem(detail::row_ptr(p.data, p.pitch, x, y), v);
@@ -2992,6 +3015,9 @@ template <class T> struct TensorWrite {
     FKD_HD static u32 row_phase_bound(const Params& p) {
         return row_phase_bound_of<T>(p.data, p.pitch, p.planes > 1 ? size_t(p.plane_pitch) * p.color_planes : 0);
     }
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(T); }
+    FKD_HD static u32 dense_phase_bound(const Params& p) { return row_phase_bound_of<T>(p.data, 0, p.planes > 1 ? size_t(p.plane_pitch) * p.color_planes : 0); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static T* plane(const Params& p, int z) {
         return reinterpret_cast<T*>(reinterpret_cast<char*>(p.data) + size_t(p.plane_pitch) * p.color_planes * z);
@@ -3041,6 +3067,8 @@ template <class T, bool TRANSPOSED = false> struct TensorSplit {
         return G::channel_elements(p) * sizeof(B) * cn_v<T> < size_t(0x7fffffffu) &&
                G::channel_elements(p) * sizeof(B) * (cn_v<T> - 1) + size_t(p.pitch) * p.height < size_t(0x7fffffffu);
     }
+    FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(B); }
+    FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
     // The power of two, at most a line, that the addresses of both ends of every row of `w` values are multiples of.
     FKD_HD static u32 row_grain(const Params& p, u32 w, u32 planes) {
         const size_t ends = reinterpret_cast<size_t>(p.data) | p.pitch | G::channel_elements(p) * sizeof(B) | (planes > 1u ? G::image_bytes(p) : 0u) | size_t(w) * sizeof(B) | kLineBytes;
@@ -3281,6 +3309,14 @@ template <int N, class W> struct BatchWrite {
         }
         return 0u;
     }
+    FKD_HD static bool dense(const Params& p, u32 w, u32 planes) requires (knows_dense<W>()) {
+        for (u32 z = 0; z < planes && z < u32(N); ++z) if (!W::dense(p.plane[z], w, 1u)) return false;
+        return planes <= u32(N);
+    }
+    FKD_HD static u32 dense_phase_bound(const Params& p) requires (knows_dense<W>() && has_row_phase<W>()) {
+        for (int i = 0; i < N; ++i) if (const u32 b = W::dense_phase_bound(p.plane[i])) return b;      // one bound per type
+        return 0u;
+    }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static void exec(int x, int y, int z, const In& v, const Params& p) { W::exec(x, y, z, v, p.plane[z]); }
 #endif
@@ -3421,6 +3457,9 @@ inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes
 }
 #endif
 
+// Whether the rows kernel can take a plane of the chain as one row (kFlatBit): both ends know when their planes are dense.
+template <class R, class W> constexpr bool flat_capable() { return any_x<R>() && knows_dense<R>() && knows_dense<W>(); }
+
 template <class R, class Ops, class W> struct Chain;
 template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     using Read = R;
@@ -3480,11 +3519,18 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
     // Bits 8 to 15: by how many elements at most the rows kernel's waves begin left of a row to store whole lines (see
     // phase_bound_for).
     // Bit 2: the launch writes no more than kSmallOutputBytes and its segments begin at the row's start.
+    // Bit 3: every plane is one row of w * h elements (kFlatBit).
     static void finalize_write(Params& p) {
         const unsigned long long elements = (unsigned long long)p.active_w * p.active_h * p.active_z;
         if constexpr (any_x<R>() && has_row_phase<W>()) p.reserved |= phase_bound_for(W::row_phase_bound(p.write), p.active_w, elements * sizeof(Value), W::kPhaseMin) << 8;
         unsigned long long stored = elements * sizeof(Value);
         if constexpr (requires { W::stored_bytes(elements); }) stored = W::stored_bytes(elements);
+        if constexpr (flat_capable<R, W>()) {
+            if (flat_fits(p.active_w, p.active_h) && R::dense(p.read, p.active_w, p.active_z) && W::dense(p.write, p.active_w, p.active_z)) {
+                p.reserved = kFlatBit;
+                if constexpr (has_row_phase<W>()) { if (stored > kSmallOutputBytes) p.reserved |= W::dense_phase_bound(p.write) << 8; }
+            }
+        }
         if (row_phase_bound(p.reserved) == 0u && stored <= kSmallOutputBytes) p.reserved |= kSmallOutputBit;
         if constexpr (requires { R::strip_ok(p.read, false, p.active_z); W::strip_ok(p.write); }) {
             const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);

@@ -329,6 +329,27 @@ int fklcase_copy_tensor(void* stream, int kind, const void* src, int pitch, int 
         }
     });
 }
+// Image of uchar3 -> planar floats, no gaps asked for by anyone: pitches are the caller's.
+int fklcase_u8x3_to_planes(void* stream_, const uint8_t* src, int pitch, int w, int h, float* out) {
+    return guarded([&] {
+        Stream stream(stream_);
+        Tensor<float> o(out, uint(w), uint(h), 1, 3, MemType::Device, 0);
+        executeOperations<TransformDPP<>>(stream, PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(src, w, h, pitch).ptr()), SaturateCast<uchar3, float3>::build(),
+                                          TensorSplit<float3>::build(o.ptr()));
+    });
+}
+// The flags (Chain::Params::reserved) a launch of copy_tensor gets for uchar3 elements, on the host alone.
+int fklcase_copy_flags(long long address, int pitch, int plane_pitch, long long out_address, int out_pitch, int out_plane_pitch, int w, int h, int planes) {
+    auto view = [&](long long at, int row, int plane) {
+        auto v = Tensor<uchar3>(reinterpret_cast<uchar3*>(at), uint(w), uint(h), uint(planes), 1u, MemType::Device, 0).ptr();
+        v.dims.pitch = uint(row);
+        v.dims.plane_pitch = uint(plane);
+        return v;
+    };
+    using R = Read<TensorRead<uchar3>>;
+    using W = Write<TensorWrite<uchar3>>;
+    return int(amd::FusedChain<R, W>::params(R{view(address, pitch, plane_pitch)}, W{view(out_address, out_pitch, out_plane_pitch)}).reserved);
+}
 // Horizontal fusion with fewer live planes than the compiled batch (BatchRead<CONDITIONAL_WITH_DEFAULT>).
 int fklcase_crop_resize_default_norm_split_b8(void* stream_, const uint8_t* src, int w, int h, int pitch, const int32_t* rects,
                                               int dw, int dh, int used_planes, const float* def, const float* sub,

@@ -241,6 +241,16 @@ def copy_tensor(kind, src, src_pitches, out, out_pitches, w, h, planes):
                                     int(out_pitches[1]), int(w), int(h), int(planes)))
 
 
+def u8x3_to_planes(src, out):
+    """(H,W,3) u8 cuda -> (3,H,W) f32 cuda, converted."""
+    _ok(cases().fklcase_u8x3_to_planes(_stream(), _p(src), _pitch(src), src.shape[1], src.shape[0], _p(out)))
+
+
+def copy_flags(address, pitches, out_address, out_pitches, w, h, planes):
+    """Chain::Params::reserved of a copy_tensor launch of uchar3 elements."""
+    return cases().fklcase_copy_flags(C.c_longlong(address), pitches[0], pitches[1], C.c_longlong(out_address), out_pitches[0], out_pitches[1], w, h, planes)
+
+
 def uncompiled_float4_resize(src, dst, out):
     """(H,W,4) f32 cuda -> bilinear -> out (dh,dw,4) f32 cuda."""
     _ok(cases().fklcase_uncompiled_float4_resize(_stream(), _p(src), src.shape[1], src.shape[0], src.stride(0) * 4, int(dst[0]), int(dst[1]),
