@@ -760,7 +760,11 @@ __device__ __forceinline__ void gather_tile(const typename Chain::Params& p, con
                 for (int i = 0; i < XI; ++i) if (xof(i) < aw) WP::put(orow, xof(i), res[i].v);
             }
         };
-        if constexpr (FKD_GATHER_DEPTH <= 2) {
+        if constexpr (YI == 1) {
+            RowTaps t;
+            request(y0, t);
+            produce(y0, t);
+        } else if constexpr (FKD_GATHER_DEPTH <= 2) {
             RowTaps t0, t1;
             request(y0, t0);
 #pragma unroll 1
@@ -829,6 +833,18 @@ __device__ __forceinline__ void gather_tile(const typename Chain::Params& p, con
     }
 }
 
+// Launches of few tiles.  A wave issues an instruction in four to five cycles at best, so where a SIMD has a wave or none the launch is as
+// long as one wave's work: four pixels of 100 instructions are 0.8 us of a launch of 3.  Such launches take tiles of 64x4 pixels (one
+// pixel per lane) or 128x4 (two); the line is at the number of 128x8 tiles the launch would have (gather_form, fkd/launch_info.hpp).
+template <class Chain> constexpr u32 gather_some_tiles() {
+    if constexpr (is_gather_chain<Chain>()) {
+        if constexpr (requires { typename ResizeRoot<typename Chain::Read>::Resize::BackOp::FusedOver; }) return kGatherSomeTilesFused;
+        else return kGatherSomeTiles;
+    } else {
+        return 0u;
+    }
+}
+
 template <class Chain, int XI, int YI, bool STREAM>
 __device__ __forceinline__ void gather_body(const typename Chain::Params& p, const TileGeom& g) {
     using Root = ResizeRoot<typename Chain::Read>;
@@ -894,7 +910,7 @@ __device__ __forceinline__ void gather_body(const typename Chain::Params& p, con
 // The launcher decides and hands the kernel one number: the number of the first workgroup that counts as started late, or
 // 0 for a launch whose waves keep the default priority.
 // (strip_first_late_workgroup, fkd/launch_info.hpp)
-constexpr int kStripRows = kGatherBY * FKD_GATHER_YI, kStripStep = 32, kStripMaxWidth = 256;
+constexpr int kStripRows = 8, kStripStep = 32, kStripMaxWidth = 256;
 constexpr int kStripThreads = kStripRows * kStripStep, kStripMaxSteps = kStripMaxWidth / kStripStep;
 static_assert(kStripThreads == kGatherBX * kGatherBY, "the two forms of the bilinear kernel share their workgroup shape");
 static_assert(kStripThreads == kStripMaxWidth, "one table column per thread");
@@ -1200,13 +1216,14 @@ template <class Chain> constexpr bool rows_have_flat() {
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
                        !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u, rows_have_flat<Chain>() ? 1u : 0u,
-                       is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u};
+                       is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u,
+                       gather_some_tiles<Chain>()};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) DivergentBody<Chain>::run(p);
@@ -1232,13 +1249,17 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
     }
     else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsLines>(p, 0u, &g);
 }
-// The kernel for small outputs (nothing for chains that have none).
-template <class Chain> __device__ __forceinline__ void jit_small_body(const typename Chain::Params& p, const TileGeom& g) {
-    if constexpr (rows_have_small<Chain>()) rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
-}
-// The kernels for planes without gaps, likewise.
-template <class Chain, bool SMALL> __device__ __forceinline__ void jit_flat_body(const typename Chain::Params& p) {
-    if constexpr (rows_have_flat<Chain>()) flat_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, SMALL>(p);
+// The module's other kernels, 1 to 3 (nothing for chains that have no such kernel).  Rows kernel: the kernel for small outputs, those for
+// planes without gaps; bilinear kernel: gather_form's forms 1 and 2.
+template <class Chain, int WHICH> __device__ __forceinline__ void jit_other_body(const typename Chain::Params& p, const TileGeom& g) {
+    if constexpr (IsDivergent<Chain>::value) {
+    } else if constexpr (is_gather_chain<Chain>()) {
+        if constexpr (WHICH < 3) gather_body<Chain, WHICH, 1, false>(p, g);
+    } else if constexpr (WHICH == 1) {
+        rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
+    } else if constexpr (rows_have_flat<Chain>()) {
+        flat_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, WHICH == 3>(p);
+    }
 }
 
 } // namespace fkd

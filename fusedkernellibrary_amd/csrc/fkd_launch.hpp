@@ -96,7 +96,7 @@ hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, Laun
 template <class Chain>
 hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int XI = FKD_GATHER_XI, YI = FKD_GATHER_YI;
-    constexpr int TW = kGatherBX * XI, TH = kGatherBY * YI;
+    static_assert(kGatherBX * XI == int(kGatherTileW[0]) && kGatherBY * YI == int(kGatherTileH[0]), "gather_form speaks of these tiles");
     constexpr bool kStreams = writer_streams<Chain>();
     const bool streamed = kStreams && (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(typename Chain::Value) > kStreamOutputBytes;
     if constexpr (strip_capable<Chain>()) {
@@ -116,6 +116,8 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
             return launch_by_pointer(&k_strip<Chain, false, false>, grid, block, stream, p, first_late);
         }
     }
+    const unsigned form = gather_form(p.active_w, p.active_h, p.active_z, gather_some_tiles<Chain>());
+    const unsigned TW = kGatherTileW[form], TH = kGatherTileH[form];
     TileGeom g;
     g.tiles_x = (p.active_w + TW - 1) / TW;
     g.tiles_y = (p.active_h + TH - 1) / TH;
@@ -126,6 +128,8 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
     if (info) *info = LaunchInfo{"gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
     if (g.n_tiles == 0) return hipSuccess;
     if (grid.z > 65535u) return hipErrorInvalidConfiguration;
+    if (form == 1u) return launch_by_pointer(&k_gather<Chain, 1, 1, false>, grid, block, stream, p, g);
+    if (form == 2u) return launch_by_pointer(&k_gather<Chain, 2, 1, false>, grid, block, stream, p, g);
     if (streamed) return launch_by_pointer(&k_gather<Chain, XI, YI, kStreams>, grid, block, stream, p, g);
     return launch_by_pointer(&k_gather<Chain, XI, YI, false>, grid, block, stream, p, g);
 }

@@ -41,15 +41,16 @@ using fkd::JitMeta;
 using fkd::TileGeom;
 using fkd::division_magic;
 using fkd::kRowsBandBlocks;
+using fkd::gather_form;
 using fkd::kAnyPitchFlag;
 using fkd::kStreamFlag;
 using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
-// A module's kernels: the chain's own, the one for small outputs (empty where JitMeta::has_small is 0), and the two for planes without gaps
-// (empty where JitMeta::has_flat is 0).
-constexpr const char* kJitSuffix[4] = {"", "_small", "_flat", "_flat_small"};
+// A module's kernels.  Rows kernel: the chain's own, the one for small outputs (empty where JitMeta::has_small is 0), and the two for
+// planes without gaps (empty where JitMeta::has_flat is 0).  Bilinear kernel: the chain's own, and those of gather_form's forms 1 and 2.
+constexpr const char* kJitSuffix[4] = {"", "_1", "_2", "_3"};
 using JitFunctions = std::array<hipFunction_t, 4>;
 
 struct JitKernel {
@@ -237,7 +238,8 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         block[1] = m.by;
         g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]) | (streamed ? kStreamFlag : 0u) | ((active[3] & 2u) != 0 ? kAnyPitchFlag : 0u);
     } else if (m.gather) {
-        const unsigned tw = 64 * m.xi, th = m.by * m.yi;
+        which = gather_form(active[0], active[1], active[2], m.some_tiles);
+        const unsigned tw = fkd::kGatherTileW[which], th = fkd::kGatherTileH[which];
         g.tiles_x = (active[0] + tw - 1) / tw;
         g.tiles_y = (active[1] + th - 1) / th;
         g.n_tiles = streamed ? kStreamFlag : 0u;       // (the kernel counts its tiles itself)
@@ -313,14 +315,10 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
         src += "(const JitChain::Params p, const TileGeom g) {\n"
                "    jit_body<JitChain>(p, g);\n"
                "}\n";
-        src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitSuffix[1] +
-               "(const JitChain::Params p, const TileGeom g) {\n"
-               "    jit_small_body<JitChain>(p, g);\n"
-               "}\n";
-        for (int i = 2; i < 4; ++i)
+        for (int i = 1; i < 4; ++i)
             src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitSuffix[i] +
-                   "(const JitChain::Params p, const TileGeom) {\n"
-                   "    jit_flat_body<JitChain, " + (i == 3 ? "true" : "false") + ">(p);\n"
+                   "(const JitChain::Params p, const TileGeom g) {\n"
+                   "    jit_other_body<JitChain, " + std::to_string(i) + ">(p, g);\n"
                    "}\n";
         hiprtcProgram prog = nullptr;
         hiprtcResult r = hiprtcCreateProgram(&prog, src.c_str(), "fkd_jit_chain.hip", kJitHeaderCount, kJitHeaderTexts, kJitHeaderNames);

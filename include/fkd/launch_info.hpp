@@ -98,6 +98,19 @@ inline unsigned flat_blocks(unsigned w, unsigned h, unsigned reserved, unsigned 
     return unsigned(((unsigned long long)w * h + rows_phase_bound(reserved) + per_block - 1u) / per_block);
 }
 
+// Which tiles a launch of the bilinear kernel's tile form takes: 128x8 pixels, or smaller ones where it would have few of those (per-wave
+// latency, see the kernels' header).  us, tiles of 128x8 / 128x4 / 64x4 pixels (in brackets: how many of 128x8): NV12 to 148x85 (22)
+// 3.23 / 2.41 / 2.09, to 320x180 (69) 2.58 / 2.05 / 1.94, to 400x300 (152) 3.23 / 2.61 / 2.69, to 1100x700 (792) 5.32 / 4.71 / 5.38, to 1333x800 (1100)
+// 6.2 / 5.1 / 6.3, to 1600x900 (1469) 6.5 / 6.0 / 7.6, to 1920x1000 (1875) 7.6 / 6.7, to 2300x1300 (2934) 11.3 / 11.6; 5 thumbnails of 128x128 (80) 3.17 / 2.46 / 2.28, of 256x256 (320) 3.41 / 2.98 / 3.17; 8 crops
+// to 64x64 (64) 2.96 / 2.38 / 2.16, to 224x64 (128) 3.09 / 2.42 / 2.63, to 224x224 (448) 3.73 / 3.46 / 3.99, to 300x200 (600) 4.07 / 3.89 / 4.34, to 384x300 (912)
+// 4.60 / 4.42, to 320x320 (960) 4.56 / 4.77 / 5.59, 64 crops to 300x64 (1536) 5.9 / 6.3 / 8.0.  Reads that work on every tap (a colour conversion) are longer and cross later.
+constexpr unsigned kGatherFewTiles = 128, kGatherSomeTiles = 920, kGatherSomeTilesFused = 2560;
+constexpr unsigned kGatherTileW[3] = {128, 64, 128}, kGatherTileH[3] = {8, 4, 4};
+inline unsigned gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) {
+    const unsigned long long tiles = (unsigned long long)((w + 127u) / 128u) * ((h + 7u) / 8u) * planes;
+    return tiles < kGatherFewTiles ? 1u : tiles < some_tiles ? 2u : 0u;
+}
+
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
     unsigned gather;          // 1: gather kernel geometry, 0: rows kernel geometry
@@ -110,6 +123,7 @@ struct JitMeta {
     unsigned has_small;       // rows kernel: 1 when the module has a kernel for small outputs (see rows_small)
     unsigned has_flat;        // rows kernel: 1 when the module has kernels for planes taken as one row (kFlatBit)
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
+    unsigned some_tiles;      // gather kernel: the last argument of gather_form
 };
 
 } // namespace fkd

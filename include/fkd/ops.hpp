@@ -2298,6 +2298,7 @@ template <class Back, class... Ops> struct FusedRead {
     static constexpr bool kAnyX = any_x<Back>();
     static constexpr int kXGroup = x_group<Back>();
     static constexpr bool kBoundedOut = bounded_out<Back>() && (finite_map<Ops>() && ...);
+    using FusedOver = Back;
     FKD_NAME("FusedRead<" + Back::name() + OpList<Ops...>::names() + ">")
     FKD_HD static bool dense(const Params& p, u32 w, u32 planes) requires (knows_dense<Back>()) { return Back::dense(p.back, w, planes); }
     FKD_HD static void advance(Params& p, ptrdiff_t n) requires (knows_dense<Back>()) { Back::advance(p.back, n); }
