@@ -929,9 +929,69 @@ template <class Chain> constexpr bool strip_capable() {
     }
 }
 
+// Planar outputs whose rows are no whole lines: the stores of a row's steps, moved on to line boundaries.
+//
+// A step's LANES values begin wherever the row does, so stored as they are they cut a line at both of their ends, and such a line
+// leaves the chip as two partial writes (64 crops to 639x639 104 us where 640x640 take 57).  Here the lanes of a step store the
+// LANES elements from a line boundary on: a lane takes its value from the lane `shift` below it (ds_bpermute), and the lanes below the shift
+// store what the step before has left.  Channel planes begin anywhere too, so each has a shift of its own.  Only the two lines at a row's ends
+// are cut.  (Whole strips collected in LDS and stored as one run cut fewer lines and were slower for all but the largest launches: 225x225
+// 13.0 against 11.5 us, 517x517 52.5 / 48.2, 639x639 75 / 81; the LDS leaves room for three or four workgroups, and stores begin when a
+// workgroup's work is over.)
+template <class Chain, int LANES> struct LineStores {
+    using Value = typename Chain::Value;
+    using WP = typename Chain::Write::Plane;
+    static constexpr int N = cn_v<Value>;
+    u32 off[N];        // byte offset of the lane's element of step 0
+    int from[N];       // the lane (times four) whose value the lane stores
+    int shift[N];      // elements between the line boundary at or before the row's first element and that element
+    u32 left[N];       // what the step before left for the lanes below the shift
+    // g: the lane's number in its row
+    template <class WPAR> __device__ __forceinline__ void open(int z, int y, bool valid, int g, const WPAR& wpar) {
+        const char* row = WP::channel_row(z, y, wpar);
+        const u32 row_off = u32(row - WP::channel_row(z, 0, wpar));
+        const int lane0 = int(threadIdx.x) - g;
+#pragma unroll
+        for (int c = 0; c < N; ++c) {
+            shift[c] = int((u32(reinterpret_cast<uintptr_t>(row + size_t(c) * WP::channel_bytes(wpar))) / 4u) & (kLineBytes / 4u - 1u));
+            off[c] = valid ? row_off + u32(g - shift[c]) * 4u : WP::kMaskedOut;
+            from[c] = (lane0 + ((g - shift[c]) & (LANES - 1))) * 4;
+            left[c] = 0u;
+        }
+    }
+    // (the offset of a lane left of its row wraps, but such a lane is masked: check)
+    template <bool STREAM, int C> __device__ __forceinline__ void store(const typename WP::PlaneRef& r, int k, int g, bool check, int aw, u32 now) {
+        const u32 v = g < shift[C] ? left[C] : now;
+        u32 at = off[C] + u32(k) * (LANES * 4u);
+        if (check) {
+            const int x = k * LANES + g - shift[C];
+            if (x < 0 || x >= aw) at = WP::kMaskedOut;
+        }
+        WP::template put_channel<STREAM, C>(r, at, v);
+        left[C] = now;
+    }
+    template <bool STREAM, int C> __device__ __forceinline__ void one(const typename WP::PlaneRef& r, int k, int g, bool check, int aw, const Value& v) {
+        store<STREAM, C>(r, k, g, check, aw, u32(__builtin_amdgcn_ds_bpermute(from[C], int(__builtin_bit_cast(u32, chan<C>(v))))));
+    }
+    template <bool STREAM> __device__ __forceinline__ void put(const typename WP::PlaneRef& r, int k, int g, bool check, int aw, const Value& v) {
+        one<STREAM, 0>(r, k, g, check, aw, v); one<STREAM, 1>(r, k, g, check, aw, v);
+        if constexpr (N > 2) one<STREAM, 2>(r, k, g, check, aw, v);
+        if constexpr (N > 3) one<STREAM, 3>(r, k, g, check, aw, v);
+    }
+    // ... and what the last step left.
+    template <bool STREAM> __device__ __forceinline__ void finish(const typename WP::PlaneRef& r, int steps, int g, int aw) {
+        store<STREAM, 0>(r, steps, g, true, aw, 0u); store<STREAM, 1>(r, steps, g, true, aw, 0u);
+        if constexpr (N > 2) store<STREAM, 2>(r, steps, g, true, aw, 0u);
+        if constexpr (N > 3) store<STREAM, 3>(r, steps, g, true, aw, 0u);
+    }
+};
+
 // ANY_PITCH: some image of the launch has rows that do not share their alignment (Chain::kStripAnyPitch).
-template <class Chain, bool STREAM, bool ANY_PITCH>
+// LINES: stores on line boundaries (LineStores); then a row may have LANES = 64 lanes, so a workgroup four rows, and MAX_STEPS steps.
+template <class Chain, bool STREAM, bool ANY_PITCH, bool LINES = false, int LANES = kStripStep, int MAX_STEPS = kStripMaxSteps>
 __device__ __forceinline__ void strip_body(const typename Chain::Params& p, const u32 first_late_workgroup) {
+    constexpr int kStripStep = LANES, kStripMaxSteps = MAX_STEPS, kStripRows = kStripThreads / LANES;
+    constexpr int kColumns = LINES ? (MAX_STEPS + 1) * LANES : kStripMaxWidth;
     using Root = ResizeRoot<typename Chain::Read>;
     using RZ = typename Root::Resize;
     using Back = typename RZ::BackOp;
@@ -939,7 +999,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     using W = typename Chain::Write;
     using WP = typename W::Plane;
     // per column: ax, bx, window offset, bytes to drop from the window (bits 0-1) | flags
-    __shared__ detail::u32x4_t column[kStripMaxWidth];
+    __shared__ detail::u32x4_t column[kColumns];
     __shared__ u32 wave_clamped[kStripThreads / 64];
     constexpr u32 kClamped = 0x80000000u, kOutsideX = 0x40000000u;
 
@@ -1003,7 +1063,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     };
 
     // ---- the lane's row ----
-    const int g = t & (kStripStep - 1), r = t >> 5;
+    const int g = t & (kStripStep - 1), r = t / kStripStep;
     const int y = int(blockIdx.x) * kStripRows + r;
     const bool yvalid = y < ah;
     const int yc = yvalid ? y : ah - 1;
@@ -1051,9 +1111,18 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     constexpr u32 kNoWindow = 0x80000000u;
     {
         bool clamped = false;
-        detail::u32x4_t e = column_entry(t, clamped);
-        if (t >= steps * kStripStep) { e.z = kNoWindow; clamped = false; }
-        column[t] = e;
+        if constexpr (LINES) {
+            // (up to a step behind the last one, which the request behind the last step meets)
+            for (int c = t; c < (steps + 1) * kStripStep; c += kStripThreads) {
+                detail::u32x4_t e = column_entry(c, clamped);
+                if (c >= steps * kStripStep) e.z = kNoWindow;
+                column[c] = e;
+            }
+        } else {
+            detail::u32x4_t e = column_entry(t, clamped);
+            if (t >= steps * kStripStep) { e.z = kNoWindow; clamped = false; }
+            column[t] = e;
+        }
         const bool any = __builtin_amdgcn_ballot_w64(clamped) != 0ull;
         if (threadIdx.x == 0) wave_clamped[threadIdx.y] = any ? 1u : 0u;
     }
@@ -1064,6 +1133,8 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     const bool some_clamped = __builtin_amdgcn_readfirstlane(met) != 0u;
 
     const auto oplane = WP::plane_ref(z, wpar);
+    LineStores<Chain, LANES> lines;
+    if constexpr (LINES) lines.open(z, yc, yvalid, g, wpar);
     // the lane's store offset in step 0; a lane without a row carries an offset beyond the resource's extent
     const u32 out0 = yvalid ? WP::row_offset(y, oplane) + WP::lane_offset(g, true) : WP::kMaskedOut;
     const bool partial = (aw & (kStripStep - 1)) != 0;             // the last step has columns beyond the output
@@ -1095,6 +1166,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
             typename Chain::Value res;
             if constexpr (STATIC) res = Chain::compute_static_ops(v, ops);
             else res = Chain::compute_checked_ops(v, ops);
+            if constexpr (LINES) { lines.template put<STREAM>(oplane, k, g, k == 0 || k == steps - 1, aw, res); return; }
             u32 off = out0 + u32(k) * WP::lane_offset(kStripStep, true);
             if (partial && k == steps - 1) {                          // wave uniform, kept a branch
                 asm volatile("" : "+v"(off));
@@ -1123,10 +1195,22 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
         if (kAnyPitch || some_clamped) run(static_tag, IntTag<1>{});
         else run(static_tag, IntTag<0>{});
     };
+    auto finish = [&] { if constexpr (LINES) lines.template finish<STREAM>(oplane, steps, g, aw); };
     if constexpr (Chain::kQuick) {
-        if (Chain::ops_static(ops)) { run_static(IntTag<1>{}); return; }
+        if (Chain::ops_static(ops)) { run_static(IntTag<1>{}); finish(); return; }
     }
     run_static(IntTag<0>{});
+    finish();
+}
+
+// (both kinds of image rows in one kernel: the instruction more per pixel and line is nothing beside the stores)
+template <class Chain, bool STREAM, int LANES>
+__device__ __forceinline__ void strip_lines_body(const typename Chain::Params& p) {
+    strip_body<Chain, STREAM, true, true, LANES, LANES == 32 ? kStripMaxSteps : int(kLinesWidth) / 64>(p, 0u);
+}
+template <class Chain, bool STREAM, int LANES>
+__global__ __launch_bounds__(kStripThreads) void k_strip_lines(const typename Chain::Params p) {
+    if constexpr (strip_capable<Chain>()) strip_lines_body<Chain, STREAM, LANES>(p);
 }
 
 template <class Chain, bool STREAM, bool ANY_PITCH>
@@ -1250,11 +1334,15 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
     else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsLines>(p, 0u, &g);
 }
 // The module's other kernels, 1 to 3 (nothing for chains that have no such kernel).  Rows kernel: the kernel for small outputs, those for
-// planes without gaps; bilinear kernel: gather_form's forms 1 and 2.
+// planes without gaps; bilinear kernel: gather_form's forms 1 and 2, and the strip form with its stores on line boundaries.
 template <class Chain, int WHICH> __device__ __forceinline__ void jit_other_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) {
     } else if constexpr (is_gather_chain<Chain>()) {
         if constexpr (WHICH < 3) gather_body<Chain, WHICH, 1, false>(p, g);
+        else if constexpr (strip_capable<Chain>()) {
+            if ((g.n_tiles & kStreamFlag) != 0u) strip_lines_body<Chain, true, 64>(p);
+            else strip_lines_body<Chain, false, 64>(p);
+        }
     } else if constexpr (WHICH == 1) {
         rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
     } else if constexpr (rows_have_flat<Chain>()) {

@@ -100,6 +100,19 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
     constexpr bool kStreams = writer_streams<Chain>();
     const bool streamed = kStreams && (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(typename Chain::Value) > kStreamOutputBytes;
     if constexpr (strip_capable<Chain>()) {
+        if (p.active_w != 0 && (p.reserved & kLinesBit) != 0u && fklhip::strip_enabled()) {
+            const unsigned lanes = lines_lanes(p.active_w, p.active_h, p.active_z), rows = kStripThreads / lanes;
+            const dim3 grid((p.active_h + rows - 1) / rows, 1, p.active_z), block(kGatherBX, kStripThreads / kGatherBX, 1);
+            if (info) *info = LaunchInfo{(p.reserved & 1u) != 0u ? "strip" : "gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned((lanes == 32u ? 9 * 32 : 11 * 64) * 16 + (kStripThreads / 64) * 4)};
+            if (grid.x == 0 || grid.z == 0) return hipSuccess;
+            if (grid.z > 65535u) return hipErrorInvalidConfiguration;
+            if (lanes == 32u) {
+                if (streamed) return launch_by_pointer(&k_strip_lines<Chain, kStreams, 32>, grid, block, stream, p);
+                return launch_by_pointer(&k_strip_lines<Chain, false, 32>, grid, block, stream, p);
+            }
+            if (streamed) return launch_by_pointer(&k_strip_lines<Chain, kStreams, 64>, grid, block, stream, p);
+            return launch_by_pointer(&k_strip_lines<Chain, false, 64>, grid, block, stream, p);
+        }
         // Narrow outputs (batches of small planes): the strip form, whose workgroups own 8 whole rows of a plane.
         // (an output without columns has no workgroup in the tile form's grid: it falls through and launches nothing)
         if (p.active_w != 0 && p.active_w <= unsigned(kStripMaxWidth) && (p.reserved & 1u) != 0 && fklhip::strip_enabled()) {

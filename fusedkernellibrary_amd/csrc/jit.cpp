@@ -49,7 +49,8 @@ using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
 // A module's kernels.  Rows kernel: the chain's own, the one for small outputs (empty where JitMeta::has_small is 0), and the two for
-// planes without gaps (empty where JitMeta::has_flat is 0).  Bilinear kernel: the chain's own, and those of gather_form's forms 1 and 2.
+// planes without gaps (empty where JitMeta::has_flat is 0).  Bilinear kernel: the chain's own, those of
+// gather_form's forms 1 and 2, and the strip form with its stores on line boundaries.
 constexpr const char* kJitSuffix[4] = {"", "_1", "_2", "_3"};
 using JitFunctions = std::array<hipFunction_t, 4>;
 
@@ -228,7 +229,16 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     unsigned grid[3], block[3] = {64, 4, 1};
     const char* kind = m.gather ? "gather_jit" : "rows_jit";
     unsigned which = 0;                      // of kJitSuffix
-    if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {
+    if (m.gather && m.strip_width != 0 && active[0] != 0 && (active[3] & fkd::kLinesBit) != 0 && strip_enabled()) {
+        // (rows of 64 lanes only)
+        kind = (active[3] & 1u) != 0u ? "strip_jit" : "gather_jit";
+        which = 3;
+        grid[0] = (active[1] + 3u) / 4u;
+        grid[1] = 1;
+        grid[2] = active[2];
+        block[1] = m.by;
+        g.n_tiles = streamed ? kStreamFlag : 0u;
+    } else if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {
         // strip form: one workgroup per m.by * m.yi output rows of a plane; tiles_x == 0 tells the kernel, and n_tiles
         // carries the launch's priority schedule
         kind = "strip_jit";

@@ -111,6 +111,14 @@ inline unsigned gather_form(unsigned w, unsigned h, unsigned planes, unsigned so
     return tiles < kGatherFewTiles ? 1u : tiles < some_tiles ? 2u : 0u;
 }
 
+// Bit 4 of a chain's Params::reserved: a launch of the bilinear kernel whose stores are moved on to line boundaries (lines_pay, LineStores in
+// the kernels' header): workgroups of eight rows of 32 lanes or of four rows of 64.  Wide rows have 64; narrow ones too where the launch would
+// have few workgroups (8 crops to 250x250, 256 of them: 4.5 us with 32 lanes, 3.7 with 64; 64 crops to 193x105, 896: 6.2 / 6.7).
+constexpr unsigned kLinesBit = 16u, kLinesWidth = 640;
+inline constexpr unsigned lines_lanes(unsigned w, unsigned h, unsigned planes) {
+    return w > 256u || (unsigned long long)((h + 7u) / 8u) * planes < 540u ? 64u : 32u;
+}
+
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
     unsigned gather;          // 1: gather kernel geometry, 0: rows kernel geometry

@@ -3135,6 +3135,12 @@ template <class T, bool TRANSPOSED = false> struct TensorSplit {
         r.pitch = p.pitch;
         return r;
     }
+    // The address of a row of the first channel plane, how far the next channel plane's is, and one channel's store (see put_masked).
+    FKD_DEV static const char* channel_row(int z, int y, const Params& p) { return reinterpret_cast<const char*>(p.data) + G::image_bytes(p) * z + size_t(y) * p.pitch; }
+    FKD_DEV static size_t channel_bytes(const Params& p) { return G::channel_elements(p) * sizeof(B); }
+    template <bool STREAM, int C> FKD_DEV static void put_channel(const PlaneRef& r, u32 off, u32 bits) {
+        __builtin_amdgcn_raw_buffer_store_b32(bits, r.rsrc, off, u32(C) * r.chan_bytes, STREAM ? 2 : (1 | 16));
+    }
     FKD_DEV static u32 lane_offset(int x, bool valid) { return valid ? u32(x) * u32(sizeof(B)) : kMaskedOut; }
     FKD_DEV static u32 row_offset(int y, const PlaneRef& r) { return u32(y) * r.pitch; }
     // STREAM: the launch writes more than the last-level cache should give up for it (kStreamOutputBytes).  The stores then
@@ -3443,6 +3449,24 @@ template <class I, class P, class O> struct IsDivOp<Div<I, P, O>> { static const
 //   3.1 / 3.6, to 256x120 3.2 / 3.7; and rows of no whole sectors that nearly fill the tile form's 128 columns are its own from a size
 //   on: 105x193 (1.3 M pixels) 8.1 / 7.6, 105x297 (2.0 M) 9.0 / 10.3, 125x437 12.5 / 15.0 (112x279 8.5 / 7.7, 95x328 9.9 / 9.7, 130x300 13.2 / 11.6).  Launches below 40 000 pixels and rows of no whole sectors keep the tile form that such images
 //   always had; the strip form would serve some of them better (8 crops to 64x39 3.0 / 2.2, 64 crops to 165x64 4.8 / 4.3, to 250x200 12.2 / 13.5).
+// Whether a launch moves its stores on to line boundaries (kLinesBit): planar outputs whose rows are no whole 16 bytes (row_grain, see
+// strip_pays), large enough for the lines they cut to cost more than the lane exchange.  us, as they are (in the better of the two forms) / moved on:
+//  32 lanes to a row: 64 crops to 75x200 (11.5 MB) 6.8 / 6.2, to 99x250 (19) 9.1 / 7.8, to 130x100 (10) 5.5 / 5.0, to 166x90 (11.5) 5.9 / 5.0, to 193x60 (8.9)
+//   4.9 / 4.6, to 217x72 (12) 6.2 / 5.2, to 225x225 (39) 13.4 / 12.5, but to 130x60 (6.0) 3.7 / 4.1, to 150x70 (8.1) 4.3 / 4.4.
+//  64 lanes, narrow rows: 8 crops to 179x273 (4.7 MB) 3.6 / 3.4, to 225x225 (4.9) 4.1 / 3.5, to 179x400 (6.9) 4.3 / 3.9, but to 129x400 (5.0) 3.6 / 3.8.
+//  Wide rows, by workgroups of four rows: 64 crops to 258x40 (640) 4.9 / 4.3, to 290x30 (512) 4.3 / 4.0, to 310x347 (83 MB) 25.9 / 23.3, to 503x209 28.8 / 22.9, to
+//   517x517 63.7 / 50.2, to 639x639 103 / 74.5, 8 crops to 303x307 (616) 4.8 / 4.4, to 509x349 (704) 6.0 / 5.75, but to 467x239 (480) 4.8 / 4.9, to 509x200 (400)
+//   4.7 / 5.0, and rows of nine and ten steps only past the last-level cache (8 crops to 601x600, 35 MB, 9.4 / 10.6, 64 to 601x100, 46 MB, 13.3 / 13.2).
+//  Rows of whole 16 bytes gain where they are wide (64 crops to 300x50 5.5 / 5.0, to 436x40 5.7 / 5.4, to 436x138 12.65 / 12.5; to 68x600 11.95 / 12.2, to
+//   236x64 4.8 / 4.8), whole sectors nowhere (to 200x300 12.65 / 12.8, 8 to 600x601 8.8 / 9.2).
+inline bool lines_pay(u32 w, u32 h, u32 planes, u32 value_bytes, u32 row_grain) {
+    const unsigned long long bytes = (unsigned long long)w * h * planes * value_bytes;
+    if (w == 0u || w > kLinesWidth || row_grain > (w > 256u ? 16u : 8u)) return false;
+    if (w > 512u) return bytes > kStreamOutputBytes;
+    if (w > 256u) return (unsigned long long)((h + 3u) / 4u) * planes >= 500u;
+    if (lines_lanes(w, h, planes) == 32u) return bytes >= 8600000u;
+    return w > 160u && bytes >= 4500000u;
+}
 inline bool strip_pays(u32 w, u32 h, u32 planes, bool any_pitch, u32 value_bytes, u32 row_grain) {
     const unsigned long long pixels = (unsigned long long)w * h * planes, workgroups = (unsigned long long)((h + 7u) / 8u) * planes;
     if (pixels * value_bytes > kStreamOutputBytes) {
@@ -3537,6 +3561,8 @@ template <class R, class... Ops, class W> struct Chain<R, OpList<Ops...>, W> {
             const bool any_pitch = !R::strip_ok(p.read, false, p.active_z);
             if (strip_pays(p.active_w, p.active_h, p.active_z, any_pitch, sizeof(Value), W::row_grain(p.write, p.active_w, p.active_z)) && W::strip_ok(p.write) &&
                 (!any_pitch || R::strip_ok(p.read, true, p.active_z))) p.reserved |= kStripChecked | (any_pitch ? kStripAnyPitch : 0u);
+            if (lines_pay(p.active_w, p.active_h, p.active_z, sizeof(Value), W::row_grain(p.write, p.active_w, p.active_z)) && W::strip_ok(p.write) &&
+                R::strip_ok(p.read, true, p.active_z)) p.reserved |= kLinesBit;
         }
     }
 #endif

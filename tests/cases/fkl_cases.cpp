@@ -659,6 +659,9 @@ int fklcase_tap_window(int elem_bytes, unsigned at, unsigned long long image_byt
 int fklcase_strip_pays(unsigned w, unsigned h, unsigned planes, int any_pitch, unsigned row_grain) {
     return fkd::strip_pays(w, h, planes, any_pitch != 0, sizeof(fkd::Vec<fkd::f32, 3>), row_grain) ? 1 : 0;
 }
+int fklcase_lines_pay(unsigned w, unsigned h, unsigned planes, unsigned row_grain) {
+    return fkd::lines_pay(w, h, planes, sizeof(fkd::Vec<fkd::f32, 3>), row_grain) ? 1 : 0;
+}
 unsigned fklcase_gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) { return fkd::gather_form(w, h, planes, some_tiles); }
 unsigned fklcase_row_grain(unsigned long long address, unsigned w, unsigned h, unsigned planes) {
     Tensor<float> t(reinterpret_cast<float*>(size_t(address)), w, h, planes, 3, MemType::Device, 0);
