@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52062000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "937d2d0004abd7c6f2ce80cbc42c82a762a529231b64b5757e3c5bde76967a60"
+TRAFFIC_C3_SOURCES_SHA256 = "903f05ea0900a84ea5cb3e414193bf51b7180698b3badcfd23e59cd93845a9cf"
 
 
 def device_sources_sha256():

@@ -259,7 +259,7 @@ template <class T> FKD_DEV void store_elem(T* p, const T& v) {
 
 template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_words(const void* p, u32 (&w)[W]) {
     constexpr int ALIGN = ALIGNED ? 4 : 1;
-    static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
+    static_assert(W >= 1 && (W <= 4 || W == 6 || W % 4 == 0), "runs are 1-4 or 6 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
         w[0] = gload<u32, ALIGN, STREAM>(p);
     } else if constexpr (W == 2) {
@@ -268,6 +268,12 @@ template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_wor
     } else if constexpr (W == 3) {
         const u32x3_t v = gload<u32x3_t, ALIGN, STREAM>(p);
         w[0] = v.x; w[1] = v.y; w[2] = v.z;
+    } else if constexpr (W == 6) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const u32x3_t v = gload<u32x3_t, ALIGN, STREAM>(gconst<u32>(p) + 3 * i);
+            w[3 * i] = v.x; w[3 * i + 1] = v.y; w[3 * i + 2] = v.z;
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
@@ -278,7 +284,7 @@ template <int W, bool STREAM = false, bool ALIGNED = true> FKD_DEV void load_wor
 }
 template <int W, bool ALIGNED = true, bool PLAIN = false> FKD_DEV void store_words(void* p, const u32 (&w)[W]) {
     constexpr int ALIGN = ALIGNED ? 4 : 1;
-    static_assert(W >= 1 && (W <= 4 || W % 4 == 0), "runs are 1-4 dwords or whole 16-byte groups");
+    static_assert(W >= 1 && (W <= 4 || W == 6 || W % 4 == 0), "runs are 1-4 or 6 dwords or whole 16-byte groups");
     if constexpr (W == 1) {
         gstore<ALIGN, PLAIN>(p, w[0]);
     } else if constexpr (W == 2) {
@@ -287,6 +293,12 @@ template <int W, bool ALIGNED = true, bool PLAIN = false> FKD_DEV void store_wor
     } else if constexpr (W == 3) {
         u32x3_t v; v.x = w[0]; v.y = w[1]; v.z = w[2];
         gstore<ALIGN, PLAIN>(p, v);
+    } else if constexpr (W == 6) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            u32x3_t v; v.x = w[3 * i]; v.y = w[3 * i + 1]; v.z = w[3 * i + 2];
+            gstore<ALIGN, PLAIN>(gmut<u32>(p) + 3 * i, v);
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < W / 4; ++i) {
@@ -361,10 +373,11 @@ template <class T, int V, int W> FKD_DEV void unpack_words(const u32 (&w)[W], Sl
 // V consecutive elements starting at p move as one wide access per <= 16 bytes (global_load_dwordx3 for four uchar3, dwordx4
 // for four floats), which consecutive lanes make contiguous, at any byte alignment of p: rows of 1279 uchar3 start at every
 // one, and moved byte by byte they were bound by the number of accesses (100 images of 510x333: 40 us byte by byte, 20 us so;
-// 4 of 1279x719: 37.2 and 25.2 us per 4 launches).  Runs that are not a whole number of dwords move element by element.
+// 4 of 1279x719: 37.2 and 25.2 us per 4 launches).  Runs that are not a whole number of dwords move element by element.  The 24 bytes of
+// four ushort3 are two dwordx3 (RGB to P010 3840x2160 sample by sample 17.1, so 13.9 us; 1278x852 4.8 / 4.2).
 template <class T> constexpr bool wide_ok(int v) {
     const int bytes = int(sizeof(T)) * v;
-    return v > 1 && bytes % 4 == 0 && (bytes <= 16 || bytes % 16 == 0) && sizeof(T) == sizeof(base_t<T>) * cn_v<T>;
+    return v > 1 && bytes % 4 == 0 && (bytes <= 16 || bytes == 24 || bytes % 16 == 0) && sizeof(T) == sizeof(base_t<T>) * cn_v<T>;
 }
 // Runs of 32, 48 or 64 bytes per lane (four float2/float3/float4) as wide accesses would leave gaps between the lanes
 // of one instruction: lane i moves 16 bytes at i * 48, and the memory pipeline sees three sparse passes over the
