@@ -344,7 +344,8 @@ __device__ __forceinline__ void flat_run(const Q& q, const WQ& wpar, const OPS& 
         for (int i = 0; i < V; ++i) row[i].v = out[r * V + i].v;
         if constexpr (!EDGE) {
             WP::template exec_row<V, STORE>(x0[r], 0, z, row, wpar);
-        } else if constexpr (has_edge_store<WP, V>()) {
+        } else if constexpr (!PLAIN && has_edge_store<WP, V>()) {
+            // (not in small launches, which are as long as their last wave: UYVY to float3 142x110 1.87 us without, 2.05 with it)
             if (first + r * kSegment < total) WP::template exec_edge<V>(first + r * kSegment, x0[r], total, 0, z, row, wpar);
         } else {
             if (x0[r] == x[r]) {
@@ -1248,6 +1249,12 @@ template <class Chain> struct RowsConfig {
     static constexpr int ROWS = (kScattered || is_scattered_read<typename Chain::Read>()) ? FKD_SCATTER_ROWS : (kManyOps ? FKD_ROWS_MANY : FKD_ROWS);
 };
 
+// Below how many workgroups a launch takes half the rows per thread (see kRowsFewBlocks).
+template <class Chain> constexpr u32 rows_few_blocks() {
+    constexpr int V = RowsConfig<Chain>::V;
+    return detail::wave_exchange_ok<typename Chain::Read::Out>(V) || detail::wave_exchange_ok<typename Chain::Write::In>(V) ? kRowsFewBlocksExchange : kRowsFewBlocks;
+}
+
 // ---- divergent batch kernel -------------------------------------------------------------------------------
 
 // Several chains in one launch of the rows kernel's geometry: plane z runs chain select[z] (wave uniform: the plane is
@@ -1300,14 +1307,14 @@ template <class Chain> constexpr bool rows_have_flat() {
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
                        !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u, rows_have_flat<Chain>() ? 1u : 0u,
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u,
-                       gather_some_tiles<Chain>()};
+                       gather_some_tiles<Chain>(), rows_few_blocks<Chain>()};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) DivergentBody<Chain>::run(p);
@@ -1333,20 +1340,26 @@ template <class Chain> __device__ __forceinline__ void jit_body(const typename C
     }
     else rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsLines>(p, 0u, &g);
 }
-// The module's other kernels, 1 to 3 (nothing for chains that have no such kernel).  Rows kernel: the kernel for small outputs, those for
-// planes without gaps; bilinear kernel: gather_form's forms 1 and 2, and the strip form with its stores on line boundaries.
+// The module's other kernels, 1 to 6 (nothing for chains that have no such kernel).  Bilinear kernel: gather_form's forms 1 and 2, and 3 the
+// strip form with its stores on line boundaries.  Rows kernel: 1 the kernel for small outputs, 2 and 3 those for planes without gaps (3: small
+// outputs), 4 and 5 the chain's own and 2 for launches of few workgroups, with half the rows per thread, as 1 and 3 have, and 6 is 1 for larger ones (rows_few_blocks;
+// compiled at run time, NV12 to float3 240x410 2.3 -> 2.1 us, 2000x1500 8.2 -> 7.6, RGB to P010 1804x218 2.9 -> 2.3).
 template <class Chain, int WHICH> __device__ __forceinline__ void jit_other_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) {
     } else if constexpr (is_gather_chain<Chain>()) {
         if constexpr (WHICH < 3) gather_body<Chain, WHICH, 1, false>(p, g);
-        else if constexpr (strip_capable<Chain>()) {
+        else if constexpr (WHICH == 3 && strip_capable<Chain>()) {
             if ((g.n_tiles & kStreamFlag) != 0u) strip_lines_body<Chain, true, 64>(p);
             else strip_lines_body<Chain, false, 64>(p);
         }
-    } else if constexpr (WHICH == 1) {
-        rows_auto_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
-    } else if constexpr (rows_have_flat<Chain>()) {
-        flat_body<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS, WHICH == 3>(p);
+    } else {
+        constexpr int V = RowsConfig<Chain>::V, ROWS = RowsConfig<Chain>::ROWS, HALF = ROWS > 1 ? ROWS / 2 : ROWS;
+        if constexpr (WHICH == 1) rows_auto_body<Chain, V, HALF, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g);
+        else if constexpr (WHICH == 6) { if constexpr (ROWS > 1) rows_auto_body<Chain, V, ROWS, rows_in_bands<Chain>(), kRowsSmall>(p, 0u, &g); }
+        else if constexpr (WHICH == 4) { if constexpr (ROWS > 1) rows_auto_body<Chain, V, HALF, rows_in_bands<Chain>(), kRowsLines>(p, 0u, &g); }
+        else if constexpr (rows_have_flat<Chain>()) {
+            if constexpr (WHICH != 5 || ROWS > 1) flat_body<Chain, V, WHICH == 2 ? ROWS : HALF, WHICH == 3>(p);
+        }
     }
 }
 

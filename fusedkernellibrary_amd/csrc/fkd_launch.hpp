@@ -19,12 +19,6 @@ inline hipError_t launch_by_pointer(Kernel kernel, dim3 grid, dim3 block, hipStr
 
 inline const char* aligned_name(bool aligned) { return aligned ? "rows" : "rows_unaligned"; }
 
-// Launches with few workgroups (a single 1080p image is 1 080 of them at two rows per thread, about four per compute unit,
-// so some units get five and some four) take half the rows per thread: twice the workgroups spread evenly, which on such
-// launches outweighs the shorter run of independent loads per thread (1080p chains 5 - 9 % faster, 4K chains 3 % slower,
-// hence the limit: below eight workgroups per compute unit of this chip).
-constexpr unsigned kRowsSmallGrid = 2048;
-
 template <class Chain, int V, int ROWS>
 hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info, bool aligned) {
     const unsigned gx = (p.active_w + rows_phase_bound(p.reserved) + kRowsBX * V - 1) / (kRowsBX * V);
@@ -56,16 +50,11 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
     return launch_by_pointer(&k_rows<Chain, V, ROWS, false, kRowsLines>, grid, block, stream, p, g);
 }
 
-// Planes without gaps (kFlatBit): a one-dimensional grid per plane.  Below four workgroups per compute unit a wave takes half the
-// segments.  us with the line at 768 / 1024 / 2048 workgroups: 4 uchar3 images of 1279x719 (1 800) 4.5 / 4.5 / 4.9, 4 of 1209x263 (624; 4
-// launches) 12.4 / 12.4 / 12.4 (at 512: 13.05), 4 of 849x880 (1 460; 4 launches) 16.2 / 16.2 / 17.9, 50 operations on 3840x2160 floats (2 025) 12.6 / 12.6 /
-// 13.6, on 3384x77 (64) 9.2 to 10.6 from run to run.
-constexpr unsigned kFlatFewBlocks = 1024;
 template <class Chain, int V, int ROWS>
 hipError_t launch_flat(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     const unsigned blocks = flat_blocks(p.active_w, p.active_h, p.reserved, ROWS);
     if constexpr (ROWS > 1) {
-        if ((unsigned long long)blocks * p.active_z < kFlatFewBlocks) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
+        if ((unsigned long long)blocks * p.active_z < rows_few_blocks<Chain>()) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
     }
     const dim3 grid(blocks, 1, p.active_z), block(kRowsBX, kRowsBY, 1);
     if (info) *info = LaunchInfo{"rows", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
@@ -88,7 +77,7 @@ hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, Laun
     if constexpr (ROWS > 1) {
         const unsigned long long gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);
         const unsigned long long gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);
-        if (gx * gy * p.active_z < kRowsSmallGrid) return launch_rows_with<Chain, V, ROWS / 2>(p, stream, info, aligned);
+        if (gx * gy * p.active_z < rows_few_blocks<Chain>()) return launch_rows_with<Chain, V, ROWS / 2>(p, stream, info, aligned);
     }
     return launch_rows_with<Chain, V, ROWS>(p, stream, info, aligned);
 }

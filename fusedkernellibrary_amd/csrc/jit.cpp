@@ -48,11 +48,9 @@ using fkd::kStreamOutputBytes;
 using fkd::rows_phase_bound;
 using fkd::strip_first_late_workgroup;
 
-// A module's kernels.  Rows kernel: the chain's own, the one for small outputs (empty where JitMeta::has_small is 0), and the two for
-// planes without gaps (empty where JitMeta::has_flat is 0).  Bilinear kernel: the chain's own, those of
-// gather_form's forms 1 and 2, and the strip form with its stores on line boundaries.
-constexpr const char* kJitSuffix[4] = {"", "_1", "_2", "_3"};
-using JitFunctions = std::array<hipFunction_t, 4>;
+// A module's kernels: the chain's own and those of jit_other_body (empty where the chain has no such kernel).
+constexpr const char* kJitSuffix[7] = {"", "_1", "_2", "_3", "_4", "_5", "_6"};
+using JitFunctions = std::array<hipFunction_t, 7>;
 
 struct JitKernel {
     std::string signature;
@@ -259,8 +257,14 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[2] = active[2];
         block[1] = m.by;
     } else if (m.has_flat != 0u && (active[3] & fkd::kFlatBit) != 0u) {
-        which = (active[3] & fkd::kSmallOutputBit) != 0u ? 3u : 2u;
-        grid[0] = fkd::flat_blocks(active[0], active[1], active[3], m.rows);
+        unsigned rows = m.rows;
+        which = 2;
+        grid[0] = fkd::flat_blocks(active[0], active[1], active[3], rows);
+        const bool few = rows > 1u && (unsigned long long)grid[0] * active[2] < m.few_blocks;
+        if ((active[3] & fkd::kSmallOutputBit) != 0u || few) {
+            which = (active[3] & fkd::kSmallOutputBit) != 0u ? 3u : 5u;
+            if (rows > 1u) grid[0] = fkd::flat_blocks(active[0], active[1], active[3], rows / 2u);
+        }
         grid[1] = 1;
         grid[2] = active[2];
     } else {
@@ -268,6 +272,12 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
         grid[0] = (active[0] + (m.max_planes != 0 ? 0u : rows_phase_bound(active[3])) + 64 * m.v - 1) / (64 * m.v);
         grid[1] = (active[1] + 4 * m.rows - 1) / (4 * m.rows);
         grid[2] = active[2];
+        if (m.max_planes == 0u && m.rows > 1u) {
+            const bool few = (unsigned long long)((active[0] + 64 * m.v - 1) / (64 * m.v)) * grid[1] * grid[2] < m.few_blocks;
+            if (which == 0u && few) which = 4u;
+            if (which == 1u && !few) which = 6u;
+            if (few) grid[1] = (active[1] + 2 * m.rows - 1) / (2 * m.rows);
+        }
         if (m.bands && (unsigned long long)grid[0] * grid[1] >= kRowsBandBlocks) {
             // as launch_rows_with: one-dimensional, eight equal runs of the plane's blocks
             if ((unsigned long long)grid[0] * grid[1] > 0x7fffff00ull) return int(hipErrorInvalidConfiguration);
@@ -325,7 +335,7 @@ static int build_and_register(const char* signature, bool may_read_cache, bool a
         src += "(const JitChain::Params p, const TileGeom g) {\n"
                "    jit_body<JitChain>(p, g);\n"
                "}\n";
-        for (int i = 1; i < 4; ++i)
+        for (int i = 1; i < 7; ++i)
             src += "extern \"C\" __global__ __launch_bounds__(256) void " + kernel_symbol(k->signature) + kJitSuffix[i] +
                    "(const JitChain::Params p, const TileGeom g) {\n"
                    "    jit_other_body<JitChain, " + std::to_string(i) + ">(p, g);\n"

@@ -98,6 +98,15 @@ inline unsigned flat_blocks(unsigned w, unsigned h, unsigned reserved, unsigned 
     return unsigned(((unsigned long long)w * h + rows_phase_bound(reserved) + per_block - 1u) / per_block);
 }
 
+// Launches of the rows kernel with few workgroups (a single 1080p image is 1 080 of them at two rows per thread, about four per compute unit,
+// so some units get five and some four) take half the rows, or segments, per thread: twice the workgroups spread evenly, which on such
+// launches outweighs the shorter run of independent loads per thread.  The line, in workgroups (rows_few_blocks in the kernels' header): chains
+// whose runs go through the LDS 2048, others 1024.  us with the line at 1024 / 2048: NV12 to float3 2000x1500 (1 504) 8.1 / 7.6, 2200x1200
+// (1 350) 7.9 / 7.2, 1922x1082 (1 088) 6.7 / 6.4; RGB to NV12 1920x1080 (1 080) 3.4 / 3.6, 2560x1440 (1 800) 4.1 / 4.6; RGB to P010 1920x1080 4.6 / 4.9,
+// 2000x1500 6.2 / 6.7.  Planes without gaps, with the line at 768 / 1024 / 2048: 4 uchar3 images of 1279x719 (1 800) 4.5 / 4.5 / 4.9, 4 of
+// 849x880 (1 460; 4 launches) 16.2 / 16.2 / 17.9, 50 operations on 3840x2160 floats (2 025) 12.6 / 12.6 / 13.6; at 512: 4 of 1209x263 (624) 12.4 -> 13.05.
+constexpr unsigned kRowsFewBlocks = 1024, kRowsFewBlocksExchange = 2048;
+
 // Which tiles a launch of the bilinear kernel's tile form takes: 128x8 pixels, or smaller ones where it would have few of those (per-wave
 // latency, see the kernels' header).  us, tiles of 128x8 / 128x4 / 64x4 pixels (in brackets: how many of 128x8): NV12 to 148x85 (22)
 // 3.23 / 2.41 / 2.09, to 320x180 (69) 2.58 / 2.05 / 1.94, to 400x300 (152) 3.23 / 2.61 / 2.69, to 1100x700 (792) 5.32 / 4.71 / 5.38, to 1333x800 (1100)
@@ -132,6 +141,7 @@ struct JitMeta {
     unsigned has_flat;        // rows kernel: 1 when the module has kernels for planes taken as one row (kFlatBit)
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
     unsigned some_tiles;      // gather kernel: the last argument of gather_form
+    unsigned few_blocks;      // rows kernel: rows_few_blocks
 };
 
 } // namespace fkd
