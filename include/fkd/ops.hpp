@@ -1634,6 +1634,10 @@ template <class T> struct Read2D {
     }
     FKD_HD static bool dense(const Params& p, u32 w, u32) { return p.pitch == size_t(w) * sizeof(T); }
     FKD_HD static void advance(Params& p, ptrdiff_t n) { p.data += n; }
+    // Byte offset of row y from the image the taps are fetched from, and what one row more adds to it.  A rectangle's row 0 is not at
+    // offset 0.
+    FKD_HD static u32 tap_row_offset(int y, const Params& p) { return u32(y) * p.pitch; }
+    FKD_HD static u32 tap_pitch(const Params& p) { return p.pitch; }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
     FKD_DEV static int height(const Params& p) { return int(p.height); }
@@ -1698,7 +1702,6 @@ template <class T> struct Read2D {
     FKD_DEV static TapImage tap_image_bounded(int, const Params& p) {
         return detail::make_tap_image(p.data, size_t(p.pitch) * (p.height - 1) + size_t(p.width) * sizeof(T));
     }
-    FKD_DEV static u32 tap_row_offset(int y, const Params& p) { return u32(y) * p.pitch; }
     FKD_DEV static PairPrep pair_prepare(const TapImage& im, int x, const Params&) {
         return detail::prepare_pair_window<T>(im, u32(x) * u32(sizeof(T)));
     }
@@ -2129,6 +2132,12 @@ template <class Back> struct Crop {
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
         if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return p.w >= 2 && p.h >= 1 && Back::strip_ok(p.back, any_pitch); else return false;
     }
+    FKD_HD static u32 tap_row_offset(int y, const Params& p) {
+        if constexpr (requires { Back::tap_pitch(p.back); }) return Back::tap_row_offset(y + p.y, p.back); else return 0u;
+    }
+    FKD_HD static u32 tap_pitch(const Params& p) {
+        if constexpr (requires { Back::tap_pitch(p.back); }) return Back::tap_pitch(p.back); else return 0u;
+    }
 #if defined(FKD_EXEC_CODE)
     static constexpr bool kFiniteTaps = finite_taps<Back>();
     FKD_DEV static int width(const Params& p) { return p.w; }
@@ -2173,9 +2182,6 @@ template <class Back> struct Crop {
     }
     FKD_DEV static TapImage tap_image_bounded(int z, const Params& p) {
         if constexpr (kTapPrepared) return Back::tap_image_bounded(z, p.back); else return TapImage{};
-    }
-    FKD_DEV static u32 tap_row_offset(int y, const Params& p) {
-        if constexpr (kTapPrepared) return Back::tap_row_offset(y + p.y, p.back); else return 0u;
     }
     FKD_DEV static PairPrep pair_prepare(const TapImage& im, int x, const Params& p) {
         if constexpr (kTapPrepared) return Back::pair_prepare(im, x + p.x, p.back); else return PairPrep{};
@@ -2318,6 +2324,12 @@ template <class Back, class... Ops> struct FusedRead {
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch) {
         if constexpr (requires { Back::strip_ok(p.back, any_pitch); }) return Back::strip_ok(p.back, any_pitch); else return false;
     }
+    FKD_HD static u32 tap_row_offset(int y, const Params& p) {
+        if constexpr (requires { Back::tap_pitch(p.back); }) return Back::tap_row_offset(y, p.back); else return 0u;
+    }
+    FKD_HD static u32 tap_pitch(const Params& p) {
+        if constexpr (requires { Back::tap_pitch(p.back); }) return Back::tap_pitch(p.back); else return 0u;
+    }
 #if defined(FKD_EXEC_CODE)
     static constexpr bool kFiniteTaps = finite_taps<Back>() && (finite_map<Ops>() && ...);
     FKD_DEV static int width(const Params& p) { return Back::width(p.back); }
@@ -2367,9 +2379,6 @@ template <class Back, class... Ops> struct FusedRead {
     }
     FKD_DEV static TapImage tap_image_bounded(int z, const Params& p) {
         if constexpr (kTapPrepared) return Back::tap_image_bounded(z, p.back); else return TapImage{};
-    }
-    FKD_DEV static u32 tap_row_offset(int y, const Params& p) {
-        if constexpr (kTapPrepared) return Back::tap_row_offset(y, p.back); else return 0u;
     }
     FKD_DEV static PairPrep pair_prepare(const TapImage& im, int x, const Params& p) {
         if constexpr (kTapPrepared) return Back::pair_prepare(im, x, p.back); else return PairPrep{};
@@ -2574,6 +2583,9 @@ template <int WT, class Back> struct Warp {
         if constexpr (requires { Back::kTapPair; }) return Back::kTapCursor && Back::kTapPair; else return false;
     }();
     FKD_NAME("Warp<" + istr(WT) + "," + Back::name() + ">")
+    // Rows of a source whose offsets a 24-bit multiplication serves, and the offset of row y of such a source.
+    FKD_HD static bool rows_fit(int sh, const Params& p) { return u32(sh) < (1u << 24) && Back::tap_pitch(p.back) < (1u << 24); }
+    FKD_HD static u32 tap_row(u32 y, const Params& p) { return Back::tap_row_offset(0, p.back) + (y & 0xffffffu) * (Back::tap_pitch(p.back) & 0xffffffu); }
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return p.dst_w; }
     FKD_DEV static int height(const Params& p) { return p.dst_h; }
@@ -2593,9 +2605,7 @@ template <int WT, class Back> struct Warp {
     // Whether the bounded form serves this image (wave uniform): at least two columns, every byte offset within 32 bits, and rows
     // and pitch within 24 bits, so that an offset costs one multiplication that does not widen (the compiler's own choice is a
     // 64-bit multiply-add, four times as long).
-    FKD_DEV static bool bounded_ok(int sw, int sh, const Params& p) {
-        return sw >= 2 && Back::tap_offsets_fit(p.back) && u32(sh) < (1u << 24) && Back::tap_row_offset(1, p.back) < (1u << 24);
-    }
+    FKD_DEV static bool bounded_ok(int sw, int sh, const Params& p) { return sw >= 2 && Back::tap_offsets_fit(p.back) && rows_fit(sh, p); }
     // 0 <= s < limit for a limit above zero, as one comparison of the bit patterns: those of negative numbers and of NaNs are above
     // every finite positive one's, and -0, which is inside, becomes +0 first.
     FKD_DEV static bool within(f32 s, f32 limit) { return __builtin_bit_cast(u32, s + 0.0f) < __builtin_bit_cast(u32, limit); }
@@ -2606,14 +2616,13 @@ template <int WT, class Back> struct Warp {
         t.cx = t.inside ? sx : 0.f; t.cy = t.inside ? sy : 0.f;
         t.fx1 = __builtin_floorf(t.cx); t.fy1 = __builtin_floorf(t.cy);
         const int x1 = int(t.fx1);
-        const u32 y1 = u32(int(t.fy1)) & 0xffffffu;
+        const u32 y1 = u32(int(t.fy1));
         t.edge = !INTERIOR && x1 >= sw - 1;           // x1 + 1 is past the line: both taps are the last pixel
         t.xp = t.edge ? sw - 2 : x1;
         using Window = typename detail::pair_bits_of<Back>::type;
         const detail::PairPrep col = Back::pair_prepare(image, t.xp, p.back);
-        const u32 pitch = Back::tap_row_offset(1, p.back) & 0xffffffu;
-        const u32 ta = col.off + col.shift + y1 * pitch;          // from the resource's base
-        const u32 tb = ta + (INTERIOR || int(y1) < sh - 1 ? pitch : 0u);
+        const u32 ta = col.off + col.shift + tap_row(y1, p);      // from the resource's base
+        const u32 tb = ta + (INTERIOR || int(y1) < sh - 1 ? Back::tap_pitch(p.back) & 0xffffffu : 0u);
         t.wa = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(ta), p.back);
         t.wb = Back::pair_load_prepared(image, 0u, detail::pair_window_at<Window>(tb), p.back);
         return t;

@@ -569,6 +569,55 @@ int fklcase_warp_batch_u8x3(void* stream_, const uint8_t* const* srcs, int w, in
     });
 }
 
+// A rectangle of an image -> warp -> float image.  kind: 0 uchar3 (the affine one compiled ahead of time), 1 float, 2 ushort3, and uchar3
+// multiplied per channel by `mul` behind (3) or ahead of (4) the crop.
+extern "C++" template <WarpType WT> WarpingParameters<WT> warp_params(const float* m, int dw, int dh) {
+    WarpingParameters<WT> params{};
+    constexpr int rows = WT == WarpType::Affine ? 2 : 3;
+    for (int r = 0; r < rows; ++r)
+        for (int c = 0; c < 3; ++c) params.transformMatrix.data[r][c] = m[r * 3 + c];
+    params.dstSize = Size(dw, dh);
+    return params;
+}
+extern "C++" template <WarpType WT> void warp_crop(void* stream_, int kind, const void* src, int w, int h, int pitch, const int32_t* rect, const float* mul, const float* m,
+                                                   int dw, int dh, void* out, int out_pitch) {
+    Stream stream(stream_);
+    const Rect crop(rect[0], rect[1], rect[2], rect[3]);
+    const auto warp = Warping<WT>::build(warp_params<WT>(m, dw, dh));
+    const auto scale = [&] { return Mul<uchar3, float3, float3>::build(make_<float3>(mul[0], mul[1], mul[2])); };
+    auto go = [&](const auto& read, auto out_tag) {
+        using O = decltype(out_tag);
+        executeOperations<TransformDPP<>>(stream, read.then(warp), PerThreadWrite<ND::_2D, O>::build(dev2d<O>(out, dw, dh, out_pitch).ptr()));
+    };
+    switch (kind) {
+    case 0: go(PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(src, w, h, pitch).ptr()).then(Crop<>::build(crop)), float3{}); break;
+    case 1: go(PerThreadRead<ND::_2D, float>::build(dev2d<float>(src, w, h, pitch).ptr()).then(Crop<>::build(crop)), float{}); break;
+    case 2: go(PerThreadRead<ND::_2D, ushort3>::build(dev2d<ushort3>(src, w, h, pitch).ptr()).then(Crop<>::build(crop)), float3{}); break;
+    case 3: go(PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(src, w, h, pitch).ptr()).then(Crop<>::build(crop)).then(scale()), float3{}); break;
+    case 4: go(PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(src, w, h, pitch).ptr()).then(scale()).then(Crop<>::build(crop)), float3{}); break;
+    default: throw std::runtime_error("fklcase_warp_crop: kind must be 0 to 4");
+    }
+}
+int fklcase_warp_crop(void* stream, int kind, const void* src, int w, int h, int pitch, const int32_t* rect, const float* mul, const float* m, int perspective,
+                      int dw, int dh, void* out, int out_pitch) {
+    return guarded([&] {
+        if (perspective) warp_crop<WarpType::Perspective>(stream, kind, src, w, h, pitch, rect, mul, m, dw, dh, out, out_pitch);
+        else warp_crop<WarpType::Affine>(stream, kind, src, w, h, pitch, rect, mul, m, dw, dh, out, out_pitch);
+    });
+}
+// Three rectangles of one image, one matrix, into a tensor.
+int fklcase_warp_crops_u8x3(void* stream_, const uint8_t* src, int w, int h, int pitch, const int32_t* rects, const float* m, int dw, int dh, float* out) {
+    return guarded([&] {
+        Stream stream(stream_);
+        Tensor<float3> o(reinterpret_cast<float3*>(out), uint(dw), uint(dh), 3, 1, MemType::Device, 0);
+        const auto warp = Warping<WarpType::Affine>::build(warp_params<WarpType::Affine>(m, dw, dh));
+        auto plane = [&](const Rect& r) { return PerThreadRead<ND::_2D, uchar3>::build(dev2d<uchar3>(src, w, h, pitch).ptr()).then(Crop<>::build(r)).then(warp); };
+        const auto crops = rects_from<3>(rects);
+        const std::array<decltype(plane(crops[0])), 3> planes{plane(crops[0]), plane(crops[1]), plane(crops[2])};
+        executeOperations<TransformDPP<>>(stream, BatchRead<PlanePolicy::PROCESS_ALL>::build(planes), TensorWrite<float3>::build(o.ptr()));
+    });
+}
+
 // Other pixel types (compiled on first use): kind 2 uchar4 -> float4, 3 ushort3 -> float3, 4 uchar -> float.
 int fklcase_warp_kind(void* stream, int kind, const void* src, int w, int h, int pitch, const float* m, int perspective, int dw, int dh,
                       float* out, int out_pitch) {
@@ -651,6 +700,31 @@ int fklcase_tap_window(int elem_bytes, unsigned at, unsigned long long image_byt
     case 4: return fill(fkd::Vec<fkd::u8, 4>{});
     case 6: return fill(fkd::Vec<fkd::u16, 3>{});
     case 8: return fill(fkd::Vec<fkd::f32, 2>{});
+    default: return 2;
+    }
+}
+// Where a warp looks for row y of a rectangle that begins at row `top` of an image of that pitch (out[0]), where the image has that row (out[1]), and
+// whether the warp goes by them (out[2]).  kind: 0 the rectangle alone, 1 and 2 with an operation behind and ahead of it, 3 a rectangle of a
+// rectangle that begins at row 5, 4 the image itself.
+int fklcase_warp_tap_row(int kind, unsigned pitch, int top, int height, int y, unsigned* out) {
+    using Px = fkd::Vec<fkd::u8, 3>;
+    using F3 = fkd::Vec<fkd::f32, 3>;
+    using Image = fkd::Read2D<Px>;
+    using Scale = fkd::Mul<Px, F3, F3>;
+    auto image = [&](Image::Params& p) { p.width = pitch / 3u; p.height = unsigned(top + height); p.pitch = pitch; };
+    auto fill = [&](const auto& p, auto warp_tag, int row) {
+        using Warp = typename decltype(warp_tag)::type;
+        out[0] = Warp::tap_row(unsigned(y), p);
+        out[1] = unsigned(row) * pitch;
+        out[2] = Warp::rows_fit(height, p) ? 1u : 0u;
+        return 0;
+    };
+    switch (kind) {
+    case 0: { using W = fkd::Warp<0, fkd::Crop<Image>>; W::Params p{}; p.back.y = top; image(p.back.back); return fill(p, std::type_identity<W>{}, y + top); }
+    case 1: { using W = fkd::Warp<0, fkd::FusedRead<fkd::Crop<Image>, Scale>>; W::Params p{}; p.back.back.y = top; image(p.back.back.back); return fill(p, std::type_identity<W>{}, y + top); }
+    case 2: { using W = fkd::Warp<0, fkd::Crop<fkd::FusedRead<Image, Scale>>>; W::Params p{}; p.back.y = top; image(p.back.back.back); return fill(p, std::type_identity<W>{}, y + top); }
+    case 3: { using W = fkd::Warp<1, fkd::Crop<fkd::Crop<Image>>>; W::Params p{}; p.back.y = top; p.back.back.y = 5; image(p.back.back.back); return fill(p, std::type_identity<W>{}, y + top + 5); }
+    case 4: { using W = fkd::Warp<1, Image>; W::Params p{}; image(p.back); return fill(p, std::type_identity<W>{}, y); }
     default: return 2;
     }
 }

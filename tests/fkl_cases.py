@@ -282,6 +282,23 @@ def warp_batch(srcs, matrices, dst, out):
                                         int(dst[0]), int(dst[1]), _p(out)))
 
 
+def warp_crop(kind, src, rect, mul, matrix, perspective, dst, out):
+    """Rectangle of an (H,W[,cn]) cuda image -> warp -> (dh,dw[,cn]) f32 cuda; see fklcase_warp_crop for the kinds."""
+    m = np.zeros(9, np.float32)
+    m[: (9 if perspective else 6)] = np.asarray(matrix, np.float32).ravel()
+    r, f = _host(rect, np.int32), _host(mul, np.float32)
+    _ok(cases().fklcase_warp_crop(_stream(), int(kind), _p(src), src.shape[1], src.shape[0], src.stride(0) * src.element_size(), r.ctypes.data_as(C.c_void_p),
+                                  f.ctypes.data_as(C.c_void_p), m.ctypes.data_as(C.c_void_p), int(bool(perspective)), int(dst[0]), int(dst[1]), _p(out),
+                                  out.stride(0) * 4))
+
+
+def warp_crops(src, rects, matrix, dst, out):
+    """Three rectangles of an (H,W,3) u8 cuda image; matrix 2x3; out (3,dh,dw,3) f32 cuda."""
+    r, m = _host(rects, np.int32), _host(matrix, np.float32)
+    _ok(cases().fklcase_warp_crops_u8x3(_stream(), _p(src), src.shape[1], src.shape[0], src.stride(0), r.ctypes.data_as(C.c_void_p),
+                                        m.ctypes.data_as(C.c_void_p), int(dst[0]), int(dst[1]), _p(out)))
+
+
 def deinterlace(src, mode, out):
     """src (H,W,3) u8 or (H,W) f32 cuda; mode 1 BLEND, 2 INTER_LINEAR keeping even lines, 3 keeping odd; out f32 same shape."""
     is_u8 = src.element_size() == 1

@@ -343,11 +343,11 @@ def oracle_batch_default_cast_mul(srcs, active, default, mul):
     return out
 
 
-def oracle_warp(src, cn, matrix, dst, perspective):
-    """Warping<Affine|Perspective> of an (H,W[,cn]) u8/f32 image into a (dh,dw[,cn]) float image."""
+def oracle_warp(src, cn, matrix, dst, perspective, crop=None, tap_ops=None):
+    """Warping<Affine|Perspective> of an (H,W[,cn]) image, or a rectangle of it, into a (dh,dw[,cn]) float image."""
     dw, dh = dst
     out = np.zeros((dh, dw, cn) if cn > 1 else (dh, dw), np.float32)
-    r = read_2d(src, cn)
+    r = read_2d(src, cn, crop=crop, tap_ops=tap_ops)
     r.warp = 2 if perspective else 1
     r.dst_w, r.dst_h = dw, dh
     m = np.zeros(9, np.float32)

@@ -90,3 +90,16 @@ def test_columns_without_a_window_touch_no_image():
     for elem, row, lo in itertools.product((1, 2, 3, 4, 6, 8), (0, 1, 2, 3, 4097, largest), range(4)):
         assert cases.cases().fklcase_tap_window(elem, 0x80000000 + row, largest, lo, out) == 0
         assert out[0] >= 0x80000000 > out[3] and out[0] + out[2] <= 0xffffffff
+
+
+@pytest.mark.parametrize("kind", range(5))
+def test_warps_look_for_a_rectangles_rows_where_the_image_has_them(kind):
+    """A warp's row offset is the first row's plus whole pitches (fkd::Warp::tap_row): rectangles at and off the image's top, with operations on
+    either side, for pitches up to the 24 bits the multiplication takes."""
+    out = (C.c_uint * 3)()
+    for pitch, top, height in itertools.product((6, 1920, 5763, 0xfffffd), (0, 1, 20, 77), (1, 2, 100)):
+        for y in (0, 1, height // 2, height - 1):
+            assert cases.cases().fklcase_warp_tap_row(kind, pitch, top, height, y, out) == 0
+            assert out[2] == 1 and out[0] == out[1] % (1 << 32), (pitch, top, y)
+    assert cases.cases().fklcase_warp_tap_row(kind, 1 << 24, 1, 10, 0, out) == 0 and out[2] == 0
+    assert cases.cases().fklcase_warp_tap_row(kind, 6, 1, 1 << 24, 0, out) == 0 and out[2] == 0
