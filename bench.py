@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52064000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "31817d8f1970b4380b277d7d12016b1f48a48e9561ef97a4341fed9229c86ee2"
+TRAFFIC_C3_SOURCES_SHA256 = "efcc07341b70ef483384aa2d3495cc91373a70fc5de421308923357761602bc3"
 
 
 def device_sources_sha256():

@@ -911,7 +911,7 @@ __device__ __forceinline__ void gather_body(const typename Chain::Params& p, con
 // The launcher decides and hands the kernel one number: the number of the first workgroup that counts as started late, or
 // 0 for a launch whose waves keep the default priority.
 // (strip_first_late_workgroup, fkd/launch_info.hpp)
-constexpr int kStripRows = 8, kStripStep = 32, kStripMaxWidth = 256;
+constexpr int kStripRows = int(kStripFormRows), kStripStep = 32, kStripMaxWidth = 256;
 constexpr int kStripThreads = kStripRows * kStripStep, kStripMaxSteps = kStripMaxWidth / kStripStep;
 static_assert(kStripThreads == kGatherBX * kGatherBY, "the two forms of the bilinear kernel share their workgroup shape");
 static_assert(kStripThreads == kStripMaxWidth, "one table column per thread");

@@ -85,7 +85,6 @@ hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, Laun
 template <class Chain>
 hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     constexpr int XI = FKD_GATHER_XI, YI = FKD_GATHER_YI;
-    static_assert(kGatherBX * XI == int(kGatherTileW[0]) && kGatherBY * YI == int(kGatherTileH[0]), "gather_form speaks of these tiles");
     constexpr bool kStreams = writer_streams<Chain>();
     const bool streamed = kStreams && (unsigned long long)p.active_w * p.active_h * p.active_z * sizeof(typename Chain::Value) > kStreamOutputBytes;
     if constexpr (strip_capable<Chain>()) {
@@ -119,7 +118,7 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
         }
     }
     const unsigned form = gather_form(p.active_w, p.active_h, p.active_z, gather_some_tiles<Chain>());
-    const unsigned TW = kGatherTileW[form], TH = kGatherTileH[form];
+    const unsigned TW = kGatherBX * gather_form_xi(form, XI), TH = kGatherBY * gather_form_yi(form, YI);
     TileGeom g;
     g.tiles_x = (p.active_w + TW - 1) / TW;
     g.tiles_y = (p.active_h + TH - 1) / TH;

@@ -39,14 +39,6 @@ namespace {
 // The launch geometry and the description of a compiled kernel are the kernels' own (fkd/launch_info.hpp).
 using fkd::JitMeta;
 using fkd::TileGeom;
-using fkd::division_magic;
-using fkd::kRowsBandBlocks;
-using fkd::gather_form;
-using fkd::kAnyPitchFlag;
-using fkd::kStreamFlag;
-using fkd::kStreamOutputBytes;
-using fkd::rows_phase_bound;
-using fkd::strip_first_late_workgroup;
 
 // A module's kernels: the chain's own and those of jit_other_body (empty where the chain has no such kernel).
 constexpr const char* kJitSuffix[7] = {"", "_1", "_2", "_3", "_4", "_5", "_6"};
@@ -222,90 +214,22 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     unsigned active[4];
     memcpy(active, blob, sizeof(active));   // Chain::Params starts with active_w, active_h, active_z, reserved (bit 0: strip form allowed, bit 1: for rows at any pitch)
     const JitMeta& m = k->meta;
-    TileGeom g{0, 0, 0, 0};
-    const bool streamed = m.gather && (unsigned long long)active[0] * active[1] * active[2] * m.stream_bytes > kStreamOutputBytes;
-    unsigned grid[3], block[3] = {64, 4, 1};
-    const char* kind = m.gather ? "gather_jit" : "rows_jit";
-    unsigned which = 0;                      // of kJitSuffix
-    if (m.gather && m.strip_width != 0 && active[0] != 0 && (active[3] & fkd::kLinesBit) != 0 && strip_enabled()) {
-        // (rows of 64 lanes only)
-        kind = (active[3] & 1u) != 0u ? "strip_jit" : "gather_jit";
-        which = 3;
-        grid[0] = (active[1] + 3u) / 4u;
-        grid[1] = 1;
-        grid[2] = active[2];
-        block[1] = m.by;
-        g.n_tiles = streamed ? kStreamFlag : 0u;
-    } else if (m.gather && m.strip_width != 0 && active[0] != 0 && active[0] <= m.strip_width && (active[3] & 1u) != 0 && strip_enabled()) {
-        // strip form: one workgroup per m.by * m.yi output rows of a plane; tiles_x == 0 tells the kernel, and n_tiles
-        // carries the launch's priority schedule
-        kind = "strip_jit";
-        grid[0] = (active[1] + m.by * m.yi - 1) / (m.by * m.yi);
-        grid[1] = 1;
-        grid[2] = active[2];
-        block[1] = m.by;
-        g.n_tiles = strip_first_late_workgroup((unsigned long long)grid[0] * grid[2]) | (streamed ? kStreamFlag : 0u) | ((active[3] & 2u) != 0 ? kAnyPitchFlag : 0u);
-    } else if (m.gather) {
-        which = gather_form(active[0], active[1], active[2], m.some_tiles);
-        const unsigned tw = fkd::kGatherTileW[which], th = fkd::kGatherTileH[which];
-        g.tiles_x = (active[0] + tw - 1) / tw;
-        g.tiles_y = (active[1] + th - 1) / th;
-        g.n_tiles = streamed ? kStreamFlag : 0u;       // (the kernel counts its tiles itself)
-        g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
-        grid[0] = (g.tiles_x * g.tiles_y + 7u) / 8u * 8u;
-        grid[1] = 1;
-        grid[2] = active[2];
-        block[1] = m.by;
-    } else if (m.has_flat != 0u && (active[3] & fkd::kFlatBit) != 0u) {
-        unsigned rows = m.rows;
-        which = 2;
-        grid[0] = fkd::flat_blocks(active[0], active[1], active[3], rows);
-        const bool few = rows > 1u && (unsigned long long)grid[0] * active[2] < m.few_blocks;
-        if ((active[3] & fkd::kSmallOutputBit) != 0u || few) {
-            which = (active[3] & fkd::kSmallOutputBit) != 0u ? 3u : 5u;
-            if (rows > 1u) grid[0] = fkd::flat_blocks(active[0], active[1], active[3], rows / 2u);
-        }
-        grid[1] = 1;
-        grid[2] = active[2];
-    } else {
-        if (m.has_small != 0u && fkd::rows_small(active[0], m.v, active[3])) which = 1u;
-        grid[0] = (active[0] + (m.max_planes != 0 ? 0u : rows_phase_bound(active[3])) + 64 * m.v - 1) / (64 * m.v);
-        grid[1] = (active[1] + 4 * m.rows - 1) / (4 * m.rows);
-        grid[2] = active[2];
-        if (m.max_planes == 0u && m.rows > 1u) {
-            const bool few = (unsigned long long)((active[0] + 64 * m.v - 1) / (64 * m.v)) * grid[1] * grid[2] < m.few_blocks;
-            if (which == 0u && few) which = 4u;
-            if (which == 1u && !few) which = 6u;
-            if (few) grid[1] = (active[1] + 2 * m.rows - 1) / (2 * m.rows);
-        }
-        if (m.bands && (unsigned long long)grid[0] * grid[1] >= kRowsBandBlocks) {
-            // as launch_rows_with: one-dimensional, eight equal runs of the plane's blocks
-            if ((unsigned long long)grid[0] * grid[1] > 0x7fffff00ull) return int(hipErrorInvalidConfiguration);
-            g.tiles_x = grid[0];
-            g.tiles_y = grid[1];
-            g.n_tiles = grid[0] * grid[1] * grid[2];
-            g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
-            grid[0] = (grid[0] * grid[1] + 7u) / 8u * 8u;
-            grid[1] = 1;
-        } else if (m.bands > 1u && fkd::rows_bands_2d(grid[0], grid[1])) {
-            g.tiles_x = grid[0];
-            g.tiles_y = grid[1];
-            g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
-        }
-    }
-    if (info) *info = fkd::LaunchInfo{kind, {grid[0], grid[1], grid[2]}, {block[0], block[1], 1}, 0};
+    const fkd::JitGeometry l = fkd::jit_geometry(m, active, strip_enabled());
+    if (l.grid_x > 0x7fffff00ull) return int(hipErrorInvalidConfiguration);
+    const unsigned grid[3] = {unsigned(l.grid_x), l.grid_y, active[2]}, block[3] = {64, l.block_y, 1};
+    if (info) *info = fkd::LaunchInfo{l.kernel, {grid[0], grid[1], grid[2]}, {block[0], block[1], 1}, 0};
     if (grid[0] == 0 || grid[1] == 0 || grid[2] == 0) return FKLHIP_OK;
     if (grid[1] > 65535u || grid[2] > 65535u) return int(hipErrorInvalidConfiguration);
     if (m.max_planes != 0 && grid[2] > m.max_planes) return int(hipErrorInvalidConfiguration);   // as launch_divergent
     hipFunction_t fn = nullptr;
-    const int rc = get_function(k, which, &fn);
+    const int rc = get_function(k, l.which, &fn);
     if (rc != FKLHIP_OK) return rc;
     // Kernel-argument segment: the parameter block, then the TileGeom at the next 4-byte boundary.  The runtime
     // copies the buffer during the call, so the caller's block may go away as soon as we return.
     const size_t geom_at = (bytes + 3) & ~size_t(3);
     std::vector<char> args(geom_at + sizeof(TileGeom));
     memcpy(args.data(), blob, bytes);
-    memcpy(args.data() + geom_at, &g, sizeof(g));
+    memcpy(args.data() + geom_at, &l.g, sizeof(l.g));
     size_t arg_bytes = args.size();
     void* config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &arg_bytes, HIP_LAUNCH_PARAM_END};
     return int(hipModuleLaunchKernel(fn, grid[0], grid[1], grid[2], block[0], block[1], block[2], 0,

@@ -114,7 +114,9 @@ constexpr unsigned kRowsFewBlocks = 1024, kRowsFewBlocksExchange = 2048;
 // to 64x64 (64) 2.96 / 2.38 / 2.16, to 224x64 (128) 3.09 / 2.42 / 2.63, to 224x224 (448) 3.73 / 3.46 / 3.99, to 300x200 (600) 4.07 / 3.89 / 4.34, to 384x300 (912)
 // 4.60 / 4.42, to 320x320 (960) 4.56 / 4.77 / 5.59, 64 crops to 300x64 (1536) 5.9 / 6.3 / 8.0.  Reads that work on every tap (a colour conversion) are longer and cross later.
 constexpr unsigned kGatherFewTiles = 128, kGatherSomeTiles = 920, kGatherSomeTilesFused = 2560;
-constexpr unsigned kGatherTileW[3] = {128, 64, 128}, kGatherTileH[3] = {8, 4, 4};
+// A lane's pixels along x and a wave's rows: form 0 has the kernels' own (FKD_GATHER_XI, FKD_GATHER_YI), 1 and 2 are named by theirs.
+inline constexpr unsigned gather_form_xi(unsigned form, unsigned own) { return form != 0u ? form : own; }
+inline constexpr unsigned gather_form_yi(unsigned form, unsigned own) { return form != 0u ? 1u : own; }
 inline unsigned gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) {
     const unsigned long long tiles = (unsigned long long)((w + 127u) / 128u) * ((h + 7u) / 8u) * planes;
     return tiles < kGatherFewTiles ? 1u : tiles < some_tiles ? 2u : 0u;
@@ -127,6 +129,9 @@ constexpr unsigned kLinesBit = 16u, kLinesWidth = 640;
 inline constexpr unsigned lines_lanes(unsigned w, unsigned h, unsigned planes) {
     return w > 256u || (unsigned long long)((h + 7u) / 8u) * planes < 540u ? 64u : 32u;
 }
+
+// Rows of a workgroup of the bilinear kernel's strip form: half a wave each.
+constexpr unsigned kStripFormRows = 8;
 
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
@@ -143,5 +148,75 @@ struct JitMeta {
     unsigned some_tiles;      // gather kernel: the last argument of gather_form
     unsigned few_blocks;      // rows kernel: rows_few_blocks
 };
+
+// Which of a run-time compiled module's kernels a launch takes, and its grid of workgroups of 64 lanes by block_y waves.  active: the extents and
+// flags the parameter block begins with; strip: whether the strip form may be taken.  (The constants a module was compiled with are the
+// module's own: everything here comes from its JitMeta.)
+struct JitGeometry {
+    const char* kernel;
+    unsigned which;                       // 0 the chain's own kernel, 1 to 6 those of jit_other_body
+    unsigned long long grid_x;
+    unsigned grid_y, block_y;
+    TileGeom g;
+};
+inline JitGeometry jit_geometry(const JitMeta& m, const unsigned (&active)[4], bool strip) {
+    JitGeometry l{m.gather ? "gather_jit" : "rows_jit", 0u, 0u, 1u, m.gather ? m.by : 4u, TileGeom{0, 0, 0, 0}};
+    const unsigned w = active[0], h = active[1], planes = active[2], flags = active[3];
+    const bool streamed = m.gather && (unsigned long long)w * h * planes * m.stream_bytes > kStreamOutputBytes;
+    strip = strip && m.gather && m.strip_width != 0u && w != 0u;
+    if (strip && (flags & kLinesBit) != 0u) {
+        // (rows of 64 lanes only)
+        l.kernel = (flags & 1u) != 0u ? "strip_jit" : "gather_jit";
+        l.which = 3u;
+        l.grid_x = (h + 3u) / 4u;
+        l.g.n_tiles = streamed ? kStreamFlag : 0u;
+    } else if (strip && w <= m.strip_width && (flags & 1u) != 0u) {
+        // strip form: tiles_x == 0 tells the kernel, and n_tiles carries the launch's priority schedule
+        l.kernel = "strip_jit";
+        l.grid_x = (h + kStripFormRows - 1u) / kStripFormRows;
+        l.g.n_tiles = strip_first_late_workgroup(l.grid_x * planes) | (streamed ? kStreamFlag : 0u) | ((flags & 2u) != 0u ? kAnyPitchFlag : 0u);
+    } else if (m.gather) {
+        l.which = gather_form(w, h, planes, m.some_tiles);
+        const unsigned tw = 64u * gather_form_xi(l.which, m.xi), th = m.by * gather_form_yi(l.which, m.yi);
+        l.g.tiles_x = (w + tw - 1u) / tw;
+        l.g.tiles_y = (h + th - 1u) / th;
+        l.g.n_tiles = streamed ? kStreamFlag : 0u;       // (the kernel counts its tiles itself)
+        l.g.tiles_x_magic = division_magic(l.g.tiles_x, l.g.tiles_x * l.g.tiles_y);
+        l.grid_x = (l.g.tiles_x * l.g.tiles_y + 7u) / 8u * 8u;
+    } else if (m.has_flat != 0u && (flags & kFlatBit) != 0u) {
+        l.which = 2u;
+        l.grid_x = flat_blocks(w, h, flags, m.rows);
+        const bool few = m.rows > 1u && l.grid_x * planes < m.few_blocks;
+        if ((flags & kSmallOutputBit) != 0u || few) {
+            l.which = (flags & kSmallOutputBit) != 0u ? 3u : 5u;
+            if (m.rows > 1u) l.grid_x = flat_blocks(w, h, flags, m.rows / 2u);
+        }
+    } else {
+        if (m.has_small != 0u && rows_small(w, m.v, flags)) l.which = 1u;
+        unsigned rows = m.rows;
+        if (m.max_planes == 0u && m.rows > 1u) {
+            const bool few = (unsigned long long)((w + 64u * m.v - 1u) / (64u * m.v)) * ((h + 4u * rows - 1u) / (4u * rows)) * planes < m.few_blocks;
+            if (l.which == 0u && few) l.which = 4u;
+            if (l.which == 1u && !few) l.which = 6u;
+            if (few) rows /= 2u;
+        }
+        const unsigned gx = (w + (m.max_planes != 0u ? 0u : rows_phase_bound(flags)) + 64u * m.v - 1u) / (64u * m.v), gy = (h + 4u * rows - 1u) / (4u * rows);
+        l.grid_x = gx;
+        l.grid_y = gy;
+        const bool bands = m.bands && (unsigned long long)gx * gy >= kRowsBandBlocks;
+        if (bands || (m.bands > 1u && rows_bands_2d(gx, gy))) {
+            l.g.tiles_x = gx;
+            l.g.tiles_y = gy;
+            l.g.tiles_x_magic = division_magic(gx, gx * gy);
+        }
+        if (bands) {
+            // as launch_rows_with: one-dimensional, eight equal runs of the plane's blocks
+            l.g.n_tiles = gx * gy * planes;
+            l.grid_x = ((unsigned long long)gx * gy + 7u) / 8u * 8u;
+            l.grid_y = 1u;
+        }
+    }
+    return l;
+}
 
 } // namespace fkd

@@ -737,6 +737,16 @@ int fklcase_lines_pay(unsigned w, unsigned h, unsigned planes, unsigned row_grai
     return fkd::lines_pay(w, h, planes, sizeof(fkd::Vec<fkd::f32, 3>), row_grain) ? 1 : 0;
 }
 unsigned fklcase_gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) { return fkd::gather_form(w, h, planes, some_tiles); }
+// The launch of a run-time compiled kernel (fkd::jit_geometry) for a module that describes itself by meta[0..8] (gather, v, rows, xi, yi, by, strip_width,
+// bands, has_flat; small outputs have a kernel): out = kernel number, grid x, grid y, waves, tiles_x, tiles_y.
+void fklcase_jit_geometry(const unsigned* meta, unsigned w, unsigned h, unsigned planes, unsigned flags, unsigned* out) {
+    fkd::JitMeta m{};
+    m.gather = meta[0]; m.v = meta[1]; m.rows = meta[2]; m.xi = meta[3]; m.yi = meta[4]; m.by = meta[5]; m.strip_width = meta[6];
+    m.bands = meta[7]; m.has_flat = meta[8]; m.has_small = 1; m.some_tiles = fkd::kGatherSomeTiles; m.few_blocks = fkd::kRowsFewBlocks;
+    const unsigned active[4] = {w, h, planes, flags};
+    const fkd::JitGeometry l = fkd::jit_geometry(m, active, true);
+    out[0] = l.which; out[1] = unsigned(l.grid_x); out[2] = l.grid_y; out[3] = l.block_y; out[4] = l.g.tiles_x; out[5] = l.g.tiles_y;
+}
 unsigned fklcase_row_grain(unsigned long long address, unsigned w, unsigned h, unsigned planes) {
     Tensor<float> t(reinterpret_cast<float*>(size_t(address)), w, h, planes, 3, MemType::Device, 0);
     const auto& d = t.ptr().dims;

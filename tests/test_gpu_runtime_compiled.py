@@ -130,6 +130,45 @@ def test_a_chain_that_would_need_scratch_memory_is_compiled_again_or_refused(dev
     assert r.returncode != 0 and "could not be compiled at run time" in r.stderr, r.stderr[-2000:]
 
 
+_DEFINES_SCRIPT = r"""
+import os, sys
+sys.path.insert(0, sys.argv[1]); sys.path.insert(0, os.path.join(sys.argv[1], "tests"))
+import numpy as np, torch
+import fkl_cases as cases
+dev = torch.device("cuda:0")
+r = np.random.RandomState(5)
+wide = torch.from_numpy(r.rand(33, 80).astype(np.float32)).to(dev)
+rows = torch.full((33, 90), -1.0, device=dev)
+cases.uncompiled_pointwise_f32(wide[:, :70], rows[:, :70])
+img = torch.from_numpy(r.rand(40, 55, 4).astype(np.float32)).to(dev)
+big = torch.full((800, 1500, 4), -1.0, device=dev)
+cases.uncompiled_float4_resize(img, (1500, 800), big)
+crop = torch.from_numpy(r.randint(0, 256, (64, 64, 4)).astype(np.uint8)).to(dev)
+small = torch.full((4, 300, 96), -1.0, device=dev)
+cases.uncompiled_resize_split(1, crop, (1, 1, 60, 60), (96, 300), 0.5, small)
+torch.cuda.synchronize()
+np.savez(sys.argv[2], rows=rows.cpu().numpy(), big=big.cpu().numpy(), small=small.cpu().numpy())
+"""
+
+
+def test_kernels_with_other_constants_cover_the_whole_output(device, tmp_path):
+    """FKLHIP_JIT_DEFINES: the launcher lays its grids out by the constants a module was compiled with (three rows per thread, other
+    tiles of the bilinear kernel), so the results are those of the constants of the build."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for n, defines in enumerate(("", "-DFKD_ROWS=3 -DFKD_GATHER_XI=1 -DFKD_GATHER_YI=1", "-DFKD_ROWS=1 -DFKD_GATHER_XI=4 -DFKD_GATHER_YI=3")):
+        res = tmp_path / f"out{n}.npz"
+        r = subprocess.run([sys.executable, "-c", _DEFINES_SCRIPT, root, str(res)], env=dict(os.environ, FKLHIP_JIT_DEFINES=defines), capture_output=True,
+                           text=True, timeout=240)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(np.load(res))
+    for other in got[1:]:
+        assert [k for k in got[0] if got[0][k].tobytes() != other[k].tobytes()] == []
+
+
 def test_a_chain_whose_parameters_exceed_the_kernel_argument_limit_is_refused_with_a_sentence(device):
     """45 000 planes of 24-byte pointers on either side are 2 MB of by-value kernel arguments: the run-time compiler
     refuses the chain (FKLHIP_EBLOB_SIZE) and its log names the limit, instead of the launch call failing later."""
