@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52064000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "efcc07341b70ef483384aa2d3495cc91373a70fc5de421308923357761602bc3"
+TRAFFIC_C3_SOURCES_SHA256 = "8fd41668694344f431a0c1837ba6648a144e24a226855372d314b76dc085f39a"
 
 
 def device_sources_sha256():

@@ -22,7 +22,7 @@ ABI_SYMBOLS = (
     "fklhip_stream_create", "fklhip_stream_destroy", "fklhip_stream_sync", "fklhip_malloc", "fklhip_malloc_pitch",
     "fklhip_free", "fklhip_host_alloc", "fklhip_host_free", "fklhip_memcpy_async", "fklhip_memcpy2d_async",
     "fklhip_memset_async", "fklhip_event_create", "fklhip_event_destroy", "fklhip_event_record", "fklhip_event_sync",
-    "fklhip_event_elapsed_ms", "fklhip_lookup", "fklhip_launch_handle", "fklhip_launch", "fklhip_last_launch",
+    "fklhip_event_elapsed_ms", "fklhip_lookup", "fklhip_launch_handle", "fklhip_launch", "fklhip_last_launch", "fklhip_last_form",
     "fklhip_signature_count", "fklhip_signature_at", "fklhip_jit_log", "fklhip_strip_form",
 )
 
@@ -50,6 +50,7 @@ def lib() -> _C.CDLL:
         l.fklhip_stream_destroy.argtypes = [_C.c_void_p]
         l.fklhip_stream_sync.argtypes = [_C.c_void_p]
         l.fklhip_last_launch.argtypes = [_C.POINTER(_C.c_char_p), _C.POINTER(_C.c_uint), _C.POINTER(_C.c_uint), _C.POINTER(_C.c_uint)]
+        l.fklhip_last_form.argtypes = [_C.POINTER(_C.c_char_p)]
         _lib = l
     return _lib
 
@@ -78,4 +79,6 @@ def last_launch() -> dict:
     b = (_C.c_uint * 3)()
     lds = _C.c_uint()
     lib().fklhip_last_launch(_C.byref(k), g, b, _C.byref(lds))
-    return {"kernel": (k.value or b"").decode(), "grid": list(g), "block": list(b), "lds_bytes": lds.value}
+    form = _C.c_char_p()
+    lib().fklhip_last_form(_C.byref(form))
+    return {"kernel": (k.value or b"").decode(), "grid": list(g), "block": list(b), "lds_bytes": lds.value, "form": (form.value or b"").decode()}

@@ -36,7 +36,7 @@ hipError_t launch_rows_with(const typename Chain::Params& p, hipStream_t stream,
             g = TileGeom{gx, gy, 0u, division_magic(gx, gx * gy)};
         }
     }
-    if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
+    if (info) *info = LaunchInfo{aligned_name(aligned), {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0, "rows"};
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
     if (grid.y > 65535u || grid.z > 65535u) return hipErrorInvalidConfiguration;
     const bool small = rows_small(p.active_w, V, p.reserved);
@@ -57,7 +57,7 @@ hipError_t launch_flat(const typename Chain::Params& p, hipStream_t stream, Laun
         if ((unsigned long long)blocks * p.active_z < rows_few_blocks<Chain>()) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
     }
     const dim3 grid(blocks, 1, p.active_z), block(kRowsBX, kRowsBY, 1);
-    if (info) *info = LaunchInfo{"rows", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
+    if (info) *info = LaunchInfo{"rows", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0, "flat"};
     if (grid.z == 0) return hipSuccess;
     if (grid.z > 65535u) return hipErrorInvalidConfiguration;
     if ((p.reserved & kSmallOutputBit) != 0u) return launch_by_pointer(&k_flat<Chain, V, ROWS, true>, grid, block, stream, p);
@@ -91,7 +91,7 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
         if (p.active_w != 0 && (p.reserved & kLinesBit) != 0u && fklhip::strip_enabled()) {
             const unsigned lanes = lines_lanes(p.active_w, p.active_h, p.active_z), rows = kStripThreads / lanes;
             const dim3 grid((p.active_h + rows - 1) / rows, 1, p.active_z), block(kGatherBX, kStripThreads / kGatherBX, 1);
-            if (info) *info = LaunchInfo{(p.reserved & 1u) != 0u ? "strip" : "gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned((lanes == 32u ? 9 * 32 : 11 * 64) * 16 + (kStripThreads / 64) * 4)};
+            if (info) *info = LaunchInfo{(p.reserved & 1u) != 0u ? "strip" : "gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned((lanes == 32u ? 9 * 32 : 11 * 64) * 16 + (kStripThreads / 64) * 4), "strip_lines"};
             if (grid.x == 0 || grid.z == 0) return hipSuccess;
             if (grid.z > 65535u) return hipErrorInvalidConfiguration;
             if (lanes == 32u) {
@@ -105,7 +105,7 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
         // (an output without columns has no workgroup in the tile form's grid: it falls through and launches nothing)
         if (p.active_w != 0 && p.active_w <= unsigned(kStripMaxWidth) && (p.reserved & 1u) != 0 && fklhip::strip_enabled()) {
             const dim3 grid((p.active_h + kStripRows - 1) / kStripRows, 1, p.active_z), block(kGatherBX, kStripThreads / kGatherBX, 1);
-            if (info) *info = LaunchInfo{"strip", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned(kStripMaxWidth * 16 + (kStripThreads / 64) * 4)};
+            if (info) *info = LaunchInfo{"strip", {grid.x, 1, grid.z}, {block.x, block.y, 1}, unsigned(kStripMaxWidth * 16 + (kStripThreads / 64) * 4), "strip"};
             if (grid.x == 0 || grid.z == 0) return hipSuccess;
             if (grid.z > 65535u) return hipErrorInvalidConfiguration;
             const unsigned first_late = strip_first_late_workgroup((unsigned long long)grid.x * grid.z);
@@ -126,7 +126,7 @@ hipError_t launch_gather(const typename Chain::Params& p, hipStream_t stream, La
     g.tiles_x_magic = division_magic(g.tiles_x, g.tiles_x * g.tiles_y);
     const unsigned chunk = (g.tiles_x * g.tiles_y + 7u) / 8u;
     const dim3 grid(chunk * 8u, 1, p.active_z), block(kGatherBX, kGatherBY, 1);
-    if (info) *info = LaunchInfo{"gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0};
+    if (info) *info = LaunchInfo{"gather", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0, "tiles"};
     if (g.n_tiles == 0) return hipSuccess;
     if (grid.z > 65535u) return hipErrorInvalidConfiguration;
     if (form == 1u) return launch_by_pointer(&k_gather<Chain, 1, 1, false>, grid, block, stream, p, g);
@@ -143,7 +143,7 @@ hipError_t launch_divergent(const typename D::Params& p, hipStream_t stream, Lau
     const unsigned gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);
     const unsigned gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);
     const dim3 grid(gx, gy, p.active_z), block(kRowsBX, kRowsBY, 1);
-    if (info) *info = LaunchInfo{"divergent", {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0};
+    if (info) *info = LaunchInfo{"divergent", {grid.x, grid.y, grid.z}, {block.x, block.y, 1}, 0, "divergent"};
     if (grid.x == 0 || grid.y == 0 || grid.z == 0) return hipSuccess;
     if (grid.y > 65535u || grid.z > unsigned(D::kMaxPlanes)) return hipErrorInvalidConfiguration;
     return launch_by_pointer(&k_divergent<D>, grid, block, stream, p);

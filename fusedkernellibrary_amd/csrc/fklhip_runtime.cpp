@@ -28,7 +28,7 @@ Table& table() {
     return *t;
 }
 
-thread_local fkd::LaunchInfo g_last = {"", {0, 0, 0}, {0, 0, 0}, 0};
+thread_local fkd::LaunchInfo g_last = {"", {0, 0, 0}, {0, 0, 0}, 0, ""};
 
 // The environment is looked at once (a function-local static: thread safe), afterwards only the atomic is read.
 std::atomic<int>& strip_setting() {
@@ -193,6 +193,12 @@ int fklhip_last_launch(const char** kernel, unsigned grid[3], unsigned block[3],
         if (block) block[i] = g_last.block[i];
     }
     if (lds_bytes) *lds_bytes = g_last.lds_bytes;
+    return FKLHIP_OK;
+}
+
+int fklhip_last_form(const char** form) {
+    if (!form) return FKLHIP_EINVAL;
+    *form = g_last.form;
     return FKLHIP_OK;
 }
 

@@ -217,7 +217,7 @@ int jit_launch(const void* ctx, const void* blob, size_t bytes, void* stream, fk
     const fkd::JitGeometry l = fkd::jit_geometry(m, active, strip_enabled());
     if (l.grid_x > 0x7fffff00ull) return int(hipErrorInvalidConfiguration);
     const unsigned grid[3] = {unsigned(l.grid_x), l.grid_y, active[2]}, block[3] = {64, l.block_y, 1};
-    if (info) *info = fkd::LaunchInfo{l.kernel, {grid[0], grid[1], grid[2]}, {block[0], block[1], 1}, 0};
+    if (info) *info = fkd::LaunchInfo{l.kernel, {grid[0], grid[1], grid[2]}, {block[0], block[1], 1}, 0, l.form};
     if (grid[0] == 0 || grid[1] == 0 || grid[2] == 0) return FKLHIP_OK;
     if (grid[1] > 65535u || grid[2] > 65535u) return int(hipErrorInvalidConfiguration);
     if (m.max_planes != 0 && grid[2] > m.max_planes) return int(hipErrorInvalidConfiguration);   // as launch_divergent

@@ -6,9 +6,12 @@
 namespace fkd {
 
 struct LaunchInfo {
-    const char* kernel;   // "rows", "rows_unaligned" (chains with a kernel of its own for such rows), "gather" or "strip"
+    const char* kernel;   // "rows", "rows_unaligned" (chains with a kernel of its own for such rows), "gather", "strip" or "divergent"
     unsigned grid[3], block[3];
     unsigned lds_bytes;
+    // The kernel by its own name, where `kernel` is the name of the form it took the place of: "rows", "flat" (planes without gaps), "tiles", "strip",
+    // "strip_lines" (stores moved on to line boundaries) or "divergent".
+    const char* form;
 };
 
 // ---- the geometry a launcher hands to kernels that renumber their workgroups ----
@@ -153,26 +156,28 @@ struct JitMeta {
 // flags the parameter block begins with; strip: whether the strip form may be taken.  (The constants a module was compiled with are the
 // module's own: everything here comes from its JitMeta.)
 struct JitGeometry {
-    const char* kernel;
+    const char *kernel, *form;            // see LaunchInfo
     unsigned which;                       // 0 the chain's own kernel, 1 to 6 those of jit_other_body
     unsigned long long grid_x;
     unsigned grid_y, block_y;
     TileGeom g;
 };
 inline JitGeometry jit_geometry(const JitMeta& m, const unsigned (&active)[4], bool strip) {
-    JitGeometry l{m.gather ? "gather_jit" : "rows_jit", 0u, 0u, 1u, m.gather ? m.by : 4u, TileGeom{0, 0, 0, 0}};
+    JitGeometry l{m.gather ? "gather_jit" : "rows_jit", m.gather ? "tiles" : (m.max_planes != 0u ? "divergent" : "rows"), 0u, 0u, 1u, m.gather ? m.by : 4u, TileGeom{0, 0, 0, 0}};
     const unsigned w = active[0], h = active[1], planes = active[2], flags = active[3];
     const bool streamed = m.gather && (unsigned long long)w * h * planes * m.stream_bytes > kStreamOutputBytes;
     strip = strip && m.gather && m.strip_width != 0u && w != 0u;
     if (strip && (flags & kLinesBit) != 0u) {
         // (rows of 64 lanes only)
         l.kernel = (flags & 1u) != 0u ? "strip_jit" : "gather_jit";
+        l.form = "strip_lines";
         l.which = 3u;
         l.grid_x = (h + 3u) / 4u;
         l.g.n_tiles = streamed ? kStreamFlag : 0u;
     } else if (strip && w <= m.strip_width && (flags & 1u) != 0u) {
         // strip form: tiles_x == 0 tells the kernel, and n_tiles carries the launch's priority schedule
         l.kernel = "strip_jit";
+        l.form = "strip";
         l.grid_x = (h + kStripFormRows - 1u) / kStripFormRows;
         l.g.n_tiles = strip_first_late_workgroup(l.grid_x * planes) | (streamed ? kStreamFlag : 0u) | ((flags & 2u) != 0u ? kAnyPitchFlag : 0u);
     } else if (m.gather) {
@@ -184,6 +189,7 @@ inline JitGeometry jit_geometry(const JitMeta& m, const unsigned (&active)[4], b
         l.g.tiles_x_magic = division_magic(l.g.tiles_x, l.g.tiles_x * l.g.tiles_y);
         l.grid_x = (l.g.tiles_x * l.g.tiles_y + 7u) / 8u * 8u;
     } else if (m.has_flat != 0u && (flags & kFlatBit) != 0u) {
+        l.form = "flat";
         l.which = 2u;
         l.grid_x = flat_blocks(w, h, flags, m.rows);
         const bool few = m.rows > 1u && l.grid_x * planes < m.few_blocks;

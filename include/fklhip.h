@@ -121,6 +121,10 @@ int fklhip_strip_form(int enable);
  * them (padding, deinterlacing, planar and circular reads; the others have one kernel for rows at every alignment).
  * grid/block receive 3 values each. */
 int fklhip_last_launch(const char **kernel, unsigned grid[3], unsigned block[3], unsigned *lds_bytes);
+/* The same launch's kernel by its own name, which fklhip_last_launch gives by the form it took the place of: "rows", "flat" (planes whose rows
+ * follow each other without gaps, taken as one row), "tiles", "strip", "strip_lines" (strips whose stores begin at line boundaries) or
+ * "divergent", ahead of time and compiled at run time alike; "" before the first launch. */
+int fklhip_last_form(const char **form);
 
 /* Number of chain signatures compiled into the library and the i-th of them with its parameter block size. */
 int fklhip_signature_count(int *count);

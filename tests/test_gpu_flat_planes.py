@@ -6,6 +6,7 @@ import pytest
 
 import fkl_cases as cases
 import oracle_lib as ol
+from fusedkernellibrary_amd import last_launch
 from test_gpu_any_alignment import FILL, Placed
 
 FLAT, SMALL = 8, 4
@@ -63,6 +64,7 @@ def test_tensors_of_any_element(device, kind, in_place):
             src_host, _, src_pitches, src_start = place(size * (n % 3), size * (n % 2), True)
             cases.copy_tensor(kind, torch.from_numpy(src_host).to(device)[src_start:], src_pitches, out[out_start:], out_pitches, w, h, planes)
         torch.cuda.synchronize()
+        assert last_launch()["form"] == ("flat" if w * h >= 4 else "rows")
         out_at[:] = data
         assert np.array_equal(out.cpu().numpy(), out_host), (w, h)
 
@@ -81,6 +83,7 @@ def test_batches_of_images(device, offset):
         cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [o.view() for o in outs])
         cases.batch_muladd_sat([s.view() for s in srcs], mul, add, [s.view() for s in srcs])      # in place
         torch.cuda.synchronize()
+        assert last_launch()["form"] == "flat"
         for a, b, c in zip(srcs, outs, want):
             assert np.array_equal(b.read(), c) and np.array_equal(a.read(), c), (w, h, offset)
 
@@ -94,6 +97,7 @@ def test_float_chains(device, n_ops):
         src, out = Placed((h, w), np.float32, 4 * (n % 4), 0, device, img), Placed((h, w), np.float32, 4 * (n % 3), 0, device)
         cases.add_mul_chain(src.view(), n_ops, 0.5, 1.0001, out.view())
         torch.cuda.synchronize()
+        assert last_launch()["form"] == "flat"
         assert out.read().tobytes() == ol.oracle_add_mul_chain(img, n_ops, np.float32(0.5), np.float32(1.0001)).tobytes(), (w, h)
 
 
@@ -108,6 +112,7 @@ def test_packed_video(device, pf, cr, cp, dtype):
         out = Placed((h, w, 3), np.float32, 4 * (n % 5), 0, device)
         cases.yuv_to_rgb(pf, cr, cp, src, w, h, out.view())
         torch.cuda.synchronize()
+        assert last_launch()["form"] == "flat"
         assert out.read().tobytes() == ol.oracle_yuv_to_rgb(pf, cr, cp, frame.view(np.uint8 if dtype == np.uint8 else np.uint16), w, h).tobytes(), (w, h)
 
 
@@ -119,4 +124,5 @@ def test_planar_output(device):
         out = torch.full((3, h, w), -1.0, dtype=torch.float32, device=device)
         cases.u8x3_to_planes(torch.from_numpy(img).to(device), out)
         torch.cuda.synchronize()
+        assert last_launch()["form"] == "flat"
         assert np.array_equal(out.cpu().numpy(), img.transpose(2, 0, 1).astype(np.float32)), (w, h)

@@ -38,7 +38,7 @@ def rects_in(rng, n, w, h):
 @pytest.mark.parametrize("width", [201, 204])
 def test_crops(device, batch, dst, width):
     import torch
-    from fusedkernellibrary_amd import lib
+    from fusedkernellibrary_amd import last_launch, lib
     assert cases.cases().fklcase_lines_pay(dst[0], dst[1], batch, 16 if dst[0] == 300 else 4) == 1
     rng = np.random.RandomState(dst[0])
     img, rects = image(width, 77, dst[1]), rects_in(np.random.RandomState(dst[1]), batch, width, 77)
@@ -57,6 +57,12 @@ def test_crops(device, batch, dst, width):
             torch.cuda.synchronize()
         finally:
             lib().fklhip_strip_form(old)
+        ll = last_launch()
+        assert ll["form"] == ("strip_lines" if on else "tiles")
+        if on:
+            # (narrow rows have 64 lanes where there would be few workgroups)
+            lanes = 64 if dst[0] > 256 or (dst[1] + 7) // 8 * batch < 540 else 32
+            assert ll["grid"] == [-(-dst[1] // (256 // lanes)), 1, batch] and ll["lds_bytes"] == (11 * 64 if lanes == 64 else 9 * 32) * 16 + 16
         got.append(buf.clone())
     assert torch.equal(got[0].view(torch.int32), got[1].view(torch.int32))
     assert (got[0][:start] == -7).all() and (got[0][start + n:] == -7).all()
@@ -78,7 +84,8 @@ def test_compiled_on_first_use(device, kind, cn, dtype, dst):
     out = torch.full((cn, dst[1], dst[0]), -7.0, dtype=torch.float32, device=device)
     cases.uncompiled_resize_split(kind, src, rect, dst, 0.5, out)
     torch.cuda.synchronize()
-    assert last_launch()["block"] == [64, 4, 1] and last_launch()["grid"][0] in ((dst[1] + 3) // 4, (dst[1] + 7) // 8)
+    ll = last_launch()
+    assert ll["form"] == "strip_lines" and ll["block"] == [64, 4, 1] and ll["grid"] == [(dst[1] + 3) // 4, 1, 1]
     want = np.zeros((cn, dst[1], dst[0]), np.float32)
     ol.execute([ol.read_2d(img, cn, crop=rect, resize=dst, ar=ol.IGNORE_AR)], [ol.op(ol.MUL, (0.5, 0.5, 0.5, 0.5))],
                [ol.write(ol.TENSOR_SPLIT, want, cn, dst[0], dst[1], 1, cn)])
@@ -94,7 +101,7 @@ def test_letterboxes(device, dst):
     bg, mul = np.float32([9, -8, 7]), np.float32([2, 0.5, 1.5])
     src = torch.from_numpy(img).to(device)
     out = torch.full((3, 3, dst[1], dst[0]), -7.0, dtype=torch.float32, device=device)
-    from fusedkernellibrary_amd import lib
+    from fusedkernellibrary_amd import last_launch, lib
     got = []
     for on in (1, 0):
         old = lib().fklhip_strip_form(on)
@@ -104,5 +111,6 @@ def test_letterboxes(device, dst):
             torch.cuda.synchronize()
         finally:
             lib().fklhip_strip_form(old)
+        assert last_launch()["form"] == ("strip_lines" if on else "tiles")
         got.append(out.cpu().numpy().tobytes())
     assert got[0] == got[1]
