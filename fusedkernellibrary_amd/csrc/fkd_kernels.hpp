@@ -1044,6 +1044,12 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
     constexpr bool kAnyPitch = Window::kShift && ANY_PITCH;
     const int steps = (aw + kStripStep - 1) / kStripStep;
     if (steps == 0) return;                                             // no columns: nothing to write (the whole workgroup leaves)
+    // With lines the launches are larger, and one whose planes are tall or share their source (large crops of one image) would have every XCD
+    // fetch all of it; as bands, us, without / with / the forms that such launches took before there were line stores: 8 crops of 1200x800 to 225x500
+    // 7.05 / 4.70 / 5.26, to 255x1000 9.4 / 6.9 / 7.4, to 331x331 6.88 / 4.90 / 5.15, to 435x435 8.6 / 6.4 / 6.6; one image of 1200x800, compiled
+    // at run time: ushort3 to 255x12001 16.7 / 10.7 / 10.6, to 333x4003 7.53 / 5.9 / 6.3, uchar4 to 129x6001 7.1 / 5.6 / 6.1.  Launches of a few
+    // microseconds pay 0.05 to 0.1 us for it (64 crops to 258x40 4.40 / 4.49 / 5.05, 8 to 299x299 4.39 / 4.55 / 5.0).
+    const u32 strip = LINES ? plane_band(blockIdx.x, dims[3], blockIdx.z) : blockIdx.x;
 
     const int t = int(threadIdx.y) * 64 + int(threadIdx.x);
     // What depends on the column: the horizontal weights, the window's byte offset in a row, and flags beside the bytes to drop.
@@ -1065,7 +1071,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
 
     // ---- the lane's row ----
     const int g = t & (kStripStep - 1), r = t / kStripStep;
-    const int y = int(blockIdx.x) * kStripRows + r;
+    const int y = int(strip) * kStripRows + r;
     const bool yvalid = y < ah;
     const int yc = yvalid ? y : ah - 1;
     const f32 sy = f32(yc - oy) * q.fy;

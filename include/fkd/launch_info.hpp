@@ -136,6 +136,14 @@ inline constexpr unsigned lines_lanes(unsigned w, unsigned h, unsigned planes) {
 // Rows of a workgroup of the bilinear kernel's strip form: half a wave each.
 constexpr unsigned kStripFormRows = 8;
 
+// Workgroup x of the gx of plane z, one row of workgroups per plane, as the number of its part of the plane: the hardware deals workgroups round-robin
+// to the 8 XCDs, so x is on XCD (z * gx + x) % 8, and XCD k takes the k-th run of parts, which share source lines, in every plane.
+inline constexpr unsigned plane_band(unsigned x, unsigned gx, unsigned z) {
+    const unsigned first = z * gx % 8u, k = (first + x) % 8u;
+    const unsigned longer = ((1u << gx % 8u) - 1u) << first;           // the XCDs with one workgroup more, round the end
+    return k * (gx / 8u) + unsigned(__builtin_popcount((longer | longer >> 8) & ((1u << k) - 1u))) + x / 8u;
+}
+
 // What the launcher of a run-time compiled kernel needs to know about it; the kernel's module publishes one.
 struct JitMeta {
     unsigned gather;          // 1: gather kernel geometry, 0: rows kernel geometry

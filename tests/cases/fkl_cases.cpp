@@ -736,6 +736,7 @@ int fklcase_strip_pays(unsigned w, unsigned h, unsigned planes, int any_pitch, u
 int fklcase_lines_pay(unsigned w, unsigned h, unsigned planes, unsigned row_grain) {
     return fkd::lines_pay(w, h, planes, sizeof(fkd::Vec<fkd::f32, 3>), row_grain) ? 1 : 0;
 }
+unsigned fklcase_plane_band(unsigned x, unsigned gx, unsigned z) { return fkd::plane_band(x, gx, z); }
 unsigned fklcase_gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) { return fkd::gather_form(w, h, planes, some_tiles); }
 // The launch of a run-time compiled kernel (fkd::jit_geometry) for a module that describes itself by meta[0..8] (gather, v, rows, xi, yi, by, strip_width,
 // bands, has_flat; small outputs have a kernel): out = kernel number, grid x, grid y, waves, tiles_x, tiles_y.

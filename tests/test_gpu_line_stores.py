@@ -17,6 +17,17 @@ def test_which_launches_move_their_stores(w, h, planes, grain, lines):
     assert cases.cases().fklcase_lines_pay(w, h, planes, grain) == lines
 
 
+def test_strips_of_a_plane_are_dealt_to_the_xcds_in_runs():
+    """fkd::plane_band: every strip once, and XCD k, which has the workgroups of number k modulo 8, the k-th run of them in every plane."""
+    band = cases.cases().fklcase_plane_band
+    for gx in list(range(1, 75)) + [160, 251, 6001]:
+        for z in (0, 1, 2, 7, 63):
+            parts = [band(x, gx, z) for x in range(gx)]
+            assert sorted(parts) == list(range(gx))
+            xcd = {p: (z * gx + x) % 8 for x, p in enumerate(parts)}
+            assert all(xcd[p] <= xcd[p + 1] for p in range(gx - 1)), (gx, z)
+
+
 def image(w, h, seed):
     return np.random.RandomState(seed).randint(0, 256, (h, w, 3)).astype(np.uint8)
 
