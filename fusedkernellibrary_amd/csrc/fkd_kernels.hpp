@@ -1261,6 +1261,23 @@ template <class Chain> constexpr u32 rows_few_blocks() {
     return detail::wave_exchange_ok<typename Chain::Read::Out>(V) || detail::wave_exchange_ok<typename Chain::Write::In>(V) ? kRowsFewBlocksExchange : kRowsFewBlocks;
 }
 
+// Chains that keep all their rows in launches of kRowsWholeFrom to kRowsWholeTo workgroups: reads of two-plane video, and images whose elements are
+// exchanged between the lanes where they are read and where they are written.
+template <class Op> constexpr bool reads_two_planes() {
+    if constexpr (requires { typename Op::FusedOver; }) return reads_two_planes<typename Op::FusedOver>();
+    else if constexpr (requires { Op::kTwoPlanes; }) return Op::kTwoPlanes;
+    else return false;
+}
+template <class Op> constexpr bool reads_exchanged(int v) {
+    if constexpr (requires { typename Op::FusedOver; }) return reads_exchanged<typename Op::FusedOver>(v);
+    else return knows_dense<Op>() && detail::wave_exchange_ok<typename Op::Out>(v);
+}
+template <class Chain> constexpr bool rows_keep_whole() {
+    using Op = typename ReadRoot<typename Chain::Read>::Op;
+    constexpr int V = RowsConfig<Chain>::V;
+    return reads_two_planes<Op>() || (reads_exchanged<Op>(V) && detail::wave_exchange_ok<typename Chain::Write::In>(V) && puts_whole<typename Chain::Write>());
+}
+
 // ---- divergent batch kernel -------------------------------------------------------------------------------
 
 // Several chains in one launch of the rows kernel's geometry: plane z runs chain select[z] (wave uniform: the plane is
@@ -1313,14 +1330,14 @@ template <class Chain> constexpr bool rows_have_flat() {
 // (JitMeta: fkd/launch_info.hpp)
 template <class Chain> constexpr JitMeta jit_meta() {
     if constexpr (IsDivergent<Chain>::value)
-        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+        return JitMeta{0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V), u32(RowsConfig<Chain>::ROWS), 0u, 0u, 0u, u32(Chain::kMaxPlanes), 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
     else
         return JitMeta{is_gather_chain<Chain>() ? 1u : 0u, u32(sizeof(typename Chain::Params)), u32(RowsConfig<Chain>::V),
                        u32(RowsConfig<Chain>::ROWS), u32(FKD_GATHER_XI), u32(FKD_GATHER_YI), u32(kGatherBY), 0u,
                        is_gather_chain<Chain>() && strip_capable<Chain>() ? u32(kStripMaxWidth) : 0u,
                        !is_gather_chain<Chain>() && rows_in_bands<Chain>() ? (rows_by_points<Chain, RowsConfig<Chain>::V, RowsConfig<Chain>::ROWS>() ? 2u : 1u) : 0u, rows_have_small<Chain>() ? 1u : 0u, rows_have_flat<Chain>() ? 1u : 0u,
                        is_gather_chain<Chain>() && writer_streams<Chain>() ? u32(sizeof(typename Chain::Value)) : 0u,
-                       gather_some_tiles<Chain>(), rows_few_blocks<Chain>()};
+                       gather_some_tiles<Chain>(), rows_few_blocks<Chain>(), rows_keep_whole<Chain>() ? 1u : 0u};
 }
 template <class Chain> __device__ __forceinline__ void jit_body(const typename Chain::Params& p, const TileGeom& g) {
     if constexpr (IsDivergent<Chain>::value) DivergentBody<Chain>::run(p);

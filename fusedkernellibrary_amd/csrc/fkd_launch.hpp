@@ -54,7 +54,7 @@ template <class Chain, int V, int ROWS>
 hipError_t launch_flat(const typename Chain::Params& p, hipStream_t stream, LaunchInfo* info) {
     const unsigned blocks = flat_blocks(p.active_w, p.active_h, p.reserved, ROWS);
     if constexpr (ROWS > 1) {
-        if ((unsigned long long)blocks * p.active_z < rows_few_blocks<Chain>()) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
+        if (rows_halved((unsigned long long)blocks * p.active_z, rows_few_blocks<Chain>(), rows_keep_whole<Chain>())) return launch_flat<Chain, V, ROWS / 2>(p, stream, info);
     }
     const dim3 grid(blocks, 1, p.active_z), block(kRowsBX, kRowsBY, 1);
     if (info) *info = LaunchInfo{"rows", {grid.x, 1, grid.z}, {block.x, block.y, 1}, 0, "flat"};
@@ -77,7 +77,7 @@ hipError_t launch_rows(const typename Chain::Params& p, hipStream_t stream, Laun
     if constexpr (ROWS > 1) {
         const unsigned long long gx = (p.active_w + kRowsBX * V - 1) / (kRowsBX * V);
         const unsigned long long gy = (p.active_h + kRowsBY * ROWS - 1) / (kRowsBY * ROWS);
-        if (gx * gy * p.active_z < rows_few_blocks<Chain>()) return launch_rows_with<Chain, V, ROWS / 2>(p, stream, info, aligned);
+        if (rows_halved(gx * gy * p.active_z, rows_few_blocks<Chain>(), rows_keep_whole<Chain>())) return launch_rows_with<Chain, V, ROWS / 2>(p, stream, info, aligned);
     }
     return launch_rows_with<Chain, V, ROWS>(p, stream, info, aligned);
 }

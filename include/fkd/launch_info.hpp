@@ -108,7 +108,17 @@ inline unsigned flat_blocks(unsigned w, unsigned h, unsigned reserved, unsigned 
 // (1 350) 7.9 / 7.2, 1922x1082 (1 088) 6.7 / 6.4; RGB to NV12 1920x1080 (1 080) 3.4 / 3.6, 2560x1440 (1 800) 4.1 / 4.6; RGB to P010 1920x1080 4.6 / 4.9,
 // 2000x1500 6.2 / 6.7.  Planes without gaps, with the line at 768 / 1024 / 2048: 4 uchar3 images of 1279x719 (1 800) 4.5 / 4.5 / 4.9, 4 of
 // 849x880 (1 460; 4 launches) 16.2 / 16.2 / 17.9, 50 operations on 3840x2160 floats (2 025) 12.6 / 12.6 / 13.6; at 512: 4 of 1209x263 (624) 12.4 -> 13.05.
-constexpr unsigned kRowsFewBlocks = 1024, kRowsFewBlocksExchange = 2048;
+// Some chains below that line are faster with all their rows where those still make a round of two to four workgroups per compute unit (rows_keep_whole
+// in the kernels' header): semi-planar video, and elements that go through the LDS at both ends.  us, all rows / half, 30 (20) buffers in turn: NV12 to
+// float3 1280x720 (450) 3.44 / 3.45, 1280x960 (600) 3.94 / 4.00, 1536x1100 (828) 4.87 / 5.20, 1600x1000 (875) 5.06 / 5.15, 1792x1080 (945) 5.16 / 5.54, P010 to float3
+// 5.43 / 5.88, 1922x1082 (1 088) 6.79 / 6.58; float3 squared, rows with gaps, 1024x600 (300) 3.81 / 3.67, 1280x960 6.55 / 6.91, 1600x800 (700) 6.59 / 7.58,
+// 1792x1080 8.66 / 10.10, 2000x1300 (1 304) 14.2 / 13.0; without gaps 1280x960 6.55 / 6.71, 1792x1080 8.64 / 10.06.  Other chains are not:
+// uchar3 to float3 1280x960 4.62 / 4.18, two fields of uchar3 to float3 1536x1100 6.01 / 5.38, float3 to uchar3 1536x1100 6.23 / 6.08.
+constexpr unsigned kRowsFewBlocks = 1024, kRowsFewBlocksExchange = 2048, kRowsWholeFrom = 512, kRowsWholeTo = 1024;
+// blocks: of a launch with all rows; few: rows_few_blocks of the chain.
+inline constexpr bool rows_halved(unsigned long long blocks, unsigned few, bool keep_whole) {
+    return blocks < few && !(keep_whole && blocks >= kRowsWholeFrom && blocks <= kRowsWholeTo);
+}
 
 // Which tiles a launch of the bilinear kernel's tile form takes: 128x8 pixels, or smaller ones where it would have few of those (per-wave
 // latency, see the kernels' header).  us, tiles of 128x8 / 128x4 / 64x4 pixels (in brackets: how many of 128x8): NV12 to 148x85 (22)
@@ -158,6 +168,7 @@ struct JitMeta {
     unsigned stream_bytes;    // gather kernel with a planar writer: bytes stored per output element (see kStreamOutputBytes), else 0
     unsigned some_tiles;      // gather kernel: the last argument of gather_form
     unsigned few_blocks;      // rows kernel: rows_few_blocks
+    unsigned keep_whole;      // rows kernel: rows_keep_whole
 };
 
 // Which of a run-time compiled module's kernels a launch takes, and its grid of workgroups of 64 lanes by block_y waves.  active: the extents and
@@ -200,7 +211,7 @@ inline JitGeometry jit_geometry(const JitMeta& m, const unsigned (&active)[4], b
         l.form = "flat";
         l.which = 2u;
         l.grid_x = flat_blocks(w, h, flags, m.rows);
-        const bool few = m.rows > 1u && l.grid_x * planes < m.few_blocks;
+        const bool few = m.rows > 1u && rows_halved(l.grid_x * planes, m.few_blocks, m.keep_whole != 0u);
         if ((flags & kSmallOutputBit) != 0u || few) {
             l.which = (flags & kSmallOutputBit) != 0u ? 3u : 5u;
             if (m.rows > 1u) l.grid_x = flat_blocks(w, h, flags, m.rows / 2u);
@@ -209,7 +220,7 @@ inline JitGeometry jit_geometry(const JitMeta& m, const unsigned (&active)[4], b
         if (m.has_small != 0u && rows_small(w, m.v, flags)) l.which = 1u;
         unsigned rows = m.rows;
         if (m.max_planes == 0u && m.rows > 1u) {
-            const bool few = (unsigned long long)((w + 64u * m.v - 1u) / (64u * m.v)) * ((h + 4u * rows - 1u) / (4u * rows)) * planes < m.few_blocks;
+            const bool few = rows_halved((unsigned long long)((w + 64u * m.v - 1u) / (64u * m.v)) * ((h + 4u * rows - 1u) / (4u * rows)) * planes, m.few_blocks, m.keep_whole != 0u);
             if (l.which == 0u && few) l.which = 4u;
             if (l.which == 1u && !few) l.which = 6u;
             if (few) rows /= 2u;

@@ -1891,6 +1891,7 @@ template <bool VU> struct ReadNV {
     static constexpr bool kAnyX = true;
     static constexpr bool kFiniteTaps = true;
     static constexpr bool kBoundedOut = true;
+    static constexpr bool kTwoPlanes = true;
     FKD_NAME(VU ? "ReadNV21" : "ReadNV12")
 #if defined(FKD_EXEC_CODE)
     FKD_DEV static int width(const Params& p) { return int(p.width); }
@@ -2015,6 +2016,7 @@ template <int PF> struct ReadYUV {
     static constexpr int kXGroup = 2;
     static constexpr bool kAnyX = true;
     static constexpr bool kTapCursor = false;
+    static constexpr bool kTwoPlanes = L::kSemiPlanar;
     FKD_NAME("ReadYUV<" + istr(PF) + ">")
     // (packed formats: two samples per pixel; the planes of the others are two images)
     FKD_HD static bool dense(const Params& p, u32 w, u32) { return !L::kSemiPlanar && w % 2 == 0 && p.pitch == size_t(w) * 2 * sizeof(B); }

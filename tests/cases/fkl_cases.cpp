@@ -738,12 +738,12 @@ int fklcase_lines_pay(unsigned w, unsigned h, unsigned planes, unsigned row_grai
 }
 unsigned fklcase_plane_band(unsigned x, unsigned gx, unsigned z) { return fkd::plane_band(x, gx, z); }
 unsigned fklcase_gather_form(unsigned w, unsigned h, unsigned planes, unsigned some_tiles) { return fkd::gather_form(w, h, planes, some_tiles); }
-// The launch of a run-time compiled kernel (fkd::jit_geometry) for a module that describes itself by meta[0..8] (gather, v, rows, xi, yi, by, strip_width,
-// bands, has_flat; small outputs have a kernel): out = kernel number, grid x, grid y, waves, tiles_x, tiles_y.
+// The launch of a run-time compiled kernel (fkd::jit_geometry) for a module that describes itself by meta[0..9] (gather, v, rows, xi, yi, by, strip_width,
+// bands, has_flat, keep_whole; small outputs have a kernel): out = kernel number, grid x, grid y, waves, tiles_x, tiles_y.
 void fklcase_jit_geometry(const unsigned* meta, unsigned w, unsigned h, unsigned planes, unsigned flags, unsigned* out) {
     fkd::JitMeta m{};
     m.gather = meta[0]; m.v = meta[1]; m.rows = meta[2]; m.xi = meta[3]; m.yi = meta[4]; m.by = meta[5]; m.strip_width = meta[6];
-    m.bands = meta[7]; m.has_flat = meta[8]; m.has_small = 1; m.some_tiles = fkd::kGatherSomeTiles; m.few_blocks = fkd::kRowsFewBlocks;
+    m.bands = meta[7]; m.has_flat = meta[8]; m.has_small = 1; m.some_tiles = fkd::kGatherSomeTiles; m.few_blocks = fkd::kRowsFewBlocksExchange; m.keep_whole = meta[9];
     const unsigned active[4] = {w, h, planes, flags};
     const fkd::JitGeometry l = fkd::jit_geometry(m, active, true);
     out[0] = l.which; out[1] = unsigned(l.grid_x); out[2] = l.grid_y; out[3] = l.block_y; out[4] = l.g.tiles_x; out[5] = l.g.tiles_y;
