@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52065000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "1fc36701f6ee9b07ef64c4d9bd2bd598e043053c903b063e6194f8d5078e64bd"
+TRAFFIC_C3_SOURCES_SHA256 = "cd4962758118c48a9d2f231269dfcfd7a7cc88a35d53a50bc5606a6ac8adbc7e"
 
 
 def device_sources_sha256():
