@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52065000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "cd4962758118c48a9d2f231269dfcfd7a7cc88a35d53a50bc5606a6ac8adbc7e"
+TRAFFIC_C3_SOURCES_SHA256 = "e11a2ee1bceb497d97dafd9b5e31031c58785908f04f9e59aa7cf7c0baeb61ba"
 
 
 def device_sources_sha256():
