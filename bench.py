@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52065000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "e11a2ee1bceb497d97dafd9b5e31031c58785908f04f9e59aa7cf7c0baeb61ba"
+TRAFFIC_C3_SOURCES_SHA256 = "fced9da442eb5af5929d19c4edc8f595e47dfa292bbc8a98d1b26c62d7a2c0c2"
 
 
 def device_sources_sha256():

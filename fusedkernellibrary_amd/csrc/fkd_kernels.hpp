@@ -425,14 +425,6 @@ template <class Op> constexpr bool reads_points() {
 template <class Chain, int V, int ROWS> constexpr bool rows_by_points() {
     return V == kRowsBY && ROWS == 1 && reads_points<typename ReadRoot<typename Chain::Read>::Op>() && puts_whole<typename Chain::Write>();
 }
-// Chains of more than 128 bytes of operation parameters.
-template <class Chain> constexpr bool many_ops() {
-    return sizeof(typename Chain::Params) - sizeof(typename Chain::Read::Params) - sizeof(typename Chain::Write::Params) > 128 + 16;
-}
-// Eight waves per SIMD: what a wave waits for is a gather.  Not for long chains (60 operations on float4 take 72 registers, and kept to 64 they need scratch
-// memory, which the build refuses), nor for run-time compiled kernels: ushort3 in 71 registers is the faster one (1474x2063 by 29 degrees 13.7 / 15.2 us,
-// perspective 13.1 / 14.5; 3840x2160 by 7 degrees 22.1 / 22.1, perspective 24.1 / 23.5).
-template <class Chain, int V, int ROWS> constexpr int rows_min_waves() { return rows_by_points<Chain, V, ROWS>() && !many_ops<Chain>() ? 8 : 1; }
 template <class Chain, int V, int FORM>
 __device__ __forceinline__ void points_body(const typename Chain::Params& p, const TileGeom& bands) {
     using Root = ReadRoot<typename Chain::Read>;
@@ -499,7 +491,7 @@ __device__ __forceinline__ void points_body(const typename Chain::Params& p, con
 }
 
 template <class Chain, int V, int ROWS, bool ALIGNED, int FORM>
-__global__ __launch_bounds__(kRowsBX * kRowsBY, (rows_min_waves<Chain, V, ROWS>())) void k_rows(const typename Chain::Params p, const TileGeom g) {
+__global__ __launch_bounds__(kRowsBX * kRowsBY) void k_rows(const typename Chain::Params p, const TileGeom g) {
     if constexpr (rows_by_points<Chain, V, ROWS>()) points_body<Chain, V, FORM>(p, g);
     else rows_body<Chain, V, ROWS, ALIGNED, rows_in_bands<Chain>(), FORM>(p, 0u, &g);
 }
@@ -1256,7 +1248,7 @@ template <class Chain> struct RowsConfig {
     static constexpr int V = kScattered ? FKD_SCATTER_V : 4;
     // Two rows per thread; chains long enough to be bound by instruction issue rather than by memory (more than 128
     // bytes of operation parameters) take four, for the independent work per thread.
-    static constexpr bool kManyOps = many_ops<Chain>();
+    static constexpr bool kManyOps = sizeof(typename Chain::Params) - sizeof(typename Chain::Read::Params) - sizeof(typename Chain::Write::Params) > 128 + 16;
 #ifndef FKD_ROWS_MANY
 #define FKD_ROWS_MANY (2 * FKD_ROWS)
 #endif
