@@ -179,9 +179,8 @@ template <class Chain> constexpr bool rows_in_bands() {
 // plane's blocks (row-major), so that neighbouring blocks, whose taps share source lines, share an L2.  With the
 // workgroups in plain row-major order a warp fetched its source 2.5 to 3.2 times, once into nearly every L2; in bands it
 // is fetched once (rocprofv3 FETCH_SIZE), and a 3840 x 2160 warp takes 25.1 instead of 30.8 us.  Launches of fewer than
-// kRowsBandBlocks blocks per plane keep the two-dimensional grid: their source comes out of the last-level cache either
-// way, and the 1080p warp measured 5 % slower in bands (9.27 against 8.83 us).  (rows_band_chunk and kRowsBandBlocks:
-// fkd/launch_info.hpp.)
+// kRowsBandBlocks blocks per plane keep the two-dimensional grid; those of warps by columns are renumbered into bands inside it
+// (rows_bands_2d).  (rows_band_chunk and kRowsBandBlocks: fkd/launch_info.hpp.)
 
 // `kernarg_offset`: where p sits inside the kernel-argument segment (0 when the chain's parameter block is the
 // kernel's first argument); long chains fetch their operations' parameters from there.  BANDS: the launch has the bands
@@ -310,7 +309,7 @@ template <int N, class PlaneOp> struct ReadRoot<BatchRead<N, PlaneOp>> { using O
 // line that two waves share, and the kernel has no rows to work out.  A wave takes ROWS segments one after the other.  Bound by the memory
 // (100 uchar3 images of 1527x794: 119 us for 728 MB) or, below 20 MB, by the launch and one trip to the memory.  us, rows / so:
 // 4 uchar3 images of 1279x719 6.1 / 4.5, 100 of 103x243 7.9 / 4.0, of 439x918 55 / 41, of 1920x1080 208 / 204; floats 4 times 1861x714 through
-// 30 operations 16.5 / 13.4, 4 of 317x63 through 100 20.6 / 11.9, 3840x2160 through 50 14.0 / 12.6.  Nothing measured got slower.
+// 30 operations 16.5 / 13.4, 4 of 317x63 through 100 20.6 / 11.9, 3840x2160 through 50 14.0 / 12.6.  Of 70 drawn sizes one got 1 % slower.
 // The arguments that every wave needs are requested together and waited for once, and what is left of an address after the wave's own
 // part is a lane's small offset.
 template <class Chain> constexpr bool rows_flat() { return flat_capable<typename Chain::Read, typename Chain::Write>(); }
@@ -1182,7 +1181,7 @@ __device__ __forceinline__ void strip_body(const typename Chain::Params& p, cons
             WP::template put_masked<STREAM>(oplane, 0u, off, res);
         };
         // One step of taps is in flight behind the step being blended.  The steps are written out (a plane has at most
-        // kStripMaxSteps of them) and the only branches leave the kernel: every step issues the same accesses in the same
+        // kStripMaxSteps of them) and the only branches leave them (for good, or with LINES for finish, which stores what is left): every step issues the same accesses in the same
         // order, so the compiler's wait for a step's taps leaves all later accesses in flight, table reads carry their step
         // in the instruction's immediate offset, and there is no loop bookkeeping.  The request behind the last step meets
         // a column without a window.
@@ -1372,6 +1371,8 @@ template <class Chain, int WHICH> __device__ __forceinline__ void jit_other_body
     } else if constexpr (is_gather_chain<Chain>()) {
         if constexpr (WHICH < 3) gather_body<Chain, WHICH, 1, false>(p, g);
         else if constexpr (WHICH == 3 && strip_capable<Chain>()) {
+            // (two column tables in LDS, 22.5 KB, where the kernels compiled ahead of time have one; with one for both, one image to 331x12001
+            // took 13.1 us as before, to 639x4003 8.35 as before, and to 255x12001 10.4 instead of 9.9)
             if ((g.n_tiles & kStreamFlag) != 0u) strip_lines_body<Chain, true, 64>(p);
             else strip_lines_body<Chain, false, 64>(p);
         }

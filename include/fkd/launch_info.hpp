@@ -125,7 +125,9 @@ inline constexpr bool rows_halved(unsigned long long blocks, unsigned few, bool 
 // 3.23 / 2.41 / 2.09, to 320x180 (69) 2.58 / 2.05 / 1.94, to 400x300 (152) 3.23 / 2.61 / 2.69, to 1100x700 (792) 5.32 / 4.71 / 5.38, to 1333x800 (1100)
 // 6.2 / 5.1 / 6.3, to 1600x900 (1469) 6.5 / 6.0 / 7.6, to 1920x1000 (1875) 7.6 / 6.7, to 2300x1300 (2934) 11.3 / 11.6; 5 thumbnails of 128x128 (80) 3.17 / 2.46 / 2.28, of 256x256 (320) 3.41 / 2.98 / 3.17; 8 crops
 // to 64x64 (64) 2.96 / 2.38 / 2.16, to 224x64 (128) 3.09 / 2.42 / 2.63, to 224x224 (448) 3.73 / 3.46 / 3.99, to 300x200 (600) 4.07 / 3.89 / 4.34, to 384x300 (912)
-// 4.60 / 4.42, to 320x320 (960) 4.56 / 4.77 / 5.59, 64 crops to 300x64 (1536) 5.9 / 6.3 / 8.0.  Reads that work on every tap (a colour conversion) are longer and cross later.
+// 4.60 / 4.42, to 320x320 (960) 4.56 / 4.77 / 5.59, 64 crops to 300x64 (1536) 5.9 / 6.3 / 8.0.  Reads with operations of their own under the resize cross later, cheap ones as well: uchar3 1920x1080
+// with a cast fused, 128x8 / 128x4, to 1333x800 5.4 / 5.3, to 1400x900 (1243) 5.5 / 5.1, to 1600x900 5.4 / 5.4, to 1800x1000 (1875) 6.6 / 6.4, to 1920x1080 (2025) 6.1 /
+// 5.7; cast, multiplication and addition 5.8 / 5.3, 6.0 / 5.5, 6.1 / 6.0, 7.4 / 7.0, 7.4 / 7.3.
 constexpr unsigned kGatherFewTiles = 128, kGatherSomeTiles = 920, kGatherSomeTilesFused = 2560;
 // A lane's pixels along x and a wave's rows: form 0 has the kernels' own (FKD_GATHER_XI, FKD_GATHER_YI), 1 and 2 are named by theirs.
 inline constexpr unsigned gather_form_xi(unsigned form, unsigned own) { return form != 0u ? form : own; }

@@ -2818,7 +2818,6 @@ template <int N, class PlaneOp> struct BatchRead {
         for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::dense(p.plane[z], w, 1u)) return false;
         return planes <= u32(N);
     }
-    static constexpr bool kPlanes = true;      // plane z is plane[z], a PlaneOp of its own
     FKD_HD static bool strip_ok(const Params& p, bool any_pitch, u32 planes) {
         if constexpr (requires { PlaneOp::strip_ok(p.plane[0], any_pitch); }) {
             for (u32 z = 0; z < planes && z < u32(N); ++z) if (!PlaneOp::strip_ok(p.plane[z], any_pitch)) return false;
