@@ -386,7 +386,7 @@ def main():
 TRAFFIC_C3_BYTES = 52065000
 TRAFFIC_C3_SOURCES = ("fusedkernellibrary_amd/csrc/fkd_kernels.hpp", "fusedkernellibrary_amd/csrc/fkd_launch.hpp",
                       "include/fkd/ops.hpp", "include/fkd/types.hpp", "include/fkd/launch_info.hpp")
-TRAFFIC_C3_SOURCES_SHA256 = "fced9da442eb5af5929d19c4edc8f595e47dfa292bbc8a98d1b26c62d7a2c0c2"
+TRAFFIC_C3_SOURCES_SHA256 = "96b79eaba81703cc4c3a8d196db2381ee570fee7326841772ba6fa395a80ceb1"
 
 
 def device_sources_sha256():
